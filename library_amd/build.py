@@ -112,7 +112,7 @@ def build_workloads():
 
 def build_oracle():
     targets = ["oracle"]
-    if os.path.isdir(os.environ.get("ASX_REFERENCE", "/root/reference")):
+    if os.path.isdir(os.path.join(os.environ.get("ASX_REFERENCE", "/root/reference"), "hygon")):
         targets.append("ref")  # only where the reference sources are mounted
     _run(["make", "-C", os.path.join(ROOT, "oracle"), "-j8", *targets])
 
