@@ -58,16 +58,16 @@ FlatLayout spmv_flat_layout(int32_t nnz, size_t sv, bool with_split)
     return L;
 }
 
-struct SpmmLayout {  // [raw xs | raw ys | xs | ys | carry_row | carry]
-    size_t raw_xs_off, raw_ys_off, xs_off, ys_off, crow_off, carry_off, bytes;
+struct SpmmLayout {  // [xs | ys | carry_row | carry]
+    size_t xs_off, ys_off, crow_off, carry_off, bytes;
 };
 SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv, bool with_split)
 {
     SpmmLayout L{};
-    const size_t ns = (size_t)spmm_segments(m, nnz);
+    const size_t ns = (size_t)spmm_segments(m, nnz, spmm_segment_items(m, nnz, ncols, sv));
     size_t off = 0;
     if (with_split) {
-        for (size_t *o : {&L.raw_xs_off, &L.raw_ys_off, &L.xs_off, &L.ys_off}) {
+        for (size_t *o : {&L.xs_off, &L.ys_off}) {
             *o = off;
             off = align_up(off + (ns + 1) * 4, kAlign);
         }
@@ -261,22 +261,18 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         if (ws_bytes < L.bytes) return ASX_STATUS_INVALID_SIZE;
         const int32_t *xs, *ys;
         if (plan) {
-            const size_t ns = (size_t)spmm_segments(m, nnz);
             xs = plan->d_meta;
-            ys = plan->d_meta + (ns + 1);
+            ys = plan->d_meta + (plan->nunits + 1);
         } else {
-            int st = launch_merge_path_search(row_ptr, m, nnz, kSpmmSegment, (int32_t *)(w + L.raw_xs_off),
-                                              (int32_t *)(w + L.raw_ys_off), s);
-            if (!st)
-                st = launch_spmm_snap_splits(m, nnz, row_ptr, (const int32_t *)(w + L.raw_xs_off),
-                                             (const int32_t *)(w + L.raw_ys_off), (int32_t *)(w + L.xs_off),
-                                             (int32_t *)(w + L.ys_off), s);
+            int st = launch_spmm_splits(m, nnz, spmm_segment_items(m, nnz, ncols, sizeof(T)), row_ptr, (int32_t *)(w + L.xs_off),
+                                        (int32_t *)(w + L.ys_off), nullptr, s);
             if (st) return st;
             xs = (const int32_t *)(w + L.xs_off);
             ys = (const int32_t *)(w + L.ys_off);
         }
         return launch_spmm_merge<T>(m, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
-                                    ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off), s);
+                                    ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
+                                    plan ? plan->carry_pass != 0 : true, s);
     }
     case ASX_SPMM_BLOCKED:
         // the blocks hold a copy of A's values and are built by asx_spmm_plan_create
@@ -447,16 +443,19 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             p->workspace_bytes = spmv_merge_layout(m, nnz, sv, false).bytes;
         }
     } else if (kernel == ASX_SPMM_MERGE) {
-        const size_t ns = (size_t)spmm_segments(m, nnz);
+        const int32_t items = spmm_segment_items(m, nnz, p->ncols, sv);
+        const size_t ns = (size_t)spmm_segments(m, nnz, items);
         p->nunits = (int32_t)ns;
         p->meta_bytes = 2 * (ns + 1) * 4;
-        int32_t *raw = nullptr;  // the merge-path points, then snapped to short-row ends
+        p->carry_pass = 1;
         st = status_of(hipMalloc((void **)&p->d_meta, p->meta_bytes));
-        if (!st) st = status_of(hipMalloc((void **)&raw, p->meta_bytes));
-        if (!st) st = launch_merge_path_search(d_row_ptr, m, nnz, kSpmmSegment, raw, raw + (ns + 1), s);
-        if (!st) st = launch_spmm_snap_splits(m, nnz, d_row_ptr, raw, raw + (ns + 1), p->d_meta, p->d_meta + (ns + 1), s);
+        // does any row stay cut?  (one int read back; creation syncs anyway)
+        int32_t *d_flag = reinterpret_cast<int32_t *>(p->d_counters + 40), h_flag = 1;
+        if (!st) st = launch_fill_i32(d_flag, 1, 0, s);
+        if (!st) st = launch_spmm_splits(m, nnz, items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
+        if (!st) st = status_of(hipMemcpyAsync(&h_flag, d_flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         if (!st) st = status_of(hipStreamSynchronize(s));
-        if (raw) (void)hipFree(raw);
+        if (!st) p->carry_pass = h_flag != 0;
         p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv, false).bytes;
     }
     if (!st) st = status_of(hipStreamSynchronize(s));

@@ -17,7 +17,7 @@ constexpr int kStreamTile = 1024;                          // stored elements pe
 constexpr int kFlatTile = 1024;                            // stored elements per flat tile
 constexpr int kLongRow = 8192;  // DEFAULT (with a plan) switches to the merge-path kernel above this row length
 // SpMM: merge items (rows + stored elements) per wave
-constexpr int kSpmmSegment = 128;
+constexpr int kSpmmSegmentSmall = 128, kSpmmSegmentMedium = 256, kSpmmSegmentLarge = 512;
 
 inline int status_of(hipError_t e)
 {
@@ -91,11 +91,12 @@ template <typename T>
 int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
-                      hipStream_t s);
+                      bool carry_pass, hipStream_t s);
 
-// merge-path split points of SpMM moved to the ends of the short rows they cut (out of place)
-int launch_spmm_snap_splits(int32_t m, int32_t nnz, const int32_t *row_ptr, const int32_t *xs, const int32_t *ys,
-                            int32_t *xs_out, int32_t *ys_out, hipStream_t s);
+// merge-path split points of SpMM, `items` apart, moved to the ends of the short rows they cut; *has_carry (may be null)
+// is set to 1 if a row stays cut
+int launch_spmm_splits(int32_t m, int32_t nnz, int32_t items, const int32_t *row_ptr, int32_t *xs, int32_t *ys,
+                       int32_t *has_carry, hipStream_t s);
 
 // ---- blocked (MFMA) SpMM (asx_blocked.hip) ----
 struct BlockedMatrix {
@@ -219,7 +220,18 @@ inline size_t window_scratch_bytes(const WindowMatrix *wm, size_t sv) { return w
 inline int32_t merge_tiles(int32_t m, int32_t nnz) { return (int32_t)ceil_div64((int64_t)m + nnz, kMergeTile); }
 inline int32_t flat_tiles(int32_t nnz) { int32_t t = (int32_t)ceil_div64(nnz, kFlatTile); return t < 1 ? 1 : t; }
 inline int32_t stream_blocks(int32_t nnz) { return (int32_t)ceil_div64(nnz, kStreamTile); }
-inline int32_t spmm_segments(int32_t m, int32_t nnz) { return (int32_t)ceil_div64((int64_t)m + nnz, kSpmmSegment); }
+// Merge items per wave of the SpMM merge kernel.  Longer segments leave fewer carries and keep the
+// lane groups of narrow N busy, shorter ones leave room for more waves (LDS) and spread small
+// matrices: 128 while 256 a wave would leave fewer than 16 waves per compute unit.  Where a row of B
+// takes 16 lanes or more of fp32 (at most four groups a wave, 8 bytes staged per element) 512 measured
+// 2 % ahead of 256 on 17 M items, elsewhere 256 is up to 16 % ahead (8 columns of fp64: 46.4 / 55.2 us).
+inline int32_t spmm_segment_items(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
+{
+    const int64_t items = (int64_t)m + nnz;
+    if (items < (int64_t)kSpmmSegmentMedium * 4096) return kSpmmSegmentSmall;
+    return sv == 4 && ncols > 32 && items >= (int64_t)kSpmmSegmentLarge * 4096 ? kSpmmSegmentLarge : kSpmmSegmentMedium;
+}
+inline int32_t spmm_segments(int32_t m, int32_t nnz, int32_t items) { return (int32_t)ceil_div64((int64_t)m + nnz, items); }
 
 }  // namespace asx
 

@@ -7,7 +7,7 @@
 // lane offset).
 //
 //   row   : one wave per (row, column tile).  Simple; long rows serialise.
-//   merge : one wave per kSpmmSegment consecutive items of the merge path over
+//   merge : one wave per segment of consecutive items of the merge path over
 //           (row ends, stored elements): bounded work per wave whatever the row lengths.
 //           Rows that end inside a segment are written by that segment, and so is a row
 //           that starts in it and ends in the next; of a longer row the part that runs past
@@ -117,172 +117,243 @@ int launch_spmm_row(int32_t m, int32_t ncols, T alpha, const int32_t *row_ptr, c
 }
 
 // ===========================================================================================
-// merge: one wave per kSpmmSegment merge items
+// merge: one wave per segment of merge items
 // ===========================================================================================
-// Boundary g of the merge path lies between segments g-1 and g, at row xs[g], element ys[g].
-// The row cut by a boundary is SHORT there if it starts inside segment g-1 and ends inside
-// segment g: then the boundary moves to the end of that row, so segment g-1 takes the whole row
-// (running up to kSpmmSegment items past its nominal end) and segment g starts after it.  Only
-// rows long enough to cover a whole segment are still cut and leave carries.
-__global__ __launch_bounds__(kBlock) void k_spmm_snap_splits(int32_t m, int32_t nseg,
-                                                             const int32_t *__restrict__ row_ptr,
-                                                             const int32_t *__restrict__ xs,
-                                                             const int32_t *__restrict__ ys,
-                                                             int32_t *__restrict__ xs_out,
-                                                             int32_t *__restrict__ ys_out)
+// Boundary g of the merge path lies between segments g-1 and g, at row x, element y (least row of
+// the diagonal g * items whose end is not behind it).  The row cut by a boundary is SHORT there if
+// it starts inside segment g-1 and ends inside segment g: then the boundary moves to the end of
+// that row, so segment g-1 takes the whole row (running up to `items` past its nominal end) and
+// segment g starts after it.  Only rows long enough to cover a whole segment are still cut and
+// leave carries.  A segment so holds at most 2 * items elements and items + 1 row ends.
+__device__ __forceinline__ void merge_point(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nnz, int64_t d,
+                                            int32_t &x, int32_t &y)
+{
+    const int64_t total = (int64_t)m + nnz;
+    d = d < 0 ? 0 : d > total ? total : d;
+    int32_t lo = (int32_t)(d > nnz ? d - nnz : 0), hi = (int32_t)(d < m ? d : m);
+    while (lo < hi) {
+        const int32_t p = lo + (hi - lo) / 2;
+        if ((int64_t)row_ptr[p + 1] < d - p)
+            lo = p + 1;
+        else
+            hi = p;
+    }
+    x = lo;
+    y = (int32_t)(d - lo);
+}
+
+// One thread per boundary searches it and its two neighbours (three independent chains of loads:
+// the latency of one) and applies the rule above; *has_carry (when wanted) is set if a row stays cut.
+__global__ __launch_bounds__(kBlock) void k_spmm_splits(int32_t m, int32_t nnz, int32_t items, int32_t nseg,
+                                                        const int32_t *__restrict__ row_ptr, int32_t *__restrict__ xs,
+                                                        int32_t *__restrict__ ys, int32_t *__restrict__ has_carry)
 {
     const int64_t g = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (g > nseg) return;
-    int32_t x = xs[g], y = ys[g];
+    int32_t x, y, xp, yp, xn, yn;
+    merge_point(row_ptr, m, nnz, (g - 1) * items, xp, yp);
+    merge_point(row_ptr, m, nnz, g * items, x, y);
+    merge_point(row_ptr, m, nnz, (g + 1) * items, xn, yn);
     if (g > 0 && g < nseg && x < m) {
         const int32_t b = row_ptr[x], e = row_ptr[x + 1];
-        if (b < y && b >= ys[g - 1] && e <= ys[g + 1] && x < xs[g + 1]) {
+        if (b < y && b >= yp && e <= yn && x < xn) {
             x += 1;
             y = e;
+        } else if (has_carry && b < y) {
+            *has_carry = 1;
         }
     }
-    xs_out[g] = x;
-    ys_out[g] = y;
+    xs[g] = x;
+    ys[g] = y;
 }
 
-int launch_spmm_snap_splits(int32_t m, int32_t nnz, const int32_t *row_ptr, const int32_t *xs, const int32_t *ys,
-                            int32_t *xs_out, int32_t *ys_out, hipStream_t s)
+int launch_spmm_splits(int32_t m, int32_t nnz, int32_t items, const int32_t *row_ptr, int32_t *xs, int32_t *ys,
+                       int32_t *has_carry, hipStream_t s)
 {
-    const int32_t nseg = spmm_segments(m, nnz);
-    hipLaunchKernelGGL(k_spmm_snap_splits, dim3((unsigned)ceil_div64((int64_t)nseg + 1, kBlock)), dim3(kBlock), 0, s, m,
-                       nseg, row_ptr, xs, ys, xs_out, ys_out);
+    const int32_t nseg = spmm_segments(m, nnz, items);
+    hipLaunchKernelGGL(k_spmm_splits, dim3((unsigned)ceil_div64((int64_t)nseg + 1, kBlock)), dim3(kBlock), 0, s, m, nnz,
+                       items, nseg, row_ptr, xs, ys, has_carry);
     return check_launch();
 }
 
-// A segment's stored elements and row ends, staged in LDS by the wave that owns the segment.
-// After snapping a segment holds at most 2 * kSpmmSegment elements and kSpmmSegment + 1 row ends.
-constexpr int kSegElems = 2 * kSpmmSegment;
-constexpr int kSegRows = kSpmmSegment + kWave;
+// VEC consecutive columns of a lane, loaded and stored as one access that needs no more alignment
+// than an element has (ldb and ldc may be anything)
+template <typename T, int VEC>
+struct VecOf {
+    typedef T type __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
+};
 
-// acc += sum over staged elements [i0, i1) (positions relative to the segment start): a * B[col, c].
-// The LDS reads are broadcasts (every lane reads the same address).
-template <typename T>
-__device__ __forceinline__ T spmm_accumulate_staged(T acc, int32_t i0, int32_t i1, bool col_ok, int64_t c,
-                                                    const int32_t *s_col, const T *s_val,
-                                                    const T *__restrict__ B, int64_t ldb)
+template <int N>
+struct Int {
+    static constexpr int value = N;
+};
+
+// Sum over staged elements i0, i0 + ST, ... below e: a * B[col, lane's columns].  Bc: B plus the lane's
+// first column.  Batches of U, then at most one of U / 2, then one of U / 2 that is not full.
+template <typename T, int VEC, int ST, int U, bool UNIFORM>
+__device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, int32_t e, const int32_t *s_col,
+                                                                    const T *s_val, const char *Bc, uint64_t ldb_bytes)
 {
+    typedef typename VecOf<T, VEC>::type V;
+    V acc = T(0);
     int32_t i = i0;
-    for (; i + kSpmmInFlight <= i1; i += kSpmmInFlight) {
-        int32_t cc[kSpmmInFlight];
-        T a[kSpmmInFlight], b[kSpmmInFlight];
+    const auto batch = [&](auto n_, auto partial_) {  // n elements; partial: those from e on repeat the first
+        constexpr int N = decltype(n_)::value;
+        constexpr bool PARTIAL = decltype(partial_)::value;
+        V b[N];
+        T a[N];
 #pragma unroll
-        for (int u = 0; u < kSpmmInFlight; ++u) {
-            cc[u] = __builtin_amdgcn_readfirstlane(s_col[i + u]);
-            a[u] = s_val[i + u];
-        }
-#pragma unroll
-        for (int u = 0; u < kSpmmInFlight; ++u) b[u] = col_ok ? B[(int64_t)cc[u] * ldb + c] : T(0);
-#pragma unroll
-        for (int u = 0; u < kSpmmInFlight; ++u) acc = fma_t<T>(a[u], b[u], acc);
-    }
-    if (i < i1) {  // the last, partial batch: all its loads are issued before the first use
-        int32_t cc[kSpmmInFlight];
-        T a[kSpmmInFlight], b[kSpmmInFlight];
-#pragma unroll
-        for (int u = 0; u < kSpmmInFlight; ++u) {
-            const int32_t iu = i + u < i1 ? i + u : i1 - 1;
-            cc[u] = __builtin_amdgcn_readfirstlane(s_col[iu]);
+        for (int u = 0; u < N; ++u) {
+            const int32_t iu = !PARTIAL || i + u * ST < e ? i + u * ST : i;
+            uint32_t c = (uint32_t)s_col[iu];
+            if (UNIFORM) c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
+            b[u] = *(const V *)(Bc + c * ldb_bytes);
             a[u] = s_val[iu];
         }
 #pragma unroll
-        for (int u = 0; u < kSpmmInFlight; ++u) b[u] = (col_ok && i + u < i1) ? B[(int64_t)cc[u] * ldb + c] : T(0);
-#pragma unroll
-        for (int u = 0; u < kSpmmInFlight; ++u)
-            if (i + u < i1) acc = fma_t<T>(a[u], b[u], acc);
-    }
+        for (int u = 0; u < N; ++u) {
+            const V sum = __builtin_elementwise_fma((V)a[u], b[u], acc);
+            acc = !PARTIAL || i + u * ST < e ? sum : acc;
+        }
+        i += N * ST;
+    };
+    while (i + (U - 1) * ST < e) batch(Int<U>{}, Int<0>{});
+    if (i + (U / 2 - 1) * ST < e) batch(Int<U / 2>{}, Int<0>{});
+    if (i < e) batch(Int<U / 2>{}, Int<1>{});
     return acc;
 }
 
-// xs, ys: the snapped split points.  The wave first stages the segment's column indices, values
-// and row ends in LDS (one round trip for all of them), so that the loads of B of one row after
-// the other follow without waiting on row offsets or stored elements in between; the old value
-// of a row of C (beta != 0) is requested before the row's loads of B.
-template <typename T>
-__global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, int32_t nseg,
-                                                       int32_t ncols, T alpha,
+// One wave per segment and tile of columns.  A lane holds VEC columns (16 bytes where N allows), so
+// G = 2^LOGG lanes span a tile and the wave's NG = 64 / G groups work on different stored elements at
+// once: one load instruction fetches NG rows of B.  (A row of B per instruction, 4 bytes per lane,
+// gets 110 G lines/s from an L2, 16 bytes per lane 240 G; with 8 columns in fp64 such a kernel left 56
+// lanes of 64 idle.)
+//   * the segment's columns, values and row ends are staged in LDS in one round trip;
+//   * rows of up to kDealt elements are dealt to the groups, one row each;
+//   * longer rows, and the row that goes on past the segment end, are taken by all groups together,
+//     element by element in turn, and joined by a butterfly over the groups.
+// A lane past the last column of the tile repeats the last VEC columns and stores nothing; a tile
+// whose width is no multiple of VEC has its last lane overlap the one before it (both compute the same
+// bits from the same old values of C, in one wave).
+// Consecutive segments run on one XCD, whose L2 then fetches the rows of B that neighbouring rows
+// of A share once.
+template <typename T, int VEC, int LOGG, int SEG>
+__global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t nseg, int32_t ncols, T alpha,
                                                        const int32_t *__restrict__ row_ptr,
-                                                       const int32_t *__restrict__ col,
-                                                       const T *__restrict__ val,
+                                                       const int32_t *__restrict__ col, const T *__restrict__ val,
                                                        const T *__restrict__ B, int64_t ldb, T beta,
                                                        T *__restrict__ C, int64_t ldc,
-                                                       const int32_t *__restrict__ xs,
-                                                       const int32_t *__restrict__ ys,
-                                                       T *__restrict__ carry,
-                                                       int32_t *__restrict__ carry_row)
+                                                       const int32_t *__restrict__ xs, const int32_t *__restrict__ ys,
+                                                       T *__restrict__ carry, int32_t *__restrict__ carry_row)
 {
-    __shared__ int32_t s_col_all[kBlock / kWave][kSegElems];
-    __shared__ T s_val_all[kBlock / kWave][kSegElems];
-    __shared__ int32_t s_end_all[kBlock / kWave][kSegRows];
+    typedef typename VecOf<T, VEC>::type V;
+    constexpr int G = 1 << LOGG, NG = kWave / G;
+    constexpr int U = 8;  // rows of B a lane has in flight
+    constexpr int kDealt = NG == 1 ? 1 << 30 : NG <= 4 ? 16 : NG <= 8 ? 32 : 64;
+    constexpr int kElems = 2 * SEG, kEnds = SEG + kWave;
+    __shared__ int32_t s_col_all[kBlock / kWave][kElems];
+    __shared__ T s_val_all[kBlock / kWave][kElems];
+    __shared__ int32_t s_end_all[kBlock / kWave][kEnds + 1];
     const int lane = threadIdx.x & (kWave - 1);
-    const int w = threadIdx.x / kWave;
-    const int64_t seg = (int64_t)blockIdx.x * (kBlock / kWave) + w;
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t per_xcd = gridDim.x / kXcds;
+    const int64_t blk = (int64_t)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    const int64_t seg = blk * (kBlock / kWave) + w;
     if (seg >= nseg) return;  // wave-uniform
-    const int64_t c = (int64_t)blockIdx.y * kWave + lane;
-    const bool col_ok = c < ncols;
-    const int32_t x0 = __builtin_amdgcn_readfirstlane(xs[seg]);
-    const int32_t y0 = __builtin_amdgcn_readfirstlane(ys[seg]);
-    const int32_t x1 = __builtin_amdgcn_readfirstlane(xs[seg + 1]);
-    const int32_t y1 = __builtin_amdgcn_readfirstlane(ys[seg + 1]);
-    const int32_t nel = y1 - y0, nrow = x1 - x0;
-
-    if (nel <= kSegElems && nrow <= kSegRows) {
-        int32_t *s_col = s_col_all[w];
-        T *s_val = s_val_all[w];
-        int32_t *s_end = s_end_all[w];
+    const int grp = lane >> LOGG, gl = lane & (G - 1);
+    const int64_t t0 = (int64_t)blockIdx.y * ncols / gridDim.y, t1 = (int64_t)(blockIdx.y + 1) * ncols / gridDim.y;
+    int64_t c = t0 + gl * VEC;
+    const bool active = c < t1;
+    c = c < t1 - VEC ? c : t1 - VEC;
+    const char *Bc = (const char *)(B + c);
+    const uint64_t ldb_bytes = (uint64_t)ldb * sizeof(T);
+    const int32_t x0 = xs[seg], y0 = ys[seg], x1 = xs[seg + 1], y1 = ys[seg + 1];
+    const int32_t nel = y1 - y0 < kElems ? y1 - y0 : kElems, nrow = x1 - x0 < kEnds ? x1 - x0 : kEnds;
+    int32_t *s_col = s_col_all[w];
+    T *s_val = s_val_all[w];
+    int32_t *s_end = s_end_all[w];  // s_end[r + 1]: end of row x0 + r, relative to y0
+    // What most segments hold - up to SEG elements and 128 rows - is requested at once, past-the-end
+    // lanes repeating the last entry; the rest follows only where there is more.
+    const auto stage = [&](auto from_, auto to_, auto rows_from_, auto rows_to_) {
+        constexpr int E0 = decltype(from_)::value, E1 = decltype(to_)::value, R0 = decltype(rows_from_)::value,
+                      R1 = decltype(rows_to_)::value;
+        constexpr int NE = (E1 - E0) / kWave, NR = (R1 - R0) / kWave;
+        int32_t tc[NE > 0 ? NE : 1], te[NR > 0 ? NR : 1];
+        T tv[NE > 0 ? NE : 1];
 #pragma unroll
-        for (int i = lane; i < kSegElems; i += kWave) {
-            if (i < nel) {
-                s_col[i] = col[y0 + i];
-                s_val[i] = val[y0 + i];
+        for (int j = 0; j < NR; ++j) {
+            const int i = R0 + j * kWave + lane;
+            te[j] = row_ptr[x0 + (i < nrow ? i + 1 : nrow)];
+        }
+#pragma unroll
+        for (int j = 0; j < NE; ++j) {
+            const int i = E0 + j * kWave + lane;
+            const int64_t k = (int64_t)y0 + (i < nel ? i : nel - 1);
+            tc[j] = col[k];
+            tv[j] = val[k];
+        }
+#pragma unroll
+        for (int j = 0; j < NR; ++j) s_end[1 + R0 + j * kWave + lane] = te[j] - y0;
+#pragma unroll
+        for (int j = 0; j < NE; ++j) {
+            s_col[E0 + j * kWave + lane] = tc[j];
+            s_val[E0 + j * kWave + lane] = tv[j];
+        }
+    };
+    if (nel > 0)
+        stage(Int<0>{}, Int<SEG>{}, Int<0>{}, Int<128>{});
+    else
+        stage(Int<0>{}, Int<0>{}, Int<0>{}, Int<128>{});
+    if (nel > SEG) stage(Int<SEG>{}, Int<kElems>{}, Int<0>{}, Int<0>{});
+    if (nrow > 128) stage(Int<0>{}, Int<0>{}, Int<128>{}, Int<kEnds>{});
+    if (lane == 0) s_end[0] = 0;
+    // the staged data is private to this wave: order its LDS writes before its LDS reads
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+
+    const auto together = [&](int32_t k, int32_t e) {  // the row's sum over all groups, in every group
+        V acc = spmm_staged<T, VEC, NG, U, NG == 1>(k + grp, e, s_col, s_val, Bc, ldb_bytes);
+#pragma unroll
+        for (int d = G; d < kWave; d <<= 1)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) acc[v] += __shfl_xor(acc[v], d, kWave);
+        return acc;
+    };
+    const bool stores = active && grp == 0;
+    for (int32_t r0 = 0; r0 < nrow; r0 += NG) {
+        const int32_t r = r0 + grp;
+        const int32_t k = r < nrow ? s_end[r] : 0, e = r < nrow ? s_end[r + 1] : 0;
+        const bool dealt = e - k <= kDealt;
+        if (r < nrow && dealt) {
+            V *out = (V *)(C + (int64_t)(x0 + r) * ldc + c);
+            V c_old = T(0);
+            if (beta != T(0)) c_old = *out;  // requested before the row's loads of B
+            const V acc = spmm_staged<T, VEC, 1, U, NG == 1>(k, e, s_col, s_val, Bc, ldb_bytes);
+            const V y = beta == T(0) ? (V)(alpha * acc) : __builtin_elementwise_fma((V)alpha, acc, (V)(beta * c_old));
+            if (active) *out = y;
+        }
+        if (NG > 1) {
+            unsigned long long todo = __ballot(!dealt && gl == 0);
+            while (todo) {  // wave-uniform
+                const int src = __builtin_ctzll(todo);
+                todo &= todo - 1;
+                const int32_t rr = r0 + (src >> LOGG);
+                const int32_t kk = __builtin_amdgcn_readlane(k, src), ee = __builtin_amdgcn_readlane(e, src);
+                V *out = (V *)(C + (int64_t)(x0 + rr) * ldc + c);
+                V c_old = T(0);
+                if (beta != T(0) && stores) c_old = *out;
+                const V acc = together(kk, ee);
+                const V y = beta == T(0) ? (V)(alpha * acc) : __builtin_elementwise_fma((V)alpha, acc, (V)(beta * c_old));
+                if (stores) *out = y;
             }
         }
-#pragma unroll
-        for (int i = lane; i < kSegRows; i += kWave)
-            if (i < nrow) s_end[i] = row_ptr[x0 + 1 + i] - y0;
-        // the staged data is private to this wave: order its LDS writes before its LDS reads
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        int32_t k = 0;
-        for (int32_t r = 0; r < nrow; ++r) {  // rows this segment finishes
-            const int32_t e = __builtin_amdgcn_readfirstlane(s_end[r]);
-            const int64_t idx = (int64_t)(x0 + r) * ldc + c;
-            const T c_old = (beta != T(0) && col_ok) ? C[idx] : T(0);
-            const T acc = spmm_accumulate_staged<T>(T(0), k, e, col_ok, c, s_col, s_val, B, ldb);
-            k = e;
-            if (col_ok) C[idx] = beta == T(0) ? alpha * acc : fma_t<T>(alpha, acc, beta * c_old);
-        }
-        const bool has_tail = nel > k;  // row x1 continues past the segment end
-        if (has_tail) {
-            const T acc = spmm_accumulate_staged<T>(T(0), k, nel, col_ok, c, s_col, s_val, B, ldb);
-            if (col_ok) carry[seg * ncols + c] = acc;
-        }
-        if (lane == 0 && blockIdx.y == 0) carry_row[seg] = has_tail ? x1 : -1;
-        return;
     }
-
-    // a segment too large to stage (cannot happen with snapped merge-path points; kept for safety)
-    int32_t k = y0;
-    T acc = T(0);
-    for (int32_t row = x0; row < x1; ++row) {
-        const int32_t e = __builtin_amdgcn_readfirstlane(row_ptr[row + 1]);
-        acc = spmm_accumulate<T>(acc, k, e, lane, col_ok, c, col, val, B, ldb);
-        k = e;
-        if (col_ok) {
-            const int64_t idx = (int64_t)row * ldc + c;
-            C[idx] = scaled_out<T>(alpha, acc, beta, C, idx);
-        }
-        acc = T(0);
-    }
-    const bool has_tail = y1 > k;
+    const int32_t k = __builtin_amdgcn_readfirstlane(s_end[nrow]);
+    const bool has_tail = nel > k;  // row x1 continues past the segment end
     if (has_tail) {
-        acc = spmm_accumulate<T>(T(0), k, y1, lane, col_ok, c, col, val, B, ldb);
-        if (col_ok) carry[seg * ncols + c] = acc;
+        const V acc = together(k, nel);
+        if (stores) *(V *)(carry + seg * ncols + c) = acc;
     }
     if (lane == 0 && blockIdx.y == 0) carry_row[seg] = has_tail ? x1 : -1;
 }
@@ -352,20 +423,68 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge_fixup(int32_t m, int32_t 
     }
 }
 
+// Lanes per row of B: the smallest power of two that spans the tile at VEC columns each; N beyond 64
+// lanes' worth is cut into equal tiles (every tile at least VEC wide).
+template <typename T, int VEC, int SEG>
+static void launch_merge_width(int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
+                               const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
+                               T *carry, int32_t *carry_row, hipStream_t s)
+{
+    const int64_t tiles = ceil_div64(ncols, kWave * VEC), lanes = ceil_div64(ceil_div64(ncols, tiles), VEC);
+    const dim3 grid((unsigned)(ceil_div64(ceil_div64(nseg, kBlock / kWave), kXcds) * kXcds), (unsigned)tiles);
+#define ASX_WIDTH(LOGG)                                                                                              \
+    if (lanes <= (1 << LOGG)) {                                                                                      \
+        hipLaunchKernelGGL((k_spmm_merge<T, VEC, LOGG, SEG>), grid, dim3(kBlock), 0, s, nseg, ncols, alpha, row_ptr, col, \
+                           val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);                                     \
+        return;                                                                                                      \
+    }
+    ASX_WIDTH(0)
+    ASX_WIDTH(1)
+    if constexpr (VEC * sizeof(T) == 16) {  // fewer columns per lane only where N is smaller than 16 bytes
+        ASX_WIDTH(2)
+        ASX_WIDTH(3)
+        ASX_WIDTH(4)
+        ASX_WIDTH(5)
+        ASX_WIDTH(6)
+    }
+#undef ASX_WIDTH
+}
+
+template <typename T, int SEG>
+static void launch_merge_seg(int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
+                             const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
+                             T *carry, int32_t *carry_row, hipStream_t s)
+{
+    constexpr int kFull = 16 / sizeof(T);
+    if (ncols >= kFull)
+        launch_merge_width<T, kFull, SEG>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+    else if (ncols >= 2)
+        launch_merge_width<T, 2, SEG>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+    else
+        launch_merge_width<T, 1, SEG>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+}
+
 template <typename T>
 int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
-                      hipStream_t s)
+                      bool carry_pass, hipStream_t s)
 {
     if (m <= 0 || ncols <= 0) return ASX_STATUS_SUCCESS;
-    const int32_t nseg = spmm_segments(m, nnz);
-    dim3 grid((unsigned)ceil_div64(nseg, kBlock / kWave), (unsigned)ceil_div64(ncols, kWave));
-    hipLaunchKernelGGL((k_spmm_merge<T>), grid, dim3(kBlock), 0, s, m, nnz, nseg, ncols, alpha, row_ptr,
-                       col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);
-    hipLaunchKernelGGL((k_spmm_merge_fixup<T>), dim3((unsigned)ceil_div64(ceil_div64(nseg, kFixupSegs), kBlock / kWave)),
-                       dim3(kBlock), 0, s, m,
-                       nseg, ncols, alpha, carry, carry_row, C, ldc);
+    const int32_t items = spmm_segment_items(m, nnz, ncols, sizeof(T)), nseg = spmm_segments(m, nnz, items);
+    const auto launch = [&](auto seg_) {
+        launch_merge_seg<T, decltype(seg_)::value>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
+                                                   carry_row, s);
+    };
+    if (items == kSpmmSegmentSmall)
+        launch(Int<kSpmmSegmentSmall>{});
+    else if (items == kSpmmSegmentMedium)
+        launch(Int<kSpmmSegmentMedium>{});
+    else if constexpr (sizeof(T) == 4)
+        launch(Int<kSpmmSegmentLarge>{});
+    if (carry_pass)
+        hipLaunchKernelGGL((k_spmm_merge_fixup<T>), dim3((unsigned)ceil_div64(ceil_div64(nseg, kFixupSegs), kBlock / kWave)),
+                           dim3(kBlock), 0, s, m, nseg, ncols, alpha, carry, carry_row, C, ldc);
     return check_launch();
 }
 
@@ -374,7 +493,7 @@ int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int3
                                     const T *, int64_t, T, T *, int64_t, hipStream_t);               \
     template int launch_spmm_merge<T>(int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
                                       const T *, const T *, int64_t, T, T *, int64_t, const int32_t *, \
-                                      const int32_t *, T *, int32_t *, hipStream_t);
+                                      const int32_t *, T *, int32_t *, bool, hipStream_t);
 ASX_INST(float)
 ASX_INST(double)
 #undef ASX_INST
