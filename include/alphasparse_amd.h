@@ -78,6 +78,13 @@ const char *asx_version(void);
  * Stands in for the device query in alphasparseGetHandle, hip/util/handle.hip:67-83. */
 int asx_device_info(int *compute_units, int *wavefront_size);
 
+/* The library keeps device memory that plans and conversions have given back (per device at most 1 GiB,
+ * blocks of at most 512 MiB) and uses it for the next ones: allocating and freeing it anew took longer
+ * than their kernels.  This frees what is kept on the current device; so does an allocation of the
+ * library that fails at first, and destroying a handle of the generic API.  No counterpart in the
+ * reference. */
+int asx_release_cached_memory(void);
+
 /* ------------------------------------------------------------------------------------
  * CSR analysis: integer outputs, bit-identical to the reference functions cited.
  * ---------------------------------------------------------------------------------- */

@@ -17,7 +17,7 @@ WORKLOADS = os.path.join(HERE, "libasx_workloads.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
 HIP_SOURCES = ["asx_analysis.hip", "asx_spmv.hip", "asx_spmm.hip", "asx_capi.hip", "asx_blocked.hip", "asx_coo.hip", "asx_convert.hip", "asx_sliced.hip", "asx_window.hip"]
-CXX_SOURCES = ["asx_rowblocks.cpp", "alphasparse_generic.cpp", "asx_mtx.cpp"]
+CXX_SOURCES = ["asx_pool.cpp", "asx_rowblocks.cpp", "alphasparse_generic.cpp", "asx_mtx.cpp"]
 
 # packed-fp32 code generation is switched off for all device code
 HIP_FLAGS = ["--offload-arch=gfx950", "-std=c++17", "-O3", "-fPIC", "-Wall", "-Wno-unused-function",

@@ -23,7 +23,7 @@ STATUS = {0: "SUCCESS", 1: "NOT_INITIALIZED", 2: "ALLOC_FAILED", 3: "INVALID_VAL
 
 # every symbol include/alphasparse_amd.h (and, last, include/alphasparse_amd_bench.h) declares
 EXPORTS = [
-    "asx_version", "asx_device_info", "asx_row_length_histogram", "asx_partition_rows_by_nnz",
+    "asx_version", "asx_device_info", "asx_release_cached_memory", "asx_row_length_histogram", "asx_partition_rows_by_nnz",
     "asx_nnz_split_rows", "asx_merge_path_search", "asx_loadbalance_nwarps",
     "asx_loadbalance_partition", "asx_csr_adaptive_row_blocks", "asx_coo2csr", "asx_coo_sort", "asx_csr_transpose", "asx_csr_rebase",
     "asx_dense_transpose", "asx_mtx_read", "asx_host_free", "asx_spmv_plan_create",

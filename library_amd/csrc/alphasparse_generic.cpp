@@ -26,6 +26,7 @@
 #include <vector>
 
 #include "../../include/alphasparse.h"
+#include "asx_pool.hpp"
 
 // Layout checks.  The numbers are those of the reference's own headers compiled with the same
 // ROCm headers (tests/golden/layout.json, written by tests/golden/make_layout.py).
@@ -291,9 +292,10 @@ const asx_plan *kept_plan(const _alphasparseSpMatDescr *A, alphasparseOperation_
 
 void free_derived(DerivedCsr &d)
 {
-    if (d.row_ptr) (void)hipFree(d.row_ptr);
-    if (d.col) (void)hipFree(d.col);
-    if (d.transposed && d.val) (void)hipFree(d.val);
+    asx::pool_wait(d.row_ptr);  // calls that read the copy may still be running on any stream
+    asx::pool_free(d.row_ptr);
+    asx::pool_free(d.col);
+    if (d.transposed) asx::pool_free(d.val);
     d.row_ptr = d.col = nullptr;
     d.val = nullptr;
 }
@@ -322,9 +324,9 @@ alphasparseStatus_t build_derived(alphasparseHandle_t h, const _alphasparseSpMat
     const size_t sv = A->data_type == ALPHA_R_64F ? 8 : 4;
     const size_t nrow = (size_t)(transposed ? A->cols : A->rows) + 1;
     const size_t nnz1 = A->nnz > 0 ? (size_t)A->nnz : 1;
-    hipError_t e = hipMalloc((void **)&d.row_ptr, nrow * sizeof(int));
-    if (e == hipSuccess) e = hipMalloc((void **)&d.col, nnz1 * sizeof(int));
-    if (e == hipSuccess && transposed) e = hipMalloc(&d.val, nnz1 * sv);
+    hipError_t e = asx::pool_malloc(&d.row_ptr, nrow * sizeof(int), false);
+    if (e == hipSuccess) e = asx::pool_malloc(&d.col, nnz1 * sizeof(int), false);
+    if (e == hipSuccess && transposed) e = asx::pool_malloc_bytes(&d.val, nnz1 * sv, false);
     if (e != hipSuccess) {
         free_derived(d);
         return from_hip(e);
@@ -597,6 +599,7 @@ alphasparseStatus_t alphasparse_destory_handle(alphasparseHandle_t handle)
         delete reg;
     }
     handle->pflat_analysis_data = nullptr;
+    asx::pool_release();  // memory kept for later analyses
     if (handle->buffer) (void)hipFree(handle->buffer);
     if (handle->sone) (void)hipFree(handle->sone);
     if (handle->done) (void)hipFree(handle->done);

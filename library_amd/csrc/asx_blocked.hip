@@ -148,16 +148,16 @@ int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, con
     out->nnz = nnz;
     const unsigned g_nnz = (unsigned)ceil_div64(nnz > 0 ? nnz : 1, kBlock);
     if (nnz > 0) {
-        ASX_TRY(hipMalloc((void **)&keys, sizeof(uint64_t) * (size_t)nnz));
-        ASX_TRY(hipMalloc((void **)&keys2, sizeof(uint64_t) * (size_t)nnz));
-        ASX_TRY(hipMalloc((void **)&idx, sizeof(int32_t) * (size_t)nnz));
-        ASX_TRY(hipMalloc((void **)&idx2, sizeof(int32_t) * (size_t)nnz));
-        ASX_TRY(hipMalloc((void **)&head, sizeof(int32_t) * (size_t)nnz));
-        ASX_TRY(hipMalloc((void **)&block_of, sizeof(int32_t) * (size_t)nnz));
+        ASX_TRY(pool_malloc(&keys, sizeof(uint64_t) * (size_t)nnz, true));
+        ASX_TRY(pool_malloc(&keys2, sizeof(uint64_t) * (size_t)nnz, true));
+        ASX_TRY(pool_malloc(&idx, sizeof(int32_t) * (size_t)nnz, true));
+        ASX_TRY(pool_malloc(&idx2, sizeof(int32_t) * (size_t)nnz, true));
+        ASX_TRY(pool_malloc(&head, sizeof(int32_t) * (size_t)nnz, true));
+        ASX_TRY(pool_malloc(&block_of, sizeof(int32_t) * (size_t)nnz, true));
         ASX_TRY(rocprim::radix_sort_pairs(nullptr, tmp_sort, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
         ASX_TRY(rocprim::inclusive_scan(nullptr, tmp_scan, head, block_of, (size_t)nnz, rocprim::plus<int32_t>(), s));
         tmp_bytes = tmp_sort > tmp_scan ? tmp_sort : tmp_scan;
-        ASX_TRY(hipMalloc(&tmp, tmp_bytes ? tmp_bytes : 1));
+        ASX_TRY(pool_malloc(&tmp, tmp_bytes, true));
         hipLaunchKernelGGL(k_block_keys, dim3(g_nnz), dim3(kBlock), 0, s, row_ptr, col, m, nnz, keys, idx);
         ASX_TRY(rocprim::radix_sort_pairs(tmp, tmp_sort, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
         hipLaunchKernelGGL(k_block_heads, dim3(g_nnz), dim3(kBlock), 0, s, keys2, nnz, head);
@@ -166,13 +166,13 @@ int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, con
         ASX_TRY(hipStreamSynchronize(s));
     }
     out->nblocks = nblocks;
-    ASX_TRY(hipMalloc((void **)&out->brow_ptr, sizeof(int32_t) * ((size_t)nbrows + 1)));
-    ASX_TRY(hipMalloc((void **)&out->bcol, sizeof(int32_t) * (size_t)(nblocks > 0 ? nblocks : 1)));
-    ASX_TRY(hipMalloc((void **)&out->bval, sizeof(T) * 64 * (size_t)(nblocks > 0 ? nblocks : 1)));
-    ASX_TRY(hipMalloc((void **)&bkey, sizeof(uint64_t) * (size_t)(nblocks > 0 ? nblocks : 1)));
+    ASX_TRY(pool_malloc(&out->brow_ptr, sizeof(int32_t) * ((size_t)nbrows + 1), false));
+    ASX_TRY(pool_malloc(&out->bcol, sizeof(int32_t) * (size_t)(nblocks > 0 ? nblocks : 1), false));
+    ASX_TRY(pool_malloc(&out->bval, sizeof(T) * 64 * (size_t)(nblocks > 0 ? nblocks : 1), false));
+    ASX_TRY(pool_malloc(&bkey, sizeof(uint64_t) * (size_t)(nblocks > 0 ? nblocks : 1), true));
     if (nblocks > 0) {
-        ASX_TRY(hipMalloc((void **)&out->upd_src, sizeof(int32_t) * (size_t)nnz));
-        ASX_TRY(hipMalloc((void **)&out->upd_dst, sizeof(int64_t) * (size_t)nnz));
+        ASX_TRY(pool_malloc(&out->upd_src, sizeof(int32_t) * (size_t)nnz, false));
+        ASX_TRY(pool_malloc(&out->upd_dst, sizeof(int64_t) * (size_t)nnz, false));
         hipLaunchKernelGGL((k_fill_zero<T>), dim3(4096), dim3(kBlock), 0, s, (T *)out->bval, (int64_t)nblocks * 64);
         hipLaunchKernelGGL(k_block_slots, dim3(g_nnz), dim3(kBlock), 0, s, keys2, idx2, block_of, nnz, bkey,
                            out->upd_src, out->upd_dst);
@@ -187,9 +187,10 @@ int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, con
     ASX_TRY(hipGetLastError());
     ASX_TRY(hipStreamSynchronize(s));
 done:
+    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
     for (void *p : {(void *)keys, (void *)keys2, (void *)idx, (void *)idx2, (void *)head, (void *)block_of, tmp,
                     (void *)bkey})
-        if (p) (void)hipFree(p);
+        pool_free(p);
     if (st) free_blocked(out);
     return st;
 }
@@ -197,11 +198,11 @@ done:
 
 void free_blocked(BlockedMatrix *b)
 {
-    if (b->brow_ptr) (void)hipFree(b->brow_ptr);
-    if (b->bcol) (void)hipFree(b->bcol);
-    if (b->bval) (void)hipFree(b->bval);
-    if (b->upd_src) (void)hipFree(b->upd_src);
-    if (b->upd_dst) (void)hipFree(b->upd_dst);
+    pool_free(b->brow_ptr);
+    pool_free(b->bcol);
+    pool_free(b->bval);
+    pool_free(b->upd_src);
+    pool_free(b->upd_dst);
     b->brow_ptr = nullptr;
     b->bcol = nullptr;
     b->bval = nullptr;

@@ -309,6 +309,12 @@ int asx_device_info(int *compute_units, int *wavefront_size)
     return ASX_STATUS_SUCCESS;
 }
 
+int asx_release_cached_memory(void)
+{
+    pool_release();
+    return ASX_STATUS_SUCCESS;
+}
+
 // ---------------------------------------------------------------- analysis
 int asx_row_length_histogram(const int32_t *d_row_ptr, int32_t m, int64_t *d_hist, int64_t *d_stats,
                              void *stream)
@@ -388,7 +394,7 @@ int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n
     p->nnz = nnz;
     p->ncols = is_spmm ? ncols_dense : 1;
     p->row_ptr = d_row_ptr;
-    int st = status_of(hipMalloc((void **)&p->d_counters, kPlanCounters * sizeof(int64_t)));
+    int st = status_of(pool_malloc(&p->d_counters, kPlanCounters * sizeof(int64_t), false));
     if (!st) st = launch_row_histogram(d_row_ptr, m, p->d_counters, p->d_counters + 33, s);
     if (!st) st = status_of(hipMemcpyAsync(p->hist, p->d_counters, 33 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
     if (!st) st = status_of(hipMemcpyAsync(p->stats, p->d_counters + 33, 4 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
@@ -416,13 +422,13 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             int32_t nb = std::max(stream_blocks(nnz), 1);
             p->nunits = nb;
             p->meta_bytes = ((size_t)nb + 1) * 8;
-            st = status_of(hipMalloc((void **)&p->d_meta, p->meta_bytes));
+            st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
             if (!st) st = launch_stream_row_blocks(d_row_ptr, m, nnz, p->d_meta, s);
         } else if (kernel == ASX_SPMV_FLAT) {
             const size_t nt = (size_t)flat_tiles(nnz);
             p->nunits = (int32_t)nt;
             p->meta_bytes = (nt + 1) * 4;
-            st = status_of(hipMalloc((void **)&p->d_meta, p->meta_bytes));
+            st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
             if (!st) st = launch_flat_seg_rows(d_row_ptr, m, nnz, p->d_meta, s);
             p->workspace_bytes = spmv_flat_layout(nnz, sv, false).bytes;
             p->carry_pass = 1;
@@ -438,7 +444,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             const size_t nt = (size_t)merge_tiles(m, nnz);
             p->nunits = (int32_t)nt;
             p->meta_bytes = 2 * (nt + 1) * 4;
-            st = status_of(hipMalloc((void **)&p->d_meta, p->meta_bytes));
+            st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
             if (!st) st = launch_merge_path_search(d_row_ptr, m, nnz, kMergeTile, p->d_meta, p->d_meta + (nt + 1), s);
             p->workspace_bytes = spmv_merge_layout(m, nnz, sv, false).bytes;
         }
@@ -448,7 +454,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         p->nunits = (int32_t)ns;
         p->meta_bytes = 2 * (ns + 1) * 4;
         p->carry_pass = 1;
-        st = status_of(hipMalloc((void **)&p->d_meta, p->meta_bytes));
+        st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
         // does any row stay cut?  (one int read back; creation syncs anyway)
         int32_t *d_flag = reinterpret_cast<int32_t *>(p->d_counters + 40), h_flag = 1;
         if (!st) st = launch_fill_i32(d_flag, 1, 0, s);
@@ -499,15 +505,16 @@ int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_
 int asx_plan_destroy(asx_plan *plan)
 {
     if (!plan) return ASX_STATUS_SUCCESS;
-    int st = ASX_STATUS_SUCCESS;
-    if (plan->d_meta) st = status_of(hipFree(plan->d_meta));
-    if (plan->d_counters) (void)hipFree(plan->d_counters);
-    if (plan->d_checksum_parts) (void)hipFree(plan->d_checksum_parts);
+    // calls through the plan may still be running on any stream
+    pool_wait(plan->d_counters ? (const void *)plan->d_counters : plan->blocked.brow_ptr);
+    pool_free(plan->d_meta);
+    pool_free(plan->d_counters);
+    pool_free(plan->d_checksum_parts);
     free_blocked(&plan->blocked);
     free_sliced(&plan->sliced);
     free_window(&plan->window);
     delete plan;
-    return st;
+    return ASX_STATUS_SUCCESS;
 }
 
 // Blocks are worth it when they are at least this full (bytes moved per stored element fall
@@ -529,11 +536,11 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
     bool probe_blocked = alg == ASX_SPMM_DEFAULT && nnz > 0 && nnz <= kBlockedProbeMaxNnz && d_col &&
                          (value_type == ASX_R_32F || value_type == ASX_R_64F);
     if (probe_blocked) {
+        Scratch scratch((hipStream_t)stream);
         int32_t *d_scratch = nullptr;
-        if (hipMalloc((void **)&d_scratch, 128 * sizeof(int32_t)) != hipSuccess) return ASX_STATUS_ALLOC_FAILED;
+        if (scratch.take(&d_scratch, 128 * sizeof(int32_t)) != hipSuccess) return ASX_STATUS_ALLOC_FAILED;
         const ColumnSample cs = sample_columns(nullptr, m, d_col, nnz, vsize(value_type), d_scratch, (hipStream_t)stream);
         probe_blocked = cs.ok && cs.spread < kScatteredMinSpread;
-        (void)hipFree(d_scratch);
     }
     if (!want_blocked && !probe_blocked)
         return asx_plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, stream);
@@ -662,7 +669,7 @@ int plan_add_slices(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
     const int st = build_sliced<T>(p->m, p->n, p->nnz, (int32_t)(kSliceBytes / sizeof(T)), rpw, cus, d_row_ptr, d_col,
                                    d_val, &sm, s);
     if (st) return st;
-    if (p->d_meta) (void)hipFree(p->d_meta);
+    pool_free(p->d_meta);
     p->d_meta = nullptr;
     p->meta_bytes = 0;
     p->alg = ASX_SPMV_SLICED;
@@ -689,7 +696,7 @@ int plan_add_window(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
     const int st = build_window<T>(p->m, p->n, p->nnz, cus * (sizeof(T) == 4 ? 2 : 1), sizeof(T) == 4 || follows_values, d_row_ptr,
                                    d_col, d_val, &wm, s);
     if (st) return st;
-    if (p->d_meta) (void)hipFree(p->d_meta);
+    pool_free(p->d_meta);
     p->d_meta = nullptr;
     p->meta_bytes = 0;
     p->alg = ASX_SPMV_WINDOW;
@@ -716,7 +723,7 @@ static bool regrouped_copy_fits(const asx_plan *p, size_t sv)
     size_t free_b = 0, total_b = 0;
     if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
     const double copy = (double)p->nnz * (double)(sv + 8) + (double)p->nnz * (double)(sv + 2) + (double)p->nnz * 4.0;
-    return (double)free_b >= 2.0 * copy;
+    return (double)free_b + (double)pool_kept_bytes() >= 2.0 * copy;
 }
 
 static bool window_may_pay(const asx_plan *p, int row_kernel)
@@ -734,7 +741,7 @@ static int keep_checksum(asx_plan *p, const void *d_val, hipStream_t s)
 {
     unsigned long long *w = checksum_words(p);
     int st = ASX_STATUS_SUCCESS;
-    if (!p->d_checksum_parts) st = status_of(hipMalloc((void **)&p->d_checksum_parts, sizeof(unsigned long long) * 2 * checksum_parts()));
+    if (!p->d_checksum_parts) st = status_of(pool_malloc(&p->d_checksum_parts, sizeof(unsigned long long) * 2 * checksum_parts(), false));
     if (!st) st = launch_checksum(d_val, (size_t)p->nnz * vsize(p->value_type), p->d_checksum_parts, w, s);
     if (!st) st = launch_checksum_commit(w, w + 2, s);
     return st;
@@ -915,11 +922,11 @@ int asx_plan_release_scratch(asx_plan *plan)
     if (!plan) return ASX_STATUS_INVALID_POINTER;
     int st = ASX_STATUS_SUCCESS;
     if (plan->sliced.partial) {
-        st = status_of(hipFree(plan->sliced.partial));
+        st = status_of(pool_return(plan->sliced.partial));
         plan->sliced.partial = nullptr;
     }
     if (plan->window.carry) {
-        const int st2 = status_of(hipFree(plan->window.carry));
+        const int st2 = status_of(pool_return(plan->window.carry));
         plan->window.carry = nullptr;
         if (!st) st = st2;
     }

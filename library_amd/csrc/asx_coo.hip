@@ -64,13 +64,13 @@ int coo_sort(int32_t *row, int32_t *col, T *val, int32_t nnz, hipStream_t s)
         st = status_of(expr);     \
         if (st) goto done;        \
     } while (0)
-    ASX_TRY(hipMalloc((void **)&keys, sizeof(uint64_t) * (size_t)nnz));
-    ASX_TRY(hipMalloc((void **)&keys2, sizeof(uint64_t) * (size_t)nnz));
-    ASX_TRY(hipMalloc((void **)&idx, sizeof(int32_t) * (size_t)nnz));
-    ASX_TRY(hipMalloc((void **)&idx2, sizeof(int32_t) * (size_t)nnz));
-    ASX_TRY(hipMalloc((void **)&val2, sizeof(T) * (size_t)nnz));
+    ASX_TRY(pool_malloc(&keys, sizeof(uint64_t) * (size_t)nnz, true));
+    ASX_TRY(pool_malloc(&keys2, sizeof(uint64_t) * (size_t)nnz, true));
+    ASX_TRY(pool_malloc(&idx, sizeof(int32_t) * (size_t)nnz, true));
+    ASX_TRY(pool_malloc(&idx2, sizeof(int32_t) * (size_t)nnz, true));
+    ASX_TRY(pool_malloc(&val2, sizeof(T) * (size_t)nnz, true));
     ASX_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
-    ASX_TRY(hipMalloc(&tmp, tmp_bytes ? tmp_bytes : 1));
+    ASX_TRY(pool_malloc(&tmp, tmp_bytes, true));
     hipLaunchKernelGGL(k_coo_keys, dim3(grid), dim3(kBlock), 0, s, row, col, nnz, keys, idx);
     ASX_TRY(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
     ASX_TRY(hipMemcpyAsync(val2, val, sizeof(T) * (size_t)nnz, hipMemcpyDeviceToDevice, s));
@@ -79,8 +79,9 @@ int coo_sort(int32_t *row, int32_t *col, T *val, int32_t nnz, hipStream_t s)
     ASX_TRY(hipStreamSynchronize(s));
 #undef ASX_TRY
 done:
+    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
     for (void *p : {(void *)keys, (void *)keys2, (void *)idx, (void *)idx2, (void *)val2, tmp})
-        if (p) (void)hipFree(p);
+        pool_free(p);
     return st;
 }
 

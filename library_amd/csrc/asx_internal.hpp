@@ -6,6 +6,7 @@
 
 #include "../../include/alphasparse_amd.h"
 #include "asx_device.hpp"
+#include "asx_pool.hpp"
 
 namespace asx {
 

@@ -1,0 +1,236 @@
+// Kept blocks of device memory (asx_pool.hpp).
+#include "asx_pool.hpp"
+
+#include <algorithm>
+#include <mutex>
+#include <unordered_map>
+#include <vector>
+
+namespace asx {
+
+namespace {
+
+struct Block {
+    void *p;
+    size_t bytes;
+    int dev;
+};
+
+struct Pool {
+    std::mutex lock;
+    std::unordered_map<const void *, Block> live;
+    std::vector<Block> kept;  // oldest first
+    std::vector<void *> pinned;
+};
+
+// Never destroyed: at process exit the HIP runtime may be gone before static objects are.
+Pool &pool()
+{
+    static Pool *p = new Pool;
+    return *p;
+}
+
+// Sizes in eighths of a power of two: requests that differ a little meet each other's blocks.
+size_t rounded(size_t bytes)
+{
+    size_t step = 65536;
+    while (step * 16 <= bytes) step *= 2;
+    return (std::max<size_t>(bytes, 1) + step - 1) / step * step;
+}
+
+class OnDevice {
+public:
+    explicit OnDevice(int dev)
+    {
+        (void)hipGetDevice(&was_);
+        if (was_ != dev) (void)hipSetDevice(dev), moved_ = true;
+    }
+    ~OnDevice()
+    {
+        if (moved_) (void)hipSetDevice(was_);
+    }
+
+private:
+    int was_ = 0;
+    bool moved_ = false;
+};
+
+// Takes blocks of `dev` out of the kept ones (all of them, or the oldest beyond the bounds).
+std::vector<Block> surplus(Pool &P, int dev, bool all)
+{
+    std::vector<Block> out;
+    size_t bytes = 0, blocks = 0;
+    for (const Block &b : P.kept)
+        if (b.dev == dev) bytes += b.bytes, ++blocks;
+    for (size_t i = 0; i < P.kept.size();) {
+        const Block b = P.kept[i];
+        if (b.dev != dev || !(all || bytes > kPoolMaxBytes || blocks > kPoolMaxBlocks)) {
+            ++i;
+            continue;
+        }
+        bytes -= b.bytes;
+        --blocks;
+        out.push_back(b);
+        P.kept.erase(P.kept.begin() + (std::ptrdiff_t)i);
+    }
+    return out;
+}
+
+}  // namespace
+
+hipError_t pool_malloc_bytes(void **p, size_t bytes, bool brief)
+{
+    *p = nullptr;
+    int dev = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e != hipSuccess) return e;
+    const size_t want = rounded(bytes);
+    Pool &P = pool();
+    {
+        std::lock_guard<std::mutex> g(P.lock);
+        const size_t most = brief ? 4 * want : want + want / 4;
+        size_t best = P.kept.size();
+        for (size_t i = 0; i < P.kept.size(); ++i) {
+            const Block &b = P.kept[i];
+            if (b.dev == dev && b.bytes >= want && b.bytes <= most && (best == P.kept.size() || b.bytes < P.kept[best].bytes)) best = i;
+        }
+        if (best < P.kept.size()) {
+            const Block b = P.kept[best];
+            P.kept.erase(P.kept.begin() + (std::ptrdiff_t)best);
+            P.live[b.p] = b;
+            *p = b.p;
+            return hipSuccess;
+        }
+    }
+    size_t got = want;
+    e = hipMalloc(p, got);
+    if (e == hipErrorOutOfMemory) {
+        (void)hipGetLastError();
+        pool_release();
+        e = hipMalloc(p, got);
+        if (e == hipErrorOutOfMemory && bytes > 0 && bytes < want) {
+            (void)hipGetLastError();
+            got = bytes;
+            e = hipMalloc(p, got);
+        }
+    }
+    if (e != hipSuccess) {
+        *p = nullptr;
+        return e;
+    }
+    std::lock_guard<std::mutex> g(P.lock);
+    P.live[*p] = Block{*p, got, dev};
+    return hipSuccess;
+}
+
+void pool_free(void *p)
+{
+    if (!p) return;
+    Pool &P = pool();
+    std::vector<Block> out;
+    {
+        std::lock_guard<std::mutex> g(P.lock);
+        const auto it = P.live.find(p);
+        if (it == P.live.end()) return;  // not a block of this pool
+        const Block b = it->second;
+        P.live.erase(it);
+        if (b.bytes > kPoolMaxBlockBytes) {
+            out.push_back(b);
+        } else {
+            P.kept.push_back(b);
+            out = surplus(P, b.dev, false);
+        }
+    }
+    for (const Block &b : out) {
+        OnDevice on(b.dev);
+        (void)hipFree(b.p);
+    }
+}
+
+void pool_wait(const void *p)
+{
+    if (!p) return;
+    Pool &P = pool();
+    int dev;
+    {
+        std::lock_guard<std::mutex> g(P.lock);
+        const auto it = P.live.find(p);
+        if (it == P.live.end()) return;
+        dev = it->second.dev;
+    }
+    OnDevice on(dev);
+    (void)hipDeviceSynchronize();
+}
+
+hipError_t pool_return(void *p)
+{
+    if (!p) return hipSuccess;
+    Pool &P = pool();
+    int dev;
+    {
+        std::lock_guard<std::mutex> g(P.lock);
+        const auto it = P.live.find(p);
+        if (it == P.live.end()) return hipErrorInvalidValue;
+        dev = it->second.dev;
+        P.live.erase(it);
+    }
+    OnDevice on(dev);
+    return hipFree(p);
+}
+
+size_t pool_kept_bytes()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return 0;
+    Pool &P = pool();
+    std::lock_guard<std::mutex> g(P.lock);
+    size_t bytes = 0;
+    for (const Block &b : P.kept)
+        if (b.dev == dev) bytes += b.bytes;
+    return bytes;
+}
+
+void pool_release()
+{
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess) return;
+    Pool &P = pool();
+    std::vector<Block> out;
+    {
+        std::lock_guard<std::mutex> g(P.lock);
+        out = surplus(P, dev, true);
+    }
+    for (const Block &b : out) (void)hipFree(b.p);
+}
+
+void *pinned_take()
+{
+    Pool &P = pool();
+    {
+        std::lock_guard<std::mutex> g(P.lock);
+        if (!P.pinned.empty()) {
+            void *p = P.pinned.back();
+            P.pinned.pop_back();
+            return p;
+        }
+    }
+    void *p = nullptr;
+    // portable: readable and writable from every device
+    return hipHostMalloc(&p, kPinnedBytes, hipHostMallocPortable) == hipSuccess ? p : nullptr;
+}
+
+void pinned_give(void *p)
+{
+    if (!p) return;
+    Pool &P = pool();
+    {
+        std::lock_guard<std::mutex> g(P.lock);
+        if (P.pinned.size() < 16) {
+            P.pinned.push_back(p);
+            return;
+        }
+    }
+    (void)hipHostFree(p);
+}
+
+}  // namespace asx

@@ -28,6 +28,7 @@
 #include <vector>
 
 #include "asx_internal.hpp"
+#include "asx_rank.hpp"
 #include "asx_scan.hpp"
 #include "asx_tiles.hpp"
 
@@ -44,12 +45,6 @@ constexpr int32_t kPadRow = 0x7fffffff;
 // every slice; a second kernel ranks the elements of a block inside their slices (stable: row
 // order, then column order, survives inside a slice), orders them by slice in LDS and writes
 // column, value, source index and row of each straight to its slot, in runs of consecutive slots.
-constexpr int kSortThreads = 512;
-constexpr int kSortWaves = kSortThreads / kWave;
-constexpr int kSortElems = 4096;  // per block
-constexpr int kSortPerLane = kSortElems / kSortThreads;
-constexpr int kSortWaveElems = kSortElems / kSortWaves;
-
 __global__ __launch_bounds__(kSortThreads) void k_sliced_count(const int32_t *__restrict__ col, int32_t nnz,
                                                                 int32_t width, int32_t nslices, int32_t nblocks,
                                                                 int32_t *__restrict__ counts)
@@ -74,40 +69,6 @@ __global__ __launch_bounds__(kBlock) void k_sliced_slice_starts(const int32_t *_
 {
     const int32_t s = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
     if (s <= nslices) pstart[s] = offs[(int64_t)s * nblocks];
-}
-
-// largest r in [lo, hi] with row_ptr[r] <= i
-__device__ __forceinline__ int32_t row_holding(const int32_t *__restrict__ row_ptr, int32_t lo, int32_t hi, int32_t i)
-{
-    while (lo < hi) {
-        const int32_t mid = lo + (hi - lo + 1) / 2;
-        if (row_ptr[mid] <= i)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    return lo;
-}
-
-// in-place exclusive sum of a[0 .. n), n <= 2 * kSortThreads, by the whole workgroup (barriers inside)
-__device__ __forceinline__ void block_exclusive_sum(int32_t *a, int n, int32_t *wave_tot)
-{
-    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const int32_t v0 = 2 * tid < n ? a[2 * tid] : 0, v1 = 2 * tid + 1 < n ? a[2 * tid + 1] : 0;
-    int32_t incl = v0 + v1;
-#pragma unroll
-    for (int d = 1; d < kWave; d <<= 1) {
-        const int32_t t = __shfl_up(incl, d, kWave);
-        if (lane >= d) incl += t;
-    }
-    if (lane == kWave - 1) wave_tot[wave] = incl;
-    __syncthreads();
-    int32_t before = 0;
-    for (int w = 0; w < wave; ++w) before += wave_tot[w];
-    const int32_t excl = before + incl - (v0 + v1);
-    if (2 * tid < n) a[2 * tid] = excl;
-    if (2 * tid + 1 < n) a[2 * tid + 1] = excl + v0;
-    __syncthreads();
 }
 
 template <typename T>
@@ -148,26 +109,10 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_scatter(
         const int64_t i = wbase + k * kWave + lane;
         c[k] = i < nnz ? col[i] : 0;
     }
-    // rank of every element among the wave's elements of its slice, in element order: the wave
-    // takes its elements 64 at a time; inside a step the lanes of one slice find each other by
-    // ballots over the bits of the slice number
+    // rank of every element among the wave's elements of its slice, in element order
 #pragma unroll
-    for (int k = 0; k < kSortPerLane; ++k) {
-        const bool valid = wbase + k * kWave + lane < nnz;
-        const int32_t key = c[k] / width;
-        unsigned long long same = __ballot(valid);
-        for (int bit = 0; bit < nbits; ++bit) {
-            const bool one = (key >> bit) & 1;
-            const unsigned long long bal = __ballot(one);
-            same &= one ? bal : ~bal;
-        }
-        const int below = lanes_below(same);  // lanes of this slice before this one
-        const int32_t prev = valid ? mycnt[key] : 0;
-        rk[k] = prev + below;
-        if (valid && below == 0) mycnt[key] = prev + __popcll(same);
-        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-        __builtin_amdgcn_wave_barrier();
-    }
+    for (int k = 0; k < kSortPerLane; ++k)
+        rk[k] = wave_rank(c[k] / width, wbase + k * kWave + lane < nnz, nbits, mycnt);
     __syncthreads();
     for (int s = tid; s < nslices; s += kSortThreads) {
         int32_t run = 0;
@@ -681,7 +626,7 @@ __global__ __launch_bounds__(kWave) void k_sliced_reduce(int32_t m, int32_t nrb,
 void free_sliced(SlicedMatrix *p)
 {
     for (void *q : {p->store, p->partial, (void *)p->prow, (void *)p->psteps})
-        if (q) (void)hipFree(q);
+        pool_free(q);
     p->store = p->val = p->partial = nullptr;
     p->cf = p->prow = nullptr;
     p->perm = p->tile_base = p->wg_tab = p->wg_pieces = p->chunk_lo = p->pstep_ptr = p->psteps = p->block_base = nullptr;
@@ -744,7 +689,7 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
         const size_t o_pstart = take((size_t)sm.nslices + 1), o_toff = take((size_t)sm.nslices + 1);
         const size_t o_lrow = take((size_t)cap64), o_tcnt = take(max_tiles + 1), o_scnt = take((size_t)sm.nrb + 1);
         const size_t o_tmp = take(scan_scratch_ints(std::max<int64_t>(ncount, (int64_t)max_tiles + 1)));
-        ASX_TRY(hipMalloc((void **)&arena, off));
+        ASX_TRY(pool_malloc(&arena, off, true));
         counts = (int32_t *)(arena + o_counts), offs = (int32_t *)(arena + o_offs), seg_row = (int32_t *)(arena + o_seg);
         d_pstart = (int32_t *)(arena + o_pstart), d_tile_off = (int32_t *)(arena + o_toff);
         lrow = (int32_t *)(arena + o_lrow), tile_cnt = (int32_t *)(arena + o_tcnt), step_cnt = (int32_t *)(arena + o_scnt);
@@ -838,7 +783,7 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
         const size_t o_cl = take(sizeof(int32_t) * (size_t)ncells), o_sp = take(sizeof(int32_t) * ((size_t)sm.nrb + 1));
         const size_t o_pos = take(sizeof(uint16_t) * (size_t)nnz);
         const size_t o_bb = take(sizeof(int32_t) * ((size_t)nblocks + 1) * (size_t)sm.nslices);
-        ASX_TRY(hipMalloc(&sm.store, off));
+        ASX_TRY(pool_malloc(&sm.store, off, false));
         char *base = static_cast<char *>(sm.store);
         sm.val = base + o_val, sm.perm = (int32_t *)(base + o_perm), sm.cf = (uint16_t *)(base + o_cf);
         sm.tile_base = (int32_t *)(base + o_tb), sm.wg_tab = (int32_t *)(base + o_wg);
@@ -871,7 +816,7 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
         ASX_TRY_ST(launch_exclusive_scan_i32(tile_cnt, sm.tile_base, (int64_t)sm.ntiles + 1, tmp, s));
         ASX_TRY(hipMemcpyAsync(&sm.npartials, sm.tile_base + sm.ntiles, sizeof(int32_t), hipMemcpyDeviceToHost, s));
         ASX_TRY(hipStreamSynchronize(s));
-        ASX_TRY(hipMalloc((void **)&sm.prow, sizeof(uint16_t) * ((size_t)sm.npartials + kSlicedReducePad)));
+        ASX_TRY(pool_malloc(&sm.prow, sizeof(uint16_t) * ((size_t)sm.npartials + kSlicedReducePad), false));
         ASX_TRY(hipMemsetAsync(sm.prow + sm.npartials, 0, sizeof(uint16_t) * kSlicedReducePad, s));
         // 5. rows of the partial sums, run-start bits, and where each row block starts inside each slice
         hipLaunchKernelGGL(k_sliced_emit, dim3(wgrid), dim3(kBlock), 0, s, lrow, sm.tile_base, d_tile_off, sm.ntiles,
@@ -888,9 +833,9 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
                            nullptr);
         ASX_TRY_ST(launch_exclusive_scan_i32(step_cnt, sm.pstep_ptr, (int64_t)sm.nrb + 1, tmp, s));
         ASX_TRY(hipMemcpyAsync(&sm.npsteps, sm.pstep_ptr + sm.nrb, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        ASX_TRY(hipMalloc(&sm.partial, sizeof(T) * ((size_t)sm.npartials + kSlicedReducePad)));  // while the kernels run
+        ASX_TRY(pool_malloc(&sm.partial, sizeof(T) * ((size_t)sm.npartials + kSlicedReducePad), false));  // while the kernels run
         ASX_TRY(hipStreamSynchronize(s));
-        ASX_TRY(hipMalloc((void **)&sm.psteps, sizeof(int32_t) * 4 * ((size_t)sm.npsteps + kSlicedStepPad)));
+        ASX_TRY(pool_malloc(&sm.psteps, sizeof(int32_t) * 4 * ((size_t)sm.npsteps + kSlicedStepPad), false));
         ASX_TRY(hipMemsetAsync(sm.psteps + 4 * (size_t)sm.npsteps, 0, sizeof(int32_t) * 4 * kSlicedStepPad, s));
         hipLaunchKernelGGL(k_sliced_pack, dim3(pgrid), dim3(kBlock), 0, s, sm.chunk_lo, sm.nrb, sm.nslices, sm.pstep_ptr,
                            nullptr, reinterpret_cast<i32x4 *>(sm.psteps));
@@ -900,7 +845,8 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
 #undef ASX_TRY
 #undef ASX_TRY_ST
 done:
-    if (arena) (void)hipFree(arena);
+    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
+    pool_free(arena);
     if (st) {
         free_sliced(&sm);
         return st;

@@ -3,6 +3,7 @@
 // runs (asx_sliced.hip: runs = (row, slice) pairs; asx_window.hip: runs = rows).
 #pragma once
 #include "asx_internal.hpp"
+#include "asx_rank.hpp"
 
 namespace asx {
 
@@ -48,11 +49,6 @@ struct TileValues<float> {
         v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
     }
 };
-
-__device__ __forceinline__ int lanes_below(unsigned long long mask)
-{
-    return __builtin_amdgcn_mbcnt_hi((unsigned)(mask >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)mask, 0));
-}
 
 // One tile's stored elements as the loads deliver them.
 template <typename T>

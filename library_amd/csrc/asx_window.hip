@@ -787,7 +787,7 @@ __global__ __launch_bounds__(kBlock) void k_window_fixup(int32_t ntiles, T alpha
 void free_window(WindowMatrix *p)
 {
     for (void *q : {p->store, p->tables, p->carry})
-        if (q) (void)hipFree(q);
+        pool_free(q);
     p->store = p->tables = p->val = p->carry = nullptr;
     p->cf = nullptr;
     p->perm = p->tile_info = p->blocks = p->pieces = p->chains = nullptr;
@@ -831,7 +831,7 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
         const auto pad64 = [](size_t v) { return (v + 63) & ~(size_t)63; };
         const size_t per_group = pad64((size_t)ngroups), per_row = pad64((size_t)m), per_seg = pad64((size_t)nseg + 1);
         const size_t per_block = pad64((size_t)max_nb + 1);
-        ASX_TRY(hipMalloc((void **)&arena, sizeof(int32_t) * (2 * per_group + per_row + per_seg + 4 * per_block + 64)));
+        ASX_TRY(pool_malloc(&arena, sizeof(int32_t) * (2 * per_group + per_row + per_seg + 4 * per_block + 64), true));
         gmin = arena, gmax = gmin + per_group, row_start = gmax + per_group, seg_row = row_start + per_row;
         bmin = seg_row + per_seg, bmax = bmin + per_block, btiles = bmax + per_block, tile_off = btiles + per_block;
         d_small = tile_off + per_block;
@@ -903,7 +903,7 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
         };
         const int64_t nbins = (2 * (int64_t)n >> 6) + 2;
         const size_t words = (size_t)(nbins + 31) / 32;
-        ASX_TRY(hipMalloc((void **)&d_bits, sizeof(uint32_t) * words));
+        ASX_TRY(pool_malloc(&d_bits, sizeof(uint32_t) * words, true));
         ASX_TRY(hipMemsetAsync(d_bits, 0, sizeof(uint32_t) * words, s));
         hipLaunchKernelGGL(k_window_offset_bins, dim3((unsigned)nseg), dim3(kBlock), 0, s, row_ptr, col, m, n, nnz, seg_row, d_bits);
         h_bits.resize(words);
@@ -1066,14 +1066,14 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
         const size_t o_val = 0, o_perm = wm.by_reference ? 0 : align_up(sizeof(T) * (size_t)slots, 256);
         const size_t o_cf = o_perm + (wm.by_reference ? 0 : align_up(sizeof(int32_t) * (size_t)slots, 256));
         const size_t o_info = o_cf + align_up(sizeof(uint16_t) * (size_t)slots, 256);
-        ASX_TRY(hipMalloc(&wm.store, o_info + sizeof(int4) * (size_t)wm.ntiles));
+        ASX_TRY(pool_malloc(&wm.store, o_info + sizeof(int4) * (size_t)wm.ntiles, false));
         char *base = static_cast<char *>(wm.store);
         wm.val = wm.by_reference ? nullptr : base + o_val;
         wm.perm = wm.by_reference ? nullptr : (int32_t *)(base + o_perm);
         wm.cf = (uint16_t *)(base + o_cf);
         wm.tile_info = (int32_t *)(base + o_info);
     }
-    ASX_TRY(hipMalloc(&wm.carry, sizeof(T) * (size_t)wm.ntiles));
+    ASX_TRY(pool_malloc(&wm.carry, sizeof(T) * (size_t)wm.ntiles, false));
     // 4. every stored element to its slot; every other slot becomes a zero that points at the zero
     //    behind the rings and opens a run of its own
     hipLaunchKernelGGL((k_window_place<T>), dim3((unsigned)ceil_div64(nnz, kBlock)), dim3(kBlock), 0, s, row_ptr, col, val,
@@ -1212,7 +1212,7 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
     {   // the tables of the blocks in one allocation (16-byte entries first)
         const size_t o_pieces = align_up(sizeof(int32_t) * blk.size(), 256);
         const size_t o_chains = o_pieces + align_up(sizeof(int32_t) * pcs.size(), 256);
-        ASX_TRY(hipMalloc(&wm.tables, o_chains + sizeof(int32_t) * chains.size()));
+        ASX_TRY(pool_malloc(&wm.tables, o_chains + sizeof(int32_t) * chains.size(), false));
         char *base = static_cast<char *>(wm.tables);
         wm.blocks = (int32_t *)base, wm.pieces = (int32_t *)(base + o_pieces), wm.chains = (int32_t *)(base + o_chains);
     }
@@ -1224,8 +1224,8 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
     wm.has_carry = h_small[0] != 0;
 #undef ASX_TRY
 done:
-    for (void *p : {(void *)arena, (void *)d_bits})
-        if (p) (void)hipFree(p);
+    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
+    for (void *p : {(void *)arena, (void *)d_bits}) pool_free(p);
     if (st) {
         free_window(&wm);
         return st;
