@@ -6,6 +6,7 @@
 #include <algorithm>
 
 #include "asx_internal.hpp"
+#include "asx_rank.hpp"
 
 namespace asx {
 
@@ -19,9 +20,8 @@ __global__ __launch_bounds__(256) void k_zero_i64(int64_t *p, int n)
     if (i < n) p[i] = 0;
 }
 
-__global__ __launch_bounds__(256) void k_row_histogram(const int32_t *__restrict__ row_ptr, int32_t m,
-                                                       unsigned long long *hist /*33*/,
-                                                       unsigned long long *stats /*4*/)
+__device__ __forceinline__ void row_histogram(const int32_t *__restrict__ row_ptr, int32_t m, int64_t block, int64_t blocks,
+                                              unsigned long long *hist /*33*/, unsigned long long *stats /*4*/)
 {
     __shared__ unsigned int s_hist[33];
     __shared__ unsigned int s_bins[3];
@@ -32,7 +32,7 @@ __global__ __launch_bounds__(256) void k_row_histogram(const int32_t *__restrict
     __syncthreads();
     int local_max = 0;
     const int lane = threadIdx.x & (kWave - 1);
-    for (int64_t r0 = (int64_t)blockIdx.x * blockDim.x; r0 < m; r0 += (int64_t)gridDim.x * blockDim.x) {  // uniform
+    for (int64_t r0 = block * 256; r0 < m; r0 += blocks * 256) {  // uniform
         const int64_t r = r0 + threadIdx.x;
         const bool valid = r < m;
         const int len = valid ? row_ptr[r + 1] - row_ptr[r] : 0;
@@ -65,18 +65,27 @@ __global__ __launch_bounds__(256) void k_row_histogram(const int32_t *__restrict
     if (threadIdx.x == 0) atomicMax(&stats[0], (unsigned long long)s_max);
 }
 
+__global__ __launch_bounds__(256) void k_row_histogram(const int32_t *__restrict__ row_ptr, int32_t m,
+                                                       unsigned long long *hist, unsigned long long *stats)
+{
+    row_histogram(row_ptr, m, blockIdx.x, gridDim.x, hist, stats);
+}
+
+static unsigned histogram_blocks(int32_t m)
+{
+    const int64_t grid = ceil_div64(m, 256 * 8);
+    return (unsigned)(grid > 4096 ? 4096 : grid);
+}
+
 int launch_row_histogram(const int32_t *d_row_ptr, int32_t m, int64_t *d_hist, int64_t *d_stats,
                          hipStream_t s)
 {
     // counters are cleared with a kernel (not a memset node) so the call can sit in a graph
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(256), 0, s, d_hist, 33);
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(256), 0, s, d_stats, 4);
-    if (m > 0) {
-        int grid = (int)ceil_div64(m, 256 * 8);
-        if (grid > 4096) grid = 4096;
-        hipLaunchKernelGGL(k_row_histogram, dim3(grid), dim3(256), 0, s, d_row_ptr, m,
+    if (m > 0)
+        hipLaunchKernelGGL(k_row_histogram, dim3(histogram_blocks(m)), dim3(256), 0, s, d_row_ptr, m,
                            (unsigned long long *)d_hist, (unsigned long long *)d_stats);
-    }
     return check_launch();
 }
 
@@ -149,22 +158,39 @@ __global__ __launch_bounds__(256) void k_nnz_split_rows(const int32_t *__restric
     out[t] = lo;
 }
 
-// same kernel for a caller-chosen segment count (nseg >= ceil(nnz/items))
+// The same with a wave per output, 64 probes at a time: few outputs leave the chip waiting for the
+// twenty dependent reads of a search (3500 outputs over 250013 rows: 7.5 us a thread each).
+__global__ __launch_bounds__(256) void k_nnz_split_rows_wave(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nseg,
+                                                             int32_t items, int32_t *__restrict__ out)
+{
+    const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+    if (t > nseg) return;  // whole waves leave
+    const int32_t r = t == nseg ? m : wave_row_holding(row_ptr, 0, m, (int32_t)(t * items));
+    if ((threadIdx.x & (kWave - 1)) == 0) out[t] = r;
+}
+
+static int launch_split_rows(const int32_t *d_row_ptr, int32_t m, int32_t nseg, int32_t items, int32_t *d_out, hipStream_t s)
+{
+    if (nseg < 65536)
+        hipLaunchKernelGGL(k_nnz_split_rows_wave, dim3((unsigned)ceil_div64(((int64_t)nseg + 1) * kWave, 256)), dim3(256), 0, s,
+                           d_row_ptr, m, nseg, items, d_out);
+    else
+        hipLaunchKernelGGL(k_nnz_split_rows, dim3((unsigned)ceil_div64((int64_t)nseg + 1, 256)), dim3(256), 0, s, d_row_ptr, m,
+                           nseg, items, d_out);
+    return check_launch();
+}
+
+// for a caller-chosen segment count (nseg >= ceil(nnz/items))
 int launch_nnz_split_rows_n(const int32_t *d_row_ptr, int32_t m, int32_t nseg, int32_t items, int32_t *d_out,
                             hipStream_t s)
 {
-    int grid = (int)ceil_div64((int64_t)nseg + 1, 256);
-    hipLaunchKernelGGL(k_nnz_split_rows, dim3(grid), dim3(256), 0, s, d_row_ptr, m, nseg, items, d_out);
-    return check_launch();
+    return launch_split_rows(d_row_ptr, m, nseg, items, d_out, s);
 }
 
 int launch_nnz_split_rows(const int32_t *d_row_ptr, int32_t m, int32_t nnz, int32_t items,
                           int32_t *d_out, hipStream_t s)
 {
-    int32_t nseg = (int32_t)ceil_div64(nnz, items);
-    int grid = (int)ceil_div64((int64_t)nseg + 1, 256);
-    hipLaunchKernelGGL(k_nnz_split_rows, dim3(grid), dim3(256), 0, s, d_row_ptr, m, nseg, items, d_out);
-    return check_launch();
+    return launch_split_rows(d_row_ptr, m, (int32_t)ceil_div64(nnz, items), items, d_out, s);
 }
 
 // -------------------------------------------------------------------------------------------
@@ -269,22 +295,41 @@ __global__ __launch_bounds__(256) void k_copy16(const u32x4 *__restrict__ src, u
 // row_ptr given also out[64 + t] = number of (row, slice) pairs among the tile's elements, slices
 // of `width` columns: an element opens a pair when it is the first of its row (or of the tile) or
 // lies in another slice than the element before it (columns ascend inside a row).
-__global__ __launch_bounds__(kBlock) void k_sample_columns(const int32_t *__restrict__ col, int64_t stride, int shift,
-                                                           const int32_t *__restrict__ row_ptr, int32_t m, int32_t width,
-                                                           int32_t *__restrict__ out)
+struct SampleArgs {
+    const int32_t *col;
+    int64_t stride;
+    int shift;
+    const int32_t *row_ptr;
+    int32_t m, width, samples;
+    int32_t *out;
+};
+__device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
 {
     constexpr int kSlots = 4096;
     __shared__ int32_t table[kSlots];
+    __shared__ uint32_t starts[kFlatTile / 32];  // bit i: element i of the tile is the first of its row
     __shared__ int32_t count, pairs;
     for (int i = threadIdx.x; i < kSlots; i += kBlock) table[i] = -1;
+    if (threadIdx.x < kFlatTile / 32) starts[threadIdx.x] = 0;
     if (threadIdx.x == 0) count = 0, pairs = 0;
     __syncthreads();
-    const int64_t first = (int64_t)blockIdx.x * stride;
-    const int32_t *from = col + first;
+    const int64_t first = (int64_t)t * q.stride;
+    const int32_t *from = q.col + first;
+    if (q.row_ptr) {
+        // the rows that start in the tile: found by two searches, marked by one read each (a search
+        // per element was a chain of twenty reads, 23 us for the whole sample)
+        const int32_t lo = wave_row_holding(q.row_ptr, 0, q.m, (int32_t)first),
+                      hi = wave_row_holding(q.row_ptr, lo, q.m, (int32_t)(first + kFlatTile - 1));
+        for (int64_t r = (int64_t)lo + threadIdx.x; r <= hi && r < q.m; r += kBlock) {
+            const int64_t at = (int64_t)q.row_ptr[r] - first;
+            if (at >= 0 && at < kFlatTile) atomicOr(&starts[at >> 5], 1u << (at & 31));
+        }
+    }
+    __syncthreads();
     int32_t mine = 0, mine_pairs = 0;
     for (int i = threadIdx.x; i < kFlatTile; i += kBlock) {
         const int32_t c = from[i];
-        const int32_t v = c >> shift;
+        const int32_t v = c >> q.shift;
         uint32_t h = ((uint32_t)v * 2654435761u) >> 20;
         for (;;) {
             const int32_t old = atomicCAS(&table[h], -1, v);
@@ -295,37 +340,50 @@ __global__ __launch_bounds__(kBlock) void k_sample_columns(const int32_t *__rest
             if (old == v) break;
             h = (h + 1) & (kSlots - 1);
         }
-        if (row_ptr) {
-            bool opens = i == 0 || c / width != from[i - 1] / width;
-            if (!opens) {  // first element of its row?
-                const int64_t e = first + i;
-                int32_t lo = 0, hi = m;  // largest r with row_ptr[r] <= e
-                while (lo < hi) {
-                    const int32_t mid = lo + (hi - lo + 1) / 2;
-                    if ((int64_t)row_ptr[mid] <= e)
-                        lo = mid;
-                    else
-                        hi = mid - 1;
-                }
-                opens = row_ptr[lo] == e;
-            }
-            mine_pairs += opens;
-        }
+        if (q.row_ptr)
+            mine_pairs += i == 0 || c / q.width != from[i - 1] / q.width || (starts[i >> 5] >> (i & 31) & 1u) != 0;
     }
     if (mine) atomicAdd(&count, mine);
     if (mine_pairs) atomicAdd(&pairs, mine_pairs);
     __syncthreads();
     if (threadIdx.x == 0) {
-        out[blockIdx.x] = count;
-        if (row_ptr) out[64 + blockIdx.x] = pairs;
+        q.out[t] = count;
+        if (q.row_ptr) q.out[64 + t] = pairs;
     }
 }
+__global__ __launch_bounds__(kBlock) void k_sample_columns(SampleArgs q) { sample_columns_tile(q, blockIdx.x); }
+
 int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const int32_t *d_row_ptr, int32_t m,
                           int32_t width, int32_t samples, int32_t *d_out, hipStream_t s)
 {
     if (samples <= 0 || samples > 64) return samples > 64 ? ASX_STATUS_INVALID_VALUE : ASX_STATUS_SUCCESS;
-    hipLaunchKernelGGL(k_sample_columns, dim3((unsigned)samples), dim3(kBlock), 0, s, d_col, stride, shift, d_row_ptr, m, width,
-                       d_out);
+    const SampleArgs q{d_col, stride, shift, d_row_ptr, m, width, samples, d_out};
+    hipLaunchKernelGGL(k_sample_columns, dim3((unsigned)samples), dim3(kBlock), 0, s, q);
+    return check_launch();
+}
+
+// What an analysis looks at first, in one launch: the sample (its workgroups first, they take longest) and the
+// histogram of the row lengths.
+__global__ __launch_bounds__(kBlock) void k_plan_stats(SampleArgs q, const int32_t *__restrict__ row_ptr, int32_t m,
+                                                       unsigned long long *hist, unsigned long long *stats)
+{
+    if ((int)blockIdx.x < q.samples)
+        sample_columns_tile(q, blockIdx.x);
+    else
+        row_histogram(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, hist, stats);
+}
+
+int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int64_t *d_hist, int64_t *d_stats,
+                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample,
+                      hipStream_t s)
+{
+    if (samples < 0 || samples > 64) return ASX_STATUS_INVALID_VALUE;
+    hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(256), 0, s, d_counters, ncounters);
+    if (m > 0) {
+        const SampleArgs q{d_col, stride, shift, d_row_ptr, m, width, samples, d_sample};
+        hipLaunchKernelGGL(k_plan_stats, dim3(histogram_blocks(m) + (unsigned)samples), dim3(kBlock), 0, s, q, d_row_ptr, m,
+                           (unsigned long long *)d_hist, (unsigned long long *)d_stats);
+    }
     return check_launch();
 }
 

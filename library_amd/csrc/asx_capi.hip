@@ -92,27 +92,33 @@ struct ColumnSample {
     double spread, pairs;
 };
 constexpr int32_t kSliceBytes = 131072;  // of x per slice: one workgroup of 16 waves per compute unit
-ColumnSample sample_columns(const int32_t *d_row_ptr, int32_t m, const int32_t *d_col, int32_t nnz, size_t sv,
-                            int32_t *d_scratch /* 128 ints */, hipStream_t s)
+int sample_tiles(int32_t nnz) { return (int)std::min<int64_t>(64, nnz / kFlatTile); }
+int64_t sample_stride(int32_t nnz) { return (int64_t)(nnz / kFlatTile) / std::max(sample_tiles(nnz), 1) * kFlatTile; }
+int line_shift(size_t sv) { return sv == 8 ? 4 : 5; }  // columns per 128-byte line of x
+// h: distinct lines of every tile, then (with row offsets) the pairs, as counted on the device
+ColumnSample sample_result(const int32_t h[128], int32_t nnz, bool with_pairs)
 {
-    ColumnSample cs{false, 0.0, 1.0};
-    const int64_t tiles = nnz / kFlatTile;
-    if (tiles < 1) return cs;
-    const int samples = (int)std::min<int64_t>(64, tiles);
-    const int64_t stride = tiles / samples;
-    int32_t h[128];
-    const int shift = sv == 8 ? 4 : 5;  // columns per 128-byte line of x
-    if (launch_sample_columns(d_col, stride * kFlatTile, shift, d_row_ptr, m, (int32_t)(kSliceBytes / sv), samples, d_scratch,
-                              s) != ASX_STATUS_SUCCESS ||
-        hipMemcpyAsync(h, d_scratch, sizeof(h), hipMemcpyDeviceToHost, s) != hipSuccess ||
-        hipStreamSynchronize(s) != hipSuccess)
-        return cs;
+    const int samples = sample_tiles(nnz);
     int64_t distinct = 0, pairs = 0;
     for (int t = 0; t < samples; ++t) distinct += h[t], pairs += h[64 + t];
-    cs.ok = true;
-    cs.spread = (double)distinct / ((double)samples * kFlatTile);
-    cs.pairs = d_row_ptr ? (double)pairs / ((double)samples * kFlatTile) : 1.0;
+    ColumnSample cs{samples > 0, 0.0, 1.0};
+    if (samples > 0) cs.spread = (double)distinct / ((double)samples * kFlatTile);
+    if (samples > 0 && with_pairs) cs.pairs = (double)pairs / ((double)samples * kFlatTile);
     return cs;
+}
+// the spread alone, counted now
+ColumnSample sample_columns(const int32_t *d_col, int32_t nnz, size_t sv, hipStream_t s)
+{
+    const ColumnSample none{false, 0.0, 1.0};
+    Scratch scratch(s);
+    int32_t *h = static_cast<int32_t *>(scratch.pinned());
+    if (sample_tiles(nnz) < 1 || !h) return none;
+    // the counts go straight into the host's memory
+    if (launch_sample_columns(d_col, sample_stride(nnz), line_shift(sv), nullptr, 0, 1, sample_tiles(nnz), h, s) != ASX_STATUS_SUCCESS ||
+        hipStreamSynchronize(s) != hipSuccess)
+        return none;
+    scratch.idle = true;
+    return sample_result(h, nnz, false);
 }
 constexpr double kScatteredMinSpread = 0.5;
 
@@ -377,11 +383,16 @@ int asx_loadbalance_partition(const int32_t *d_row_ptr, int32_t m, int32_t nnz, 
 
 namespace {
 
-// A plan with sizes and the row-length histogram, no kernel chosen yet.  The counters on the device
-// stay with the plan (33 histogram bins, 4 stats, spare words for what else the build reads back):
-// freeing them here would cost more than the build's kernels.
+// A plan with sizes and the row-length histogram, no kernel chosen yet; with d_col also the column
+// sample of an analysis that may regroup A, and whether the device has room for that.  One round trip.
+// The counters on the device stay with the plan (33 histogram bins, 4 stats, spare words for what
+// else the build reads back): freeing them here would cost more than the build's kernels.
+struct PlanStats {
+    ColumnSample sample;
+    size_t free_bytes;
+};
 int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n, int32_t nnz, const int32_t *d_row_ptr,
-               int32_t ncols_dense, hipStream_t s)
+               int32_t ncols_dense, const int32_t *d_col, PlanStats *more, hipStream_t s)
 {
     asx_plan *p = new (std::nothrow) asx_plan();
     if (!p) return ASX_STATUS_ALLOC_FAILED;
@@ -394,15 +405,31 @@ int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n
     p->nnz = nnz;
     p->ncols = is_spmm ? ncols_dense : 1;
     p->row_ptr = d_row_ptr;
-    int st = status_of(pool_malloc(&p->d_counters, kPlanCounters * sizeof(int64_t), false));
-    if (!st) st = launch_row_histogram(d_row_ptr, m, p->d_counters, p->d_counters + 33, s);
-    if (!st) st = status_of(hipMemcpyAsync(p->hist, p->d_counters, 33 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    if (!st) st = status_of(hipMemcpyAsync(p->stats, p->d_counters + 33, 4 * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    const size_t sv = vsize(value_type);
+    const int samples = d_col && m > 0 ? sample_tiles(nnz) : 0;
+    Scratch scratch(s);
+    int64_t *h = static_cast<int64_t *>(scratch.pinned());
+    static_assert(kPlanCounters * sizeof(int64_t) <= kPinnedBytes, "the counters are read back through page-locked memory");
+    int st = h ? status_of(pool_malloc(&p->d_counters, kPlanCounters * sizeof(int64_t), false)) : ASX_STATUS_ALLOC_FAILED;
+    if (!st)
+        st = launch_plan_stats(d_row_ptr, m, p->d_counters, kPlanCounters, p->d_counters, p->d_counters + 33, d_col, sample_stride(nnz),
+                               line_shift(sv), (int32_t)(kSliceBytes / sv), samples,
+                               reinterpret_cast<int32_t *>(p->d_counters + 64), s);
+    if (!st) st = status_of(hipMemcpyAsync(h, p->d_counters, kPlanCounters * sizeof(int64_t), hipMemcpyDeviceToHost, s));
+    if (more) {  // asked while the device counts
+        size_t total = 0;
+        if (hipMemGetInfo(&more->free_bytes, &total) != hipSuccess) more->free_bytes = 0;
+        more->free_bytes += pool_kept_bytes();
+    }
     if (!st) st = status_of(hipStreamSynchronize(s));
     if (st) {
         asx_plan_destroy(p);
         return st;
     }
+    scratch.idle = true;
+    std::memcpy(p->hist, h, sizeof(p->hist));
+    std::memcpy(p->stats, h + 33, sizeof(p->stats));
+    if (more) more->sample = samples > 0 ? sample_result(reinterpret_cast<const int32_t *>(h + 64), nnz, true) : ColumnSample{false, 0.0, 1.0};
     *out = p;
     return ASX_STATUS_SUCCESS;
 }
@@ -417,6 +444,17 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
     p->alg = kernel;
     p->workspace_bytes = 0;
     if (m == 0) return ASX_STATUS_SUCCESS;  // nothing to analyse: calls with m == 0 return before any launch
+    // zero since plan_begin; set by the kernels that look for rows cut between units of work
+    int32_t *d_flag = reinterpret_cast<int32_t *>(p->d_counters + 40);
+    const auto read_flag = [&]() {
+        Scratch scratch(s);
+        int32_t *h = static_cast<int32_t *>(scratch.pinned());
+        if (!h) return (int)ASX_STATUS_ALLOC_FAILED;
+        int rc = status_of(hipMemcpyAsync(h, d_flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
+        if (!rc) rc = status_of(hipStreamSynchronize(s));
+        if (!rc) p->carry_pass = *h != 0, scratch.idle = true;
+        return rc;
+    };
     if (!p->is_spmm) {
         if (kernel == ASX_SPMV_STREAM) {
             int32_t nb = std::max(stream_blocks(nnz), 1);
@@ -433,12 +471,8 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             p->workspace_bytes = spmv_flat_layout(nnz, sv, false).bytes;
             p->carry_pass = 1;
             if (!st) {  // is any row cut by a tile boundary?  (one int read back; creation syncs anyway)
-                int32_t *d_flag = reinterpret_cast<int32_t *>(p->d_counters + 40), h_flag = 1;
-                st = launch_fill_i32(d_flag, 1, 0, s);
-                if (!st) st = launch_flat_has_carry(d_row_ptr, m, nnz, p->d_meta, d_flag, s);
-                if (!st) st = status_of(hipMemcpyAsync(&h_flag, d_flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-                if (!st) st = status_of(hipStreamSynchronize(s));
-                if (!st) p->carry_pass = h_flag != 0;
+                st = launch_flat_has_carry(d_row_ptr, m, nnz, p->d_meta, d_flag, s);
+                if (!st) st = read_flag();
             }
         } else if (kernel == ASX_SPMV_MERGE) {
             const size_t nt = (size_t)merge_tiles(m, nnz);
@@ -456,12 +490,8 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         p->carry_pass = 1;
         st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
         // does any row stay cut?  (one int read back; creation syncs anyway)
-        int32_t *d_flag = reinterpret_cast<int32_t *>(p->d_counters + 40), h_flag = 1;
-        if (!st) st = launch_fill_i32(d_flag, 1, 0, s);
         if (!st) st = launch_spmm_splits(m, nnz, items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
-        if (!st) st = status_of(hipMemcpyAsync(&h_flag, d_flag, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        if (!st) st = status_of(hipStreamSynchronize(s));
-        if (!st) p->carry_pass = h_flag != 0;
+        if (!st) st = read_flag();
         p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv, false).bytes;
     }
     if (!st) st = status_of(hipStreamSynchronize(s));
@@ -482,7 +512,7 @@ int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_
     if (m > 0 && !d_row_ptr) return ASX_STATUS_INVALID_POINTER;
     hipStream_t s = (hipStream_t)stream;
     asx_plan *p = nullptr;
-    int st = plan_begin(&p, is_spmm, value_type, m, n, nnz, d_row_ptr, ncols_dense, s);
+    int st = plan_begin(&p, is_spmm, value_type, m, n, nnz, d_row_ptr, ncols_dense, nullptr, nullptr, s);
     if (st) return st;
     int kernel;
     if (!is_spmm)
@@ -536,10 +566,7 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
     bool probe_blocked = alg == ASX_SPMM_DEFAULT && nnz > 0 && nnz <= kBlockedProbeMaxNnz && d_col &&
                          (value_type == ASX_R_32F || value_type == ASX_R_64F);
     if (probe_blocked) {
-        Scratch scratch((hipStream_t)stream);
-        int32_t *d_scratch = nullptr;
-        if (scratch.take(&d_scratch, 128 * sizeof(int32_t)) != hipSuccess) return ASX_STATUS_ALLOC_FAILED;
-        const ColumnSample cs = sample_columns(nullptr, m, d_col, nnz, vsize(value_type), d_scratch, (hipStream_t)stream);
+        const ColumnSample cs = sample_columns(d_col, nnz, vsize(value_type), (hipStream_t)stream);
         probe_blocked = cs.ok && cs.spread < kScatteredMinSpread;
     }
     if (!want_blocked && !probe_blocked)
@@ -718,12 +745,10 @@ int plan_add_window(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
 // bytes per stored element more for a while.
 // DEFAULT only makes one while twice that is free: a caller who sized the device for one copy of A
 // is not pushed to the edge by an analysis call.
-static bool regrouped_copy_fits(const asx_plan *p, size_t sv)
+static bool regrouped_copy_fits(const asx_plan *p, size_t sv, size_t free_bytes)
 {
-    size_t free_b = 0, total_b = 0;
-    if (hipMemGetInfo(&free_b, &total_b) != hipSuccess) return false;
     const double copy = (double)p->nnz * (double)(sv + 8) + (double)p->nnz * (double)(sv + 2) + (double)p->nnz * 4.0;
-    return (double)free_b + (double)pool_kept_bytes() >= 2.0 * copy;
+    return (double)free_bytes >= 2.0 * copy;
 }
 
 static bool window_may_pay(const asx_plan *p, int row_kernel)
@@ -765,12 +790,14 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
     }
     hipStream_t s = (hipStream_t)stream;
     asx_plan *p = nullptr;
-    int st = plan_begin(&p, 0, value_type, m, n, nnz, d_row_ptr, 1, s);
+    PlanStats ps{ColumnSample{false, 0.0, 1.0}, 0};
+    const bool may_regroup = alg == ASX_SPMV_DEFAULT && d_col && d_val && m > 0 && n > 0 && nnz >= kSlicedMinNnz;
+    const bool sample = may_regroup || alg == ASX_SPMV_SLICED;
+    int st = plan_begin(&p, 0, value_type, m, n, nnz, d_row_ptr, 1, sample ? d_col : nullptr, sample ? &ps : nullptr, s);
     if (st) return st;
     if (alg == ASX_SPMV_DEFAULT) row_kernel = choose_spmv_from_stats(p->hist, p->stats, m, nnz);
     const bool f64 = value_type == ASX_R_64F;
     const size_t sv = vsize(value_type);
-    int32_t *d_sample = reinterpret_cast<int32_t *>(p->d_counters + 64);  // 128 ints
     const auto add_slices = [&](double pairs) {
         return f64 ? plan_add_slices<double>(p, d_row_ptr, d_col, (const double *)d_val, pairs, s)
                    : plan_add_slices<float>(p, d_row_ptr, d_col, (const float *)d_val, pairs, s);
@@ -779,20 +806,18 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
         return f64 ? plan_add_window<double>(p, d_row_ptr, d_col, (const double *)d_val, checked, s)
                    : plan_add_window<float>(p, d_row_ptr, d_col, (const float *)d_val, checked, s);
     };
-    const bool can_regroup = alg == ASX_SPMV_DEFAULT && d_col && d_val && m > 0 && n > 0 && nnz >= kSlicedMinNnz &&
-                             regrouped_copy_fits(p, sv);
+    const bool can_regroup = may_regroup && regrouped_copy_fits(p, sv, ps.free_bytes);
+    const ColumnSample &cs = ps.sample;
     bool done = false;
     if (alg == ASX_SPMV_WINDOW) {
         st = add_window();
         done = true;
     } else if (alg == ASX_SPMV_SLICED) {
-        const ColumnSample cs = sample_columns(d_row_ptr, m, d_col, nnz, sv, d_sample, s);  // sizes the row blocks of pass 2
-        st = add_slices(cs.pairs);
+        st = add_slices(cs.pairs);  // the sample sizes the row blocks of pass 2
         done = true;
     } else if (can_regroup) {
         // DEFAULT: a regrouped copy where it is estimated to pay; a build that fails (out of memory,
         // a matrix the kernel does not take) is not an error: the next choice stands
-        const ColumnSample cs = sample_columns(d_row_ptr, m, d_col, nnz, sv, d_sample, s);
         if (cs.ok) {
             // the row-block kernel needs columns near each other; whether they fit its windows the
             // build finds out (NOT_SUPPORTED when some 256 rows reach further)

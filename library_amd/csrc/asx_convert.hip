@@ -114,13 +114,7 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_count(const int32_t 
         const int64_t i = first + k * kSortThreads + threadIdx.x;
         if (i < nnz) atomicAdd(&hist[(col[i] - base) >> shift], 1);  // integer counts: the order does not matter
     }
-    // the row holding every 512th element (and m behind the last): one lane each, while the others count
-    if (threadIdx.x < kSortWaves) {
-        const int64_t e = first + (int64_t)threadIdx.x * kSortWaveElems;
-        const int64_t g = (int64_t)blockIdx.x * kSortWaves + threadIdx.x;
-        seg_row[g] = e < nnz ? row_holding(row_ptr, 0, m - 1, (int32_t)e + base) : m - 1;
-        if (blockIdx.x == gridDim.x - 1 && threadIdx.x == kSortWaves - 1) seg_row[g + 1] = m - 1;
-    }
+    block_seg_rows(row_ptr, m, nnz, base, seg_row);
     __syncthreads();
     for (int s = threadIdx.x; s < nbuckets; s += kSortThreads) counts[(int64_t)s * nblocks + blockIdx.x] = hist[s];
     if (blockIdx.x == 0 && threadIdx.x == 0) counts[(int64_t)nbuckets * nblocks] = 0;
@@ -157,7 +151,10 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_bucket(const int32_t
         v[k] = val[at];
     }
     const int64_t g = (int64_t)b * kSortWaves + wave;
-    const int32_t r_lo = seg_row[g], r_hi = seg_row[g + 1];
+    const int32_t r_lo = __builtin_amdgcn_readfirstlane(seg_row[g]), r_hi = __builtin_amdgcn_readfirstlane(seg_row[g + 1]);
+    int32_t *row_s = reinterpret_cast<int32_t *>(stage);
+    int32_t r[kSortPerLane];
+    wave_rows(row_ptr, base, r_lo, r_hi, wbase, nnz, row_s + wave * kSortWaveElems, r);
     __syncthreads();
     uint16_t *mycnt = cnt + wave * nbuckets;
 #pragma unroll
@@ -177,7 +174,6 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_bucket(const int32_t
     __syncthreads();
     block_exclusive_sum(lofs, nbuckets, wave_tot);
     for (int s = tid; s < nbuckets; s += kSortThreads) to[s] -= lofs[s];
-    int32_t *row_s = reinterpret_cast<int32_t *>(stage);
 #pragma unroll
     for (int k = 0; k < kSortPerLane; ++k) {
         const int64_t i = wbase + k * kWave + lane;
@@ -185,7 +181,7 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_bucket(const int32_t
             const int32_t s = c[k] >> shift;
             p[k] += lofs[s] + mycnt[s];
             col_s[p[k]] = c[k];
-            row_s[p[k]] = row_holding(row_ptr, r_lo, r_hi, (int32_t)i + base);
+            row_s[p[k]] = r[k];
         }
     }
     __syncthreads();
@@ -321,14 +317,15 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_rows(const int32_t *
     }
 }
 
-// Columns of a bucket, as a power of two: buckets of about kSortElems elements, fewer where that leaves too few
-// workgroups, more where kBuckets of them are not enough.  -1: the sort by keys takes the matrix, because a bucket would
+// Columns of a bucket, as a power of two: buckets of up to two turns of kSortElems elements (a run of 8 elements per
+// block and bucket in pass 2; 3.6 M elements: 33 us there against 40 with buckets of one turn), fewer where that
+// leaves less than a workgroup per compute unit, more where kBuckets of them are not enough.  -1: the sort by keys takes the matrix, because a bucket would
 // span more than kBucketColumns columns or few columns hold so much that their buckets' workgroups would work in turn
 // (one workgroup takes about 2 us per 4096 elements).
 int bucket_shift(int32_t n, int32_t nnz)
 {
     if (nnz > 0x7fff0000) return -1;  // element numbers past the last one have to fit as well
-    const double per_bucket = std::min<double>(3700.0, std::max<double>(1024.0, nnz / 512.0));
+    const double per_bucket = std::min<double>(7600.0, std::max<double>(1024.0, nnz / 256.0));
     int shift = 0;
     while ((1 << (shift + 1)) <= kBucketColumns && (double)nnz / (double)ceil_div64(n, (int64_t)1 << (shift + 1)) <= per_bucket) ++shift;
     while (ceil_div64(n, (int64_t)1 << shift) > kBuckets) ++shift;

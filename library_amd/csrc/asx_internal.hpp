@@ -62,6 +62,10 @@ int launch_checksum(const void *d_data, size_t bytes, unsigned long long *d_part
 int launch_checksum_commit(const unsigned long long *d_now, unsigned long long *d_kept, hipStream_t s);
 int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const int32_t *d_row_ptr, int32_t m,
                           int32_t width, int32_t samples, int32_t *d_out, hipStream_t s);
+// the counters set to zero, then launch_row_histogram and launch_sample_columns in one launch (samples = 0: no sample)
+int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int64_t *d_hist, int64_t *d_stats,
+                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample,
+                      hipStream_t s);
 int launch_gather_lines(const void *d_buf, size_t bytes, int group_lanes, int per_lane, void *d_out, int *nthreads,
                         hipStream_t s);
 
@@ -156,7 +160,7 @@ struct SlicedMatrix {
     uint16_t *pos;          // nnz: position of each stored element among its block's elements in slice order
     int32_t *block_base;    // (nsort_blocks + 1) x nslices: slot of a block's first element of each slice (last row: the slices' ends)
     int32_t *wg_pieces;     // nwg x 8: first piece, end piece of each workgroup, 0, 0, then the first piece's four
-                            // words again (behind wg_tab in the store)
+                            // words again
     uint16_t *prow;         // npartials + kSlicedReducePad: row of each partial sum inside its row block
     int32_t *chunk_lo;      // (nrb + 1) x nslices: first partial sum of row block b in slice s
     int32_t npsteps;        // steps of pass 2, all row blocks

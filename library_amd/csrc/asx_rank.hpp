@@ -50,6 +50,82 @@ __device__ __forceinline__ int32_t row_holding(const int32_t *__restrict__ row_p
     return lo;
 }
 
+// The same for one i, by the whole wave: 64 probes at a time, so that a million rows take four
+// dependent reads instead of twenty (every lane gets the answer; lo, hi, i uniform).
+__device__ __forceinline__ int32_t wave_row_holding(const int32_t *__restrict__ row_ptr, int32_t lo, int32_t hi, int32_t i)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    while (lo < hi) {
+        const int32_t step = (hi - lo + kWave - 1) / kWave;
+        const int64_t p = lo + (int64_t)(lane + 1) * step;
+        const int n = __popcll(__ballot(p <= hi && row_ptr[p <= hi ? p : hi] <= i));
+        lo += n * step;
+        hi = hi - lo < step - 1 ? hi : lo + step - 1;
+    }
+    return lo;
+}
+
+// seg_row[g] = the row holding stored element g * kSortWaveElems (m - 1 behind the last element), written by the workgroup
+// of block blockIdx.x for its kSortWaves segments, one a wave, and the last workgroup's for the end of the array.
+__device__ __forceinline__ void block_seg_rows(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nnz, int32_t base,
+                                               int32_t *__restrict__ seg_row)
+{
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), lane = threadIdx.x & (kWave - 1);
+    const int64_t g = (int64_t)blockIdx.x * kSortWaves + wave, e = g * kSortWaveElems;
+    const int32_t r = e < nnz ? wave_row_holding(row_ptr, 0, m - 1, (int32_t)e + base) : m - 1;
+    if (lane == 0) seg_row[g] = r;
+    if (blockIdx.x == gridDim.x - 1 && threadIdx.x == 0) seg_row[(int64_t)gridDim.x * kSortWaves] = m - 1;
+}
+
+// Rows of the wave's kSortWaveElems consecutive elements from wbase on: rr[k] = row of element
+// wbase + k * 64 + lane, all of them in rows r_lo .. r_hi (uniform; r_lo holds element wbase).  The starts
+// of the rows are marked in `mark` (kSortWaveElems ints of LDS, the wave's own) and a running maximum
+// spreads them: one read of row_ptr per row instead of a binary search per element.  A long run of
+// empty rows falls back to the search.
+__device__ __forceinline__ void wave_rows(const int32_t *__restrict__ row_ptr, int32_t base, int32_t r_lo, int32_t r_hi,
+                                          int64_t wbase, int64_t nnz, int32_t *mark, int32_t (&rr)[kSortPerLane])
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    if (r_hi - r_lo > 8 * kSortWaveElems) {  // uniform
+#pragma unroll
+        for (int k = 0; k < kSortPerLane; ++k) {
+            const int64_t i = wbase + k * kWave + lane;
+            rr[k] = row_holding(row_ptr, r_lo, r_hi, (int32_t)(i < nnz ? i : nnz - 1) + base);
+        }
+        return;
+    }
+#pragma unroll
+    for (int k = 0; k < kSortPerLane; ++k) mark[k * kWave + lane] = 0;
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    for (int32_t r = r_lo + 1 + lane; r <= r_hi; r += kWave) {
+        const int64_t at = (int64_t)row_ptr[r] - base - wbase;
+        if (at >= 0 && at < kSortWaveElems) atomicMax(&mark[at], r - r_lo);  // of rows that start alike the last one holds the element
+    }
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    int32_t before = 0;
+#pragma unroll
+    for (int k = 0; k < kSortPerLane; ++k) {
+        int32_t v = mark[k * kWave + lane];
+#define ASX_MAX_STEP(CTRL, ROW_MASK)                     \
+    {                                                    \
+        const int32_t u = dpp0_i32<CTRL, ROW_MASK>(v);   \
+        v = v > u ? v : u;                               \
+    }
+        ASX_MAX_STEP(0x111, 0xF)  // row_shr:1
+        ASX_MAX_STEP(0x112, 0xF)  // row_shr:2
+        ASX_MAX_STEP(0x114, 0xF)  // row_shr:4
+        ASX_MAX_STEP(0x118, 0xF)  // row_shr:8
+        ASX_MAX_STEP(0x142, 0xA)  // row_bcast15 into rows 1 and 3
+        ASX_MAX_STEP(0x143, 0xC)  // row_bcast31 into rows 2 and 3
+#undef ASX_MAX_STEP
+        v = v > before ? v : before;
+        rr[k] = r_lo + v;
+        before = __builtin_amdgcn_readlane(v, kWave - 1);
+    }
+}
+
 // in-place exclusive sum of a[0 .. n), n <= 2 * kSortThreads, by the whole workgroup (barriers inside)
 __device__ __forceinline__ void block_exclusive_sum(int32_t *a, int n, int32_t *wave_tot)
 {

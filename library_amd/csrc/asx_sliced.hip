@@ -25,7 +25,6 @@
 // No global atomics; results are bit-reproducible.  The reference has no counterpart (its CSR
 // kernels gather x from global memory: hip/kernel/level2/alphasparse_spmv_csr_vector.h:99-126).
 #include <algorithm>
-#include <vector>
 
 #include "asx_internal.hpp"
 #include "asx_rank.hpp"
@@ -37,6 +36,7 @@ namespace asx {
 namespace {
 
 constexpr int32_t kPadRow = 0x7fffffff;
+static_assert(kSlicedReducePad == kBlock, "k_sliced_emit writes one pad entry a thread");
 
 // ---- plan build ---------------------------------------------------------------------------
 // The regrouping is a stable counting sort by slice, written for this purpose: the stored
@@ -45,9 +45,10 @@ constexpr int32_t kPadRow = 0x7fffffff;
 // every slice; a second kernel ranks the elements of a block inside their slices (stable: row
 // order, then column order, survives inside a slice), orders them by slice in LDS and writes
 // column, value, source index and row of each straight to its slot, in runs of consecutive slots.
-__global__ __launch_bounds__(kSortThreads) void k_sliced_count(const int32_t *__restrict__ col, int32_t nnz,
+__global__ __launch_bounds__(kSortThreads) void k_sliced_count(const int32_t *__restrict__ row_ptr, int32_t m,
+                                                                const int32_t *__restrict__ col, int32_t nnz,
                                                                 int32_t width, int32_t nslices, int32_t nblocks,
-                                                                int32_t *__restrict__ counts)
+                                                                int32_t *__restrict__ counts, int32_t *__restrict__ seg_row)
 {
     __shared__ int32_t hist[kSlicedMaxSlices];
     for (int s = threadIdx.x; s < nslices; s += kSortThreads) hist[s] = 0;
@@ -58,17 +59,126 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_count(const int32_t *__
         const int64_t i = base + k * kSortThreads + threadIdx.x;
         if (i < nnz) atomicAdd(&hist[col[i] / width], 1);  // integer counts: the order does not matter
     }
+    block_seg_rows(row_ptr, m, nnz, 0, seg_row);
     __syncthreads();
     for (int s = threadIdx.x; s < nslices; s += kSortThreads) counts[(int64_t)s * nblocks + blockIdx.x] = hist[s];
     if (blockIdx.x == 0 && threadIdx.x == 0) counts[(int64_t)nslices * nblocks] = 0;
 }
 
-// pstart[s] = stored elements in slices before s (s = nslices: all of them)
-__global__ __launch_bounds__(kBlock) void k_sliced_slice_starts(const int32_t *__restrict__ offs, int32_t nslices,
-                                                                 int32_t nblocks, int32_t *__restrict__ pstart)
+// exclusive sum of one value per thread over a workgroup of kLayoutThreads; *total: of all (barriers inside)
+constexpr int kLayoutThreads = 1024;
+__device__ __forceinline__ int32_t layout_exclusive(int32_t v, int32_t *wave_tot, int32_t *total)
 {
-    const int32_t s = (int32_t)(blockIdx.x * blockDim.x + threadIdx.x);
-    if (s <= nslices) pstart[s] = offs[(int64_t)s * nblocks];
+    const int lane = threadIdx.x & (kWave - 1), wave = threadIdx.x / kWave;
+    int32_t incl = v;
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) {
+        const int32_t t = __shfl_up(incl, d, kWave);
+        if (lane >= d) incl += t;
+    }
+    __syncthreads();
+    if (lane == kWave - 1) wave_tot[wave] = incl;
+    __syncthreads();
+    int32_t before = 0, all = 0;
+    for (int w = 0; w < kLayoutThreads / kWave; ++w) {
+        before += w < wave ? wave_tot[w] : 0;
+        all += wave_tot[w];
+    }
+    *total = all;
+    return before + incl - v;
+}
+
+// The tables that follow from the slices' sizes, by one workgroup (on the host they cost a round trip in the middle of
+// the build).  pstart[s] = stored elements in slices before s, tile_off[s] = tiles before it: every slice starts a new
+// tile.  Workgroups of pass 1: about `target` equal shares of the tiles, whatever slices they lie in (a share per slice,
+// rounded, left 270 workgroups for 256 compute units where 54 slices wanted 4.7 each: two rounds).  A cut that falls
+// within 32 tiles of the start of a slice moves there; a share that still reaches over such a start is worked off as
+// several pieces, one slice of x after the other.  No share smaller than 32 tiles unless there is only one.
+// Workgroups next to each other share slices of x: they go to one XCD, whose L2 then fetches a slice once
+// (workgroup i runs on XCD i mod kXcds; share j goes to position (j mod per_xcd) * kXcds + j / per_xcd).
+// info: tiles, workgroups, pieces, whether a slice is empty.
+__global__ __launch_bounds__(kLayoutThreads) void k_sliced_layout(const int32_t *__restrict__ offs, int32_t nslices,
+                                                                  int32_t nblocks, int32_t target, int32_t *__restrict__ pstart,
+                                                                  int32_t *__restrict__ tile_off, int4 *__restrict__ tab,
+                                                                  int4 *__restrict__ wgs, int32_t *__restrict__ info)
+{
+    __shared__ int32_t toff[kLayoutThreads + 1], cuts[kLayoutThreads + 1], wave_tot[kLayoutThreads / kWave];
+    const int tid = threadIdx.x;
+    const int32_t from = tid <= nslices ? offs[(int64_t)tid * nblocks] : 0;
+    const int32_t cnt = tid < nslices ? offs[(int64_t)(tid + 1) * nblocks] - from : 0;
+    if (tid < nslices) pstart[tid] = from;
+    if (tid == nslices - 1) pstart[nslices] = from + cnt;
+    int32_t nt;
+    const int32_t before = layout_exclusive((cnt + kSlicedTile - 1) / kSlicedTile, wave_tot, &nt);
+    if (tid < nslices) toff[tid] = tile_off[tid] = before;
+    if (tid == 0) toff[nslices] = tile_off[nslices] = nt;
+    const int empty = __syncthreads_or(tid < nslices && cnt == 0);
+    const int32_t most = nt / 32 < target ? nt / 32 : target;
+    const int32_t shares = most < 1 ? 1 : most < kLayoutThreads ? most : kLayoutThreads;
+    if (tid < shares) {
+        int32_t c = (int32_t)((int64_t)nt * tid / shares);
+        int32_t lo = 0, hi = nslices;  // first slice start at or behind c (the last entry is nt >= c)
+        while (lo < hi) {
+            const int32_t mid = (lo + hi) / 2;
+            if (toff[mid] < c)
+                lo = mid + 1;
+            else
+                hi = mid;
+        }
+        const int32_t above = toff[lo] - c, below = lo > 0 ? c - toff[lo - 1] : 32;
+        if (above < 32 && above <= below)
+            c += above;
+        else if (below < 32)
+            c -= below;
+        cuts[tid] = tid == 0 ? 0 : c;
+    }
+    if (tid == 0) cuts[shares] = nt;
+    for (int d = 1; d < shares; d <<= 1) {  // no cut before the one in front of it
+        __syncthreads();
+        const int32_t v = tid >= d && tid < shares ? cuts[tid - d] : 0;
+        __syncthreads();
+        if (tid >= d && tid < shares && v > cuts[tid]) cuts[tid] = v;
+    }
+    __syncthreads();
+    const int32_t lo = tid < shares ? cuts[tid] : 0, hi = tid < shares ? cuts[tid + 1] : 0;
+    int32_t first = 0, pieces = 0;  // slice that holds tile lo; slices with tiles in lo .. hi - 1
+    if (hi > lo) {
+        int32_t a = 0, z = nslices - 1;  // largest s with toff[s] <= lo
+        while (a < z) {
+            const int32_t mid = a + (z - a + 1) / 2;
+            if (toff[mid] <= lo)
+                a = mid;
+            else
+                z = mid - 1;
+        }
+        first = a;
+        for (int32_t s = first; s < nslices && toff[s] < hi; ++s) pieces += toff[s + 1] > toff[s];
+    }
+    int32_t nwg, npieces;
+    const int32_t j = layout_exclusive(hi > lo ? 1 : 0, wave_tot, &nwg);
+    int32_t at = layout_exclusive(pieces, wave_tot, &npieces);
+    if (hi > lo) {
+        const int32_t per_xcd = nwg / kXcds;
+        const int32_t i = nwg % kXcds == 0 ? (j % per_xcd) * kXcds + j / per_xcd : j;
+        wgs[2 * i] = make_int4(at, at + pieces, 0, 0);
+        bool is_first = true;
+        for (int32_t s = first; s < nslices && toff[s] < hi; ++s) {
+            if (toff[s + 1] == toff[s]) continue;
+            const int4 piece = make_int4(s, lo > toff[s] ? lo : toff[s], hi < toff[s + 1] ? hi : toff[s + 1], 0);
+            tab[at++] = piece;
+            if (is_first) wgs[2 * i + 1] = piece;  // the first piece again
+            is_first = false;
+        }
+    }
+    if (tid == 0) info[0] = nt, info[1] = nwg, info[2] = npieces, info[3] = empty;
+}
+
+// what the host reads after it has waited: info and the number of partial sums, into page-locked memory
+__global__ __launch_bounds__(kWave) void k_sliced_publish(const int32_t *__restrict__ info, const int32_t *__restrict__ last,
+                                                          int32_t *__restrict__ host)
+{
+    if (threadIdx.x < 4) host[threadIdx.x] = info[threadIdx.x];
+    if (threadIdx.x == 4) host[4] = *last;
 }
 
 template <typename T>
@@ -87,11 +197,12 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_scatter(
     uint16_t *__restrict__ cf, T *__restrict__ val_out, int32_t *__restrict__ perm, uint16_t *__restrict__ pos,
     int32_t *__restrict__ block_base)
 {
-    __shared__ int32_t cnt[kSortWaves * MAXS];  // per wave and slice: count, then first rank of the wave's elements
-    __shared__ int32_t lofs[MAXS];              // per slice: the block's count, then its first position in slice order
-    __shared__ int32_t gbase[MAXS];             // per slice: slot of the block's first element of the slice
+    // 54 KB for up to 256 slices: three workgroups a compute unit
+    __shared__ uint16_t cnt[kSortWaves * MAXS];  // per wave and slice: count, then first rank of the wave's elements
+    __shared__ int32_t lofs[MAXS];               // per slice: the block's count, then its first position in slice order
+    __shared__ int32_t to[MAXS];                 // per slice: slot of the block's first element of the slice, minus lofs
     __shared__ int32_t wave_tot[kSortWaves];
-    __shared__ int32_t dest[kSortElems];        // slot of the element at each position of the block in slice order
+    __shared__ uint16_t slice_s[kSortElems];     // slice of the element at each position of the block in slice order
     __shared__ __align__(16) unsigned char stage_raw[kSortElems * 10];
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     // consecutive blocks write neighbouring slots of every slice: keep them on one XCD, whose L2
@@ -101,13 +212,26 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_scatter(
     if (b >= nblocks) return;  // the whole workgroup leaves
     for (int i = tid; i < kSortWaves * nslices; i += kSortThreads) cnt[i] = 0;
     __syncthreads();
-    int32_t *mycnt = cnt + wave * nslices;
+    uint16_t *mycnt = cnt + wave * nslices;
     const int64_t wbase = (int64_t)b * kSortElems + (int64_t)wave * kSortWaveElems;
     int32_t c[kSortPerLane], rk[kSortPerLane];
 #pragma unroll
     for (int k = 0; k < kSortPerLane; ++k) {
         const int64_t i = wbase + k * kWave + lane;
         c[k] = i < nnz ? col[i] : 0;
+    }
+    // rows: the wave's 512 elements lie in rows seg_row[g] .. seg_row[g + 1]
+    int32_t *row_s = reinterpret_cast<int32_t *>(stage_raw), *src_s = row_s + kSortElems;
+    int32_t r[kSortPerLane];
+    {
+        const int64_t g = wbase / kSortWaveElems;
+        int32_t r_lo = m - 1, r_hi = m - 1;
+        if (wbase < nnz) {
+            r_lo = __builtin_amdgcn_readfirstlane(seg_row[g]);
+            r_hi = __builtin_amdgcn_readfirstlane(seg_row[g + 1]);
+            r_hi = r_hi > m - 1 ? m - 1 : r_hi;
+        }
+        wave_rows(row_ptr, 0, r_lo, r_hi, wbase, nnz, row_s + wave * kSortWaveElems, r);
     }
     // rank of every element among the wave's elements of its slice, in element order
 #pragma unroll
@@ -119,39 +243,30 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_scatter(
 #pragma unroll
         for (int w = 0; w < kSortWaves; ++w) {
             const int32_t t = cnt[w * nslices + s];
-            cnt[w * nslices + s] = run;
+            cnt[w * nslices + s] = (uint16_t)run;
             run += t;
         }
         lofs[s] = run;
-        gbase[s] = tile_off[s] * kSlicedTile + offs[(int64_t)s * nblocks + b] - offs[(int64_t)s * nblocks];
+        to[s] = tile_off[s] * kSlicedTile + offs[(int64_t)s * nblocks + b] - offs[(int64_t)s * nblocks];
         // for k_sliced_rescatter: where the block's elements of every slice start (row nblocks: where the slice's end)
-        block_base[(int64_t)b * nslices + s] = gbase[s];
+        block_base[(int64_t)b * nslices + s] = to[s];
         if (b == nblocks - 1)
             block_base[(int64_t)nblocks * nslices + s] =
                 tile_off[s] * kSlicedTile + offs[(int64_t)s * nblocks + nblocks] - offs[(int64_t)s * nblocks];
     }
     __syncthreads();
     block_exclusive_sum(lofs, nslices, wave_tot);
-    // rows: the wave's 512 elements lie in rows seg_row[g] .. seg_row[g + 1]
-    const int64_t g = wbase / kSortWaveElems;
-    int32_t r_lo = 0, r_hi = m - 1;
-    if (wbase < nnz) {
-        r_lo = seg_row[g];
-        r_hi = seg_row[g + 1];
-        r_hi = r_hi > m - 1 ? m - 1 : r_hi;
-    }
-    int32_t *row_s = reinterpret_cast<int32_t *>(stage_raw), *src_s = row_s + kSortElems;
+    for (int s = tid; s < nslices; s += kSortThreads) to[s] -= lofs[s];
 #pragma unroll
     for (int k = 0; k < kSortPerLane; ++k) {
         const int64_t i = wbase + k * kWave + lane;
         if (i < nnz) {
             const int32_t key = c[k] / width;
-            const int32_t in_slice = mycnt[key] + rk[k];
-            const int32_t p = lofs[key] + in_slice;
+            const int32_t p = lofs[key] + mycnt[key] + rk[k];
             rk[k] = p;
             pos[i] = (uint16_t)p;
-            dest[p] = gbase[key] + in_slice;
-            row_s[p] = row_holding(row_ptr, r_lo, r_hi, (int32_t)i);
+            slice_s[p] = (uint16_t)key;
+            row_s[p] = r[k];
             src_s[p] = (int32_t)i;
         }
     }
@@ -159,7 +274,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_scatter(
     const int64_t left = (int64_t)nnz - (int64_t)b * kSortElems;
     const int32_t count = left < kSortElems ? (int32_t)left : kSortElems;
     for (int j = tid; j < count; j += kSortThreads) {
-        const int64_t d = dest[j];
+        const int64_t d = to[slice_s[j]] + j;
         lrow[d] = row_s[j];
         perm[slot_val_pos<T>(d)] = src_s[j];
     }
@@ -181,7 +296,7 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_scatter(
     }
     __syncthreads();
     for (int j = tid; j < count; j += kSortThreads) {
-        const int64_t d = dest[j];
+        const int64_t d = to[slice_s[j]] + j;
         val_out[slot_val_pos<T>(d)] = val_s[j];
         cf[d] = cf_s[j];
     }
@@ -225,16 +340,19 @@ struct TileRuns {
     }
 };
 
-__global__ __launch_bounds__(kBlock) void k_sliced_tile_runs(const int32_t *__restrict__ lrow, int32_t ntiles,
-                                                              int32_t *__restrict__ tile_cnt)
+__global__ __launch_bounds__(kBlock) void k_sliced_tile_runs(const int32_t *__restrict__ lrow, const int32_t *__restrict__ info,
+                                                              int32_t max_tiles, int32_t *__restrict__ tile_cnt)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    if (t >= ntiles) return;  // whole waves leave
+    if (t > max_tiles) return;  // whole waves leave
+    if (t >= info[0]) {         // behind the last tile: nothing to count
+        if (lane == 0) tile_cnt[t] = 0;
+        return;
+    }
     TileRuns tr;
     tr.load(lrow, t, lane);
     if (lane == 0) tile_cnt[t] = tr.total;
-    if (t == 0 && lane == 0) tile_cnt[ntiles] = 0;
 }
 
 // Per run: its row inside the row block (prow); per slot: the run-start bit of cf; per (row
@@ -246,20 +364,13 @@ __global__ __launch_bounds__(kBlock) void k_sliced_emit(const int32_t *__restric
                                                          const int32_t *__restrict__ tile_off, int32_t ntiles,
                                                          int32_t nslices, int32_t rpw, int32_t nrb,
                                                          uint16_t *__restrict__ cf, uint16_t *__restrict__ prow,
-                                                         int32_t *__restrict__ chunk_lo)
+                                                         int32_t *__restrict__ chunk_lo, int32_t npartials)
 {
+    if (blockIdx.x == 0) prow[npartials + threadIdx.x] = 0;  // kSlicedReducePad readable entries behind the last one
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t t = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
     if (t >= ntiles) return;  // whole waves leave
-    int32_t lo = 0, hi = nslices - 1;  // slice of tile t: largest s with tile_off[s] <= t (uniform)
-    while (lo < hi) {
-        const int32_t mid = lo + (hi - lo + 1) / 2;
-        if (tile_off[mid] <= t)
-            lo = mid;
-        else
-            hi = mid - 1;
-    }
-    const int32_t s = lo;
+    const int32_t s = wave_row_holding(tile_off, 0, nslices - 1, (int32_t)t);  // slice of tile t: largest s with tile_off[s] <= t
     const bool first_tile = t == tile_off[s], last_tile = t + 1 == tile_off[s + 1];
     TileRuns tr;
     tr.load(lrow, t, lane);
@@ -452,16 +563,32 @@ constexpr int kPieces = 3;
 typedef int32_t i32x4 __attribute__((ext_vector_type(4)));
 
 // One wave per row block walks the block's ranges (loaded 64 slices at a time, then read lane by
-// lane: the walk itself is serial); `psteps == nullptr`: only count.
+// lane: the walk itself is serial) and leaves its steps at a place of its own in `raw`: a block with e
+// entries takes at most e / 64 + nslices / 3 + 1 steps (every other step that is cut short has used up
+// three ranges), so the steps of block b may start at (entries before it) / 64 + b (nslices / 3 + 2).
+// k_sliced_steps moves them together once their counts are summed up.
+__device__ __forceinline__ int64_t raw_steps_at(const int32_t *__restrict__ chunk_lo, int32_t nslices, int64_t b, int lane)
+{
+    int32_t before = 0;
+    for (int32_t s = lane; s < nslices; s += kWave) before += chunk_lo[b * nslices + s] - chunk_lo[s];
+#pragma unroll
+    for (int d = 1; d < kWave; d <<= 1) before += __shfl_xor(before, d, kWave);
+    return (int64_t)(before / kWave) + b * (nslices / 3 + 2);
+}
+inline int64_t raw_steps_most(int64_t npartials, int64_t nrb, int64_t nslices) { return npartials / kWave + nrb * (nslices / 3 + 2); }
+
 __global__ __launch_bounds__(kBlock) void k_sliced_pack(const int32_t *__restrict__ chunk_lo, int32_t nrb,
-                                                         int32_t nslices, const int32_t *__restrict__ pstep_ptr,
-                                                         int32_t *__restrict__ count, i32x4 *__restrict__ psteps)
+                                                         int32_t nslices, int32_t *__restrict__ count,
+                                                         i32x4 *__restrict__ raw)
 {
     const int lane = threadIdx.x & (kWave - 1);
     const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
-    if (b >= nrb) return;  // whole waves leave
+    if (b >= nrb) {  // whole waves leave
+        if (b == nrb && lane == 0) count[nrb] = 0;
+        return;
+    }
     const int32_t *lo_row = chunk_lo + b * nslices, *hi_row = lo_row + nslices;
-    i32x4 *out = psteps ? psteps + pstep_ptr[b] : nullptr;
+    i32x4 *out = raw + raw_steps_at(chunk_lo, nslices, b, lane);
     int32_t nsteps = 0, fill = 0, pieces = 0;
     int32_t base0 = 0, base1 = 0, base2 = 0, first1 = kWave, first2 = kWave;
     for (int32_t s0 = 0; s0 < nslices; s0 += kWave) {
@@ -475,7 +602,7 @@ __global__ __launch_bounds__(kBlock) void k_sliced_pack(const int32_t *__restric
             int32_t lo = __builtin_amdgcn_readlane(lo_v, j), len = __builtin_amdgcn_readlane(len_v, j);
             while (len > 0) {
                 if (pieces == kPieces || fill == kWave) {
-                    if (out && lane == 0) out[nsteps] = i32x4{base0, base1, base2, first1 | first2 << 8 | fill << 16};
+                    if (lane == 0) out[nsteps] = i32x4{base0, base1, base2, first1 | first2 << 8 | fill << 16};
                     ++nsteps;
                     fill = pieces = 0;
                     first1 = first2 = kWave;
@@ -495,12 +622,32 @@ __global__ __launch_bounds__(kBlock) void k_sliced_pack(const int32_t *__restric
         }
     }
     if (fill > 0) {
-        if (out && lane == 0) out[nsteps] = i32x4{base0, base1, base2, first1 | first2 << 8 | fill << 16};
+        if (lane == 0) out[nsteps] = i32x4{base0, base1, base2, first1 | first2 << 8 | fill << 16};
         ++nsteps;
     }
-    if (!psteps && lane == 0) count[b] = nsteps;
+    if (lane == 0) count[b] = nsteps;
 }
 
+// The steps of all row blocks one after the other, kSlicedStepPad empty ones behind the last; their number for the host.
+__global__ __launch_bounds__(kBlock) void k_sliced_steps(const int32_t *__restrict__ chunk_lo, int32_t nrb, int32_t nslices,
+                                                          const int32_t *__restrict__ pstep_ptr,
+                                                          const i32x4 *__restrict__ raw, i32x4 *__restrict__ psteps,
+                                                          int32_t *__restrict__ host)
+{
+    const int lane = threadIdx.x & (kWave - 1);
+    const int64_t b = ((int64_t)blockIdx.x * blockDim.x + threadIdx.x) / kWave;
+    if (b > nrb) return;  // whole waves leave
+    const int32_t s0 = pstep_ptr[b];
+    if (b == nrb) {
+        if (lane == 0) *host = s0;
+        psteps[(int64_t)s0 + lane] = i32x4{0, 0, 0, 0};
+        return;
+    }
+    const int32_t n = pstep_ptr[b + 1] - s0;
+    const i32x4 *from = raw + raw_steps_at(chunk_lo, nslices, b, lane);
+    for (int32_t i = lane; i < n; i += kWave) psteps[(int64_t)s0 + i] = from[i];
+}
+static_assert(kSlicedStepPad == kWave, "k_sliced_steps writes one empty step a lane");
 
 // U steps whose loads are issued together.
 template <typename T, int U>
@@ -649,25 +796,28 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
     int nbits = 0;
     while ((1 << nbits) < sm.nslices) ++nbits;
     const int32_t nblocks = (int32_t)ceil_div64(nnz, kSortElems);
-    const int32_t nseg = (int32_t)ceil_div64(nnz, kSortWaveElems);
     const int64_t ncount = (int64_t)sm.nslices * nblocks + 1;
     const int64_t cap64 = (int64_t)nnz + (int64_t)(kSlicedTile - 1) * sm.nslices;  // the most slots there can be
     const int64_t ncells = ((int64_t)sm.nrb + 1) * sm.nslices;
-    if (cap64 > 0x7fffffff || ncount > 0x7fffffff || ncells > 0x7fffffff) return ASX_STATUS_INVALID_SIZE;
+    if (cap64 > 0x7fffffff - kSlicedTile || ncount > 0x7fffffff || ncells > 0x7fffffff) return ASX_STATUS_INVALID_SIZE;
+    const int32_t max_tiles = (int32_t)ceil_div64(cap64, kSlicedTile);
+    const size_t max_slots = (size_t)max_tiles * kSlicedTile;
+    const size_t max_pieces = (size_t)std::min(target_wgs, kLayoutThreads) + (size_t)sm.nslices;
 
     int st = ASX_STATUS_SUCCESS;
+    // The build waits for the device twice: for the number of partial sums, which sizes what follows, and at its
+    // end.  Everything else is sized by what there can be at most (255 spare slots a slice).
+    Scratch scratch(s);
+    int32_t *host = static_cast<int32_t *>(scratch.pinned());
+    if (!host) return ASX_STATUS_ALLOC_FAILED;
     // Scratch of the build in one allocation: per-(slice, block) counts and their scan, the row
     // holding every 512th stored element, slice offsets (elements, tiles), the row of every slot,
     // per-tile and per-row-block counts, the scans' block sums.
     char *arena = nullptr;
     int32_t *counts = nullptr, *offs = nullptr, *seg_row = nullptr, *d_pstart = nullptr, *d_tile_off = nullptr;
     int32_t *lrow = nullptr, *tile_cnt = nullptr, *step_cnt = nullptr;
-    int32_t *tmp = nullptr;
-    std::vector<int32_t> pstart((size_t)sm.nslices + 1), tile_off((size_t)sm.nslices + 1, 0);
-    std::vector<int32_t> tab, wgs;
-    int64_t slots = 0;
-    bool empty_slice = false;
-    const size_t max_tiles = (size_t)ceil_div64(cap64, kSlicedTile);
+    int32_t *tmp = nullptr, *info = nullptr;
+    i32x4 *raw = nullptr;
 #define ASX_TRY(expr)         \
     do {                      \
         st = status_of(expr); \
@@ -685,90 +835,15 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
             off += align_up(count * sizeof(int32_t), 256);
             return at;
         };
-        const size_t o_counts = take((size_t)ncount), o_offs = take((size_t)ncount), o_seg = take((size_t)nseg + 1);
-        const size_t o_pstart = take((size_t)sm.nslices + 1), o_toff = take((size_t)sm.nslices + 1);
-        const size_t o_lrow = take((size_t)cap64), o_tcnt = take(max_tiles + 1), o_scnt = take((size_t)sm.nrb + 1);
-        const size_t o_tmp = take(scan_scratch_ints(std::max<int64_t>(ncount, (int64_t)max_tiles + 1)));
-        ASX_TRY(pool_malloc(&arena, off, true));
+        const size_t o_counts = take((size_t)ncount), o_offs = take((size_t)ncount), o_seg = take((size_t)nblocks * kSortWaves + 1);
+        const size_t o_pstart = take((size_t)sm.nslices + 1), o_toff = take((size_t)sm.nslices + 1), o_info = take(4);
+        const size_t o_lrow = take(max_slots), o_tcnt = take((size_t)max_tiles + 1), o_scnt = take((size_t)sm.nrb + 1);
+        const size_t o_tmp = take(scan_scratch_ints(std::max<int64_t>(ncount, std::max<int64_t>(max_tiles, sm.nrb) + 1)));
+        ASX_TRY(scratch.take(&arena, off));
         counts = (int32_t *)(arena + o_counts), offs = (int32_t *)(arena + o_offs), seg_row = (int32_t *)(arena + o_seg);
-        d_pstart = (int32_t *)(arena + o_pstart), d_tile_off = (int32_t *)(arena + o_toff);
+        d_pstart = (int32_t *)(arena + o_pstart), d_tile_off = (int32_t *)(arena + o_toff), info = (int32_t *)(arena + o_info);
         lrow = (int32_t *)(arena + o_lrow), tile_cnt = (int32_t *)(arena + o_tcnt), step_cnt = (int32_t *)(arena + o_scnt);
         tmp = (int32_t *)(arena + o_tmp);
-    }
-
-    // 1. every block's stored elements per slice, and from their scan the block's place in each slice
-    hipLaunchKernelGGL(k_sliced_count, dim3((unsigned)nblocks), dim3(kSortThreads), 0, s, col, nnz, width, sm.nslices,
-                       nblocks, counts);
-    ASX_TRY_ST(launch_exclusive_scan_i32(counts, offs, ncount, tmp, s));
-    hipLaunchKernelGGL(k_sliced_slice_starts, dim3((unsigned)ceil_div64((int64_t)sm.nslices + 1, kBlock)), dim3(kBlock), 0, s,
-                       offs, sm.nslices, nblocks, d_pstart);
-    ASX_TRY(hipMemcpyAsync(pstart.data(), d_pstart, sizeof(int32_t) * pstart.size(), hipMemcpyDeviceToHost, s));
-    ASX_TRY_ST(launch_nnz_split_rows(row_ptr, m, nnz, kSortWaveElems, seg_row, s));  // runs while the host waits
-    ASX_TRY(hipStreamSynchronize(s));
-
-    // 2. tiles: every slice starts a new tile
-    for (int32_t sl = 0; sl < sm.nslices; ++sl) {
-        tile_off[sl + 1] = tile_off[sl] + (int32_t)ceil_div64(pstart[sl + 1] - pstart[sl], kSlicedTile);
-        empty_slice |= pstart[sl + 1] == pstart[sl];
-    }
-    sm.ntiles = tile_off[sm.nslices];
-    slots = (int64_t)sm.ntiles * kSlicedTile;
-    ASX_TRY(hipMemcpyAsync(d_tile_off, tile_off.data(), sizeof(int32_t) * tile_off.size(), hipMemcpyHostToDevice, s));
-    //    workgroups of pass 1: about `target_wgs` equal shares of the tiles, whatever slices they lie
-    //    in (a share per slice, rounded, left 270 workgroups for 256 compute units where 54 slices
-    //    wanted 4.7 each: two rounds).  A cut that falls within 32 tiles of the start of a slice
-    //    moves there; a share that still reaches over such a start is worked off as two pieces,
-    //    one slice of x after the other.  No share smaller than 32 tiles unless there is only one.
-    {
-        const int64_t nt = sm.ntiles;
-        const int32_t shares = (int32_t)std::max<int64_t>(1, std::min<int64_t>(target_wgs, nt / 32));
-        std::vector<int32_t> cuts((size_t)shares + 1);
-        for (int32_t k = 0; k <= shares; ++k) {
-            int32_t c = (int32_t)(nt * k / shares);
-            // the start of a slice nearest to c, when fewer than 32 tiles away
-            const auto at = std::lower_bound(tile_off.begin(), tile_off.end(), c);
-            const int32_t above = at != tile_off.end() ? *at - c : 32, below = at != tile_off.begin() ? c - *(at - 1) : 32;
-            if (above < 32 && above <= below)
-                c += above;
-            else if (below < 32)
-                c -= below;
-            cuts[(size_t)k] = k == 0 ? 0 : k == shares ? (int32_t)nt : std::max(c, cuts[(size_t)k - 1]);
-        }
-        int32_t sl = 0;
-        for (int32_t k = 0; k < shares; ++k) {
-            const int32_t lo = cuts[(size_t)k], hi = cuts[(size_t)k + 1];
-            if (hi <= lo) continue;
-            const int32_t first_piece = (int32_t)(tab.size() / 4);
-            while (tile_off[(size_t)sl + 1] <= lo) ++sl;  // the slice that holds tile lo
-            for (int32_t a = lo; a < hi;) {
-                while (tile_off[(size_t)sl + 1] <= a) ++sl;
-                const int32_t z = std::min(hi, tile_off[(size_t)sl + 1]);
-                tab.push_back(sl);
-                tab.push_back(a);
-                tab.push_back(z);
-                tab.push_back(0);
-                a = z;
-            }
-            wgs.push_back(first_piece);
-            wgs.push_back((int32_t)(tab.size() / 4));
-            wgs.push_back(0);
-            wgs.push_back(0);
-            for (int q = 0; q < 4; ++q) wgs.push_back(tab[(size_t)first_piece * 4 + q]);  // the first piece again
-        }
-        sm.npieces = (int32_t)(tab.size() / 4);
-        sm.nwg = (int32_t)(wgs.size() / 8);
-        // Workgroups next to each other in this list share slices of x: keep them on one XCD, whose
-        // L2 then fetches a slice once (workgroup i runs on XCD i mod kXcds; entry j of the list goes
-        // to position (j mod per_xcd) * kXcds + j / per_xcd, so consecutive entries share an XCD).
-        if (sm.nwg % kXcds == 0 && sm.nwg > 0) {
-            const int32_t per_xcd = sm.nwg / kXcds;
-            std::vector<int32_t> placed(wgs.size());
-            for (int32_t j = 0; j < sm.nwg; ++j) {
-                const int32_t i = (j % per_xcd) * kXcds + j / per_xcd;
-                for (int q = 0; q < 8; ++q) placed[(size_t)i * 8 + q] = wgs[(size_t)j * 8 + q];
-            }
-            wgs.swap(placed);
-        }
     }
     {   // what the plan keeps and whose size is known by now, in one allocation
         size_t off = 0;
@@ -777,23 +852,28 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
             off += align_up(bytes, 256);
             return at;
         };
-        const size_t o_val = take(sizeof(T) * (size_t)slots), o_perm = take(sizeof(int32_t) * (size_t)slots);
-        const size_t o_cf = take(sizeof(uint16_t) * (size_t)slots), o_tb = take(sizeof(int32_t) * ((size_t)sm.ntiles + 1));
-        const size_t o_wg = take(sizeof(int32_t) * std::max<size_t>(tab.size() + wgs.size(), 4));
+        const size_t o_val = take(sizeof(T) * max_slots), o_perm = take(sizeof(int32_t) * max_slots);
+        const size_t o_cf = take(sizeof(uint16_t) * max_slots), o_tb = take(sizeof(int32_t) * ((size_t)max_tiles + 1));
+        const size_t o_wg = take(16 * max_pieces), o_wp = take(32 * max_pieces);
         const size_t o_cl = take(sizeof(int32_t) * (size_t)ncells), o_sp = take(sizeof(int32_t) * ((size_t)sm.nrb + 1));
         const size_t o_pos = take(sizeof(uint16_t) * (size_t)nnz);
         const size_t o_bb = take(sizeof(int32_t) * ((size_t)nblocks + 1) * (size_t)sm.nslices);
         ASX_TRY(pool_malloc(&sm.store, off, false));
         char *base = static_cast<char *>(sm.store);
         sm.val = base + o_val, sm.perm = (int32_t *)(base + o_perm), sm.cf = (uint16_t *)(base + o_cf);
-        sm.tile_base = (int32_t *)(base + o_tb), sm.wg_tab = (int32_t *)(base + o_wg);
+        sm.tile_base = (int32_t *)(base + o_tb), sm.wg_tab = (int32_t *)(base + o_wg), sm.wg_pieces = (int32_t *)(base + o_wp);
         sm.chunk_lo = (int32_t *)(base + o_cl), sm.pstep_ptr = (int32_t *)(base + o_sp);
-        sm.wg_pieces = sm.wg_tab + tab.size();
         sm.pos = (uint16_t *)(base + o_pos), sm.block_base = (int32_t *)(base + o_bb);
         sm.nnz = nnz, sm.nsort_blocks = nblocks;
-        ASX_TRY(hipMemcpyAsync(sm.wg_tab, tab.data(), sizeof(int32_t) * tab.size(), hipMemcpyHostToDevice, s));
-        ASX_TRY(hipMemcpyAsync(sm.wg_pieces, wgs.data(), sizeof(int32_t) * wgs.size(), hipMemcpyHostToDevice, s));
     }
+
+    // 1. every block's stored elements per slice, and from their scan the block's place in each slice
+    hipLaunchKernelGGL(k_sliced_count, dim3((unsigned)nblocks), dim3(kSortThreads), 0, s, row_ptr, m, col, nnz, width, sm.nslices,
+                       nblocks, counts, seg_row);
+    ASX_TRY_ST(launch_exclusive_scan_i32(counts, offs, ncount, tmp, s));
+    // 2. tiles, and the workgroups of pass 1
+    hipLaunchKernelGGL(k_sliced_layout, dim3(1), dim3(kLayoutThreads), 0, s, offs, sm.nslices, nblocks, target_wgs, d_pstart,
+                       d_tile_off, reinterpret_cast<int4 *>(sm.wg_tab), reinterpret_cast<int4 *>(sm.wg_pieces), info);
     // 3. every stored element to its slot; the pads behind every slice
     {
         const unsigned sgrid = (unsigned)(ceil_div64(nblocks, kXcds) * kXcds);
@@ -810,47 +890,50 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
                            sm.cf, (T *)sm.val, sm.perm);
     }
     // 4. partial sums: one per run start; tile_base = the run starts before each tile
+    hipLaunchKernelGGL(k_sliced_tile_runs, dim3((unsigned)ceil_div64(((int64_t)max_tiles + 1) * kWave, kBlock)), dim3(kBlock), 0, s,
+                       lrow, info, max_tiles, tile_cnt);
+    ASX_TRY_ST(launch_exclusive_scan_i32(tile_cnt, sm.tile_base, (int64_t)max_tiles + 1, tmp, s));
+    hipLaunchKernelGGL(k_sliced_publish, dim3(1), dim3(kWave), 0, s, info, sm.tile_base + max_tiles, host);
+    ASX_TRY(hipGetLastError());
+    ASX_TRY(hipStreamSynchronize(s));
+    sm.ntiles = host[0], sm.nwg = host[1], sm.npieces = host[2], sm.npartials = host[4];
     {
-        const unsigned wgrid = (unsigned)ceil_div64((int64_t)sm.ntiles * kWave, kBlock);
-        hipLaunchKernelGGL(k_sliced_tile_runs, dim3(wgrid), dim3(kBlock), 0, s, lrow, sm.ntiles, tile_cnt);
-        ASX_TRY_ST(launch_exclusive_scan_i32(tile_cnt, sm.tile_base, (int64_t)sm.ntiles + 1, tmp, s));
-        ASX_TRY(hipMemcpyAsync(&sm.npartials, sm.tile_base + sm.ntiles, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        ASX_TRY(hipStreamSynchronize(s));
+        const int64_t most_steps = raw_steps_most(sm.npartials, sm.nrb, sm.nslices);
+        if (most_steps > 0x7fffffff - kSlicedStepPad) {
+            st = ASX_STATUS_INVALID_SIZE;
+            goto done;
+        }
+        ASX_TRY(scratch.take(&raw, sizeof(i32x4) * (size_t)most_steps));
         ASX_TRY(pool_malloc(&sm.prow, sizeof(uint16_t) * ((size_t)sm.npartials + kSlicedReducePad), false));
-        ASX_TRY(hipMemsetAsync(sm.prow + sm.npartials, 0, sizeof(uint16_t) * kSlicedReducePad, s));
         // 5. rows of the partial sums, run-start bits, and where each row block starts inside each slice
-        hipLaunchKernelGGL(k_sliced_emit, dim3(wgrid), dim3(kBlock), 0, s, lrow, sm.tile_base, d_tile_off, sm.ntiles,
-                           sm.nslices, rows_per_wave, sm.nrb, sm.cf, sm.prow, sm.chunk_lo);
-        if (empty_slice)
+        hipLaunchKernelGGL(k_sliced_emit, dim3((unsigned)ceil_div64((int64_t)sm.ntiles * kWave, kBlock)), dim3(kBlock), 0, s, lrow,
+                           sm.tile_base, d_tile_off, sm.ntiles, sm.nslices, rows_per_wave, sm.nrb, sm.cf, sm.prow, sm.chunk_lo,
+                           sm.npartials);
+        if (host[3])
             hipLaunchKernelGGL(k_sliced_empty_slices, dim3((unsigned)ceil_div64(ncells, kBlock)), dim3(kBlock), 0, s,
                                sm.tile_base, d_tile_off, sm.nslices, sm.nrb, sm.chunk_lo);
-    }
-    // 6. the steps in which pass 2 reads each row block's ranges
-    {
-        const unsigned pgrid = (unsigned)ceil_div64((int64_t)sm.nrb * kWave, kBlock);
-        ASX_TRY(hipMemsetAsync(step_cnt + sm.nrb, 0, sizeof(int32_t), s));
-        hipLaunchKernelGGL(k_sliced_pack, dim3(pgrid), dim3(kBlock), 0, s, sm.chunk_lo, sm.nrb, sm.nslices, nullptr, step_cnt,
-                           nullptr);
+        // 6. the steps in which pass 2 reads each row block's ranges
+        const unsigned pgrid = (unsigned)ceil_div64(((int64_t)sm.nrb + 1) * kWave, kBlock);
+        hipLaunchKernelGGL(k_sliced_pack, dim3(pgrid), dim3(kBlock), 0, s, sm.chunk_lo, sm.nrb, sm.nslices, step_cnt, raw);
         ASX_TRY_ST(launch_exclusive_scan_i32(step_cnt, sm.pstep_ptr, (int64_t)sm.nrb + 1, tmp, s));
-        ASX_TRY(hipMemcpyAsync(&sm.npsteps, sm.pstep_ptr + sm.nrb, sizeof(int32_t), hipMemcpyDeviceToHost, s));
-        ASX_TRY(pool_malloc(&sm.partial, sizeof(T) * ((size_t)sm.npartials + kSlicedReducePad), false));  // while the kernels run
-        ASX_TRY(hipStreamSynchronize(s));
-        ASX_TRY(pool_malloc(&sm.psteps, sizeof(int32_t) * 4 * ((size_t)sm.npsteps + kSlicedStepPad), false));
-        ASX_TRY(hipMemsetAsync(sm.psteps + 4 * (size_t)sm.npsteps, 0, sizeof(int32_t) * 4 * kSlicedStepPad, s));
-        hipLaunchKernelGGL(k_sliced_pack, dim3(pgrid), dim3(kBlock), 0, s, sm.chunk_lo, sm.nrb, sm.nslices, sm.pstep_ptr,
-                           nullptr, reinterpret_cast<i32x4 *>(sm.psteps));
+        ASX_TRY(pool_malloc(&sm.psteps, sizeof(i32x4) * ((size_t)most_steps + kSlicedStepPad), false));
+        hipLaunchKernelGGL(k_sliced_steps, dim3(pgrid), dim3(kBlock), 0, s, sm.chunk_lo, sm.nrb, sm.nslices, sm.pstep_ptr, raw,
+                           reinterpret_cast<i32x4 *>(sm.psteps), host + 5);
+        ASX_TRY(pool_malloc(&sm.partial, sizeof(T) * ((size_t)sm.npartials + kSlicedReducePad), false));
     }
-    ASX_TRY(hipStreamSynchronize(s));
     ASX_TRY(hipGetLastError());
+    ASX_TRY(hipStreamSynchronize(s));
+    sm.npsteps = host[5];
 #undef ASX_TRY
 #undef ASX_TRY_ST
 done:
-    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
-    pool_free(arena);
     if (st) {
+        (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
         free_sliced(&sm);
+        scratch.idle = true;
         return st;
     }
+    scratch.idle = true;
     *out = sm;
     return ASX_STATUS_SUCCESS;
 }
