@@ -8,11 +8,13 @@ from __future__ import annotations
 import os
 import subprocess
 import sys
+import sysconfig
 
 HERE = os.path.dirname(os.path.abspath(__file__))
 ROOT = os.path.dirname(HERE)
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libalphasparse_amd.so")
+CALLS = os.path.join(HERE, "_calls.so")
 WORKLOADS = os.path.join(HERE, "libasx_workloads.so")
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 
@@ -104,6 +106,12 @@ def build_library(verbose=False):
     return LIB
 
 
+def build_calls():
+    """The Python module behind capi.py's inner-loop calls (csrc/py_calls.c)."""
+    _run(["gcc", "-O2", "-fPIC", "-shared", "-Wall", "-I" + sysconfig.get_paths()["include"], "-o", CALLS, os.path.join(CSRC, "py_calls.c")])
+    return CALLS
+
+
 def build_workloads():
     _run(["gcc", "-O2", "-ffp-contract=off", "-fopenmp", "-fPIC", "-shared", "-Wall", "-o", WORKLOADS,
           os.path.join(CSRC, "workload_gen.c"), "-lm"])
@@ -144,6 +152,7 @@ def build_cli():
 def build_all():
     build_workloads()
     build_library()
+    build_calls()
     build_cli()
     build_oracle()
 

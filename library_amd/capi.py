@@ -45,6 +45,35 @@ class AsxError(RuntimeError):
 
 
 _lib = None
+_fast = None  # _Calls of the library that is loaded
+
+
+class _Calls:
+    """Addresses of the functions of one loaded library for csrc/py_calls.c, and what it needs from torch."""
+
+    def __init__(self, L):
+        import torch
+        try:
+            from . import _calls
+        except ImportError as e:
+            raise RuntimeError("library_amd/_calls.so is not built (python -m library_amd.build)") from e
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None) or (lambda d: torch.cuda.current_stream(d).cuda_stream)
+        _calls.streams_from(getattr(torch._C, "_cuda_getDevice", None) or torch.cuda.current_device, raw)
+        at = lambda f: C.cast(f, C.c_void_p).value
+        self.spmv, self.spmm, self.plan_values = _calls.spmv, _calls.spmm, _calls.plan_values
+        self.f64 = {torch.float32: False, torch.float64: True}
+        self.spmv_fn = {torch.float32: at(L.asx_spmv_csr_f32), torch.float64: at(L.asx_spmv_csr_f64)}
+        self.spmm_fn = {torch.float32: at(L.asx_spmm_csr_f32), torch.float64: at(L.asx_spmm_csr_f64)}
+        self.update, self.refresh = at(L.asx_plan_update_values), at(L.asx_plan_refresh_if_changed)
+
+
+def _loaded():
+    global _fast
+    L = lib()
+    if _fast is None or _fast.of is not L:
+        _fast = _Calls(L)
+        _fast.of = L
+    return _fast
 
 
 def lib():
@@ -128,10 +157,16 @@ def _stream():
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
+_VALUE_TYPES = {np.dtype(np.float32): R_32F, np.dtype(np.float64): R_64F}
+
+
 def value_type(dtype):
     import torch
-    return {torch.float32: R_32F, torch.float64: R_64F, np.dtype(np.float32): R_32F,
-            np.dtype(np.float64): R_64F}[dtype]
+    vt = _VALUE_TYPES.get(dtype)
+    if vt is None:
+        _VALUE_TYPES.update({torch.float32: R_32F, torch.float64: R_64F})
+        vt = _VALUE_TYPES[dtype]
+    return vt
 
 
 # ------------------------------------------------------------------------------ analysis
@@ -309,10 +344,16 @@ class Plan:
 
     def refresh_if_changed(self, val):
         """asx_plan_refresh_if_changed: checksums of val, and the plan's copy refreshed on the device where they differ."""
-        _check(lib().asx_plan_refresh_if_changed(self.h, _ptr(val), _stream()), "asx_plan_refresh_if_changed")
+        f = _loaded()
+        st = f.plan_values(f.refresh, self.h.value, val)
+        if st:
+            raise AsxError(st, "asx_plan_refresh_if_changed")
 
     def update_values(self, val):
-        _check(lib().asx_plan_update_values(self.h, _ptr(val), _stream()), "asx_plan_update_values")
+        f = _loaded()
+        st = f.plan_values(f.update, self.h.value, val)
+        if st:
+            raise AsxError(st, "asx_plan_update_values")
         self._keep = (self._keep[0], self._keep[1], val)
 
     INFO = {"tiles": 0, "slices": 1, "partial_sums": 2, "rows_per_wave": 3, "rows_per_block": 4, "bands": 5,
@@ -368,33 +409,32 @@ def _workspace(nbytes, device):
 def spmv(row_ptr, col, val, x, y, alpha, beta, alg=SPMV_DEFAULT, plan=None, workspace=None, n=None):
     """y <- alpha*A*x + beta*y in place (torch CUDA tensors).  Returns y.  workspace=None allocates
     what the call needs; workspace=False passes none (a sliced or window plan then uses its own buffer)."""
-    m = row_ptr.numel() - 1
-    n = x.numel() if n is None else n
-    nnz = col.numel()
-    vt = value_type(val.dtype)
-    need = plan.workspace_bytes if plan is not None else lib().asx_spmv_workspace_bytes(alg, vt, m, nnz)
+    f = _loaded()
+    dt = val.dtype
     if workspace is None:
-        workspace = _workspace(need, val.device)
-    ws_ptr, ws_bytes = (None, 0) if workspace is False else (_ptr(workspace), workspace.numel() * workspace.element_size())
-    fn = lib().asx_spmv_csr_f64 if vt == R_64F else lib().asx_spmv_csr_f32
-    _check(fn(plan.h if plan is not None else None, alg, m, n, nnz, alpha, _ptr(row_ptr), _ptr(col), _ptr(val),
-              _ptr(x), beta, _ptr(y), ws_ptr, ws_bytes, _stream()), "asx_spmv_csr")
+        need = plan.workspace_bytes if plan is not None else lib().asx_spmv_workspace_bytes(alg, value_type(dt), row_ptr.numel() - 1, col.numel())
+        if need or plan is None:
+            workspace = _workspace(need, val.device)
+    elif workspace is False:
+        workspace = None
+    st = f.spmv(f.spmv_fn[dt], f.f64[dt], None if plan is None else plan.h.value, alg, row_ptr, col, val, x, y, alpha, beta, n, workspace)
+    if st:
+        raise AsxError(st, "asx_spmv_csr")
     return y
 
 
 def spmm(row_ptr, col, val, B, Cm, ncols, alpha, beta, alg=SPMM_DEFAULT, plan=None, workspace=None,
          ldb=None, ldc=None, k=None):
     """C <- alpha*A*B + beta*C in place; B (k x ncols), C (m x ncols) row-major torch CUDA tensors."""
-    m = row_ptr.numel() - 1
-    nnz = col.numel()
-    ldb = ncols if ldb is None else ldb
-    ldc = ncols if ldc is None else ldc
-    k = B.numel() // ldb if k is None else k
-    vt = value_type(val.dtype)
-    need = plan.workspace_bytes if plan is not None else lib().asx_spmm_workspace_bytes(alg, vt, m, nnz, ncols)
+    f = _loaded()
+    dt = val.dtype
     if workspace is None:
-        workspace = _workspace(need, val.device)
-    fn = lib().asx_spmm_csr_f64 if vt == R_64F else lib().asx_spmm_csr_f32
-    _check(fn(plan.h if plan is not None else None, alg, m, k, nnz, ncols, alpha, _ptr(row_ptr), _ptr(col), _ptr(val),
-              _ptr(B), ldb, beta, _ptr(Cm), ldc, _ptr(workspace), workspace.numel(), _stream()), "asx_spmm_csr")
+        need = (plan.workspace_bytes if plan is not None
+                else lib().asx_spmm_workspace_bytes(alg, value_type(dt), row_ptr.numel() - 1, col.numel(), ncols))
+        if need or plan is None:
+            workspace = _workspace(need, val.device)
+    st = f.spmm(f.spmm_fn[dt], f.f64[dt], None if plan is None else plan.h.value, alg, row_ptr, col, val, B, Cm, ncols, alpha, beta,
+                ldb, ldc, k, workspace)
+    if st:
+        raise AsxError(st, "asx_spmm_csr")
     return Cm
