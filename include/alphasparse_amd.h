@@ -190,8 +190,8 @@ int asx_plan_create(asx_plan **plan, int is_spmm, int alg, int value_type, int32
  * hip/kernel/level3/alphasparse_spmm_tc4csr.h:38-153; the plan then holds a COPY of the values:
  * asx_plan_update_values after changing them; repeated (row, column) entries are summed; B must
  * be finite, see below).  alg = ASX_SPMM_DEFAULT measures the block fill nnz / (64 * blocks) and
- * picks the blocked kernel when it is at least 1/8, else the merge kernel.  Other algorithms
- * behave as asx_plan_create.  Synchronises `stream`. */
+ * picks the blocked kernel when it is at least 1/8 (rows of B of 256 bytes and more; 0.2, 0.3 and 0.4
+ * down to 128, 64 and fewer bytes), else the merge kernel.  Other algorithms behave as asx_plan_create.  Synchronises `stream`. */
 int asx_spmm_plan_create(asx_plan **plan, int alg, int value_type, int32_t m, int32_t k, int32_t nnz,
                          const int32_t *d_row_ptr, const int32_t *d_col, const void *d_val, int32_t ncols,
                          void *stream);

@@ -278,7 +278,8 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         }
         return launch_spmm_merge<T>(m, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
                                     ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
-                                    plan ? plan->carry_pass != 0 : true, s);
+                                    plan ? plan->carry_pass != 0 : true,
+                                    spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
     }
     case ASX_SPMM_BLOCKED:
         // the blocks hold a copy of A's values and are built by asx_spmm_plan_create
@@ -547,9 +548,15 @@ int asx_plan_destroy(asx_plan *plan)
     return ASX_STATUS_SUCCESS;
 }
 
-// Blocks are worth it when they are at least this full (bytes moved per stored element fall
-// below the merge kernel's from about 1/8 upwards, see asx_blocked.hip).
-static const double kBlockedMinFill = 0.125;
+// Blocks are worth it when they are at least this full.  The wider the rows of B, the more of the time goes into them,
+// four a block instead of one a stored element; where they are narrow, A's zeros weigh more.  Measured against the merge
+// kernel (bands of 3, 7 and 19, fill 0.125, 0.29 and 0.475, 200000 rows): 256 bytes of B a row 27 / 26, 27 / 30 and
+// 30 / 112 us, 128 bytes 18 / 15, 18 / 21 and 20 / 30, 64 bytes 13.2 / 7.9, 13.0 / 12.3 and 14.5 / 18.8, 16 bytes
+// 11.5 / 5.9, 11.3 / 6.7 and 13.0 / 18.2.
+static double blocked_min_fill(size_t row_bytes)
+{
+    return row_bytes >= 256 ? 0.125 : row_bytes >= 128 ? 0.2 : row_bytes >= 64 ? 0.3 : 0.4;
+}
 static const int32_t kBlockedProbeMaxNnz = 1 << 28;
 
 int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int32_t k, int32_t nnz,
@@ -563,14 +570,20 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
     const bool want_blocked = kernel == ASX_SPMM_BLOCKED;
     // scattered columns (a sample of tiles of 1024 stored elements touches mostly distinct
     // 128-byte lines) cannot fill 16x4 blocks: the blocks are not even built then
+    int columns = kColumnsUnknown;
     bool probe_blocked = alg == ASX_SPMM_DEFAULT && nnz > 0 && nnz <= kBlockedProbeMaxNnz && d_col &&
                          (value_type == ASX_R_32F || value_type == ASX_R_64F);
     if (probe_blocked) {
         const ColumnSample cs = sample_columns(d_col, nnz, vsize(value_type), (hipStream_t)stream);
         probe_blocked = cs.ok && cs.spread < kScatteredMinSpread;
+        if (cs.ok) columns = probe_blocked ? kColumnsNear : kColumnsScattered;
     }
-    if (!want_blocked && !probe_blocked)
-        return asx_plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, stream);
+    const auto row_ordered = [&]() {
+        const int st = asx_plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, stream);
+        if (!st && (*out)->alg == ASX_SPMM_MERGE) (*out)->columns = columns;
+        return st;
+    };
+    if (!want_blocked && !probe_blocked) return row_ordered();
     if (m < 0 || k < 0 || nnz < 0 || ncols < 1) return ASX_STATUS_INVALID_SIZE;
     if (value_type != ASX_R_32F && value_type != ASX_R_64F) return ASX_STATUS_NOT_SUPPORTED;
     if ((m > 0 && !d_row_ptr) || (nnz > 0 && (!d_col || !d_val))) return ASX_STATUS_INVALID_POINTER;
@@ -581,9 +594,9 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
                  : build_blocked<float>(m, k, nnz, d_row_ptr, d_col, (const float *)d_val, &bm, s);
     if (st) return st;
     const double fill = bm.nblocks > 0 ? (double)nnz / (64.0 * (double)bm.nblocks) : 0.0;
-    if (!want_blocked && fill < kBlockedMinFill) {
+    if (!want_blocked && fill < blocked_min_fill((size_t)ncols * vsize(value_type))) {
         free_blocked(&bm);
-        return asx_plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, stream);
+        return row_ordered();
     }
     asx_plan *p = new (std::nothrow) asx_plan();
     if (!p) {

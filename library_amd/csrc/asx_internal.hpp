@@ -96,7 +96,7 @@ template <typename T>
 int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
-                      bool carry_pass, hipStream_t s);
+                      bool carry_pass, int tile_bytes, hipStream_t s);
 
 // merge-path split points of SpMM, `items` apart, moved to the ends of the short rows they cut; *has_carry (may be null)
 // is set to 1 if a row stays cut
@@ -225,6 +225,22 @@ inline size_t window_scratch_bytes(const WindowMatrix *wm, size_t sv) { return w
 inline int32_t merge_tiles(int32_t m, int32_t nnz) { return (int32_t)ceil_div64((int64_t)m + nnz, kMergeTile); }
 inline int32_t flat_tiles(int32_t nnz) { int32_t t = (int32_t)ceil_div64(nnz, kFlatTile); return t < 1 ? 1 : t; }
 inline int32_t stream_blocks(int32_t nnz) { return (int32_t)ceil_div64(nnz, kStreamTile); }
+// What an SpMM plan knows of A's columns: nothing, that neighbouring rows share most of them, or that they do not.
+enum { kColumnsUnknown = 0, kColumnsNear = 1, kColumnsScattered = 2 };
+// How many bytes of a row of B a wave takes at once; the tiles of columns are worked off one after the other, so what an
+// L2 (4 MB, one per XCD) or L1 (32 KB) can keep of B is the narrower the more rows of it.
+//   Rows of B that start on 128-byte lines can be cut between lines: 128 bytes while all of B's tile is small
+//   (k = 30000, 256 columns fp32: 58 us against 77 with 256 bytes and 102 with 1 KB; k = 100000: 173 / 197 / 228;
+//   k = 200000: 459 / 446 / 499), else 256 (fewer reads of A; near columns: 2-D stencil 193 us against 214).
+//   Other rows begin and end inside lines wherever they are cut, 100 columns fp32 are 4.1 lines in one piece and 5.1 in
+//   two: 1 KB for scattered columns, 512 bytes for near ones (7-point stencil, 200 columns: 223 us against 244) or
+//   when nothing is known.
+inline int spmm_tile_bytes(int columns, int64_t k, const void *B, size_t pitch)
+{
+    if (pitch % 128 == 0 && (uintptr_t)B % 128 == 0) return columns != kColumnsNear && k * 128 <= (16 << 20) ? 128 : 256;
+    return columns == kColumnsScattered ? 1024 : 512;
+}
+
 // Merge items per wave of the SpMM merge kernel.  Longer segments leave fewer carries and keep the
 // lane groups of narrow N busy, shorter ones leave room for more waves (LDS) and spread small
 // matrices: 128 while 256 a wave would leave fewer than 16 waves per compute unit.  Where a row of B
@@ -255,7 +271,8 @@ struct asx_plan {
     int32_t *d_meta;         // split points / row blocks (layout depends on alg)
     size_t meta_bytes;
     int32_t nunits;  // tiles / row blocks / segments
-    int carry_pass;  // flat kernel: 0 when no row is cut by a tile boundary
+    int carry_pass;  // flat and SpMM merge kernel: 0 when no row is cut between units of work
+    int columns;     // SpMM merge kernel: kColumns*
     int64_t hist[33];
     int64_t stats[4];
     size_t workspace_bytes;

@@ -14,6 +14,8 @@
 //           a segment end is kept as a carry row and added by an ordered pass afterwards.  No atomics (the reference's default SpMM,
 //           hip/kernel/level3/alphasparse_spmm_csr_nnz_split.h:283-409, scales C in a
 //           separate pass and joins segments with atomicAdd).
+#include <algorithm>
+
 #include "asx_internal.hpp"
 
 namespace asx {
@@ -423,14 +425,14 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge_fixup(int32_t m, int32_t 
     }
 }
 
-// Lanes per row of B: the smallest power of two that spans the tile at VEC columns each; N beyond 64
-// lanes' worth is cut into equal tiles (every tile at least VEC wide).
+// N is cut into equal tiles of at most tile_bytes of a row of B (every tile at least VEC wide); lanes per row of B: the
+// smallest power of two that spans a tile at VEC columns each.
 template <typename T, int VEC, int SEG>
-static void launch_merge_width(int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
+static void launch_merge_width(int tile_bytes, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
                                const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
                                T *carry, int32_t *carry_row, hipStream_t s)
 {
-    const int64_t tiles = ceil_div64(ncols, kWave * VEC), lanes = ceil_div64(ceil_div64(ncols, tiles), VEC);
+    const int64_t tiles = ceil_div64(ncols, std::max<int64_t>(tile_bytes / (int64_t)sizeof(T), VEC)), lanes = ceil_div64(ceil_div64(ncols, tiles), VEC);
     const dim3 grid((unsigned)(ceil_div64(ceil_div64(nseg, kBlock / kWave), kXcds) * kXcds), (unsigned)tiles);
 #define ASX_WIDTH(LOGG)                                                                                              \
     if (lanes <= (1 << LOGG)) {                                                                                      \
@@ -451,29 +453,29 @@ static void launch_merge_width(int32_t nseg, int32_t ncols, T alpha, const int32
 }
 
 template <typename T, int SEG>
-static void launch_merge_seg(int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
+static void launch_merge_seg(int tile_bytes, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
                              const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
                              T *carry, int32_t *carry_row, hipStream_t s)
 {
     constexpr int kFull = 16 / sizeof(T);
     if (ncols >= kFull)
-        launch_merge_width<T, kFull, SEG>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_merge_width<T, kFull, SEG>(tile_bytes, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
     else if (ncols >= 2)
-        launch_merge_width<T, 2, SEG>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_merge_width<T, 2, SEG>(tile_bytes, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
     else
-        launch_merge_width<T, 1, SEG>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_merge_width<T, 1, SEG>(tile_bytes, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
 }
 
 template <typename T>
 int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
-                      bool carry_pass, hipStream_t s)
+                      bool carry_pass, int tile_bytes, hipStream_t s)
 {
     if (m <= 0 || ncols <= 0) return ASX_STATUS_SUCCESS;
     const int32_t items = spmm_segment_items(m, nnz, ncols, sizeof(T)), nseg = spmm_segments(m, nnz, items);
     const auto launch = [&](auto seg_) {
-        launch_merge_seg<T, decltype(seg_)::value>(nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
+        launch_merge_seg<T, decltype(seg_)::value>(tile_bytes, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
                                                    carry_row, s);
     };
     if (items == kSpmmSegmentSmall)
@@ -493,7 +495,7 @@ int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int3
                                     const T *, int64_t, T, T *, int64_t, hipStream_t);               \
     template int launch_spmm_merge<T>(int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
                                       const T *, const T *, int64_t, T, T *, int64_t, const int32_t *, \
-                                      const int32_t *, T *, int32_t *, bool, hipStream_t);
+                                      const int32_t *, T *, int32_t *, bool, int, hipStream_t);
 ASX_INST(float)
 ASX_INST(double)
 #undef ASX_INST

@@ -1,4 +1,4 @@
-"""The merge-path SpMM kernel at the edges of its dispatch: widths of C on both sides of every lane group and column tile,
+"""The SpMM kernels at the edges of their dispatch: widths of C on both sides of every lane group and column tile,
 row lengths around what one lane group takes alone, segment sizes, padded leading dimensions.  Against the CPU oracle;
 tolerance: a row's products in another order, tol * (|alpha| sum |a b| + |beta c|) with tol = 1e-12 (fp64), 1e-5 (fp32)."""
 import numpy as np
@@ -13,14 +13,14 @@ pytestmark = pytest.mark.gpu
 TOL = {np.dtype(np.float64): 1e-12, np.dtype(np.float32): 1e-5}
 
 
-def _check(oracle, rp, col, val, k, n, ldb, ldc, beta, planned, what):
+def _check(oracle, rp, col, val, k, n, ldb, ldc, beta, planned, what, alg=capi.SPMM_MERGE):
     rng = np.random.default_rng(n)
     m, dtype = rp.size - 1, val.dtype
     B = rng.uniform(-1, 1, (k - 1) * ldb + n).astype(dtype)   # ends with the last column of the last row
     C0 = rng.uniform(-1, 1, (m - 1) * ldc + n).astype(dtype)
     d = [torch.from_numpy(a).cuda() for a in (rp, col, val, B, C0)]
-    plan = capi.Plan(True, capi.SPMM_MERGE, dtype, m, k, col.size, d[0], ncols=n) if planned else None
-    capi.spmm(d[0], d[1], d[2], d[3], d[4], n, 1.5, beta, alg=capi.SPMM_MERGE, plan=plan, ldb=ldb, ldc=ldc, k=k)
+    plan = capi.Plan(True, alg, dtype, m, k, col.size, d[0], ncols=n, col=d[1], val=d[2]) if planned else None
+    capi.spmm(d[0], d[1], d[2], d[3], d[4], n, 1.5, beta, alg=alg, plan=plan, ldb=ldb, ldc=ldc, k=k)
     torch.cuda.synchronize()
     got = d[4].cpu().numpy()
     ref = oracle.spmm(rp, col, val, B, n, 1.5, beta, C0, 8, ldb=ldb, ldc=ldc)
@@ -51,3 +51,17 @@ def test_spmm_merge_segment_sizes(oracle, dtype, m, n):
     rp, col, val = W.csr_fixed(m, 50000, 16, dtype, seed=3)
     for planned in (False, True):
         _check(oracle, rp, col, val, 50000, n, n, n, 1.0, planned, f"m={m} n={n} planned={planned}")
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("n", [1, 5, 16, 17, 31, 33, 63, 65, 66, 127, 129, 130, 193, 257])
+def test_spmm_blocked_widths(oracle, dtype, n):
+    """The blocked kernel at the edges of its column tiles, with and without spare columns behind the rows, k no multiple of 4."""
+    rng = np.random.default_rng(6)
+    m, k = 83, 61
+    A = sp.random(m, k, density=0.3, random_state=7, format="csr", dtype=dtype)
+    A[40:60] = 0  # block rows without blocks
+    A.eliminate_zeros()
+    rp, col, val = A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data.astype(dtype)
+    for ldb, ldc, beta in ((n, n, 0.0), (n, n, 1.0), (n + 1, n + 3, 0.5)):
+        _check(oracle, rp, col, val, k, n, ldb, ldc, beta, True, f"blocked n={n} ldb={ldb} beta={beta}", alg=capi.SPMM_BLOCKED)
