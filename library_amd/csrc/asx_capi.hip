@@ -58,20 +58,14 @@ FlatLayout spmv_flat_layout(int32_t nnz, size_t sv, bool with_split)
     return L;
 }
 
-struct SpmmLayout {  // [xs | ys | carry_row | carry]
-    size_t xs_off, ys_off, crow_off, carry_off, bytes;
+struct SpmmLayout {  // [carry_row | carry]
+    size_t crow_off, carry_off, bytes;
 };
-SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv, bool with_split)
+SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
 {
     SpmmLayout L{};
     const size_t ns = (size_t)spmm_segments(m, nnz, spmm_segment_items(m, nnz, ncols, sv));
     size_t off = 0;
-    if (with_split) {
-        for (size_t *o : {&L.xs_off, &L.ys_off}) {
-            *o = off;
-            off = align_up(off + (ns + 1) * 4, kAlign);
-        }
-    }
     L.crow_off = off;
     off = align_up(off + std::max<size_t>(ns, 1) * 4, kAlign);
     L.carry_off = off;
@@ -200,15 +194,13 @@ int spmv_impl(const asx_plan *plan, int alg, int32_t m, int32_t n, int32_t nnz, 
         const FlatLayout L = spmv_flat_layout(nnz, sizeof(T), plan == nullptr);
         if (!ws) return ASX_STATUS_INVALID_POINTER;
         if (ws_bytes < L.bytes) return ASX_STATUS_INVALID_SIZE;
-        const int32_t *seg;
-        if (plan) {
-            seg = plan->d_meta;
-        } else {
-            int st = launch_flat_seg_rows(row_ptr, m, nnz, (int32_t *)(w + L.seg_off), s);
+        int32_t *seg = plan ? plan->d_meta : (int32_t *)(w + L.seg_off);
+        const bool search = !plan && flat_tiles(nnz) <= kFlatSelfSearchMost;
+        if (!plan && !search) {
+            int st = launch_flat_seg_rows(row_ptr, m, nnz, seg, s);
             if (st) return st;
-            seg = (const int32_t *)(w + L.seg_off);
         }
-        return launch_spmv_flat<T>(m, nnz, alpha, row_ptr, col, val, x, beta, y, seg, (T *)(w + L.carry_off),
+        return launch_spmv_flat<T>(m, nnz, alpha, row_ptr, col, val, x, beta, y, seg, search, (T *)(w + L.carry_off),
                                    plan ? plan->carry_pass != 0 : true, s);
     }
     case ASX_SPMV_SLICED: {
@@ -262,7 +254,7 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
     case ASX_SPMM_ROW:
         return launch_spmm_row<T>(m, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, s);
     case ASX_SPMM_MERGE: {
-        const SpmmLayout L = spmm_merge_layout(m, nnz, ncols, sizeof(T), plan == nullptr);
+        const SpmmLayout L = spmm_merge_layout(m, nnz, ncols, sizeof(T));
         if (!ws) return ASX_STATUS_INVALID_POINTER;
         if (ws_bytes < L.bytes) return ASX_STATUS_INVALID_SIZE;
         const int32_t *xs, *ys;
@@ -270,11 +262,7 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
             xs = plan->d_meta;
             ys = plan->d_meta + (plan->nunits + 1);
         } else {
-            int st = launch_spmm_splits(m, nnz, spmm_segment_items(m, nnz, ncols, sizeof(T)), row_ptr, (int32_t *)(w + L.xs_off),
-                                        (int32_t *)(w + L.ys_off), nullptr, s);
-            if (st) return st;
-            xs = (const int32_t *)(w + L.xs_off);
-            ys = (const int32_t *)(w + L.ys_off);
+            xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
         return launch_spmm_merge<T>(m, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
                                     ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
@@ -493,7 +481,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         // does any row stay cut?  (one int read back; creation syncs anyway)
         if (!st) st = launch_spmm_splits(m, nnz, items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
         if (!st) st = read_flag();
-        p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv, false).bytes;
+        p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv).bytes;
     }
     if (!st) st = status_of(hipStreamSynchronize(s));
     return st;
@@ -1216,7 +1204,7 @@ int asx_spmm_resolve_alg(int alg, int32_t m, int32_t nnz, int32_t ncols)
 size_t asx_spmm_workspace_bytes(int alg, int value_type, int32_t m, int32_t nnz, int32_t ncols)
 {
     const int kernel = asx_spmm_resolve_alg(alg, m, nnz, ncols);
-    if (kernel == ASX_SPMM_MERGE) return spmm_merge_layout(m, nnz, ncols, vsize(value_type), true).bytes;
+    if (kernel == ASX_SPMM_MERGE) return spmm_merge_layout(m, nnz, ncols, vsize(value_type)).bytes;
     return 0;
 }
 

@@ -83,8 +83,8 @@ int launch_spmv_stream(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, 
 
 template <typename T>
 int launch_spmv_flat(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, const int32_t *col,
-                     const T *val, const T *x, T beta, T *y, const int32_t *seg_row, T *carry,
-                     bool carry_pass, hipStream_t s);
+                     const T *val, const T *x, T beta, T *y, int32_t *seg_row, bool search, T *carry,
+                     bool carry_pass, hipStream_t s);  // search: seg_row is written by the call
 int launch_flat_has_carry(const int32_t *d_row_ptr, int32_t m, int32_t nnz, const int32_t *d_seg_row,
                           int32_t *d_flag, hipStream_t s);
 
@@ -223,6 +223,10 @@ int launch_spmv_window(int32_t m, int32_t n, T alpha, const WindowMatrix *wm, co
 inline size_t window_scratch_bytes(const WindowMatrix *wm, size_t sv) { return wm->has_carry ? (size_t)wm->ntiles * sv : 0; }
 
 inline int32_t merge_tiles(int32_t m, int32_t nnz) { return (int32_t)ceil_div64((int64_t)m + nnz, kMergeTile); }
+// Without a plan the flat kernel's tiles look up their own rows up to this many tiles; beyond it the search's latency at the
+// start of every workgroup costs more than a launch of its own (4700 tiles 32 us against 35, 16400 104 against 98, 78000 412
+// against 333).
+constexpr int32_t kFlatSelfSearchMost = 8192;
 inline int32_t flat_tiles(int32_t nnz) { int32_t t = (int32_t)ceil_div64(nnz, kFlatTile); return t < 1 ? 1 : t; }
 inline int32_t stream_blocks(int32_t nnz) { return (int32_t)ceil_div64(nnz, kStreamTile); }
 // What an SpMM plan knows of A's columns: nothing, that neighbouring rows share most of them, or that they do not.

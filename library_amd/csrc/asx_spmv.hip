@@ -20,6 +20,7 @@
 // _flat.h, _merge_ginkgo.h, _adaptive.h) join partial rows with floating-point atomicAdd and
 // recompute their split points in every call; neither is done here.
 #include "asx_internal.hpp"
+#include "asx_rank.hpp"
 
 namespace asx {
 
@@ -525,10 +526,6 @@ int launch_spmv_merge(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, c
 constexpr int kFlatItemsPerThread = kFlatTile / kBlock;
 static_assert(kFlatItemsPerThread == 4, "the vector loads below read 4 elements per thread");
 constexpr int kFlatRowCap = 1024;  // rows of one tile kept in LDS
-#ifndef ASX_FLAT_TPG
-#define ASX_FLAT_TPG 1
-#endif
-constexpr int kFlatTilesPerGroup = ASX_FLAT_TPG;
 
 template <typename T>
 struct Vec4;
@@ -633,8 +630,8 @@ struct FlatShared {
 template <typename T, bool NT>
 __device__ __forceinline__ void flat_tile(FlatShared<T> &sh, int t, int32_t m, int32_t nnz, T alpha,
                                           const int32_t *__restrict__ row_ptr, const int32_t c[4], T p[4],
-                                          const T *__restrict__ x, T beta, T *__restrict__ y,
-                                          const int32_t *__restrict__ seg_row, T *__restrict__ carry)
+                                          const T *__restrict__ x, T beta, T *__restrict__ y, int32_t rs, int32_t re,
+                                          T *__restrict__ carry)
 {
     int32_t *s_rend = sh.rend;
     T *s_out = sh.out;
@@ -646,8 +643,6 @@ __device__ __forceinline__ void flat_tile(FlatShared<T> &sh, int t, int32_t m, i
     const int32_t n1 = nnz - base < kFlatTile ? (int32_t)(nnz - base) : kFlatTile;
     const int32_t k0 = tid * 4;
     // ---- rows met by the tile: rs .. re; re (if < m) continues into the next tile ----
-    const int32_t rs = t == 0 ? 0 : seg_row[t];
-    const int32_t re = seg_row[t + 1];
     const int32_t nwritten = re - rs;                   // rows that end inside this tile
     const int32_t rcount = nwritten + (re < m ? 1 : 0);  // plus the one left open
     const bool fits = rcount <= kFlatRowCap + 1;  // 1024 one-element rows plus the open row still fit
@@ -771,32 +766,42 @@ __device__ __forceinline__ void flat_tile(FlatShared<T> &sh, int t, int32_t m, i
     }
 }
 
-// kFlatTilesPerGroup consecutive tiles per workgroup: the loads of all of them are issued before
-// the first is reduced, so the reduction of one tile overlaps the memory latency of the next.
-template <typename T, bool VEC, bool NT, int TPG>
+// SEARCH: the call has no plan and seg_row is written here - two waves look up the rows at the tile's ends, 64 probes at a
+// time, while the tile's loads are in flight (a launch of its own for the search took 5 us and the gap behind it); the carry
+// pass reads them.
+template <typename T, bool VEC, bool NT, bool SEARCH>
 __global__ __launch_bounds__(kBlock) void k_spmv_flat(int32_t m, int32_t nnz, int32_t ntiles, T alpha,
                                                       const int32_t *__restrict__ row_ptr,
                                                       const int32_t *__restrict__ col,
                                                       const T *__restrict__ val,
                                                       const T *__restrict__ x, T beta,
                                                       T *__restrict__ y,
-                                                      const int32_t *__restrict__ seg_row,
+                                                      int32_t *__restrict__ seg_row,
                                                       T *__restrict__ carry)
 {
     __shared__ FlatShared<T> sh;
-    const int t0 = blockIdx.x * TPG;
-    int32_t c[TPG][4];
-    T p[TPG][4];
-#pragma unroll
-    for (int u = 0; u < TPG; ++u)
-        if (t0 + u < ntiles) flat_load<T, VEC, NT>(t0 + u, nnz, col, val, c[u], p[u]);
-#pragma unroll
-    for (int u = 0; u < TPG; ++u) {
-        if (t0 + u < ntiles) {  // uniform over the workgroup
-            if (u > 0) __syncthreads();  // the previous tile is done with the LDS buffers
-            flat_tile<T, NT>(sh, t0 + u, m, nnz, alpha, row_ptr, c[u], p[u], x, beta, y, seg_row, carry);
+    const int t = blockIdx.x;
+    int32_t c[4];
+    T p[4];
+    flat_load<T, VEC, NT>(t, nnz, col, val, c, p);
+    int32_t rs, re;
+    if (SEARCH) {
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        if (w < 2) {
+            const int64_t e = (int64_t)(t + w) * kFlatTile;
+            const int32_t r = t + w == 0 ? 0 : t + w == ntiles ? m : wave_row_holding(row_ptr, 0, m, (int32_t)e);
+            if ((threadIdx.x & (kWave - 1)) == 0) {
+                sh.wk[w] = r;
+                if (w == 0 || t == ntiles - 1) seg_row[t + w] = r;
+            }
         }
+        __syncthreads();
+        rs = sh.wk[0], re = sh.wk[1];
+    } else {
+        rs = t == 0 ? 0 : seg_row[t];
+        re = seg_row[t + 1];
     }
+    flat_tile<T, NT>(sh, t, m, nnz, alpha, row_ptr, c, p, x, beta, y, rs, re, carry);
 }
 
 // seg_row[t] = row holding stored element t*kFlatTile for t < nt, seg_row[nt] = m,
@@ -830,7 +835,7 @@ int launch_flat_has_carry(const int32_t *d_row_ptr, int32_t m, int32_t nnz, cons
 
 template <typename T>
 int launch_spmv_flat(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, const int32_t *col,
-                     const T *val, const T *x, T beta, T *y, const int32_t *seg_row, T *carry,
+                     const T *val, const T *x, T beta, T *y, int32_t *seg_row, bool search, T *carry,
                      bool carry_pass, hipStream_t s)
 {
     if (m <= 0) return ASX_STATUS_SUCCESS;
@@ -839,10 +844,15 @@ int launch_spmv_flat(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, co
     // a caller may pass an offset view)
     const bool aligned = ((uintptr_t)col % 16 == 0) && ((uintptr_t)val % 16 == 0);
     const bool nt = use_nontemporal(nnz, sizeof(T));
-#define ASX_FLAT(VEC, NT)                                                                             \
-    hipLaunchKernelGGL((k_spmv_flat<T, VEC, NT, kFlatTilesPerGroup>),                                 \
-                       dim3((unsigned)ceil_div64(ntiles, kFlatTilesPerGroup)), dim3(kBlock), 0, s, m, nnz, \
-                       ntiles, alpha, row_ptr, col, val, x, beta, y, seg_row, carry)
+#define ASX_FLAT(VEC, NT)                                                                                              \
+    do {                                                                                                               \
+        if (search)                                                                                                    \
+            hipLaunchKernelGGL((k_spmv_flat<T, VEC, NT, true>), dim3((unsigned)ntiles), dim3(kBlock), 0, s, m, nnz, ntiles, \
+                               alpha, row_ptr, col, val, x, beta, y, seg_row, carry);                                  \
+        else                                                                                                           \
+            hipLaunchKernelGGL((k_spmv_flat<T, VEC, NT, false>), dim3((unsigned)ntiles), dim3(kBlock), 0, s, m, nnz, ntiles, \
+                               alpha, row_ptr, col, val, x, beta, y, seg_row, carry);                                  \
+    } while (0)
     if (aligned && nt) ASX_FLAT(true, true);
     else if (aligned) ASX_FLAT(true, false);
     else if (nt) ASX_FLAT(false, true);
@@ -863,7 +873,7 @@ int launch_spmv_flat(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, co
                                       const T *, const T *, T, T *, const int32_t *, const int32_t *, \
                                       T *, hipStream_t);                                             \
     template int launch_spmv_flat<T>(int32_t, int32_t, T, const int32_t *, const int32_t *, const T *, \
-                                     const T *, T, T *, const int32_t *, T *, bool, hipStream_t);
+                                     const T *, T, T *, int32_t *, bool, T *, bool, hipStream_t);
 ASX_INST(float)
 ASX_INST(double)
 #undef ASX_INST
