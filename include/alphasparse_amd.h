@@ -45,7 +45,7 @@ enum { ASX_R_32F = 0, ASX_R_64F = 1 };
  * (include/alphasparse/spdef.h:345-365); how each reference algorithm id maps onto these
  * kernels is decided by asx_spmv_resolve_alg. */
 enum {
-    ASX_SPMV_DEFAULT = 0, /* pick from the row-length histogram (plan) or from m, nnz */
+    ASX_SPMV_DEFAULT = 0, /* pick from the matrix (plan) or from m, nnz */
     ASX_SPMV_VECTOR = 6,  /* wave64 sub-groups, one group per row */
     ASX_SPMV_STREAM = 3,  /* LDS-staged row blocks, segmented reduction */
     ASX_SPMV_MERGE = 9,   /* merge-path tiles + ordered carry fix-up */
@@ -199,18 +199,18 @@ int asx_spmm_plan_create(asx_plan **plan, int alg, int value_type, int32_t m, in
  * elements by column slice (128 KiB of x per slice) for the kernel that holds its slice of x in
  * LDS.  The plan then holds a COPY of the columns and values (asx_plan_update_values after
  * changing the values) and the buffer for the partial sums of a call: calls through one plan
- * must not overlap.  alg = ASX_SPMV_DEFAULT picks that kernel when nnz >= 2^21, the columns are
- * scattered (a sample of 64 tiles of 1024 stored elements touches on average more than 512
- * distinct 128-byte lines of x per tile) and a cost model over the row-length histogram and the
- * sizes puts it at least 10 % ahead of the row-ordered kernels; the choice depends on the matrix
- * alone, not on timings.  Otherwise as asx_plan_create.  No counterpart in the reference (its
+ * must not overlap.  alg = ASX_SPMV_DEFAULT estimates every kernel's time from the sizes, the row-length
+ * histogram and a sample of the columns (64 tiles of 1024 stored elements) and picks the lowest: a row-ordered
+ * kernel, or for nnz >= 2^21 that kernel where it is ahead of them (by 10 % below 2^22, where the copy saves less
+ * than it costs a caller to build); the choice depends on the matrix alone, not on timings.  A plan for the vector
+ * kernel also lists the long rows where a few rows are much longer than the rest.  Other algorithms as
+ * asx_plan_create.  No counterpart in the reference (its
  * alphasparseSpMV_analysis is a stub).  alg = ASX_SPMV_WINDOW builds the row-block copy for the
  * kernel that keeps sliding windows of x in LDS (again a COPY of columns and values, and the
  * carry slots of a call; a matrix without rows of fewer than two stored elements needs no copy of
  * the values: an fp32 plan, or a plan made by asx_spmv_plan_create_checked, then reads A's values
  * in every call, ASX_PLAN_INFO_BY_REFERENCE = 1, and holds 2 bytes per stored element instead of
- * 14 or 10); DEFAULT picks it, when the sliced kernel is not chosen, for nnz >= 2^21
- * whenever the matrix qualifies: every 256 consecutive rows reach
+ * 14 or 10); DEFAULT picks it for nnz >= 2^21 where it is estimated ahead and the matrix qualifies: every 256 consecutive rows reach
  * over fewer than 16376 columns, or the stored elements lie on at most 4 bands of diagonals whose
  * windows fit the LDS together (stencils on three-dimensional grids); otherwise
  * ASX_STATUS_NOT_SUPPORTED for the explicit id, the row-ordered plan for DEFAULT.  Synchronises

@@ -156,7 +156,8 @@ int spmv_impl(const asx_plan *plan, int alg, int32_t m, int32_t n, int32_t nnz, 
     char *w = (char *)ws;
     switch (kernel) {
     case ASX_SPMV_VECTOR:
-        return launch_spmv_vector<T>(m, nnz, alpha, row_ptr, col, val, x, beta, y, s);
+        return launch_spmv_vector<T>(m, nnz, alpha, row_ptr, col, val, x, beta, y,
+                                     plan ? LongRows{plan->d_meta, plan->nwide, plan->nlong, plan->long_len} : LongRows{}, s);
     case ASX_SPMV_STREAM: {
         const int32_t *blocks;
         if (plan) {
@@ -373,7 +374,7 @@ int asx_loadbalance_partition(const int32_t *d_row_ptr, int32_t m, int32_t nnz, 
 namespace {
 
 // A plan with sizes and the row-length histogram, no kernel chosen yet; with d_col also the column
-// sample of an analysis that may regroup A, and whether the device has room for that.  One round trip.
+// sample, and, when asked, how much memory is free.  One round trip.
 // The counters on the device stay with the plan (33 histogram bins, 4 stats, spare words for what
 // else the build reads back): freeing them here would cost more than the build's kernels.
 struct PlanStats {
@@ -381,7 +382,7 @@ struct PlanStats {
     size_t free_bytes;
 };
 int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n, int32_t nnz, const int32_t *d_row_ptr,
-               int32_t ncols_dense, const int32_t *d_col, PlanStats *more, hipStream_t s)
+               int32_t ncols_dense, const int32_t *d_col, PlanStats *more, bool ask_memory, hipStream_t s)
 {
     asx_plan *p = new (std::nothrow) asx_plan();
     if (!p) return ASX_STATUS_ALLOC_FAILED;
@@ -405,7 +406,7 @@ int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n
                                line_shift(sv), (int32_t)(kSliceBytes / sv), samples,
                                reinterpret_cast<int32_t *>(p->d_counters + 64), s);
     if (!st) st = status_of(hipMemcpyAsync(h, p->d_counters, kPlanCounters * sizeof(int64_t), hipMemcpyDeviceToHost, s));
-    if (more) {  // asked while the device counts
+    if (ask_memory) {  // while the device counts
         size_t total = 0;
         if (hipMemGetInfo(&more->free_bytes, &total) != hipSuccess) more->free_bytes = 0;
         more->free_bytes += pool_kept_bytes();
@@ -501,7 +502,7 @@ int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_
     if (m > 0 && !d_row_ptr) return ASX_STATUS_INVALID_POINTER;
     hipStream_t s = (hipStream_t)stream;
     asx_plan *p = nullptr;
-    int st = plan_begin(&p, is_spmm, value_type, m, n, nnz, d_row_ptr, ncols_dense, nullptr, nullptr, s);
+    int st = plan_begin(&p, is_spmm, value_type, m, n, nnz, d_row_ptr, ncols_dense, nullptr, nullptr, false, s);
     if (st) return st;
     int kernel;
     if (!is_spmm)
@@ -609,58 +610,110 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
 
 }  // extern "C"
 
-// ---- what DEFAULT picks when it may regroup A --------------------------------------------
+// ---- what DEFAULT picks when it may look at the columns ----------------------------------
 // Decided from figures that do not change from one plan build to the next (the row-length
 // histogram, the sizes, the column sample), never from timings: two analyses of one matrix keep the
-// same kernel.  Estimated times (rates fitted to measurements on MI355X over families of matrices:
-// uniform and power-law rows, bands, stencils, clustered columns):
-//   row-ordered kernels   5 us + max(nnz spread' / g, bytes / 4.0 TB/s); g = gathers of x an L2
-//                         serves per second: 180 G while x fits one (<= 3 MiB), 62 G once it does
-//                         not (>= 6 MiB), linear in between; spread' = the sample's spread, at least
-//                         0.05 (neighbouring columns share a line); bytes = nnz (sv + 4) + n sv + m (sv + 4)
-//   column-sliced kernel  8 us + bytes / 6.0 TB/s, bytes = nnz (sv + 2) + P (2 sv + 2) + n sv + 2 m sv,
-//                         P = nnz times the sample's pairs per stored element
-//   row-block kernel      8 us + bytes / 5.0 TB/s (3.7 TB/s when rows longer than 16 are cut by
-//                         tiles), bytes = (nnz + empty rows) (sv + 2) + n sv + 2 m sv; only for
-//                         columns that are not scattered, and whether every block's columns fit a
-//                         window is known once its build was tried
-// A regrouped kernel is taken when its estimate is at least 3 % below the row-ordered one; of the
-// two, the sliced one unless the row-block one is estimated more than 5 % faster.
-constexpr int32_t kSlicedMinNnz = 1 << 21;
+// same kernel.  Estimated times, fitted to 306 matrices timed with every kernel on MI355X, three copies
+// of each in turn (uniform, power-law, banded, near-diagonal rows and stencils of 60 000 to 32 M stored
+// elements in both types; the kernel chosen is on average 2.4 % behind the fastest).  In microseconds, with
+//   gathers(r) = nnz spread' / r thousand, r falling to 62 while x grows from 3 to 6 MB (an L2 holds 4);
+//                spread' = the sample's spread, at least 0.05 (neighbouring columns share a line)
+//   bytes      = nnz (sv + 4) + n sv + m (sv + 4)
+// and a + b read as their smooth maximum (a^4 + b^4)^(1/4):
+//   vector  at least 4; 2.1 + (gathers(158) + bytes / (the lower of 4.3 TB/s u and 2.7 TB/s)), u = the share of a
+//           group's lanes that a mean row fills; + 0.125 per turn of a group in which only the longest row is left
+//   stream  at least 4; 3.0 + (gathers(171) + bytes / 3.6 TB/s); + 0.018 per element of the longest row beyond
+//           twice the mean (its block sums it with the few lanes its short neighbours want)
+//   flat    6.0 + (gathers(190) + bytes / 3.9 TB/s), + 3.4 where rows longer than 32 make tiles walk
+//   merge   7.8 + (gathers(164) + (nnz (sv + 4) + n sv + m (sv + 1)) / 2.9 TB/s)
+//   sliced  9.9 + bytes / 5.6 TB/s, bytes = nnz (sv + 2) + P (2 sv + 2) + n sv + 2 m sv, P = nnz times the
+//           sample's pairs per stored element
+//   window  8 + bytes / 5.9 TB/s in fp64, 15 + bytes / 5.6 TB/s in fp32 (11 + 5.1 TB/s and 15 + 4.6 TB/s where rows longer
+//           than 16 are cut by tiles), bytes = (nnz + slots rows shorter than two leave free) (sv + 2) + n sv + 2 m sv; only for columns
+//           that are not scattered, and whether every block's columns fit a window is known once its build was tried
+// With a list of its long rows the vector kernel costs 0.5 more and 0.0004 per element of the longest row instead of the
+// turns, u divided by the turns a wave of the other rows takes.
+// A regrouped kernel is taken when its estimate is 3 % below the row-ordered ones: 10 % below 4 M stored elements, where it
+// saves little for what its build costs, and above up to 10 % slower where neighbours do not share lines (spread > 0.1), because
+// what gathers cost the row-ordered kernels is estimated less well than what a copy streams.  Of the two, the sliced one unless
+// the window one is estimated more than 5 % faster - or, in fp32 with rows the tiles do not cut, not more than 9 % slower: its
+// plan reads A's values where the caller keeps them, and a caller who changes them before every multiply has nothing to bring up
+// to date (7 per row, 22 M elements: 48 us against 95).
+constexpr int32_t kRegroupMinNnz = 1 << 21;
+// The vector kernel with a list of long rows: eight turns of a lane group are long, kWideRow elements take a workgroup (a
+// power of two each, so that the histogram holds their numbers), and with a row of more than kMostWideRow the kernels
+// that cut rows are ahead: one workgroup walks it alone.
+constexpr int32_t kWideRow = 2048, kMostWideRow = 8192;
+static int32_t long_row_len(const asx_plan *p) { return 8 * vector_lanes(p->m, p->nnz); }
+static int64_t rows_of_at_least(const asx_plan *p, int32_t len /* a power of two */)
+{
+    int64_t n = 0;
+    for (int b = 1; b <= 32; ++b)
+        if (((int64_t)1 << (b - 1)) >= len) n += p->hist[b];
+    return n;
+}
 struct KernelEstimates {
     // seconds; infinity where the kernel does not apply.  window: with one ring of x per block;
     // window_bands: with rings per band of diagonals, window_stacked: with three bands on stacked
     // planes; which of the three it is only the build finds out
     double rows, sliced, window, window_bands, window_stacked;
+    int row_kernel;  // of the row-ordered ones
+    bool long_rows;  // the vector kernel with a list of its long rows
 };
 static KernelEstimates estimate_kernels(const asx_plan *p, size_t sv, const ColumnSample &cs, bool window_ok, bool checked)
 {
     const double inf = 1e30;
     const double nnz = (double)p->nnz, m = (double)p->m, n = (double)p->n, dsv = (double)sv;
+    const double longest = (double)p->stats[0], mean = nnz / m;
     const double xbytes = n * dsv;
     const double lo = 3.0 * 1048576.0, hi = 6.0 * 1048576.0;
     const double f = xbytes <= lo ? 0.0 : xbytes >= hi ? 1.0 : (xbytes - lo) / (hi - lo);
-    const double gather_rate = 180e9 + f * (62e9 - 180e9);
+    const double spread = std::max(cs.ok ? cs.spread : 0.5, 0.05);
+    const auto gathers = [&](double rate) { return nnz * spread / ((rate + f * (62.0 - rate)) * 1e9); };
+    const auto both = [](double a, double b) { return std::sqrt(std::hypot(a * a, b * b)); };
+    const double bytes = nnz * (dsv + 4) + xbytes + m * (dsv + 4);
+    const double lanes = vector_lanes(p->m, p->nnz);
+    // a wave's turns are those of the longest of its 64 / lanes rows (long rows aside, which a list may take)
+    double turns = 0.0, below = 0.0;
+    for (int b = 0; b <= 32; ++b) {
+        const double len = b == 0 ? 0.0 : 1.4 * std::ldexp(1.0, b - 1);
+        if (len >= long_row_len(p)) break;
+        const double upto = below + (double)p->hist[b] / m;
+        turns += std::max(1.0, std::ceil(std::min(len, longest) / lanes)) * (std::pow(upto, 64.0 / lanes) - std::pow(below, 64.0 / lanes));
+        below = upto;
+    }
+    turns = std::max(1.0, turns);
+    const auto by_lanes = [&](double filled) { return both(gathers(158), bytes / std::min(2.7e12, 4.3e12 * filled)); };
+    const double vector = std::max(4e-6, 2.1e-6 + by_lanes(mean / lanes)) +
+                          0.125e-6 * std::max(0.0, longest / lanes - std::max(1.0, mean / lanes));
+    const double stream = std::max(4e-6, 3e-6 + both(gathers(171), bytes / 3.6e12)) +
+                          0.018e-6 * std::max(0.0, std::min(longest, 1024.0) - std::max(32.0, 2 * mean));
+    const double flat = 6e-6 + both(gathers(190), bytes / 3.9e12) + (longest > 32 ? 3.4e-6 : 0.0);
+    const double merge = 7.8e-6 + both(gathers(164), (bytes - 3 * m) / 2.9e12);
+    const double with_list = std::max(4e-6, 2.6e-6 + by_lanes(mean / (lanes * turns))) + 0.4e-9 * longest;
     KernelEstimates e;
-    e.rows = 5e-6 + std::max(nnz * std::max(cs.spread, 0.05) / gather_rate, (nnz * (dsv + 4) + n * dsv + m * (dsv + 4)) / 4.0e12);
+    e.row_kernel = ASX_SPMV_VECTOR, e.rows = vector, e.long_rows = false;
+    if (longest >= long_row_len(p) && longest <= kMostWideRow && with_list < vector)
+        e.rows = with_list, e.long_rows = true;
+    if (stream < e.rows) e.row_kernel = ASX_SPMV_STREAM, e.rows = stream;
+    if (flat < e.rows) e.row_kernel = ASX_SPMV_FLAT, e.rows = flat;
+    if (merge < e.rows) e.row_kernel = ASX_SPMV_MERGE, e.rows = merge;
+    // Mostly empty rows: only the merge-path kernel counts row ends as work
+    if (p->hist[0] > (int64_t)p->m / 2) e.row_kernel = ASX_SPMV_MERGE, e.rows = merge;
     const int64_t nslices = ceil_div64((int64_t)p->n * (int64_t)sv, kSliceBytes);
     e.sliced = nslices > kSlicedMaxSlices
                    ? inf
-                   : 8e-6 + (nnz * (dsv + 2) + cs.pairs * nnz * (2 * dsv + 2) + n * dsv + 2 * m * dsv) / 6.0e12;
-    // The row-block copy gives every row at least two slots.  Rates measured over the audit's
-    // families (what the copy moves / (time - 8 us)): one ring 5.8e12 with rows the tiles do not cut
-    // (5-point stencil, band of 9), 5.0 and 4.6e12 with rows of 19 and 65; rings per band, x fetched
-    // about 1.5 times: 4.7e12 (7-point stencil) and 3.9e12 (27-point).
+                   : 9.9e-6 + (nnz * (dsv + 2) + cs.pairs * nnz * (2 * dsv + 2) + n * dsv + 2 * m * dsv) / 5.6e12;
+    // The row-block copy gives every row at least two slots.  Rings per band fetch x about 1.5 times, stacked planes 1.3
+    // times; in fp32 the time goes with the slots and not with the bytes.
     const double wslots = nnz + 2.0 * (double)p->hist[0] + (double)p->hist[1];
-    const bool uncut = p->stats[0] <= 16;
-    e.window = !window_ok ? inf : 8e-6 + (wslots * (dsv + 2) + n * dsv + 2 * m * dsv) / (uncut ? 5.6e12 : 4.8e12);
-    e.window_bands = !window_ok ? inf : 8e-6 + (wslots * (dsv + 2) + 1.5 * n * dsv + 2 * m * dsv) / (uncut ? 4.6e12 : 3.9e12);
-    // three bands on stacked planes (x fetched about 1.3 times): 7-point stencil on 160^3 5.6e12 in
-    // fp64 but 3.5e12 in fp32, where the time goes with the slots and not with the bytes; 27-point
-    // on 96^3 (rows of 27, cut by tiles) 4.2e12
-    e.window_stacked = !window_ok ? inf
-                                  : 8e-6 + (wslots * (dsv + 2) + 1.3 * n * dsv + 2 * m * dsv) /
-                                               (sv == 8 ? (uncut ? 5.6e12 : 4.2e12) : (uncut ? 3.5e12 : 3.0e12));
+    const bool uncut = p->stats[0] <= 16, f64 = sv == 8;
+    const auto window = [&](double x_times, double base, double uncut_rate, double cut_rate) {
+        return !window_ok ? inf : base + (wslots * (dsv + 2) + x_times * n * dsv + 2 * m * dsv) / (uncut ? uncut_rate : cut_rate);
+    };
+    e.window = window(1.0, f64 ? (uncut ? 8e-6 : 11e-6) : 15e-6, f64 ? 5.9e12 : 5.6e12, f64 ? 5.1e12 : 4.6e12);
+    e.window_bands = window(1.5, f64 ? 8e-6 : 20e-6, 4.6e12, 3.9e12);
+    e.window_stacked = window(1.3, f64 ? 8e-6 : 15e-6, f64 ? 5.6e12 : 3.5e12, f64 ? 4.2e12 : 3.0e12);
     if (checked) {
         // a checked plan reads the caller's values once more in every call (a stream of its own
         // kernel: 6.3 TB/s measured) and launches three small kernels
@@ -672,6 +725,22 @@ static KernelEstimates estimate_kernels(const asx_plan *p, size_t sv, const Colu
             e.window *= 1.06, e.window_bands *= 1.06, e.window_stacked *= 1.06;
     }
     return e;
+}
+
+// The list of long rows onto a plan for the vector kernel; one round trip, after which the plan can be used on any stream.
+static int plan_long_rows(asx_plan *p, hipStream_t s)
+{
+    const int32_t len = long_row_len(p);
+    const int64_t nwide = rows_of_at_least(p, kWideRow), nlong = rows_of_at_least(p, len) - nwide;
+    if (len > kWideRow || nwide + nlong == 0) return ASX_STATUS_SUCCESS;
+    p->meta_bytes = (size_t)(nwide + nlong) * sizeof(int32_t);
+    int st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
+    if (!st)
+        st = launch_long_rows(p->row_ptr, p->m, len, kWideRow, (int32_t)nwide, reinterpret_cast<int32_t *>(p->d_counters + 41),
+                              p->d_meta, s);
+    if (!st) st = status_of(hipStreamSynchronize(s));
+    p->nwide = (int32_t)nwide, p->nlong = (int32_t)nlong, p->long_len = len;
+    return st;
 }
 
 // Builds the sliced copy onto a plan that already holds the histogram (`p` takes the slices over;
@@ -735,8 +804,7 @@ int plan_add_window(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
     return ASX_STATUS_SUCCESS;
 }
 
-// DEFAULT tries the row-block copy for matrices the flat or merge-path kernel would take, without
-// rows past the carry pass's limit, and with few rows of fewer than two stored elements: the copy
+// DEFAULT tries the row-block copy for matrices with few rows of fewer than two stored elements: the copy
 // gives every row at least two slots (a value, a column word and a source index each, read in every
 // call), so a matrix where that padding exceeds a quarter of its stored elements stays with the
 // other kernels.
@@ -752,11 +820,7 @@ static bool regrouped_copy_fits(const asx_plan *p, size_t sv, size_t free_bytes)
     return (double)free_bytes >= 2.0 * copy;
 }
 
-static bool window_may_pay(const asx_plan *p, int row_kernel)
-{
-    return (row_kernel == ASX_SPMV_FLAT || row_kernel == ASX_SPMV_MERGE) &&
-           2 * p->hist[0] + p->hist[1] <= (int64_t)p->nnz / 4;
-}
+static bool window_may_pay(const asx_plan *p) { return 2 * p->hist[0] + p->hist[1] <= (int64_t)p->nnz / 4; }
 
 // the checksum words of a plan: of the values as they are now (2), of the values its copy holds (2)
 static unsigned long long *checksum_words(const asx_plan *p) { return reinterpret_cast<unsigned long long *>(p->d_counters + 44); }
@@ -792,9 +856,10 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
     hipStream_t s = (hipStream_t)stream;
     asx_plan *p = nullptr;
     PlanStats ps{ColumnSample{false, 0.0, 1.0}, 0};
-    const bool may_regroup = alg == ASX_SPMV_DEFAULT && d_col && d_val && m > 0 && n > 0 && nnz >= kSlicedMinNnz;
-    const bool sample = may_regroup || alg == ASX_SPMV_SLICED;
-    int st = plan_begin(&p, 0, value_type, m, n, nnz, d_row_ptr, 1, sample ? d_col : nullptr, sample ? &ps : nullptr, s);
+    const bool looks = alg == ASX_SPMV_DEFAULT && d_col && d_val && m > 0 && n > 0 && nnz > 0;  // DEFAULT with the columns at hand
+    const bool may_regroup = looks && nnz >= kRegroupMinNnz;
+    const int32_t *sampled = looks || alg == ASX_SPMV_SLICED ? d_col : nullptr;
+    int st = plan_begin(&p, 0, value_type, m, n, nnz, d_row_ptr, 1, sampled, &ps, may_regroup, s);
     if (st) return st;
     if (alg == ASX_SPMV_DEFAULT) row_kernel = choose_spmv_from_stats(p->hist, p->stats, m, nnz);
     const bool f64 = value_type == ASX_R_64F;
@@ -809,38 +874,49 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
     };
     const bool can_regroup = may_regroup && regrouped_copy_fits(p, sv, ps.free_bytes);
     const ColumnSample &cs = ps.sample;
-    bool done = false;
+    bool done = false, list_long_rows = false;
     if (alg == ASX_SPMV_WINDOW) {
         st = add_window();
         done = true;
     } else if (alg == ASX_SPMV_SLICED) {
         st = add_slices(cs.pairs);  // the sample sizes the row blocks of pass 2
         done = true;
-    } else if (can_regroup) {
+    } else if (looks) {
         // DEFAULT: a regrouped copy where it is estimated to pay; a build that fails (out of memory,
-        // a matrix the kernel does not take) is not an error: the next choice stands
-        if (cs.ok) {
-            // the row-block kernel needs columns near each other; whether they fit its windows the
-            // build finds out (NOT_SUPPORTED when some 256 rows reach further)
-            const bool window_ok = window_may_pay(p, row_kernel) && cs.spread < kScatteredMinSpread;
-            const KernelEstimates e = estimate_kernels(p, sv, cs, window_ok, checked);
-            const bool sliced_pays = e.sliced < 0.97 * e.rows, window_pays = e.window < 0.97 * e.rows;
-            if (window_pays && e.window < e.sliced / 1.05) done = add_window() == ASX_STATUS_SUCCESS;
-            if (done && p->window.nbands > 1 && sliced_pays &&
-                !((p->window.stack_rows > 0 ? e.window_stacked : e.window_bands) < e.sliced / 1.05)) {
-                // the build needed a ring per band of diagonals; with those the slices are ahead
-                WindowMatrix built = p->window;
-                p->window = WindowMatrix{};
-                if (add_slices(cs.pairs) == ASX_STATUS_SUCCESS)
-                    free_window(&built);
-                else
-                    p->window = built, p->alg = ASX_SPMV_WINDOW;
+        // a matrix the kernel does not take) is not an error: the next choice stands.  The row-block
+        // kernel needs columns near each other; whether they fit its windows the build finds out
+        // (NOT_SUPPORTED when some 256 rows reach further)
+        const bool window_ok = can_regroup && cs.ok && window_may_pay(p) && cs.spread < kScatteredMinSpread;
+        const KernelEstimates e = estimate_kernels(p, sv, cs, window_ok, checked);
+        row_kernel = e.row_kernel;
+        list_long_rows = e.long_rows;
+        if (can_regroup && cs.ok) {
+            const double ahead = (nnz < (1 << 22) ? 0.9 : cs.spread > 0.1 ? 1.1 : 0.97) * e.rows;
+            const bool sliced_pays = e.sliced < ahead, window_pays = e.window < ahead;
+            const bool in_place = !f64 && p->hist[0] + p->hist[1] == 0 && p->stats[0] <= 16;
+            const double slices_for_window = e.sliced * (in_place ? 1.09 : 1 / 1.05);
+            if (window_pays && e.window < slices_for_window) done = add_window() == ASX_STATUS_SUCCESS;
+            if (done && p->window.nbands > 1) {
+                // the build needed a ring per band of diagonals: estimated again
+                const double built_for = p->window.stack_rows > 0 ? e.window_stacked : e.window_bands;
+                const bool slices = sliced_pays && !(built_for < slices_for_window), rows = !slices && !(built_for < ahead);
+                if (slices || rows) {
+                    WindowMatrix built = p->window;
+                    p->window = WindowMatrix{};
+                    if (rows || add_slices(cs.pairs) == ASX_STATUS_SUCCESS) {
+                        free_window(&built);
+                        done = !rows;
+                    } else {
+                        p->window = built, p->alg = ASX_SPMV_WINDOW;
+                    }
+                }
             }
             if (!done && sliced_pays) done = add_slices(cs.pairs) == ASX_STATUS_SUCCESS;
-            if (!done && window_pays && !(e.window < e.sliced / 1.05)) done = add_window() == ASX_STATUS_SUCCESS;
+            if (!done && window_pays && !(e.window < slices_for_window)) done = add_window() == ASX_STATUS_SUCCESS;
         }
     }
     if (!done) st = plan_row_ordered(p, row_kernel, s);
+    if (!done && !st && row_kernel == ASX_SPMV_VECTOR && list_long_rows) st = plan_long_rows(p, s);
     if (!st && checked && asx_plan_holds_values(p)) {
         // the values must lie on a 16-byte boundary for the checksum's loads (every allocation does);
         // a view that does not keeps an unchecked plan out: row-ordered instead

@@ -70,9 +70,17 @@ int launch_gather_lines(const void *d_buf, size_t bytes, int group_lanes, int pe
                         hipStream_t s);
 
 // ---- SpMV launchers (asx_spmv.hip) ----
+// Rows that the vector kernel gives more than a lane group: nwide rows a workgroup each, then nlong rows a wave each, all of
+// long_len elements or more (rows == nullptr: none).
+struct LongRows {
+    const int32_t *rows;
+    int32_t nwide, nlong, long_len;
+};
+int launch_long_rows(const int32_t *d_row_ptr, int32_t m, int32_t long_len, int32_t wide_len, int32_t nwide, int32_t *d_at,
+                     int32_t *d_out, hipStream_t s);
 template <typename T>
 int launch_spmv_vector(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, const int32_t *col,
-                       const T *val, const T *x, T beta, T *y, hipStream_t s);
+                       const T *val, const T *x, T beta, T *y, const LongRows &long_rows, hipStream_t s);
 template <typename T>
 int launch_spmv_merge(int32_t m, int32_t nnz, T alpha, const int32_t *row_ptr, const int32_t *col,
                       const T *val, const T *x, T beta, T *y, const int32_t *xs, const int32_t *ys,
@@ -222,6 +230,13 @@ int launch_spmv_window(int32_t m, int32_t n, T alpha, const WindowMatrix *wm, co
                        hipStream_t s);
 inline size_t window_scratch_bytes(const WindowMatrix *wm, size_t sv) { return wm->has_carry ? (size_t)wm->ntiles * sv : 0; }
 
+// lanes per row of the vector kernel: the power of two that holds a mean row
+inline int vector_lanes(int32_t m, int32_t nnz)
+{
+    int l = 2;
+    while (l < 64 && (double)nnz > (double)l * (double)m) l *= 2;
+    return l;
+}
 inline int32_t merge_tiles(int32_t m, int32_t nnz) { return (int32_t)ceil_div64((int64_t)m + nnz, kMergeTile); }
 // Without a plan the flat kernel's tiles look up their own rows up to this many tiles; beyond it the search's latency at the
 // start of every workgroup costs more than a launch of its own (4700 tiles 32 us against 35, 16400 104 against 98, 78000 412
@@ -268,7 +283,7 @@ struct asx_plan {
     int value_type;
     int32_t m, n, nnz, ncols;
     const int32_t *row_ptr;  // the device array the plan was built from (identity check only)
-    int64_t *d_counters;     // kPlanCounters words on the device: histogram (33), stats (4), a flag (40), checksums of the values:
+    int64_t *d_counters;     // kPlanCounters words on the device: histogram (33), stats (4), a flag (40), counts of long rows (41), checksums of the values:
                              // of this call (44, 45) and of the copy the plan holds (46, 47), 64 sample counts (64..95)
     int checked;             // the plan holds a copy of A's values and a checksum of them (asx_spmv_plan_create_checked)
     unsigned long long *d_checksum_parts;  // checked plans: the workgroups' partial sums of one checksum run
@@ -276,6 +291,7 @@ struct asx_plan {
     size_t meta_bytes;
     int32_t nunits;  // tiles / row blocks / segments
     int carry_pass;  // flat and SpMM merge kernel: 0 when no row is cut between units of work
+    int32_t nwide, nlong, long_len;  // vector kernel: d_meta lists the long rows (asx::LongRows)
     int columns;     // SpMM merge kernel: kColumns*
     int64_t hist[33];
     int64_t stats[4];

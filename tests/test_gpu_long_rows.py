@@ -1,0 +1,42 @@
+"""SpMV plans that list their long rows, at the edges of the list: row lengths on both sides of eight turns of a lane group,
+of what takes a workgroup and of the longest row the list is for; every lane group.  Against float64 sums on the host;
+tolerance: a row's products in another order, len u (|alpha| sum |a x|) + 3 u |beta y| with u = 2^-24 or 2^-53."""
+import numpy as np
+import pytest
+import torch
+
+from conftest import csr_from_lengths
+from library_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("lanes", [2, 4, 8, 16, 32])
+@pytest.mark.parametrize("wide", [(), (2047, 2048, 2049), (8191, 8192)])
+def test_long_row_list(dtype, lanes, wide):
+    rng = np.random.default_rng(lanes)
+    cut = 8 * lanes
+    n = 9001
+    short = rng.integers(0, 2 * lanes - 2, 3001)
+    lens = np.r_[short[:1500], cut - 1, cut, cut + 1, 0, wide, cut, 1900, short[1500:]].astype(int)
+    while lens.sum() > lanes * lens.size:  # keep the mean row inside the lane group
+        lens = np.r_[lens, np.ones(1000, int)]
+    rp, col, val = csr_from_lengths(lens, n, 3, dtype)
+    x, y0 = rng.uniform(-1, 1, n).astype(dtype), rng.uniform(-1, 1, lens.size).astype(dtype)
+    d = [torch.from_numpy(a).cuda() for a in (rp, col, val, x)]
+    plan = capi.Plan(False, capi.SPMV_DEFAULT, val.dtype, lens.size, n, col.size, d[0], col=d[1], val=d[2])
+    assert plan.alg == capi.SPMV_VECTOR
+    u = 2.0 ** (-53 if dtype == np.float64 else -24)
+    rows = np.repeat(np.arange(lens.size), lens)
+    prod = val.astype(np.longdouble) * x[col].astype(np.longdouble)
+    exact, size = np.zeros(lens.size, np.longdouble), np.zeros(lens.size, np.longdouble)
+    np.add.at(exact, rows, prod)
+    np.add.at(size, rows, np.abs(prod))
+    for beta in (0.0, 0.5):
+        y = torch.from_numpy(y0).cuda()
+        capi.spmv(d[0], d[1], d[2], d[3], y, 1.5, beta, plan=plan)
+        torch.cuda.synchronize()
+        bound = (lens + 3) * u * 1.5 * size + 3 * u * np.abs(beta * y0)
+        assert np.all(np.abs(y.cpu().numpy() - (1.5 * exact + beta * y0)) <= bound), (lanes, beta)
+    plan.destroy()
