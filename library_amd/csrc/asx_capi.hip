@@ -633,12 +633,12 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
 //           that are not scattered, and whether every block's columns fit a window is known once its build was tried
 // With a list of its long rows the vector kernel costs 0.5 more and 0.0004 per element of the longest row instead of the
 // turns, u divided by the turns a wave of the other rows takes.
-// A regrouped kernel is taken when its estimate is 3 % below the row-ordered ones: 10 % below 4 M stored elements, where it
-// saves little for what its build costs, and above up to 10 % slower where neighbours do not share lines (spread > 0.1), because
-// what gathers cost the row-ordered kernels is estimated less well than what a copy streams.  Of the two, the sliced one unless
-// the window one is estimated more than 5 % faster - or, in fp32 with rows the tiles do not cut, not more than 9 % slower: its
-// plan reads A's values where the caller keeps them, and a caller who changes them before every multiply has nothing to bring up
-// to date (7 per row, 22 M elements: 48 us against 95).
+// A regrouped kernel is taken when its estimate is 3 % below the row-ordered ones: 5 % (window 15 %, the dearest to build)
+// below 4 M stored elements, where it saves little for what its build costs, and above that even when up to 10 % slower where
+// the columns are neither neighbours nor scattered, because there what gathers cost the row-ordered kernels is estimated less
+// well than what a copy streams.  Of the two, the sliced one unless the window one is estimated more than 5 % faster - or, in
+// fp32 with rows the tiles do not cut, not more than 9 % slower: its plan reads A's values where the caller keeps them, and a
+// caller who changes them before every multiply has nothing to bring up to date (7 per row, 22 M elements: 48 us against 95).
 constexpr int32_t kRegroupMinNnz = 1 << 21;
 // The vector kernel with a list of long rows: eight turns of a lane group are long, kWideRow elements take a workgroup (a
 // power of two each, so that the histogram holds their numbers), and with a row of more than kMostWideRow the kernels
@@ -891,8 +891,8 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
         row_kernel = e.row_kernel;
         list_long_rows = e.long_rows;
         if (can_regroup && cs.ok) {
-            const double ahead = (nnz < (1 << 22) ? 0.9 : cs.spread > 0.1 ? 1.1 : 0.97) * e.rows;
-            const bool sliced_pays = e.sliced < ahead, window_pays = e.window < ahead;
+            const double ahead = (nnz < (1 << 22) ? 0.95 : cs.spread > 0.1 && cs.spread < kScatteredMinSpread ? 1.1 : 0.97) * e.rows;
+            const bool sliced_pays = e.sliced < ahead, window_pays = e.window < ahead * (nnz < (1 << 22) ? 0.9 : 1.0);
             const bool in_place = !f64 && p->hist[0] + p->hist[1] == 0 && p->stats[0] <= 16;
             const double slices_for_window = e.sliced * (in_place ? 1.09 : 1 / 1.05);
             if (window_pays && e.window < slices_for_window) done = add_window() == ASX_STATUS_SUCCESS;
