@@ -152,6 +152,11 @@ def _ptr(t):
     return None if t is None else C.c_void_p(t.data_ptr())
 
 
+def _handle(h):
+    """The address in a plan's handle: a c_void_p or, from an adopted plan, an integer; None of a destroyed plan."""
+    return h.value if isinstance(h, C.c_void_p) else h
+
+
 def _stream():
     import torch
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
@@ -345,13 +350,13 @@ class Plan:
     def refresh_if_changed(self, val):
         """asx_plan_refresh_if_changed: checksums of val, and the plan's copy refreshed on the device where they differ."""
         f = _loaded()
-        st = f.plan_values(f.refresh, self.h.value, val)
+        st = f.plan_values(f.refresh, _handle(self.h), val)
         if st:
             raise AsxError(st, "asx_plan_refresh_if_changed")
 
     def update_values(self, val):
         f = _loaded()
-        st = f.plan_values(f.update, self.h.value, val)
+        st = f.plan_values(f.update, _handle(self.h), val)
         if st:
             raise AsxError(st, "asx_plan_update_values")
         self._keep = (self._keep[0], self._keep[1], val)
@@ -417,7 +422,7 @@ def spmv(row_ptr, col, val, x, y, alpha, beta, alg=SPMV_DEFAULT, plan=None, work
             workspace = _workspace(need, val.device)
     elif workspace is False:
         workspace = None
-    st = f.spmv(f.spmv_fn[dt], f.f64[dt], None if plan is None else plan.h.value, alg, row_ptr, col, val, x, y, alpha, beta, n, workspace)
+    st = f.spmv(f.spmv_fn[dt], f.f64[dt], None if plan is None else _handle(plan.h), alg, row_ptr, col, val, x, y, alpha, beta, n, workspace)
     if st:
         raise AsxError(st, "asx_spmv_csr")
     return y
@@ -433,7 +438,7 @@ def spmm(row_ptr, col, val, B, Cm, ncols, alpha, beta, alg=SPMM_DEFAULT, plan=No
                 else lib().asx_spmm_workspace_bytes(alg, value_type(dt), row_ptr.numel() - 1, col.numel(), ncols))
         if need or plan is None:
             workspace = _workspace(need, val.device)
-    st = f.spmm(f.spmm_fn[dt], f.f64[dt], None if plan is None else plan.h.value, alg, row_ptr, col, val, B, Cm, ncols, alpha, beta,
+    st = f.spmm(f.spmm_fn[dt], f.f64[dt], None if plan is None else _handle(plan.h), alg, row_ptr, col, val, B, Cm, ncols, alpha, beta,
                 ldb, ldc, k, workspace)
     if st:
         raise AsxError(st, "asx_spmm_csr")
