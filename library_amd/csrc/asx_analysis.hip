@@ -20,8 +20,25 @@ __global__ __launch_bounds__(256) void k_zero_i64(int64_t *p, int n)
     if (i < n) p[i] = 0;
 }
 
+// Row blocks of the stream kernel (k_stream_row_blocks: the same pairs) marked by row r, which starts at element s and ends
+// at e: r + 1 is the first row at or behind every boundary after s up to e.  The boundaries up to the first row's start are
+// row 0's, those behind the last row's end (nnz larger than row_ptr[m]) and the last pair are (m, row_ptr[m]).
+__device__ __forceinline__ void mark_blocks(int64_t r, int32_t m, int32_t s, int32_t e, int32_t nb, int2 *__restrict__ blocks)
+{
+    if (r == 0)
+        for (int64_t t = 0; t < nb && t * kStreamTile <= s; ++t) blocks[t] = make_int2(0, s);
+    int64_t t = s < 0 ? 0 : s / kStreamTile + 1;
+    for (; t < nb && t * kStreamTile <= e; ++t) blocks[t] = make_int2((int32_t)r + 1, e);
+    if (r == m - 1) {
+        for (; t < nb; ++t) blocks[t] = make_int2(m, e);
+        blocks[nb] = make_int2(m, e);
+    }
+}
+
+template <bool MARK = false>
 __device__ __forceinline__ void row_histogram(const int32_t *__restrict__ row_ptr, int32_t m, int64_t block, int64_t blocks,
-                                              unsigned long long *hist /*33*/, unsigned long long *stats /*4*/)
+                                              unsigned long long *hist /*33*/, unsigned long long *stats /*4*/,
+                                              int32_t nb = 0, int2 *__restrict__ row_blocks = nullptr)
 {
     __shared__ unsigned int s_hist[33];
     __shared__ unsigned int s_bins[3];
@@ -35,7 +52,9 @@ __device__ __forceinline__ void row_histogram(const int32_t *__restrict__ row_pt
     for (int64_t r0 = block * 256; r0 < m; r0 += blocks * 256) {  // uniform
         const int64_t r = r0 + threadIdx.x;
         const bool valid = r < m;
-        const int len = valid ? row_ptr[r + 1] - row_ptr[r] : 0;
+        const int32_t from = valid ? row_ptr[r] : 0, to = valid ? row_ptr[r + 1] : 0;
+        const int len = to - from;
+        if (MARK && valid) mark_blocks(r, m, from, to, nb, row_blocks);
         const int bin = len <= 0 ? 0 : 32 - __clz(len);
         // one LDS atomic per distinct bin among the wave's 64 rows (rows of one length would
         // otherwise serialise 64 atomics on one address)
@@ -314,7 +333,15 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
     if (threadIdx.x == 0) count = 0, pairs = 0;
     __syncthreads();
     const int64_t first = (int64_t)t * q.stride;
-    const int32_t *from = q.col + first;
+    // the columns are requested before the searches, so that their latency passes during those
+    constexpr int kPer = kFlatTile / kBlock;
+    int32_t c[kPer], left[kPer];
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = u * kBlock + threadIdx.x;
+        c[u] = q.col[first + i];
+        left[u] = q.col[first + (i > 0 ? i - 1 : 0)];
+    }
     if (q.row_ptr) {
         // the rows that start in the tile: found by two searches, marked by one read each (a search
         // per element was a chain of twenty reads, 23 us for the whole sample)
@@ -327,9 +354,10 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
     }
     __syncthreads();
     int32_t mine = 0, mine_pairs = 0;
-    for (int i = threadIdx.x; i < kFlatTile; i += kBlock) {
-        const int32_t c = from[i];
-        const int32_t v = c >> q.shift;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) {
+        const int i = u * kBlock + threadIdx.x;
+        const int32_t v = c[u] >> q.shift;
         uint32_t h = ((uint32_t)v * 2654435761u) >> 20;
         for (;;) {
             const int32_t old = atomicCAS(&table[h], -1, v);
@@ -341,7 +369,7 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
             h = (h + 1) & (kSlots - 1);
         }
         if (q.row_ptr)
-            mine_pairs += i == 0 || c / q.width != from[i - 1] / q.width || (starts[i >> 5] >> (i & 31) & 1u) != 0;
+            mine_pairs += i == 0 || c[u] / q.width != left[u] / q.width || (starts[i >> 5] >> (i & 31) & 1u) != 0;
     }
     if (mine) atomicAdd(&count, mine);
     if (mine_pairs) atomicAdd(&pairs, mine_pairs);
@@ -363,26 +391,30 @@ int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const
 }
 
 // What an analysis looks at first, in one launch: the sample (its workgroups first, they take longest) and the
-// histogram of the row lengths.
+// histogram of the row lengths; with row_blocks also the row blocks of the stream kernel, which come with the row offsets
+// that are read anyway (searched for afterwards they took a kernel of 7 us and a second wait for the device).
 __global__ __launch_bounds__(kBlock) void k_plan_stats(SampleArgs q, const int32_t *__restrict__ row_ptr, int32_t m,
-                                                       unsigned long long *hist, unsigned long long *stats)
+                                                       unsigned long long *hist, unsigned long long *stats, int32_t nb,
+                                                       int2 *__restrict__ row_blocks)
 {
     if ((int)blockIdx.x < q.samples)
         sample_columns_tile(q, blockIdx.x);
+    else if (row_blocks)
+        row_histogram<true>(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, hist, stats, nb, row_blocks);
     else
         row_histogram(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, hist, stats);
 }
 
 int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int64_t *d_hist, int64_t *d_stats,
                       const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample,
-                      hipStream_t s)
+                      int32_t nb, int32_t *d_row_blocks, hipStream_t s)
 {
     if (samples < 0 || samples > 64) return ASX_STATUS_INVALID_VALUE;
     hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(256), 0, s, d_counters, ncounters);
     if (m > 0) {
         const SampleArgs q{d_col, stride, shift, d_row_ptr, m, width, samples, d_sample};
         hipLaunchKernelGGL(k_plan_stats, dim3(histogram_blocks(m) + (unsigned)samples), dim3(kBlock), 0, s, q, d_row_ptr, m,
-                           (unsigned long long *)d_hist, (unsigned long long *)d_stats);
+                           (unsigned long long *)d_hist, (unsigned long long *)d_stats, nb, reinterpret_cast<int2 *>(d_row_blocks));
     }
     return check_launch();
 }

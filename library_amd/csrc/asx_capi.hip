@@ -377,12 +377,16 @@ namespace {
 // sample, and, when asked, how much memory is free.  One round trip.
 // The counters on the device stay with the plan (33 histogram bins, 4 stats, spare words for what
 // else the build reads back): freeing them here would cost more than the build's kernels.
+// Where DEFAULT may choose the stream kernel, its row blocks come along behind the counters, in the same block of the pool
+// (which is 64 KB at least); searched for afterwards they took another launch and
+// another wait for the device: 300 000 x 400 000, 16 per row, f64, analysed, multiplied once and dropped: 95 us, now 75.
+constexpr int32_t kMarkedBlocksMost = (65536 - kPlanCounters * (int32_t)sizeof(int64_t)) / (int32_t)sizeof(int2) - 1;
 struct PlanStats {
     ColumnSample sample;
     size_t free_bytes;
 };
 int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n, int32_t nnz, const int32_t *d_row_ptr,
-               int32_t ncols_dense, const int32_t *d_col, PlanStats *more, bool ask_memory, hipStream_t s)
+               int32_t ncols_dense, const int32_t *d_col, PlanStats *more, bool ask_memory, bool mark_blocks, hipStream_t s)
 {
     asx_plan *p = new (std::nothrow) asx_plan();
     if (!p) return ASX_STATUS_ALLOC_FAILED;
@@ -400,11 +404,15 @@ int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n
     Scratch scratch(s);
     int64_t *h = static_cast<int64_t *>(scratch.pinned());
     static_assert(kPlanCounters * sizeof(int64_t) <= kPinnedBytes, "the counters are read back through page-locked memory");
-    int st = h ? status_of(pool_malloc(&p->d_counters, kPlanCounters * sizeof(int64_t), false)) : ASX_STATUS_ALLOC_FAILED;
+    const int32_t nb = std::max(stream_blocks(nnz), 1);
+    p->nmarked = mark_blocks && samples > 0 && nb <= kMarkedBlocksMost ? nb : 0;
+    const size_t marked_bytes = p->nmarked > 0 ? ((size_t)nb + 1) * sizeof(int2) : 0;
+    int st = h ? status_of(pool_malloc(&p->d_counters, kPlanCounters * sizeof(int64_t) + marked_bytes, false)) : ASX_STATUS_ALLOC_FAILED;
     if (!st)
         st = launch_plan_stats(d_row_ptr, m, p->d_counters, kPlanCounters, p->d_counters, p->d_counters + 33, d_col, sample_stride(nnz),
                                line_shift(sv), (int32_t)(kSliceBytes / sv), samples,
-                               reinterpret_cast<int32_t *>(p->d_counters + 64), s);
+                               reinterpret_cast<int32_t *>(p->d_counters + 64), nb,
+                               p->nmarked > 0 ? reinterpret_cast<int32_t *>(p->d_counters + kPlanCounters) : nullptr, s);
     if (!st) st = status_of(hipMemcpyAsync(h, p->d_counters, kPlanCounters * sizeof(int64_t), hipMemcpyDeviceToHost, s));
     if (ask_memory) {  // while the device counts
         size_t total = 0;
@@ -434,6 +442,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
     p->alg = kernel;
     p->workspace_bytes = 0;
     if (m == 0) return ASX_STATUS_SUCCESS;  // nothing to analyse: calls with m == 0 return before any launch
+    if (kernel == ASX_SPMV_VECTOR && !p->is_spmm) return ASX_STATUS_SUCCESS;  // needs no split points
     // zero since plan_begin; set by the kernels that look for rows cut between units of work
     int32_t *d_flag = reinterpret_cast<int32_t *>(p->d_counters + 40);
     const auto read_flag = [&]() {
@@ -450,6 +459,10 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             int32_t nb = std::max(stream_blocks(nnz), 1);
             p->nunits = nb;
             p->meta_bytes = ((size_t)nb + 1) * 8;
+            if (p->nmarked == nb) {  // made by plan_begin, which has waited for them; pool_free leaves them to the counters
+                p->d_meta = reinterpret_cast<int32_t *>(p->d_counters + kPlanCounters);
+                return ASX_STATUS_SUCCESS;
+            }
             st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
             if (!st) st = launch_stream_row_blocks(d_row_ptr, m, nnz, p->d_meta, s);
         } else if (kernel == ASX_SPMV_FLAT) {
@@ -462,7 +475,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             p->carry_pass = 1;
             if (!st) {  // is any row cut by a tile boundary?  (one int read back; creation syncs anyway)
                 st = launch_flat_has_carry(d_row_ptr, m, nnz, p->d_meta, d_flag, s);
-                if (!st) st = read_flag();
+                return st ? st : read_flag();  // which waits
             }
         } else if (kernel == ASX_SPMV_MERGE) {
             const size_t nt = (size_t)merge_tiles(m, nnz);
@@ -480,9 +493,9 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         p->carry_pass = 1;
         st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
         // does any row stay cut?  (one int read back; creation syncs anyway)
-        if (!st) st = launch_spmm_splits(m, nnz, items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
-        if (!st) st = read_flag();
         p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv).bytes;
+        if (!st) st = launch_spmm_splits(m, nnz, items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
+        return st ? st : read_flag();  // which waits
     }
     if (!st) st = status_of(hipStreamSynchronize(s));
     return st;
@@ -502,7 +515,7 @@ int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_
     if (m > 0 && !d_row_ptr) return ASX_STATUS_INVALID_POINTER;
     hipStream_t s = (hipStream_t)stream;
     asx_plan *p = nullptr;
-    int st = plan_begin(&p, is_spmm, value_type, m, n, nnz, d_row_ptr, ncols_dense, nullptr, nullptr, false, s);
+    int st = plan_begin(&p, is_spmm, value_type, m, n, nnz, d_row_ptr, ncols_dense, nullptr, nullptr, false, false, s);
     if (st) return st;
     int kernel;
     if (!is_spmm)
@@ -859,7 +872,7 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
     const bool looks = alg == ASX_SPMV_DEFAULT && d_col && d_val && m > 0 && n > 0 && nnz > 0;  // DEFAULT with the columns at hand
     const bool may_regroup = looks && nnz >= kRegroupMinNnz;
     const int32_t *sampled = looks || alg == ASX_SPMV_SLICED ? d_col : nullptr;
-    int st = plan_begin(&p, 0, value_type, m, n, nnz, d_row_ptr, 1, sampled, &ps, may_regroup, s);
+    int st = plan_begin(&p, 0, value_type, m, n, nnz, d_row_ptr, 1, sampled, &ps, may_regroup, looks, s);
     if (st) return st;
     if (alg == ASX_SPMV_DEFAULT) row_kernel = choose_spmv_from_stats(p->hist, p->stats, m, nnz);
     const bool f64 = value_type == ASX_R_64F;

@@ -62,9 +62,10 @@ int launch_checksum(const void *d_data, size_t bytes, unsigned long long *d_part
 int launch_checksum_commit(const unsigned long long *d_now, unsigned long long *d_kept, hipStream_t s);
 int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const int32_t *d_row_ptr, int32_t m,
                           int32_t width, int32_t samples, int32_t *d_out, hipStream_t s);
-// the counters set to zero, then launch_row_histogram and launch_sample_columns in one launch (samples = 0: no sample)
+// the counters set to zero, then launch_row_histogram and launch_sample_columns in one launch (samples = 0: no sample);
+// d_row_blocks: the nb row blocks of launch_stream_row_blocks too (null: not wanted)
 int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int64_t *d_hist, int64_t *d_stats,
-                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample,
+                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample, int32_t nb, int32_t *d_row_blocks,
                       hipStream_t s);
 int launch_gather_lines(const void *d_buf, size_t bytes, int group_lanes, int per_lane, void *d_out, int *nthreads,
                         hipStream_t s);
@@ -287,6 +288,7 @@ struct asx_plan {
                              // of this call (44, 45) and of the copy the plan holds (46, 47), 64 sample counts (64..95)
     int checked;             // the plan holds a copy of A's values and a checksum of them (asx_spmv_plan_create_checked)
     unsigned long long *d_checksum_parts;  // checked plans: the workgroups' partial sums of one checksum run
+    int32_t nmarked;         // row blocks of the stream kernel behind the counters (0: none)
     int32_t *d_meta;         // split points / row blocks (layout depends on alg)
     size_t meta_bytes;
     int32_t nunits;  // tiles / row blocks / segments
