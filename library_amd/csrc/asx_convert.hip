@@ -120,20 +120,24 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_count(const int32_t 
     if (blockIdx.x == 0 && threadIdx.x == 0) counts[(int64_t)nbuckets * nblocks] = 0;
 }
 
+// Four workgroups a compute unit in fp32 (37 KB of LDS, 64 registers), three in fp64 (53 KB): its chain of dependent steps
+// is long, and 3.6 M elements are 879 workgroups - two rounds with 57 KB.  BKT_FIG
 template <typename T>
-__global__ __launch_bounds__(kSortThreads) void k_transpose_bucket(const int32_t *__restrict__ row_ptr,
+__global__ __launch_bounds__(kSortThreads, sizeof(T) == 4 ? 8 : 6) void k_transpose_bucket(const int32_t *__restrict__ row_ptr,
                                                                    const int32_t *__restrict__ col, const T *__restrict__ val,
                                                                    const int32_t *__restrict__ seg_row, int32_t nnz, int32_t base,
                                                                    int shift, int32_t nbuckets, int nbits, int32_t nblocks,
                                                                    const int32_t *__restrict__ offs, int32_t *__restrict__ brow,
                                                                    uint16_t *__restrict__ bcol, T *__restrict__ bval)
 {
-    __shared__ uint16_t cnt[kSortWaves * kBuckets];  // per wave and bucket: count, then first rank of the wave's elements
-    __shared__ int32_t lofs[kBuckets];               // per bucket: the block's count, then its first position in bucket order
-    __shared__ int32_t to[kBuckets];                 // per bucket: place of the block's first element minus lofs
+    // per wave and bucket: count, then first rank of the wave's elements; when those are used up, the columns in bucket order
+    __shared__ __align__(16) unsigned char lds[kSortElems * sizeof(int32_t)];
+    static_assert(sizeof(uint16_t) * kSortWaves * kBuckets <= sizeof(lds), "the counters lie where the columns go");
+    __shared__ int32_t lofs[kBuckets];  // per bucket: the block's count, then its first position in bucket order, then its place minus that
     __shared__ int32_t wave_tot[kSortWaves];
-    __shared__ int32_t col_s[kSortElems];
     __shared__ __align__(16) unsigned char stage[kSortElems * (sizeof(T) > 4 ? sizeof(T) : 4)];
+    uint16_t *cnt = reinterpret_cast<uint16_t *>(lds);
+    int32_t *col_s = reinterpret_cast<int32_t *>(lds);
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     // consecutive blocks write neighbouring places of every bucket: keep them on one XCD, whose L2
     // then merges their pieces of a cache line (the grid is a multiple of kXcds workgroups)
@@ -153,14 +157,24 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_bucket(const int32_t
     const int64_t g = (int64_t)b * kSortWaves + wave;
     const int32_t r_lo = __builtin_amdgcn_readfirstlane(seg_row[g]), r_hi = __builtin_amdgcn_readfirstlane(seg_row[g + 1]);
     int32_t *row_s = reinterpret_cast<int32_t *>(stage);
+    int32_t *my_rows = row_s + wave * kSortWaveElems;
     int32_t r[kSortPerLane];
-    wave_rows(row_ptr, base, r_lo, r_hi, wbase, nnz, row_s + wave * kSortWaveElems, r);
+    wave_rows(row_ptr, base, r_lo, r_hi, wbase, nnz, my_rows, r);
+    // the rows wait in LDS: in registers they would cost waves
+#pragma unroll
+    for (int k = 0; k < kSortPerLane; ++k) my_rows[k * kWave + lane] = r[k];
     __syncthreads();
     uint16_t *mycnt = cnt + wave * nbuckets;
 #pragma unroll
     for (int k = 0; k < kSortPerLane; ++k) p[k] = wave_rank(c[k] >> shift, wbase + k * kWave + lane < nnz, nbits, mycnt);
     __syncthreads();
-    for (int s = tid; s < nbuckets; s += kSortThreads) {
+    constexpr int kPer = kBuckets / kSortThreads;
+    int32_t place[kPer];  // of the block's first element in buckets tid, tid + kSortThreads, ...
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int s = tid + q * kSortThreads;
+        if (s >= nbuckets) break;
+        place[q] = offs[(int64_t)s * nblocks + b];
         int32_t run = 0;
 #pragma unroll
         for (int w = 0; w < kSortWaves; ++w) {
@@ -169,17 +183,24 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_bucket(const int32_t
             run += t;
         }
         lofs[s] = run;
-        to[s] = offs[(int64_t)s * nblocks + b];
     }
     __syncthreads();
     block_exclusive_sum(lofs, nbuckets, wave_tot);
-    for (int s = tid; s < nbuckets; s += kSortThreads) to[s] -= lofs[s];
 #pragma unroll
     for (int k = 0; k < kSortPerLane; ++k) {
-        const int64_t i = wbase + k * kWave + lane;
-        if (i < nnz) {
-            const int32_t s = c[k] >> shift;
-            p[k] += lofs[s] + mycnt[s];
+        if (wbase + k * kWave + lane < nnz) p[k] += lofs[c[k] >> shift] + mycnt[c[k] >> shift];
+        r[k] = my_rows[k * kWave + lane];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kPer; ++q) {
+        const int s = tid + q * kSortThreads;
+        if (s < nbuckets) lofs[s] = place[q] - lofs[s];
+    }
+    const int32_t *to = lofs;
+#pragma unroll
+    for (int k = 0; k < kSortPerLane; ++k) {
+        if (wbase + k * kWave + lane < nnz) {
             col_s[p[k]] = c[k];
             row_s[p[k]] = r[k];
         }
