@@ -327,10 +327,10 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
     constexpr int kSlots = 4096;
     __shared__ int32_t table[kSlots];
     __shared__ uint32_t starts[kFlatTile / 32];  // bit i: element i of the tile is the first of its row
-    __shared__ int32_t count, pairs;
+    __shared__ int32_t count, pairs, lowest, highest;
     for (int i = threadIdx.x; i < kSlots; i += kBlock) table[i] = -1;
     if (threadIdx.x < kFlatTile / 32) starts[threadIdx.x] = 0;
-    if (threadIdx.x == 0) count = 0, pairs = 0;
+    if (threadIdx.x == 0) count = 0, pairs = 0, lowest = 0x7fffffff, highest = 0;
     __syncthreads();
     const int64_t first = (int64_t)t * q.stride;
     // the columns are requested before the searches, so that their latency passes during those
@@ -371,12 +371,19 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
         if (q.row_ptr)
             mine_pairs += i == 0 || c[u] / q.width != left[u] / q.width || (starts[i >> 5] >> (i & 31) & 1u) != 0;
     }
+    if (!q.row_ptr) {
+        int32_t lo = c[0], hi = c[0];
+#pragma unroll
+        for (int u = 1; u < kPer; ++u) lo = c[u] < lo ? c[u] : lo, hi = c[u] > hi ? c[u] : hi;
+        atomicMin(&lowest, lo);
+        atomicMax(&highest, hi);
+    }
     if (mine) atomicAdd(&count, mine);
     if (mine_pairs) atomicAdd(&pairs, mine_pairs);
     __syncthreads();
     if (threadIdx.x == 0) {
         q.out[t] = count;
-        if (q.row_ptr) q.out[64 + t] = pairs;
+        q.out[64 + t] = q.row_ptr ? pairs : highest - lowest;
     }
 }
 __global__ __launch_bounds__(kBlock) void k_sample_columns(SampleArgs q) { sample_columns_tile(q, blockIdx.x); }

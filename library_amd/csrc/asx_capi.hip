@@ -81,9 +81,10 @@ SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
 //   pairs   (row, slice) pairs per stored element, for column slices of 128 KiB of x: the partial
 //           sums the column-sliced kernel would carry through memory.  16 random columns per row
 //           over 32 slices give 0.8, a band matrix about 1 / (row length).
+//   span    columns between a tile's first and last, on average (instead of the pairs, for SpMM).
 struct ColumnSample {
     bool ok;
-    double spread, pairs;
+    double spread, pairs, span;
 };
 constexpr int32_t kSliceBytes = 131072;  // of x per slice: one workgroup of 16 waves per compute unit
 int sample_tiles(int32_t nnz) { return (int)std::min<int64_t>(64, nnz / kFlatTile); }
@@ -95,15 +96,16 @@ ColumnSample sample_result(const int32_t h[128], int32_t nnz, bool with_pairs)
     const int samples = sample_tiles(nnz);
     int64_t distinct = 0, pairs = 0;
     for (int t = 0; t < samples; ++t) distinct += h[t], pairs += h[64 + t];
-    ColumnSample cs{samples > 0, 0.0, 1.0};
+    ColumnSample cs{samples > 0, 0.0, 1.0, 0.0};
     if (samples > 0) cs.spread = (double)distinct / ((double)samples * kFlatTile);
     if (samples > 0 && with_pairs) cs.pairs = (double)pairs / ((double)samples * kFlatTile);
+    if (samples > 0 && !with_pairs) cs.span = (double)pairs / (double)samples;
     return cs;
 }
-// the spread alone, counted now
+// the spread and the span, counted now
 ColumnSample sample_columns(const int32_t *d_col, int32_t nnz, size_t sv, hipStream_t s)
 {
-    const ColumnSample none{false, 0.0, 1.0};
+    const ColumnSample none{false, 0.0, 1.0, 0.0};
     Scratch scratch(s);
     int32_t *h = static_cast<int32_t *>(scratch.pinned());
     if (sample_tiles(nnz) < 1 || !h) return none;
@@ -114,8 +116,6 @@ ColumnSample sample_columns(const int32_t *d_col, int32_t nnz, size_t sv, hipStr
     scratch.idle = true;
     return sample_result(h, nnz, false);
 }
-constexpr double kScatteredMinSpread = 0.5;
-
 constexpr int32_t kSmallNnz = 1 << 18;
 constexpr int64_t kSmallMaxRow = 2048;
 
@@ -265,7 +265,7 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         } else {
             xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
-        return launch_spmm_merge<T>(m, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
+        return launch_spmm_merge<T>(m, nnz, plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T)), ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
                                     ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
                                     plan ? plan->carry_pass != 0 : true,
                                     spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
@@ -427,7 +427,7 @@ int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n
     scratch.idle = true;
     std::memcpy(p->hist, h, sizeof(p->hist));
     std::memcpy(p->stats, h + 33, sizeof(p->stats));
-    if (more) more->sample = samples > 0 ? sample_result(reinterpret_cast<const int32_t *>(h + 64), nnz, true) : ColumnSample{false, 0.0, 1.0};
+    if (more) more->sample = samples > 0 ? sample_result(reinterpret_cast<const int32_t *>(h + 64), nnz, true) : ColumnSample{false, 0.0, 1.0, 0.0};
     *out = p;
     return ASX_STATUS_SUCCESS;
 }
@@ -486,27 +486,32 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             p->workspace_bytes = spmv_merge_layout(m, nnz, sv, false).bytes;
         }
     } else if (kernel == ASX_SPMM_MERGE) {
-        const int32_t items = spmm_segment_items(m, nnz, p->ncols, sv);
-        const size_t ns = (size_t)spmm_segments(m, nnz, items);
-        p->nunits = (int32_t)ns;
-        p->meta_bytes = 2 * (ns + 1) * 4;
-        p->carry_pass = 1;
-        st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
-        // does any row stay cut?  (one int read back; creation syncs anyway)
+        const int32_t usual = spmm_segment_items(m, nnz, p->ncols, sv);
         p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv).bytes;
-        if (!st) st = launch_spmm_splits(m, nnz, items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
-        return st ? st : read_flag();  // which waits
+        // B's rows one after the other, from the start of a line on, as nearly every caller has them
+        const int tile_bytes = spmm_tile_bytes(p->columns, p->n, nullptr, (size_t)p->ncols * sv);
+        p->items = spmm_plan_items(usual, p->columns, spmm_tiling(p->ncols, tile_bytes, sv).groups, m, nnz, p->stats[0]);
+        for (;; p->items = usual) {
+            const size_t ns = (size_t)spmm_segments(m, nnz, p->items);
+            p->nunits = (int32_t)ns;
+            p->meta_bytes = 2 * (ns + 1) * 4;
+            p->carry_pass = 1;
+            st = status_of(pool_malloc(&p->d_meta, p->meta_bytes, false));
+            // does any row stay cut?  (one int read back; creation syncs anyway)
+            if (!st) st = launch_spmm_splits(m, nnz, p->items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
+            if (!st) st = read_flag();
+            if (st || p->items == usual || !p->carry_pass) return st;
+            pool_free(p->d_meta);  // read_flag has waited; the flag stays set, so that the carry pass runs
+            p->d_meta = nullptr;
+        }
     }
     if (!st) st = status_of(hipStreamSynchronize(s));
     return st;
 }
 
-}  // namespace
-
-extern "C" {
-
-int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m, int32_t n,
-                    int32_t nnz, const int32_t *d_row_ptr, int32_t ncols_dense, void *stream)
+// columns: kColumns* of an SpMM plan
+int plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m, int32_t n, int32_t nnz,
+                const int32_t *d_row_ptr, int32_t ncols_dense, int columns, void *stream)
 {
     if (!out) return ASX_STATUS_INVALID_POINTER;
     *out = nullptr;
@@ -526,6 +531,7 @@ int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_
         asx_plan_destroy(p);
         return ASX_STATUS_NOT_SUPPORTED;
     }
+    if (kernel == ASX_SPMM_MERGE && is_spmm) p->columns = columns;
     st = plan_row_ordered(p, kernel, s);
     if (st) {
         asx_plan_destroy(p);
@@ -533,6 +539,16 @@ int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_
     }
     *out = p;
     return ASX_STATUS_SUCCESS;
+}
+
+}  // namespace
+
+extern "C" {
+
+int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m, int32_t n,
+                    int32_t nnz, const int32_t *d_row_ptr, int32_t ncols_dense, void *stream)
+{
+    return plan_create(out, is_spmm, alg, value_type, m, n, nnz, d_row_ptr, ncols_dense, kColumnsUnknown, stream);
 }
 
 int asx_plan_destroy(asx_plan *plan)
@@ -578,12 +594,10 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
     if (probe_blocked) {
         const ColumnSample cs = sample_columns(d_col, nnz, vsize(value_type), (hipStream_t)stream);
         probe_blocked = cs.ok && cs.spread < kScatteredMinSpread;
-        if (cs.ok) columns = probe_blocked ? kColumnsNear : kColumnsScattered;
+        if (cs.ok) columns = spmm_columns(cs.spread, cs.span, (double)nnz / std::max(m, 1), vsize(value_type));
     }
     const auto row_ordered = [&]() {
-        const int st = asx_plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, stream);
-        if (!st && (*out)->alg == ASX_SPMM_MERGE) (*out)->columns = columns;
-        return st;
+        return plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, columns, stream);
     };
     if (!want_blocked && !probe_blocked) return row_ordered();
     if (m < 0 || k < 0 || nnz < 0 || ncols < 1) return ASX_STATUS_INVALID_SIZE;
@@ -868,7 +882,7 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
     }
     hipStream_t s = (hipStream_t)stream;
     asx_plan *p = nullptr;
-    PlanStats ps{ColumnSample{false, 0.0, 1.0}, 0};
+    PlanStats ps{ColumnSample{false, 0.0, 1.0, 0.0}, 0};
     const bool looks = alg == ASX_SPMV_DEFAULT && d_col && d_val && m > 0 && n > 0 && nnz > 0;  // DEFAULT with the columns at hand
     const bool may_regroup = looks && nnz >= kRegroupMinNnz;
     const int32_t *sampled = looks || alg == ASX_SPMV_SLICED ? d_col : nullptr;

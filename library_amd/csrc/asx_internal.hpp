@@ -19,6 +19,7 @@ constexpr int kFlatTile = 1024;                            // stored elements pe
 constexpr int kLongRow = 8192;  // DEFAULT (with a plan) switches to the merge-path kernel above this row length
 // SpMM: merge items (rows + stored elements) per wave
 constexpr int kSpmmSegmentSmall = 128, kSpmmSegmentMedium = 256, kSpmmSegmentLarge = 512;
+constexpr double kScatteredMinSpread = 0.5;  // of a column sample: from here on the columns count as scattered
 
 inline int status_of(hipError_t e)
 {
@@ -102,7 +103,7 @@ template <typename T>
 int launch_spmm_row(int32_t m, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col,
                     const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s);
 template <typename T>
-int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
+int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
                       bool carry_pass, int tile_bytes, hipStream_t s);
@@ -245,20 +246,35 @@ inline int32_t merge_tiles(int32_t m, int32_t nnz) { return (int32_t)ceil_div64(
 constexpr int32_t kFlatSelfSearchMost = 8192;
 inline int32_t flat_tiles(int32_t nnz) { int32_t t = (int32_t)ceil_div64(nnz, kFlatTile); return t < 1 ? 1 : t; }
 inline int32_t stream_blocks(int32_t nnz) { return (int32_t)ceil_div64(nnz, kStreamTile); }
-// What an SpMM plan knows of A's columns: nothing, that neighbouring rows share most of them, or that they do not.
-enum { kColumnsUnknown = 0, kColumnsNear = 1, kColumnsScattered = 2 };
+// What an SpMM plan knows of A's columns: nothing; that neighbouring rows share most of them (stencils, narrow bands); that
+// they share few, but a stretch of rows stays within a part of B that an L2 can keep; that they lie all over B.
+enum { kColumnsUnknown = 0, kColumnsNear = 1, kColumnsScattered = 2, kColumnsSpread = 3 };
 // How many bytes of a row of B a wave takes at once; the tiles of columns are worked off one after the other, so what an
 // L2 (4 MB, one per XCD) or L1 (32 KB) can keep of B is the narrower the more rows of it.
 //   Rows of B that start on 128-byte lines can be cut between lines: 128 bytes while all of B's tile is small
 //   (k = 30000, 256 columns fp32: 58 us against 77 with 256 bytes and 102 with 1 KB; k = 100000: 173 / 197 / 228;
-//   k = 200000: 459 / 446 / 499), else 256 (fewer reads of A; near columns: 2-D stencil 193 us against 214).
+//   k = 200000: 459 / 446 / 499) or the part of it that a stretch of rows needs is, unless that fits 256 bytes wide as well
+//   (64 columns fp64, 20 per row within 30000 of the diagonal: 187 us against 232; within 1000, 128 columns: 128 against
+//   118), else 256 (fewer reads of A; near columns: 2-D stencil 193 us against 214).
 //   Other rows begin and end inside lines wherever they are cut, 100 columns fp32 are 4.1 lines in one piece and 5.1 in
 //   two: 1 KB for scattered columns, 512 bytes for near ones (7-point stencil, 200 columns: 223 us against 244) or
 //   when nothing is known.
+constexpr int64_t kSmallTileOfB = 16 << 20;
 inline int spmm_tile_bytes(int columns, int64_t k, const void *B, size_t pitch)
 {
-    if (pitch % 128 == 0 && (uintptr_t)B % 128 == 0) return columns != kColumnsNear && k * 128 <= (16 << 20) ? 128 : 256;
+    if (pitch % 128 == 0 && (uintptr_t)B % 128 == 0)
+        return columns == kColumnsSpread || (columns != kColumnsNear && k * 128 <= kSmallTileOfB) ? 128 : 256;
     return columns == kColumnsScattered ? 1024 : 512;
+}
+// spread: distinct 128-byte lines of a vector of the value type per stored element of a sample tile; span: columns between a
+// tile's first and last; mean: elements per row.  Rows that share little touch more than 4 new columns each, counting whole
+// lines (2-D stencils 3.4, 20 per row within 300 and 1000 of the diagonal 13 and 40); shorter ones than 8 do not repay the
+// second read of A (4 per row within 10000: 66 us against 64), longer ones than 30 leave lane groups idle (32: 352 / 352).
+inline int spmm_columns(double spread, double span, double mean, size_t sv)
+{
+    if (mean >= 8.0 && mean <= 30.0 && spread * mean * (128 / sv) > 4.0 && span * 256 > (4 << 20) && span * 128 <= kSmallTileOfB)
+        return kColumnsSpread;
+    return spread < kScatteredMinSpread ? kColumnsNear : kColumnsScattered;
 }
 
 // Merge items per wave of the SpMM merge kernel.  Longer segments leave fewer carries and keep the
@@ -271,6 +287,42 @@ inline int32_t spmm_segment_items(int32_t m, int32_t nnz, int32_t ncols, size_t 
     const int64_t items = (int64_t)m + nnz;
     if (items < (int64_t)kSpmmSegmentMedium * 4096) return kSpmmSegmentSmall;
     return sv == 4 && ncols > 32 && items >= (int64_t)kSpmmSegmentLarge * 4096 ? kSpmmSegmentLarge : kSpmmSegmentMedium;
+}
+// Columns of B a lane takes, tiles of columns, and lane groups of a wave (which take a row of A each) when a wave takes at most
+// tile_bytes of a row of B.
+struct SpmmTiling {
+    int vec;
+    int64_t tiles;
+    int log_lanes, groups;
+};
+inline SpmmTiling spmm_tiling(int64_t ncols, int tile_bytes, size_t sv)
+{
+    SpmmTiling t;
+    t.vec = ncols >= (int64_t)(16 / sv) ? (int)(16 / sv) : ncols >= 2 ? 2 : 1;
+    const int64_t most = tile_bytes / (int64_t)sv;
+    t.tiles = ceil_div64(ncols, most > t.vec ? most : t.vec);
+    const int64_t lanes = ceil_div64(ceil_div64(ncols, t.tiles), t.vec);
+    for (t.log_lanes = 0; ((int64_t)1 << t.log_lanes) < lanes;) ++t.log_lanes;
+    t.groups = kWave >> t.log_lanes;
+    return t;
+}
+// Rows of up to this many elements are taken by one lane group each, longer ones by all groups together.  32 against 16 with
+// up to 4 groups: 40 columns fp64, 20 per row within 2000 of the diagonal 170 -> 148 us, 64 columns fp32 over scattered rows
+// of 25 141 -> 135 us, power-law rows 207.7 -> 204.1 us.
+constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 4 ? 32 : 64; }
+// Segments of a plan whose columns are near or spread, where they leave no row cut (carries of more segments would not fit the
+// workspace that callers size without a plan).  They are short, so that fewer rows of B are in use at a time, and where rows are
+// of one length (the longest at most a quarter above the mean) they hold as many as the wave's groups take in full turns.
+// 64 columns fp32, 20 per row within 1000 of the diagonal: 94.9 us with segments of 512 items, 54.2 with two turns of 84;
+// 7-point stencil 78.7 -> 59.7, 5-point stencil 128.7 -> 85.7; 13 per row 50.2 -> 42.3.
+inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest)
+{
+    if (columns != kColumnsNear && columns != kColumnsSpread) return usual;
+    const int32_t least = usual == kSpmmSegmentLarge ? kSpmmSegmentSmall : usual;
+    const int64_t turn = groups * (longest + 1);
+    const int32_t most = usual == kSpmmSegmentLarge && turn > kSpmmSegmentSmall ? kSpmmSegmentMedium : least;
+    if (longest > spmm_dealt(groups) || turn > most || 4 * (longest + 1) * m > 5 * ((int64_t)m + nnz)) return least;
+    return (int32_t)(most / turn * turn);
 }
 inline int32_t spmm_segments(int32_t m, int32_t nnz, int32_t items) { return (int32_t)ceil_div64((int64_t)m + nnz, items); }
 
@@ -295,6 +347,7 @@ struct asx_plan {
     int carry_pass;  // flat and SpMM merge kernel: 0 when no row is cut between units of work
     int32_t nwide, nlong, long_len;  // vector kernel: d_meta lists the long rows (asx::LongRows)
     int columns;     // SpMM merge kernel: kColumns*
+    int32_t items;   // SpMM merge kernel: merge items per segment
     int64_t hist[33];
     int64_t stats[4];
     size_t workspace_bytes;

@@ -260,7 +260,7 @@ __device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, 
     return acc;
 }
 
-// One wave per segment and tile of columns.  A lane holds VEC columns (16 bytes where N allows), so
+// One wave per segment (of `items` merge items, at most SEG) and tile of columns.  A lane holds VEC columns (16 bytes where N allows), so
 // G = 2^LOGG lanes span a tile and the wave's NG = 64 / G groups work on different stored elements at
 // once: one load instruction fetches NG rows of B.  (A row of B per instruction, 4 bytes per lane,
 // gets 110 G lines/s from an L2, 16 bytes per lane 240 G; with 8 columns in fp64 such a kernel left 56
@@ -275,7 +275,7 @@ __device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, 
 // Consecutive segments run on one XCD, whose L2 then fetches the rows of B that neighbouring rows
 // of A share once.
 template <typename T, int VEC, int LOGG, int SEG>
-__global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, int32_t nseg, int32_t ncols, T alpha,
+__global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
                                                        const int32_t *__restrict__ row_ptr,
                                                        const int32_t *__restrict__ col, const T *__restrict__ val,
                                                        const T *__restrict__ B, int64_t ldb, T beta,
@@ -286,7 +286,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     typedef typename VecOf<T, VEC>::type V;
     constexpr int G = 1 << LOGG, NG = kWave / G;
     constexpr int U = 8;  // rows of B a lane has in flight
-    constexpr int kDealt = NG == 1 ? 1 << 30 : NG <= 4 ? 16 : NG <= 8 ? 32 : 64;
+    constexpr int kDealt = spmm_dealt(NG);
     constexpr int kElems = 2 * SEG, kEnds = SEG + kWave;
     __shared__ int32_t s_col_all[kBlock / kWave][kElems];
     __shared__ T s_val_all[kBlock / kWave][kElems];
@@ -308,7 +308,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     if (xs)  // uniform
         x0 = xs[seg], y0 = ys[seg], x1 = xs[seg + 1], y1 = ys[seg + 1];
     else
-        segment_ends(row_ptr, m, nnz, SEG, nseg, seg, x0, y0, x1, y1);
+        segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1);
     const int32_t nel = y1 - y0 < kElems ? y1 - y0 : kElems, nrow = x1 - x0 < kEnds ? x1 - x0 : kEnds;
     int32_t *s_col = s_col_all[w];
     T *s_val = s_val_all[w];
@@ -391,12 +391,13 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
         }
     }
     const int32_t k = __builtin_amdgcn_readfirstlane(s_end[nrow]);
-    const bool has_tail = nel > k;  // row x1 continues past the segment end
+    // row x1 continues past the segment end (without a carry pass: elements behind the last row's end, which count nowhere)
+    const bool has_tail = nel > k && carry_row;
     if (has_tail) {
         const V acc = together(k, nel);
         if (stores) *(V *)(carry + seg * ncols + c) = acc;
     }
-    if (lane == 0 && blockIdx.y == 0) carry_row[seg] = has_tail ? x1 : -1;
+    if (carry_row && lane == 0 && blockIdx.y == 0) carry_row[seg] = has_tail ? x1 : -1;
 }
 
 // Every wave looks at kFixupSegs consecutive segments (one lane each) for the first segment of a run
@@ -467,15 +468,14 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge_fixup(int32_t m, int32_t 
 // N is cut into equal tiles of at most tile_bytes of a row of B (every tile at least VEC wide); lanes per row of B: the
 // smallest power of two that spans a tile at VEC columns each.
 template <typename T, int VEC, int SEG>
-static void launch_merge_width(int tile_bytes, int32_t m, int32_t nnz, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
+static void launch_merge_width(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
                                const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
                                T *carry, int32_t *carry_row, hipStream_t s)
 {
-    const int64_t tiles = ceil_div64(ncols, std::max<int64_t>(tile_bytes / (int64_t)sizeof(T), VEC)), lanes = ceil_div64(ceil_div64(ncols, tiles), VEC);
-    const dim3 grid((unsigned)(ceil_div64(ceil_div64(nseg, kBlock / kWave), kXcds) * kXcds), (unsigned)tiles);
+    const dim3 grid((unsigned)(ceil_div64(ceil_div64(nseg, kBlock / kWave), kXcds) * kXcds), (unsigned)tiling.tiles);
 #define ASX_WIDTH(LOGG)                                                                                              \
-    if (lanes <= (1 << LOGG)) {                                                                                      \
-        hipLaunchKernelGGL((k_spmm_merge<T, VEC, LOGG, SEG>), grid, dim3(kBlock), 0, s, m, nnz, nseg, ncols, alpha, row_ptr, col, \
+    if (tiling.log_lanes <= LOGG) {                                                                                      \
+        hipLaunchKernelGGL((k_spmm_merge<T, VEC, LOGG, SEG>), grid, dim3(kBlock), 0, s, m, nnz, items, nseg, ncols, alpha, row_ptr, col, \
                            val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);                                     \
         return;                                                                                                      \
     }
@@ -492,34 +492,36 @@ static void launch_merge_width(int tile_bytes, int32_t m, int32_t nnz, int32_t n
 }
 
 template <typename T, int SEG>
-static void launch_merge_seg(int tile_bytes, int32_t m, int32_t nnz, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
+static void launch_merge_seg(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
                              const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
                              T *carry, int32_t *carry_row, hipStream_t s)
 {
     constexpr int kFull = 16 / sizeof(T);
-    if (ncols >= kFull)
-        launch_merge_width<T, kFull, SEG>(tile_bytes, m, nnz, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
-    else if (ncols >= 2)
-        launch_merge_width<T, 2, SEG>(tile_bytes, m, nnz, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+    if (tiling.vec == kFull)
+        launch_merge_width<T, kFull, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+    else if (tiling.vec == 2)
+        launch_merge_width<T, 2, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
     else
-        launch_merge_width<T, 1, SEG>(tile_bytes, m, nnz, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_merge_width<T, 1, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
 }
 
 template <typename T>
-int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
+int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
                       bool carry_pass, int tile_bytes, hipStream_t s)
 {
     if (m <= 0 || ncols <= 0) return ASX_STATUS_SUCCESS;
-    const int32_t items = spmm_segment_items(m, nnz, ncols, sizeof(T)), nseg = spmm_segments(m, nnz, items);
+    const int32_t nseg = spmm_segments(m, nnz, items);
+    const SpmmTiling tiling = spmm_tiling(ncols, tile_bytes, sizeof(T));
+    if (!carry_pass) carry = nullptr, carry_row = nullptr;  // no row is cut: nothing is left for the pass
     const auto launch = [&](auto seg_) {
-        launch_merge_seg<T, decltype(seg_)::value>(tile_bytes, m, nnz, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
+        launch_merge_seg<T, decltype(seg_)::value>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
                                                    carry_row, s);
     };
-    if (items == kSpmmSegmentSmall)
+    if (items <= kSpmmSegmentSmall)
         launch(Int<kSpmmSegmentSmall>{});
-    else if (items == kSpmmSegmentMedium)
+    else if (items <= kSpmmSegmentMedium)
         launch(Int<kSpmmSegmentMedium>{});
     else if constexpr (sizeof(T) == 4)
         launch(Int<kSpmmSegmentLarge>{});
@@ -532,7 +534,7 @@ int launch_spmm_merge(int32_t m, int32_t nnz, int32_t ncols, T alpha, const int3
 #define ASX_INST(T)                                                                                  \
     template int launch_spmm_row<T>(int32_t, int32_t, T, const int32_t *, const int32_t *, const T *, \
                                     const T *, int64_t, T, T *, int64_t, hipStream_t);               \
-    template int launch_spmm_merge<T>(int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
+    template int launch_spmm_merge<T>(int32_t, int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
                                       const T *, const T *, int64_t, T, T *, int64_t, const int32_t *, \
                                       const int32_t *, T *, int32_t *, bool, int, hipStream_t);
 ASX_INST(float)
