@@ -58,8 +58,8 @@ MEASURED_TRAFFIC_BYTES = {
     "uniform16_f64": 478_017_157,  # profiles/spmv_sliced_uniform16_f64.md
     "powerlaw_f64": 730_483_835,  # profiles/spmv_sliced_powerlaw_f64.md
     "stencil5_f64": 1_142_530_786,  # profiles/spmv_window_stencil5_f64.md
-    "spmm_zipf_f32": 4_965_331_333,  # profiles/spmm_merge_spmm_zipf_f32.md
-    "spmm_banded_f32": 1_870_263_890,  # profiles/spmm_blocked_spmm_banded_f32.md
+    "spmm_zipf_f32": 4_923_160_191,  # profiles/spmm_merge_spmm_zipf_f32.md
+    "spmm_banded_f32": 1_322_809_550,  # profiles/spmm_blocked_spmm_banded_f32.md
     "stencil7_f64": 1_630_404_585,  # profiles/spmv_window_stencil7_256_f64.md
 }
 
