@@ -1,10 +1,8 @@
 // CSR x dense SpMM for gfx950, C = alpha*A*B + beta*C with B (k x N) and C (m x N) row-major.
 //
-// Lanes of a wavefront are the 64 columns of a column tile, so every read of a row of B and
-// every access to a row of C is one fully coalesced 256-byte (fp32) / 512-byte (fp64) access.
-// The stored elements of A are read 64 at a time, one per lane, and broadcast lane by lane
-// through v_readlane, which also makes the row address of B wave-uniform (scalar base +
-// lane offset).
+// Every access to a row of B or C covers consecutive columns: 64 lanes of one element in the row kernel, whose stored elements
+// are read 64 at a time and broadcast through v_readlane (the address of the row of B is then wave-uniform), 16 bytes a lane
+// in the merge kernel, whose lane groups work on different rows of A.
 //
 //   row   : one wave per (row, column tile).  Simple; long rows serialise.
 //   merge : one wave per segment of consecutive items of the merge path over
