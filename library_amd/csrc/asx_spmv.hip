@@ -83,8 +83,10 @@ __device__ __forceinline__ T strided_dot(int64_t k, int64_t e, const int32_t *__
     return (s[0] + s[1]) + (s[2] + s[3]);
 }
 
-// The rows of workgroup b, a lane group each; rows of long_len elements or more are somebody else's.
-template <typename T, int LANES>
+// The rows of workgroup b, a lane group each; with a list, rows of long_len elements or more are somebody else's.  Without
+// one a row may hold everything that int32 offsets can count (2^31 - 1 elements): nothing is compared, and positions are
+// unsigned, so that the step past the row's end does not overflow.
+template <typename T, int LANES, bool LISTED>
 __device__ __forceinline__ void vector_rows(int64_t b, int32_t m, T alpha, const int32_t *__restrict__ row_ptr,
                                             const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ x,
                                             T beta, T *__restrict__ y, int32_t long_len)
@@ -94,9 +96,9 @@ __device__ __forceinline__ void vector_rows(int64_t b, int32_t m, T alpha, const
     T sum = T(0);
     bool mine = row < m;
     if (mine) {
-        const int32_t e = row_ptr[row + 1];
-        int32_t k = row_ptr[row];
-        mine = e - k < long_len;
+        const uint32_t e = (uint32_t)row_ptr[row + 1];
+        uint32_t k = (uint32_t)row_ptr[row];
+        mine = !LISTED || (int32_t)(e - k) < long_len;
         k = mine ? k + lane : e;
         // two independent chains per lane keep more gathers in flight on long rows
         T s0 = T(0), s1 = T(0);
@@ -119,7 +121,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_vector(int32_t m, T alpha,
                                                         const T *__restrict__ x, T beta,
                                                         T *__restrict__ y)
 {
-    vector_rows<T, LANES>(blockIdx.x, m, alpha, row_ptr, col, val, x, beta, y, 0x7fffffff);
+    vector_rows<T, LANES, false>(blockIdx.x, m, alpha, row_ptr, col, val, x, beta, y, 0);
 }
 
 // The same with a plan's list of long rows: nwide rows for a workgroup each, then nlong for a wave each, so that no lane group
@@ -151,7 +153,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_vector_long(int32_t m, T alpha,
         const T sum = group_sum<kWave>(strided_dot<T, kWave>((int64_t)s + lane, e, col, val, x));
         if (lane == 0) y[r] = axpby_out<T>(alpha, sum, beta, y, r);
     } else {
-        vector_rows<T, LANES>(b - nblocks, m, alpha, row_ptr, col, val, x, beta, y, long_len);
+        vector_rows<T, LANES, true>(b - nblocks, m, alpha, row_ptr, col, val, x, beta, y, long_len);
     }
 }
 

@@ -40,3 +40,15 @@ def test_long_row_list(dtype, lanes, wide):
         bound = (lens + 3) * u * 1.5 * size + 3 * u * np.abs(beta * y0)
         assert np.all(np.abs(y.cpu().numpy() - (1.5 * exact + beta * y0)) <= bound), (lanes, beta)
     plan.destroy()
+
+
+def test_one_row_of_every_element_int32_offsets_can_count():
+    """2^31 - 1 ones: 64 lanes with two sums each add 2^24 of them at most, exact in float32; joined they round to 2^31."""
+    nnz = 2**31 - 1
+    row_ptr = torch.tensor([0, nnz], dtype=torch.int32, device="cuda")
+    col = torch.zeros(nnz, dtype=torch.int32, device="cuda")
+    val = torch.ones(nnz, dtype=torch.float32, device="cuda")
+    x, y = torch.ones(1, device="cuda"), torch.full((1,), -7.0, device="cuda")
+    capi.spmv(row_ptr, col, val, x, y, 1.0, 0.0, alg=capi.SPMV_VECTOR)
+    torch.cuda.synchronize()
+    assert y.item() == 2.0**31
