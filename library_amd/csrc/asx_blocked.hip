@@ -250,23 +250,29 @@ struct ColsOf {
     typedef T type __attribute__((ext_vector_type(VEC), aligned(sizeof(T))));
 };
 
+// Waves a SIMD by the bytes of a row of B that a lane holds: two batches of wide rows want the registers (two waves, 200
+// columns fp64: 29 us against 38 with one), and where 16 bytes a lane leave room for eight waves, six keep the rows of B
+// that neighbours share longer in the L2 (65 per row, N = 64, fp32: 226 us against 230).
+constexpr int blocked_waves(size_t bytes) { return bytes > 32 ? 2 : bytes > 16 ? 3 : bytes == 16 ? 6 : 8; }
+
 // One wave per (block row, tile of up to 16 * VEC * NT columns of C).  Lane (kq, j) = (lane / 16, lane % 16) loads, of row
 // kq of a block's four rows of B, the VEC columns from j * VEC on (16 bytes where N allows: one instruction
 // fetches the four rows of 64 fp32 columns, where 4 bytes a lane took four) and feeds its v-th column to the v-th
 // MFMA: accumulator v holds columns v, VEC + v, 2 VEC + v, ..., so a lane ends up with VEC consecutive columns of
 // four rows of C.
 // U blocks are in flight while the U before them are multiplied; every load is unconditional (past the end the
-// last block is fetched again, a quad that reaches over B's last row repeats that row against A's zeros).
+// last block is fetched again, a quad that reaches over B's last row repeats that row).  What is fetched so is not
+// multiplied, or an infinity in B would meet other zeros of A than those that fill its own block: the last batch leaves
+// out blocks past the end, and in the last block, the only one that can hold the partial quad, rows past B's end are zeros.
 // Lanes past the last column repeat the last VEC columns and store nothing; where the width is no multiple of
 // VEC the last lane overlaps the one before it (same bits, same wave).
 // Consecutive block rows run on one XCD: they share most of their rows of B, which its L2 then fetches once.
 // Bound by memory: 65 per row, N = 64, fp32 (1.2 GB past the L2s with C read and written): 312 -> 228 us.
 template <typename T, int VEC, int NT>
-__global__ __launch_bounds__(kBlock) void k_spmm_blocked(int32_t m, int32_t kdim, int32_t ncols, int32_t nbrows,
-                                                         T alpha, const int32_t *__restrict__ brow_ptr,
-                                                         const int32_t *__restrict__ bcol,
-                                                         const T *__restrict__ bval, const T *__restrict__ B,
-                                                         int64_t ldb, T beta, T *__restrict__ C, int64_t ldc)
+__global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2, blocked_waves(VEC * NT * sizeof(T)))))
+void k_spmm_blocked(int32_t m, int32_t kdim, int32_t ncols, int32_t nbrows, T alpha, const int32_t *__restrict__ brow_ptr,
+                    const int32_t *__restrict__ bcol, const T *__restrict__ bval, const T *__restrict__ B, int64_t ldb,
+                    T beta, T *__restrict__ C, int64_t ldc)
 {
     typedef typename Acc4<T>::type acc_t;
     typedef typename ColsOf<T, VEC>::type V;
@@ -305,26 +311,42 @@ __global__ __launch_bounds__(kBlock) void k_spmm_blocked(int32_t m, int32_t kdim
             for (int t = 0; t < NT; ++t) q.b[u][t] = *(const V *)(row + col[t]);
         }
     };
-    const auto multiply = [&](const Batch &q, int32_t first) {
+    const auto multiply = [&](T a, const V (&bq)[NT]) {
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) acc[t * VEC + v] = mfma16x16x4(a, bq[t][v], acc[t * VEC + v]);
+    };
+    const auto multiply_all = [&](const Batch &q) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) multiply(q.a[u], q.b[u]);
+    };
+    const auto multiply_last = [&](Batch &q, int32_t first) {
+        const bool there = bcol[last] * 4 + kq < kdim;
 #pragma unroll
         for (int u = 0; u < U; ++u) {
-            const T a = first + u < b1 ? q.a[u] : T(0);
+            const bool counts = first + u < last || (first + u == last && there);
 #pragma unroll
-            for (int t = 0; t < NT; ++t)
-#pragma unroll
-                for (int v = 0; v < VEC; ++v) acc[t * VEC + v] = mfma16x16x4(a, q.b[u][t][v], acc[t * VEC + v]);
+            for (int t = 0; t < NT; ++t) q.b[u][t] = counts ? q.b[u][t] : (V)T(0);
+            multiply(counts ? q.a[u] : T(0), q.b[u]);
         }
     };
     if (b0 < b1) {
         fetch(cur, b0);
         int32_t b = b0;
-        for (; b + U < b1; b += 2 * U) {  // uniform
+        for (; b + 2 * U < b1; b += 2 * U) {  // uniform
             fetch(next, b + U);
-            multiply(cur, b);
+            multiply_all(cur);
             fetch(cur, b + 2 * U);
-            multiply(next, b + U);
+            multiply_all(next);
         }
-        if (b < b1) multiply(cur, b);
+        if (b + U < b1) {
+            fetch(next, b + U);
+            multiply_all(cur);
+            multiply_last(next, b + U);
+        } else {
+            multiply_last(cur, b);
+        }
     }
     // every old value before the first store: the overlapping columns may belong to two tiles t of one lane row
     V old[NT][4];
