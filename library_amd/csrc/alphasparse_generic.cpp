@@ -292,10 +292,10 @@ const asx_plan *kept_plan(const _alphasparseSpMatDescr *A, alphasparseOperation_
 
 void free_derived(DerivedCsr &d)
 {
-    asx::pool_wait(d.row_ptr);  // calls that read the copy may still be running on any stream
-    asx::pool_free(d.row_ptr);
-    asx::pool_free(d.col);
-    if (d.transposed) asx::pool_free(d.val);
+    const bool idle = asx::pool_wait(d.row_ptr);  // calls that read the copy may still be running on any stream
+    asx::pool_free(d.row_ptr, idle);
+    asx::pool_free(d.col, idle);
+    if (d.transposed) asx::pool_free(d.val, idle);
     d.row_ptr = d.col = nullptr;
     d.val = nullptr;
 }

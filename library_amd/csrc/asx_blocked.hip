@@ -137,6 +137,7 @@ int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, con
     void *tmp = nullptr;
     size_t tmp_sort = 0, tmp_scan = 0, tmp_bytes = 0;
     int32_t nblocks = 0;
+    Scratch scratch(s);
     const int32_t nbrows = (int32_t)ceil_div64(m, 16);
     out->nbrows = nbrows;
     out->nblocks = 0;
@@ -148,16 +149,16 @@ int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, con
     out->nnz = nnz;
     const unsigned g_nnz = (unsigned)ceil_div64(nnz > 0 ? nnz : 1, kBlock);
     if (nnz > 0) {
-        ASX_TRY(pool_malloc(&keys, sizeof(uint64_t) * (size_t)nnz, true));
-        ASX_TRY(pool_malloc(&keys2, sizeof(uint64_t) * (size_t)nnz, true));
-        ASX_TRY(pool_malloc(&idx, sizeof(int32_t) * (size_t)nnz, true));
-        ASX_TRY(pool_malloc(&idx2, sizeof(int32_t) * (size_t)nnz, true));
-        ASX_TRY(pool_malloc(&head, sizeof(int32_t) * (size_t)nnz, true));
-        ASX_TRY(pool_malloc(&block_of, sizeof(int32_t) * (size_t)nnz, true));
+        ASX_TRY(scratch.take(&keys, sizeof(uint64_t) * (size_t)nnz));
+        ASX_TRY(scratch.take(&keys2, sizeof(uint64_t) * (size_t)nnz));
+        ASX_TRY(scratch.take(&idx, sizeof(int32_t) * (size_t)nnz));
+        ASX_TRY(scratch.take(&idx2, sizeof(int32_t) * (size_t)nnz));
+        ASX_TRY(scratch.take(&head, sizeof(int32_t) * (size_t)nnz));
+        ASX_TRY(scratch.take(&block_of, sizeof(int32_t) * (size_t)nnz));
         ASX_TRY(rocprim::radix_sort_pairs(nullptr, tmp_sort, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
         ASX_TRY(rocprim::inclusive_scan(nullptr, tmp_scan, head, block_of, (size_t)nnz, rocprim::plus<int32_t>(), s));
         tmp_bytes = tmp_sort > tmp_scan ? tmp_sort : tmp_scan;
-        ASX_TRY(pool_malloc(&tmp, tmp_bytes, true));
+        ASX_TRY(scratch.take(&tmp, tmp_bytes));
         hipLaunchKernelGGL(k_block_keys, dim3(g_nnz), dim3(kBlock), 0, s, row_ptr, col, m, nnz, keys, idx);
         ASX_TRY(rocprim::radix_sort_pairs(tmp, tmp_sort, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
         hipLaunchKernelGGL(k_block_heads, dim3(g_nnz), dim3(kBlock), 0, s, keys2, nnz, head);
@@ -169,7 +170,7 @@ int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, con
     ASX_TRY(pool_malloc(&out->brow_ptr, sizeof(int32_t) * ((size_t)nbrows + 1), false));
     ASX_TRY(pool_malloc(&out->bcol, sizeof(int32_t) * (size_t)(nblocks > 0 ? nblocks : 1), false));
     ASX_TRY(pool_malloc(&out->bval, sizeof(T) * 64 * (size_t)(nblocks > 0 ? nblocks : 1), false));
-    ASX_TRY(pool_malloc(&bkey, sizeof(uint64_t) * (size_t)(nblocks > 0 ? nblocks : 1), true));
+    ASX_TRY(scratch.take(&bkey, sizeof(uint64_t) * (size_t)(nblocks > 0 ? nblocks : 1)));
     if (nblocks > 0) {
         ASX_TRY(pool_malloc(&out->upd_src, sizeof(int32_t) * (size_t)nnz, false));
         ASX_TRY(pool_malloc(&out->upd_dst, sizeof(int64_t) * (size_t)nnz, false));
@@ -186,23 +187,16 @@ int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, con
     }
     ASX_TRY(hipGetLastError());
     ASX_TRY(hipStreamSynchronize(s));
+    scratch.idle = true;
 done:
-    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
-    for (void *p : {(void *)keys, (void *)keys2, (void *)idx, (void *)idx2, (void *)head, (void *)block_of, tmp,
-                    (void *)bkey})
-        pool_free(p);
-    if (st) free_blocked(out);
+    if (st) free_blocked(out, scratch.settle());
     return st;
 }
 #undef ASX_TRY
 
-void free_blocked(BlockedMatrix *b)
+void free_blocked(BlockedMatrix *b, bool idle)
 {
-    pool_free(b->brow_ptr);
-    pool_free(b->bcol);
-    pool_free(b->bval);
-    pool_free(b->upd_src);
-    pool_free(b->upd_dst);
+    for (void *q : {(void *)b->brow_ptr, (void *)b->bcol, b->bval, (void *)b->upd_src, (void *)b->upd_dst}) pool_free(q, idle);
     b->brow_ptr = nullptr;
     b->bcol = nullptr;
     b->bval = nullptr;

@@ -501,7 +501,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             if (!st) st = launch_spmm_splits(m, nnz, p->items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
             if (!st) st = read_flag();
             if (st || p->items == usual || !p->carry_pass) return st;
-            pool_free(p->d_meta);  // read_flag has waited; the flag stays set, so that the carry pass runs
+            pool_free(p->d_meta, true);  // read_flag has waited; the flag stays set, so that the carry pass runs
             p->d_meta = nullptr;
         }
     }
@@ -555,13 +555,13 @@ int asx_plan_destroy(asx_plan *plan)
 {
     if (!plan) return ASX_STATUS_SUCCESS;
     // calls through the plan may still be running on any stream
-    pool_wait(plan->d_counters ? (const void *)plan->d_counters : plan->blocked.brow_ptr);
-    pool_free(plan->d_meta);
-    pool_free(plan->d_counters);
-    pool_free(plan->d_checksum_parts);
-    free_blocked(&plan->blocked);
-    free_sliced(&plan->sliced);
-    free_window(&plan->window);
+    const bool idle = pool_wait(plan->d_counters ? (const void *)plan->d_counters : plan->blocked.brow_ptr);
+    pool_free(plan->d_meta, idle);
+    pool_free(plan->d_counters, idle);
+    pool_free(plan->d_checksum_parts, idle);
+    free_blocked(&plan->blocked, idle);
+    free_sliced(&plan->sliced, idle);
+    free_window(&plan->window, idle);
     delete plan;
     return ASX_STATUS_SUCCESS;
 }
@@ -611,12 +611,12 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
     if (st) return st;
     const double fill = bm.nblocks > 0 ? (double)nnz / (64.0 * (double)bm.nblocks) : 0.0;
     if (!want_blocked && fill < blocked_min_fill((size_t)ncols * vsize(value_type))) {
-        free_blocked(&bm);
+        free_blocked(&bm, true);
         return row_ordered();
     }
     asx_plan *p = new (std::nothrow) asx_plan();
     if (!p) {
-        free_blocked(&bm);
+        free_blocked(&bm, true);
         return ASX_STATUS_ALLOC_FAILED;
     }
     std::memset(p, 0, sizeof(*p));
@@ -793,7 +793,7 @@ int plan_add_slices(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
     const int st = build_sliced<T>(p->m, p->n, p->nnz, (int32_t)(kSliceBytes / sizeof(T)), rpw, cus, d_row_ptr, d_col,
                                    d_val, &sm, s);
     if (st) return st;
-    pool_free(p->d_meta);
+    pool_free(p->d_meta, true);
     p->d_meta = nullptr;
     p->meta_bytes = 0;
     p->alg = ASX_SPMV_SLICED;
@@ -820,7 +820,7 @@ int plan_add_window(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
     const int st = build_window<T>(p->m, p->n, p->nnz, cus * (sizeof(T) == 4 ? 2 : 1), sizeof(T) == 4 || follows_values, d_row_ptr,
                                    d_col, d_val, &wm, s);
     if (st) return st;
-    pool_free(p->d_meta);
+    pool_free(p->d_meta, true);
     p->d_meta = nullptr;
     p->meta_bytes = 0;
     p->alg = ASX_SPMV_WINDOW;
@@ -931,7 +931,7 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
                     WindowMatrix built = p->window;
                     p->window = WindowMatrix{};
                     if (rows || add_slices(cs.pairs) == ASX_STATUS_SUCCESS) {
-                        free_window(&built);
+                        free_window(&built, true);
                         done = !rows;
                     } else {
                         p->window = built, p->alg = ASX_SPMV_WINDOW;

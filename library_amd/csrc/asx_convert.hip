@@ -428,18 +428,19 @@ int csr_transpose(int32_t m, int32_t n, int32_t nnz, int32_t base, const int32_t
     size_t tmp_bytes = 0;
     const unsigned grid = (unsigned)ceil_div64(nnz, kBlock);
     const int end_bit = 32 + bits_for(n);
+    Scratch scratch(s);
 #define ASX_TRY(expr)             \
     do {                          \
         st = status_of(expr);     \
-        if (st) goto done;        \
+        if (st) return st;        \
     } while (0)
-    ASX_TRY(pool_malloc(&keys, sizeof(uint64_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&keys2, sizeof(uint64_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&idx, sizeof(int32_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&idx2, sizeof(int32_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&trow, sizeof(int32_t) * (size_t)nnz, true));
+    ASX_TRY(scratch.take(&keys, sizeof(uint64_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&keys2, sizeof(uint64_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&idx, sizeof(int32_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&idx2, sizeof(int32_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&trow, sizeof(int32_t) * (size_t)nnz));
     ASX_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)end_bit, s));
-    ASX_TRY(pool_malloc(&tmp, tmp_bytes, true));
+    ASX_TRY(scratch.take(&tmp, tmp_bytes));
     hipLaunchKernelGGL(k_transpose_keys, dim3(grid), dim3(kBlock), 0, s, row_ptr, col, m, nnz, base, keys, idx);
     ASX_TRY(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)end_bit, s));
     hipLaunchKernelGGL((k_transpose_apply<T>), dim3(grid), dim3(kBlock), 0, s, keys2, idx2, val, nnz, trow, col_t,
@@ -449,10 +450,7 @@ int csr_transpose(int32_t m, int32_t n, int32_t nnz, int32_t base, const int32_t
     ASX_TRY(hipGetLastError());
     ASX_TRY(hipStreamSynchronize(s));
 #undef ASX_TRY
-done:
-    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
-    for (void *p : {(void *)keys, (void *)keys2, (void *)idx, (void *)idx2, (void *)trow, tmp})
-        pool_free(p);
+    scratch.idle = true;
     return st;
 }
 

@@ -59,18 +59,19 @@ int coo_sort(int32_t *row, int32_t *col, T *val, int32_t nnz, hipStream_t s)
     void *tmp = nullptr;
     size_t tmp_bytes = 0;
     const unsigned grid = (unsigned)ceil_div64(nnz, kBlock);
+    Scratch scratch(s);
 #define ASX_TRY(expr)             \
     do {                          \
         st = status_of(expr);     \
-        if (st) goto done;        \
+        if (st) return st;        \
     } while (0)
-    ASX_TRY(pool_malloc(&keys, sizeof(uint64_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&keys2, sizeof(uint64_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&idx, sizeof(int32_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&idx2, sizeof(int32_t) * (size_t)nnz, true));
-    ASX_TRY(pool_malloc(&val2, sizeof(T) * (size_t)nnz, true));
+    ASX_TRY(scratch.take(&keys, sizeof(uint64_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&keys2, sizeof(uint64_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&idx, sizeof(int32_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&idx2, sizeof(int32_t) * (size_t)nnz));
+    ASX_TRY(scratch.take(&val2, sizeof(T) * (size_t)nnz));
     ASX_TRY(rocprim::radix_sort_pairs(nullptr, tmp_bytes, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
-    ASX_TRY(pool_malloc(&tmp, tmp_bytes, true));
+    ASX_TRY(scratch.take(&tmp, tmp_bytes));
     hipLaunchKernelGGL(k_coo_keys, dim3(grid), dim3(kBlock), 0, s, row, col, nnz, keys, idx);
     ASX_TRY(rocprim::radix_sort_pairs(tmp, tmp_bytes, keys, keys2, idx, idx2, (size_t)nnz, 0u, (unsigned)64, s));
     ASX_TRY(hipMemcpyAsync(val2, val, sizeof(T) * (size_t)nnz, hipMemcpyDeviceToDevice, s));
@@ -78,10 +79,7 @@ int coo_sort(int32_t *row, int32_t *col, T *val, int32_t nnz, hipStream_t s)
     ASX_TRY(hipGetLastError());
     ASX_TRY(hipStreamSynchronize(s));
 #undef ASX_TRY
-done:
-    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
-    for (void *p : {(void *)keys, (void *)keys2, (void *)idx, (void *)idx2, (void *)val2, tmp})
-        pool_free(p);
+    scratch.idle = true;
     return st;
 }
 

@@ -127,7 +127,7 @@ struct BlockedMatrix {
 template <typename T>
 int build_blocked(int32_t m, int32_t k, int32_t nnz, const int32_t *row_ptr, const int32_t *col,
                   const T *val, BlockedMatrix *out, hipStream_t s);
-void free_blocked(BlockedMatrix *b);
+void free_blocked(BlockedMatrix *b, bool idle);  // idle: as for pool_free
 template <typename T>
 int blocked_update_values(const BlockedMatrix *bm, const T *val, hipStream_t s);
 template <typename T>
@@ -182,7 +182,7 @@ constexpr int kSlicedReducePad = 256;  // entries of prow / partial that pass 2 
 template <typename T>
 int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_per_wave, int32_t target_wgs,
                  const int32_t *row_ptr, const int32_t *col, const T *val, SlicedMatrix *out, hipStream_t s);
-void free_sliced(SlicedMatrix *p);
+void free_sliced(SlicedMatrix *p, bool idle);
 template <typename T>
 int sliced_update_values(const SlicedMatrix *sm, const T *val, hipStream_t s, const unsigned long long *unless_equal = nullptr);
 template <typename T>
@@ -224,7 +224,7 @@ struct WindowMatrix {
 template <typename T>
 int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_place, const int32_t *row_ptr,
                  const int32_t *col, const T *val, WindowMatrix *out, hipStream_t s);
-void free_window(WindowMatrix *p);
+void free_window(WindowMatrix *p, bool idle);
 template <typename T>
 int window_update_values(const WindowMatrix *wm, const T *val, hipStream_t s, const unsigned long long *unless_equal = nullptr);
 template <typename T>

@@ -123,9 +123,13 @@ hipError_t pool_malloc_bytes(void **p, size_t bytes, bool brief)
     return hipSuccess;
 }
 
-void pool_free(void *p)
+void pool_free(void *p, bool idle)
 {
     if (!p) return;
+    if (!idle) {
+        (void)pool_return(p);
+        return;
+    }
     Pool &P = pool();
     std::vector<Block> out;
     {
@@ -147,19 +151,19 @@ void pool_free(void *p)
     }
 }
 
-void pool_wait(const void *p)
+bool pool_wait(const void *p)
 {
-    if (!p) return;
+    if (!p) return true;
     Pool &P = pool();
     int dev;
     {
         std::lock_guard<std::mutex> g(P.lock);
         const auto it = P.live.find(p);
-        if (it == P.live.end()) return;
+        if (it == P.live.end()) return true;
         dev = it->second.dev;
     }
     OnDevice on(dev);
-    (void)hipDeviceSynchronize();
+    return hipDeviceSynchronize() == hipSuccess;
 }
 
 hipError_t pool_return(void *p)
@@ -219,11 +223,11 @@ void *pinned_take()
     return hipHostMalloc(&p, kPinnedBytes, hipHostMallocPortable) == hipSuccess ? p : nullptr;
 }
 
-void pinned_give(void *p)
+void pinned_give(void *p, bool idle)
 {
     if (!p) return;
     Pool &P = pool();
-    {
+    if (idle) {
         std::lock_guard<std::mutex> g(P.lock);
         if (P.pinned.size() < 16) {
             P.pinned.push_back(p);

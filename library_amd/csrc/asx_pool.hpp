@@ -25,11 +25,13 @@ hipError_t pool_malloc(P **p, size_t bytes, bool brief)
     *p = static_cast<P *>(q);
     return e;
 }
-// Nothing on the device may still use the block: the caller has synchronised the streams that did,
-// or calls pool_wait first.  Null is allowed.
-void pool_free(void *p);
-// Waits until everything queued on the device that owns p has run (as hipFree does).
-void pool_wait(const void *p);
+// idle: nothing on the device uses the block any more - the caller has synchronised the streams that did, or pool_wait
+// says so - and it may be kept.  Otherwise it goes back through hipFree, which waits by itself, and is never handed out
+// again.  Null is allowed.
+void pool_free(void *p, bool idle);
+// Waits until everything queued on the device that owns p has run (as hipFree does); false where that was refused, for
+// instance while a stream is being captured.
+bool pool_wait(const void *p);
 // Back to the device at once (waits as hipFree does).
 hipError_t pool_return(void *p);
 // Bytes kept on the current device; gives all of them back.
@@ -40,19 +42,25 @@ void pool_release();
 // reads after it has synchronised the stream; null if there is none to be had.
 constexpr size_t kPinnedBytes = 8192;
 void *pinned_take();
-void pinned_give(void *p);
+void pinned_give(void *p, bool idle);  // idle: as for pool_free
 
 // Scratch of one call on one stream, handed back when the scope ends: after a wait for the stream
-// unless the call has already waited (`idle`).
+// unless the call has already waited (`idle`).  What a refused wait leaves in doubt is not kept.
 class Scratch {
 public:
     explicit Scratch(hipStream_t s) : s_(s) {}
     ~Scratch()
     {
         if (n_ == 0 && !pinned_) return;
-        if (!idle) (void)hipStreamSynchronize(s_);
-        for (int i = 0; i < n_; ++i) pool_free(p_[i]);
-        pinned_give(pinned_);
+        settle();
+        for (int i = 0; i < n_; ++i) pool_free(p_[i], idle);
+        pinned_give(pinned_, idle);
+    }
+    // waits unless the call has; whether nothing queued on the stream is left that could use the scratch
+    bool settle()
+    {
+        if (!idle) idle = hipStreamSynchronize(s_) == hipSuccess;
+        return idle;
     }
     Scratch(const Scratch &) = delete;
     Scratch &operator=(const Scratch &) = delete;

@@ -770,10 +770,10 @@ __global__ __launch_bounds__(kWave) void k_sliced_reduce(int32_t m, int32_t nrb,
 
 }  // namespace
 
-void free_sliced(SlicedMatrix *p)
+void free_sliced(SlicedMatrix *p, bool idle)
 {
     for (void *q : {p->store, p->partial, (void *)p->prow, (void *)p->psteps})
-        pool_free(q);
+        pool_free(q, idle);
     p->store = p->val = p->partial = nullptr;
     p->cf = p->prow = nullptr;
     p->perm = p->tile_base = p->wg_tab = p->wg_pieces = p->chunk_lo = p->pstep_ptr = p->psteps = p->block_base = nullptr;
@@ -928,9 +928,7 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
 #undef ASX_TRY_ST
 done:
     if (st) {
-        (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
-        free_sliced(&sm);
-        scratch.idle = true;
+        free_sliced(&sm, scratch.settle());
         return st;
     }
     scratch.idle = true;

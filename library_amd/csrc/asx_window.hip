@@ -784,10 +784,10 @@ __global__ __launch_bounds__(kBlock) void k_window_fixup(int32_t ntiles, T alpha
 
 }  // namespace
 
-void free_window(WindowMatrix *p)
+void free_window(WindowMatrix *p, bool idle)
 {
     for (void *q : {p->store, p->tables, p->carry})
-        pool_free(q);
+        pool_free(q, idle);
     p->store = p->tables = p->val = p->carry = nullptr;
     p->cf = nullptr;
     p->perm = p->tile_info = p->blocks = p->pieces = p->chains = nullptr;
@@ -819,6 +819,7 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
     const int32_t max_nb = (int32_t)ceil_div64(m, 256);
     const int32_t ngroups = (int32_t)ceil_div64(m, kSpanGroup);
     const int32_t nseg = (int32_t)ceil_div64(nnz, kBlock);
+    Scratch scratch(s);
 #define ASX_TRY(expr)         \
     do {                      \
         st = status_of(expr); \
@@ -831,7 +832,7 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
         const auto pad64 = [](size_t v) { return (v + 63) & ~(size_t)63; };
         const size_t per_group = pad64((size_t)ngroups), per_row = pad64((size_t)m), per_seg = pad64((size_t)nseg + 1);
         const size_t per_block = pad64((size_t)max_nb + 1);
-        ASX_TRY(pool_malloc(&arena, sizeof(int32_t) * (2 * per_group + per_row + per_seg + 4 * per_block + 64), true));
+        ASX_TRY(scratch.take(&arena, sizeof(int32_t) * (2 * per_group + per_row + per_seg + 4 * per_block + 64)));
         gmin = arena, gmax = gmin + per_group, row_start = gmax + per_group, seg_row = row_start + per_row;
         bmin = seg_row + per_seg, bmax = bmin + per_block, btiles = bmax + per_block, tile_off = btiles + per_block;
         d_small = tile_off + per_block;
@@ -903,7 +904,7 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
         };
         const int64_t nbins = (2 * (int64_t)n >> 6) + 2;
         const size_t words = (size_t)(nbins + 31) / 32;
-        ASX_TRY(pool_malloc(&d_bits, sizeof(uint32_t) * words, true));
+        ASX_TRY(scratch.take(&d_bits, sizeof(uint32_t) * words));
         ASX_TRY(hipMemsetAsync(d_bits, 0, sizeof(uint32_t) * words, s));
         hipLaunchKernelGGL(k_window_offset_bins, dim3((unsigned)nseg), dim3(kBlock), 0, s, row_ptr, col, m, n, nnz, seg_row, d_bits);
         h_bits.resize(words);
@@ -1224,10 +1225,9 @@ int build_window(int32_t m, int32_t n, int32_t nnz, int32_t target_wgs, bool in_
     wm.has_carry = h_small[0] != 0;
 #undef ASX_TRY
 done:
-    if (st) (void)hipStreamSynchronize(s);  // nothing queued may still use what is freed
-    for (void *p : {(void *)arena, (void *)d_bits}) pool_free(p);
+    scratch.idle = !st;
     if (st) {
-        free_window(&wm);
+        free_window(&wm, scratch.settle());
         return st;
     }
     *out = wm;
