@@ -1,5 +1,5 @@
 // The pool of device memory on a HIP that is played here: memory is the host's, streams are always done, and what waits is
-// refused while `capturing`.  Usage: pool_check CASE; exit status 0 where the case holds.
+// refused while `capturing`; while it is `relaxed`, only a wait for the device as such is, and the capture is lost by it.  Usage: pool_check CASE; exit status 0 where the case holds.
 #include <stdio.h>
 #include <stdlib.h>
 #include <string.h>
@@ -9,7 +9,7 @@
 #include "../../library_amd/csrc/asx_pool.hpp"
 
 namespace {
-bool capturing = false;  // a stream is being captured: nothing may wait
+bool capturing = false, relaxed = false, lost = false;
 std::map<void *, size_t> device_blocks, host_blocks;
 int frees_refused = 0;
 }  // namespace
@@ -20,6 +20,7 @@ hipError_t hipSetDevice(int) { return hipSuccess; }
 hipError_t hipGetLastError() { return hipSuccess; }
 hipError_t hipMalloc(void **p, size_t n)
 {
+    if (capturing) return *p = nullptr, hipErrorStreamCaptureUnsupported;
     *p = malloc(n);
     device_blocks[*p] = n;
     return hipSuccess;
@@ -44,7 +45,11 @@ hipError_t hipHostFree(void *p)
     free(p);
     return hipSuccess;
 }
-hipError_t hipDeviceSynchronize() { return capturing ? hipErrorStreamCaptureUnsupported : hipSuccess; }
+hipError_t hipDeviceSynchronize()
+{
+    lost |= relaxed;
+    return capturing || relaxed ? hipErrorStreamCaptureUnsupported : hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return capturing ? hipErrorStreamCaptureUnsupported : hipSuccess; }
 }
 
@@ -87,6 +92,15 @@ static void refused_wait_of_a_plan()
     CHECK(pool_kept_bytes() == 0);
     CHECK(block(100000) != a && block(300000) != b);
 }
+// a capture in relaxed mode survives the wait for a plan's last call
+static void relaxed_capture()
+{
+    void *a = block(100000);
+    relaxed = true;
+    CHECK(pool_wait(a));
+    pool_free(a, true);
+    CHECK(!lost && block(100000) == a);
+}
 static void refused_wait_of_a_call()
 {
     void *a = nullptr, *pinned = nullptr;
@@ -107,7 +121,7 @@ int main(int argc, char **argv)
     const struct {
         const char *name;
         void (*run)();
-    } cases[] = {{"kept", kept}, {"refused_wait_of_a_plan", refused_wait_of_a_plan}, {"refused_wait_of_a_call", refused_wait_of_a_call}};
+    } cases[] = {{"kept", kept}, {"refused_wait_of_a_plan", refused_wait_of_a_plan}, {"refused_wait_of_a_call", refused_wait_of_a_call}, {"relaxed_capture", relaxed_capture}};
     for (const auto &c : cases)
         if (argc == 2 && !strcmp(argv[1], c.name)) return c.run(), 0;
     return 2;
