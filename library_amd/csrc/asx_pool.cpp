@@ -1,6 +1,8 @@
 // Kept blocks of device memory (asx_pool.hpp).
 #include "asx_pool.hpp"
 
+#include <stdint.h>
+
 #include <algorithm>
 #include <mutex>
 #include <unordered_map>
@@ -14,13 +16,18 @@ struct Block {
     void *p;
     size_t bytes;
     int dev;
+    uint64_t id;
+};
+struct Pinned {
+    void *p;
+    uint64_t id;
 };
 
 struct Pool {
     std::mutex lock;
     std::unordered_map<const void *, Block> live;
     std::vector<Block> kept;  // oldest first
-    std::vector<void *> pinned;
+    std::vector<Pinned> pinned;
 };
 
 // Never destroyed: at process exit the HIP runtime may be gone before static objects are.
@@ -28,6 +35,23 @@ Pool &pool()
 {
     static Pool *p = new Pool;
     return *p;
+}
+
+// HIP's number of the allocation at p; every allocation has another one, also at the address of an earlier one (0: there is
+// none).  hipDeviceReset takes all memory of the device, and what lies at a kept address afterwards, if anything, is
+// somebody else's: a block counts as the pool's only while its number is the one it was allocated with.
+uint64_t allocation_id(const void *p)
+{
+    uint64_t id = 0;
+    if (hipPointerGetAttribute(&id, HIP_POINTER_ATTRIBUTE_BUFFER_ID, const_cast<void *>(p)) == hipSuccess) return id;
+    (void)hipGetLastError();  // or the next launch would seem to have failed
+    return 0;
+}
+
+hipError_t device_free(const Block &b)
+{
+    if (allocation_id(b.p) != b.id) return hipErrorInvalidValue;
+    return hipFree(b.p);
 }
 
 // Sizes in eighths of a power of two: requests that differ a little meet each other's blocks.
@@ -86,21 +110,25 @@ hipError_t pool_malloc_bytes(void **p, size_t bytes, bool brief)
     if (e != hipSuccess) return e;
     const size_t want = rounded(bytes);
     Pool &P = pool();
-    {
-        std::lock_guard<std::mutex> g(P.lock);
-        const size_t most = brief ? 4 * want : want + want / 4;
-        size_t best = P.kept.size();
-        for (size_t i = 0; i < P.kept.size(); ++i) {
-            const Block &b = P.kept[i];
-            if (b.dev == dev && b.bytes >= want && b.bytes <= most && (best == P.kept.size() || b.bytes < P.kept[best].bytes)) best = i;
-        }
-        if (best < P.kept.size()) {
-            const Block b = P.kept[best];
+    const size_t most = brief ? 4 * want : want + want / 4;
+    for (;;) {
+        Block b;
+        {
+            std::lock_guard<std::mutex> g(P.lock);
+            size_t best = P.kept.size();
+            for (size_t i = 0; i < P.kept.size(); ++i) {
+                const Block &k = P.kept[i];
+                if (k.dev == dev && k.bytes >= want && k.bytes <= most && (best == P.kept.size() || k.bytes < P.kept[best].bytes)) best = i;
+            }
+            if (best == P.kept.size()) break;
+            b = P.kept[best];
             P.kept.erase(P.kept.begin() + (std::ptrdiff_t)best);
-            P.live[b.p] = b;
-            *p = b.p;
-            return hipSuccess;
         }
+        if (allocation_id(b.p) != b.id) continue;  // lost in a reset of the device
+        std::lock_guard<std::mutex> g(P.lock);
+        P.live[b.p] = b;
+        *p = b.p;
+        return hipSuccess;
     }
     size_t got = want;
     e = hipMalloc(p, got);
@@ -118,8 +146,9 @@ hipError_t pool_malloc_bytes(void **p, size_t bytes, bool brief)
         *p = nullptr;
         return e;
     }
+    const uint64_t id = allocation_id(*p);
     std::lock_guard<std::mutex> g(P.lock);
-    P.live[*p] = Block{*p, got, dev};
+    P.live[*p] = Block{*p, got, dev, id};
     return hipSuccess;
 }
 
@@ -147,7 +176,7 @@ void pool_free(void *p, bool idle)
     }
     for (const Block &b : out) {
         OnDevice on(b.dev);
-        (void)hipFree(b.p);
+        (void)device_free(b);
     }
 }
 
@@ -174,16 +203,16 @@ hipError_t pool_return(void *p)
 {
     if (!p) return hipSuccess;
     Pool &P = pool();
-    int dev;
+    Block b;
     {
         std::lock_guard<std::mutex> g(P.lock);
         const auto it = P.live.find(p);
         if (it == P.live.end()) return hipErrorInvalidValue;
-        dev = it->second.dev;
+        b = it->second;
         P.live.erase(it);
     }
-    OnDevice on(dev);
-    return hipFree(p);
+    OnDevice on(b.dev);
+    return device_free(b);
 }
 
 size_t pool_kept_bytes()
@@ -208,19 +237,21 @@ void pool_release()
         std::lock_guard<std::mutex> g(P.lock);
         out = surplus(P, dev, true);
     }
-    for (const Block &b : out) (void)hipFree(b.p);
+    for (const Block &b : out) (void)device_free(b);
 }
 
 void *pinned_take()
 {
     Pool &P = pool();
-    {
-        std::lock_guard<std::mutex> g(P.lock);
-        if (!P.pinned.empty()) {
-            void *p = P.pinned.back();
+    for (;;) {
+        Pinned k;
+        {
+            std::lock_guard<std::mutex> g(P.lock);
+            if (P.pinned.empty()) break;
+            k = P.pinned.back();
             P.pinned.pop_back();
-            return p;
         }
+        if (allocation_id(k.p) == k.id) return k.p;
     }
     void *p = nullptr;
     // portable: readable and writable from every device
@@ -232,9 +263,10 @@ void pinned_give(void *p, bool idle)
     if (!p) return;
     Pool &P = pool();
     if (idle) {
+        const uint64_t id = allocation_id(p);
         std::lock_guard<std::mutex> g(P.lock);
         if (P.pinned.size() < 16) {
-            P.pinned.push_back(p);
+            P.pinned.push_back(Pinned{p, id});
             return;
         }
     }

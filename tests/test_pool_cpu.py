@@ -17,7 +17,7 @@ def pool_check(tmp_path_factory):
     return str(exe)
 
 
-@pytest.mark.parametrize("case", ["kept", "refused_wait_of_a_plan", "refused_wait_of_a_call", "relaxed_capture"])
+@pytest.mark.parametrize("case", ["kept", "refused_wait_of_a_plan", "refused_wait_of_a_call", "relaxed_capture", "device_reset"])
 def test_pool(pool_check, case):
     run = subprocess.run([pool_check, case], capture_output=True, text=True, timeout=60)
     assert run.returncode == 0, run.stdout
