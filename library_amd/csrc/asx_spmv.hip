@@ -84,8 +84,8 @@ __device__ __forceinline__ T strided_dot(int64_t k, int64_t e, const int32_t *__
 }
 
 // The rows of workgroup b, a lane group each; with a list, rows of long_len elements or more are somebody else's.  Without
-// one a row may hold everything that int32 offsets can count (2^31 - 1 elements): nothing is compared, and positions are
-// unsigned, so that the step past the row's end does not overflow.
+// one a row may hold everything that int32 offsets can count (2^31 - 1 elements): nothing is compared, and what is left of a
+// row is counted, because the position past its end may not be an int32.
 template <typename T, int LANES, bool LISTED>
 __device__ __forceinline__ void vector_rows(int64_t b, int32_t m, T alpha, const int32_t *__restrict__ row_ptr,
                                             const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ x,
@@ -96,17 +96,18 @@ __device__ __forceinline__ void vector_rows(int64_t b, int32_t m, T alpha, const
     T sum = T(0);
     bool mine = row < m;
     if (mine) {
-        const uint32_t e = (uint32_t)row_ptr[row + 1];
-        uint32_t k = (uint32_t)row_ptr[row];
-        mine = !LISTED || (int32_t)(e - k) < long_len;
-        k = mine ? k + lane : e;
+        const int32_t from = row_ptr[row], len = row_ptr[row + 1] - from;
+        mine = !LISTED || len < long_len;
+        int32_t left = mine ? len - lane : 0;
+        const int32_t *c = col + (from + (int64_t)lane);
+        const T *v = val + (from + (int64_t)lane);
         // two independent chains per lane keep more gathers in flight on long rows
         T s0 = T(0), s1 = T(0);
-        for (; k + LANES < e; k += 2 * LANES) {
-            s0 = fma_t<T>(val[k], x[col[k]], s0);
-            s1 = fma_t<T>(val[k + LANES], x[col[k + LANES]], s1);
+        for (; left > LANES; left -= 2 * LANES, c += 2 * LANES, v += 2 * LANES) {
+            s0 = fma_t<T>(v[0], x[c[0]], s0);
+            s1 = fma_t<T>(v[LANES], x[c[LANES]], s1);
         }
-        if (k < e) s0 = fma_t<T>(val[k], x[col[k]], s0);
+        if (left > 0) s0 = fma_t<T>(v[0], x[c[0]], s0);
         sum = s0 + s1;
     }
     sum = group_sum<LANES>(sum);  // all lanes stay active for the cross-lane moves
