@@ -647,14 +647,18 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
 //                spread' = the sample's spread, at least 0.05 (neighbouring columns share a line)
 //   bytes      = nnz (sv + 4) + n sv + m (sv + 4)
 // and a + b read as their smooth maximum (a^4 + b^4)^(1/4):
-//   vector  at least 4; 2.1 + (gathers(158) + bytes / (the lower of 4.3 TB/s u and 2.7 TB/s)), u = the share of a
-//           group's lanes that a mean row fills; + 0.125 per turn of a group in which only the longest row is left
-//   stream  at least 4; 3.0 + (gathers(171) + bytes / 3.6 TB/s); + 0.018 per element of the longest row beyond
-//           twice the mean (its block sums it with the few lanes its short neighbours want)
-//   flat    6.0 + (gathers(190) + bytes / 3.9 TB/s), + 3.4 where rows longer than 32 make tiles walk
+//   vector  at least 4; 2.1 + (gathers(158) + bytes / (the lower of 4.3 TB/s u and 2.7 TB/s) + 0.125 per turn a group takes
+//           over a mean row, if it is more than one), u = the share of a group's lanes that a mean row fills; + 0.125 per
+//           turn of a group in which only the longest row is left
+//   stream  at least 4.4; 3.0 + (gathers(171) + bytes / 3.6 TB/s + 0.97 per thousand elements of the longest row beyond a
+//           block, which one workgroup adds up alone: a row of 1 M takes 990 us); + 0.018 per element of the longest
+//           row up to a block's size beyond twice the mean (its block sums it with the few lanes its short neighbours want)
+//   flat    6.0 + (gathers(190) + bytes / 3.9 TB/s), + 3.4 where rows longer than 32 make tiles walk; not with a row of
+//           more than kLongRow, whose carries it adds up slower than merge (20 rows of 100000: 17.4 us against 15.1)
 //   merge   7.8 + (gathers(164) + (nnz (sv + 4) + n sv + m (sv + 1)) / 2.9 TB/s)
 //   sliced  9.9 + bytes / 5.6 TB/s, bytes = nnz (sv + 2) + P (2 sv + 2) + n sv + 2 m sv, P = nnz times the
-//           sample's pairs per stored element
+//           sample's pairs per stored element; + 0.13 for every 64 tiles of a block of rows, each of which leaves a partial
+//           sum to the one wave that owns the block (3 rows, 2.5 M elements: 38 us against 18 with merge)
 //   window  8 + bytes / 5.9 TB/s in fp64, 15 + bytes / 5.6 TB/s in fp32 (11 + 5.1 TB/s and 15 + 4.6 TB/s where rows longer
 //           than 16 are cut by tiles), bytes = (nnz + slots rows shorter than two leave free) (sv + 2) + n sv + 2 m sv; only for columns
 //           that are not scattered, and whether every block's columns fit a window is known once its build was tried
@@ -711,11 +715,12 @@ static KernelEstimates estimate_kernels(const asx_plan *p, size_t sv, const Colu
     }
     turns = std::max(1.0, turns);
     const auto by_lanes = [&](double filled) { return both(gathers(158), bytes / std::min(2.7e12, 4.3e12 * filled)); };
-    const double vector = std::max(4e-6, 2.1e-6 + by_lanes(mean / lanes)) +
+    const double vector = std::max(4e-6, 2.1e-6 + both(by_lanes(mean / lanes), mean > lanes ? 0.125e-6 * mean / lanes : 0.0)) +
                           0.125e-6 * std::max(0.0, longest / lanes - std::max(1.0, mean / lanes));
-    const double stream = std::max(4e-6, 3e-6 + both(gathers(171), bytes / 3.6e12)) +
+    const double alone = 0.97e-9 * std::max(0.0, longest - kStreamTile);
+    const double stream = std::max(4.4e-6, 3e-6 + both(both(gathers(171), bytes / 3.6e12), alone)) +
                           0.018e-6 * std::max(0.0, std::min(longest, 1024.0) - std::max(32.0, 2 * mean));
-    const double flat = 6e-6 + both(gathers(190), bytes / 3.9e12) + (longest > 32 ? 3.4e-6 : 0.0);
+    const double flat = longest > kLongRow ? inf : 6e-6 + both(gathers(190), bytes / 3.9e12) + (longest > 32 ? 3.4e-6 : 0.0);
     const double merge = 7.8e-6 + both(gathers(164), (bytes - 3 * m) / 2.9e12);
     const double with_list = std::max(4e-6, 2.6e-6 + by_lanes(mean / (lanes * turns))) + 0.4e-9 * longest;
     KernelEstimates e;
@@ -730,7 +735,8 @@ static KernelEstimates estimate_kernels(const asx_plan *p, size_t sv, const Colu
     const int64_t nslices = ceil_div64((int64_t)p->n * (int64_t)sv, kSliceBytes);
     e.sliced = nslices > kSlicedMaxSlices
                    ? inf
-                   : 9.9e-6 + (nnz * (dsv + 2) + cs.pairs * nnz * (2 * dsv + 2) + n * dsv + 2 * m * dsv) / 5.6e12;
+                   : 9.9e-6 + (nnz * (dsv + 2) + cs.pairs * nnz * (2 * dsv + 2) + n * dsv + 2 * m * dsv) / 5.6e12 +
+                         0.13e-6 * nnz / kSlicedTile / (double)ceil_div64(p->m, 256) / kWave;
     // The row-block copy gives every row at least two slots.  Rings per band fetch x about 1.5 times, stacked planes 1.3
     // times; in fp32 the time goes with the slots and not with the bytes.
     const double wslots = nnz + 2.0 * (double)p->hist[0] + (double)p->hist[1];

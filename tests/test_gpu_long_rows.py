@@ -52,3 +52,27 @@ def test_one_row_of_every_element_int32_offsets_can_count():
     capi.spmv(row_ptr, col, val, x, y, 1.0, 0.0, alg=capi.SPMV_VECTOR)
     torch.cuda.synchronize()
     assert y.item() == 2.0**31
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("rows, length, longest, n", [(1, 0, 1000000, 1200000), (1, 0, 30000, 40000), (3, 9000, 9000, 10000),
+                                                      (20, 100000, 100000, 200000), (64, 30000, 30000, 100000),
+                                                      (1800, 500, 1000000, 1200000), (2, 300000, 2000000, 2500000)])
+def test_default_cuts_very_long_rows(dtype, rows, length, longest, n):
+    """Few rows, or one among shorter ones, that a single workgroup would walk alone: DEFAULT, with the columns at hand, takes a
+    kernel that cuts rows between workgroups.  Integers, so that every order of the sums gives the same bits."""
+    rng = np.random.default_rng(rows)
+    lens = np.r_[np.full(rows, length, int), longest]
+    rp = np.r_[0, np.cumsum(lens)].astype(np.int32)
+    col = np.concatenate([np.sort(rng.choice(n, k, replace=False)) for k in lens]).astype(np.int32)
+    val, x = rng.integers(-2, 3, col.size).astype(dtype), rng.integers(-2, 3, n).astype(dtype)
+    d = [torch.from_numpy(a).cuda() for a in (rp, col, val, x)]
+    plan = capi.Plan(False, capi.SPMV_DEFAULT, val.dtype, lens.size, n, col.size, d[0], col=d[1], val=d[2])
+    assert plan.alg in (capi.SPMV_FLAT, capi.SPMV_MERGE, capi.SPMV_SLICED, capi.SPMV_WINDOW), plan.alg
+    y = torch.zeros(lens.size, dtype=d[2].dtype, device="cuda")
+    capi.spmv(*d, y, 1.0, 0.0, plan=plan)
+    torch.cuda.synchronize()
+    prod = val.astype(np.float64) * x[col]
+    expect = [prod[a:b].sum() for a, b in zip(rp[:-1], rp[1:])]
+    assert np.array_equal(y.cpu().numpy(), np.array(expect, dtype))
+    plan.destroy()
