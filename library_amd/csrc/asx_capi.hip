@@ -664,12 +664,17 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
 //           that are not scattered, and whether every block's columns fit a window is known once its build was tried
 // With a list of its long rows the vector kernel costs 0.5 more and 0.0004 per element of the longest row instead of the
 // turns, u divided by the turns a wave of the other rows takes.
-// A regrouped kernel is taken when its estimate is 3 % below the row-ordered ones: 5 % (window 15 %, the dearest to build)
-// below 4 M stored elements, where it saves little for what its build costs, and above that even when up to 10 % slower where
-// the columns are neither neighbours nor scattered, because there what gathers cost the row-ordered kernels is estimated less
-// well than what a copy streams.  Of the two, the sliced one unless the window one is estimated more than 5 % faster - or, in
+// A regrouped kernel is taken when its estimate is 3 % below the row-ordered ones; 5 % (window 15 %, the dearest to build)
+// below 4 M stored elements, where it saves little for what its build costs.  Two exceptions, because what gathers cost the
+// row-ordered kernels is estimated less well than what a copy streams: from 4 M on up to 10 % slower will do where the columns
+// are neither neighbours nor scattered, and up to 4 % where they are scattered (239797 x 47, fp64, values checked in every
+// call: 69 us against 85 with stream) - below 4 M as well where a slice holds seven elements and more of a row, so that the
+// slices have few partial sums to carry (60363 x 37 over 37213 columns, fp64: 14.1 us against 17.2; 246858 x 14 near the
+// diagonal 20.2 against 22.8; where the pairs are more the slices fell behind: 61822 x 34 over 120316 columns 18.0 against
+// 16.6).  Of the two, the sliced one unless the window one is estimated more than 5 % faster - or, in
 // fp32 with rows the tiles do not cut, not more than 9 % slower: its plan reads A's values where the caller keeps them, and a
-// caller who changes them before every multiply has nothing to bring up to date (7 per row, 22 M elements: 48 us against 95).
+// caller who changes them before every multiply has nothing to bring up to date (7 per row, 22 M elements: 48 us against 95;
+// 12 per row, 30 M: 53 against 119).  A caller who never changes them loses a little: those 30 M take 53.5 us, 50.7 in slices.
 constexpr int32_t kRegroupMinNnz = 1 << 21;
 // The vector kernel with a list of long rows: eight turns of a lane group are long, kWideRow elements take a workgroup (a
 // power of two each, so that the histogram holds their numbers), and with a row of more than kMostWideRow the kernels
@@ -924,7 +929,9 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
         row_kernel = e.row_kernel;
         list_long_rows = e.long_rows;
         if (can_regroup && cs.ok) {
-            const double ahead = (nnz < (1 << 22) ? 0.95 : cs.spread > 0.1 && cs.spread < kScatteredMinSpread ? 1.1 : 0.97) * e.rows;
+            const bool large = nnz >= (1 << 22), scattered = cs.spread >= kScatteredMinSpread;
+            const double between = large && cs.spread > 0.1 && !scattered ? 1.1 : large ? 0.97 : 0.95;
+            const double ahead = (scattered && (large || cs.pairs < 0.15) ? 1.04 : between) * e.rows;
             const bool sliced_pays = e.sliced < ahead, window_pays = e.window < ahead * (nnz < (1 << 22) ? 0.9 : 1.0);
             const bool in_place = !f64 && p->hist[0] + p->hist[1] == 0 && p->stats[0] <= 16;
             const double slices_for_window = e.sliced * (in_place ? 1.09 : 1 / 1.05);
