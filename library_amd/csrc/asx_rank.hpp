@@ -56,7 +56,7 @@ __device__ __forceinline__ int32_t wave_row_holding(const int32_t *__restrict__ 
 {
     const int lane = threadIdx.x & (kWave - 1);
     while (lo < hi) {
-        const int32_t step = (hi - lo + kWave - 1) / kWave;
+        const int32_t step = (int32_t)(((uint32_t)(hi - lo) + kWave - 1) / kWave);  // unsigned: hi may be 2^31 - 1
         const int64_t p = lo + (int64_t)(lane + 1) * step;
         const int n = __popcll(__ballot(p <= hi && row_ptr[p <= hi ? p : hi] <= i));
         lo += n * step;
@@ -98,9 +98,9 @@ __device__ __forceinline__ void wave_rows(const int32_t *__restrict__ row_ptr, i
     for (int k = 0; k < kSortPerLane; ++k) mark[k * kWave + lane] = 0;
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    for (int32_t r = r_lo + 1 + lane; r <= r_hi; r += kWave) {
-        const int64_t at = (int64_t)row_ptr[r] - base - wbase;
-        if (at >= 0 && at < kSortWaveElems) atomicMax(&mark[at], r - r_lo);  // of rows that start alike the last one holds the element
+    for (int32_t d = 1 + lane; d <= r_hi - r_lo; d += kWave) {  // counted from r_lo: r_hi may be close to 2^31
+        const int64_t at = (int64_t)row_ptr[(int64_t)r_lo + d] - base - wbase;
+        if (at >= 0 && at < kSortWaveElems) atomicMax(&mark[at], d);  // of rows that start alike the last one holds the element
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
