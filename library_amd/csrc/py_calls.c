@@ -20,30 +20,83 @@ typedef int (*values_t)(void *, const void *, void *);
 
 static PyObject *s_data_ptr, *s_numel, *s_element_size;
 static PyObject *get_device, *get_stream; /* the current device's number; the stream of a device, as an integer */
+static PyObject *argument_error;          /* ctypes.ArgumentError */
 
-/* result of a method without arguments, as an integer; -1 with an exception set on failure */
-static int64_t ask(PyObject *o, PyObject *method)
+/* Each of these writes *out and returns 1, or leaves an exception set and returns 0, after which nothing else of Python may
+ * be called: they are joined by &&.  Arguments of a wrong type raise what they raise through ctypes. */
+static int wrong_type(void)
+{
+    if (PyErr_ExceptionMatches(PyExc_TypeError)) {
+        PyObject *type, *value, *trace;
+        PyErr_Fetch(&type, &value, &trace);
+        PyErr_Format(argument_error, "%S", value ? value : Py_None);
+        Py_XDECREF(type);
+        Py_XDECREF(value);
+        Py_XDECREF(trace);
+    }
+    return 0;
+}
+static int integer(PyObject *o, int64_t *out)
+{
+    *out = PyLong_AsLongLong(o);
+    return *out != -1 || !PyErr_Occurred() || wrong_type();
+}
+static int real(PyObject *o, double *out)
+{
+    *out = PyFloat_AsDouble(o);
+    return *out != -1.0 || !PyErr_Occurred() || wrong_type();
+}
+/* int32 argument: sizes beyond it are an error, as they are for ctypes' c_int32 callers that check */
+static int fits32(int64_t v, int32_t *out)
+{
+    *out = (int32_t)v;
+    if (*out != v) PyErr_Format(PyExc_OverflowError, "%lld does not fit int32", (long long)v);
+    return *out == v;
+}
+static int integer32(PyObject *o, int32_t *out)
+{
+    int64_t v;
+    return integer(o, &v) && fits32(v, out);
+}
+/* of a method without arguments */
+static int ask(PyObject *o, PyObject *method, int64_t *out)
 {
     PyObject *r = PyObject_CallMethodNoArgs(o, method);
-    if (!r) return -1;
-    const int64_t v = (int64_t)PyLong_AsUnsignedLongLongMask(r);
+    if (!r) return 0;
+    *out = (int64_t)PyLong_AsUnsignedLongLongMask(r);
     Py_DECREF(r);
-    return v;
+    return *out != -1 || !PyErr_Occurred();
 }
-static void *address(PyObject *o) { return o == Py_None ? NULL : (void *)(uintptr_t)ask(o, s_data_ptr); }
-static int64_t number(PyObject *o) { return PyLong_AsLongLong(o); }
-static void *pointer(PyObject *o) { return o == Py_None ? NULL : (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(o); }
-
-static void *stream(void)
+static int ask32(PyObject *o, PyObject *method, int64_t less, int32_t *out)
+{
+    int64_t v;
+    return ask(o, method, &v) && fits32(v - less, out);
+}
+/* a tensor's memory, or NULL for None */
+static int address(PyObject *o, void **out)
+{
+    int64_t v = 0;
+    const int ok = o == Py_None || ask(o, s_data_ptr, &v);
+    *out = (void *)(uintptr_t)v;
+    return ok;
+}
+/* an address as an integer, or NULL for None */
+static int pointer(PyObject *o, void **out)
+{
+    const unsigned long long v = o == Py_None ? 0 : PyLong_AsUnsignedLongLongMask(o);
+    *out = (void *)(uintptr_t)v;
+    return v != (unsigned long long)-1 || !PyErr_Occurred() || wrong_type();
+}
+static int stream(void **out)
 {
     PyObject *d = PyObject_CallNoArgs(get_device);
-    if (!d) return NULL;
+    if (!d) return 0;
     PyObject *r = PyObject_CallOneArg(get_stream, d);
     Py_DECREF(d);
-    if (!r) return NULL;
-    void *s = (void *)(uintptr_t)PyLong_AsUnsignedLongLongMask(r);
+    if (!r) return 0;
+    const int ok = pointer(r, out);
     Py_DECREF(r);
-    return s;
+    return ok;
 }
 
 static PyObject *streams_from(PyObject *self, PyObject *const *a, Py_ssize_t n)
@@ -57,21 +110,14 @@ static PyObject *streams_from(PyObject *self, PyObject *const *a, Py_ssize_t n)
     Py_RETURN_NONE;
 }
 
-/* int32 argument: sizes beyond it are an error, as they are for ctypes' c_int32 callers that check */
-static int32_t size32(int64_t v)
+/* None (no buffer) or a tensor */
+static int workspace(PyObject *o, void **p, size_t *bytes)
 {
-    if ((v < INT32_MIN || v > INT32_MAX) && !PyErr_Occurred()) PyErr_Format(PyExc_OverflowError, "%lld does not fit int32", (long long)v);
-    return (int32_t)v;
-}
-
-/* workspace: None (no buffer) or a tensor */
-static void workspace_of(PyObject *o, void **p, size_t *bytes)
-{
+    int64_t n = 0, each = 0;
     *p = NULL;
-    *bytes = 0;
-    if (o == Py_None) return;
-    *p = address(o);
-    *bytes = (size_t)(ask(o, s_numel) * ask(o, s_element_size));
+    if (o != Py_None && !(address(o, p) && ask(o, s_numel, &n) && ask(o, s_element_size, &each))) return 0;
+    *bytes = (size_t)(n * each);
+    return 1;
 }
 
 /* spmv(fn, f64, plan, alg, row_ptr, col, val, x, y, alpha, beta, n or None, workspace or None) -> status */
@@ -79,22 +125,21 @@ static PyObject *spmv(PyObject *self, PyObject *const *a, Py_ssize_t n)
 {
     (void)self;
     if (n != 13 || !get_stream) return PyErr_Format(PyExc_TypeError, "spmv: 13 arguments, after streams_from");
-    void *fn = pointer(a[0]), *plan = pointer(a[2]), *ws;
-    const int f64 = a[1] == Py_True, alg = (int)number(a[3]);
+    void *fn, *plan, *rp, *col, *val, *x, *y, *ws, *s;
+    const int f64 = a[1] == Py_True;
     size_t ws_bytes;
-    const int32_t m = size32(ask(a[4], s_numel) - 1), nnz = size32(ask(a[5], s_numel));
-    const int32_t cols = size32(a[11] == Py_None ? ask(a[7], s_numel) : number(a[11]));
-    const int32_t *rp = address(a[4]), *col = address(a[5]);
-    const void *val = address(a[6]), *x = address(a[7]);
-    void *y = address(a[8]);
-    const double alpha = PyFloat_AsDouble(a[9]), beta = PyFloat_AsDouble(a[10]);
-    workspace_of(a[12], &ws, &ws_bytes);
-    void *s = stream();
-    if (PyErr_Occurred()) return NULL;
+    int32_t m, nnz, cols;
+    int64_t alg;
+    double alpha, beta;
+    if (!(pointer(a[0], &fn) && pointer(a[2], &plan) && integer(a[3], &alg) && ask32(a[4], s_numel, 1, &m) &&
+          ask32(a[5], s_numel, 0, &nnz) && (a[11] == Py_None ? ask32(a[7], s_numel, 0, &cols) : integer32(a[11], &cols)) &&
+          address(a[4], &rp) && address(a[5], &col) && address(a[6], &val) && address(a[7], &x) && address(a[8], &y) &&
+          real(a[9], &alpha) && real(a[10], &beta) && workspace(a[12], &ws, &ws_bytes) && stream(&s)))
+        return NULL;
     int st;
     Py_BEGIN_ALLOW_THREADS;
-    st = f64 ? ((spmv64_t)fn)(plan, alg, m, cols, nnz, alpha, rp, col, val, x, beta, y, ws, ws_bytes, s)
-             : ((spmv32_t)fn)(plan, alg, m, cols, nnz, (float)alpha, rp, col, val, x, (float)beta, y, ws, ws_bytes, s);
+    st = f64 ? ((spmv64_t)fn)(plan, (int)alg, m, cols, nnz, alpha, rp, col, val, x, beta, y, ws, ws_bytes, s)
+             : ((spmv32_t)fn)(plan, (int)alg, m, cols, nnz, (float)alpha, rp, col, val, x, (float)beta, y, ws, ws_bytes, s);
     Py_END_ALLOW_THREADS;
     return PyLong_FromLong(st);
 }
@@ -104,30 +149,26 @@ static PyObject *spmm(PyObject *self, PyObject *const *a, Py_ssize_t n)
 {
     (void)self;
     if (n != 16 || !get_stream) return PyErr_Format(PyExc_TypeError, "spmm: 16 arguments, after streams_from");
-    void *fn = pointer(a[0]), *plan = pointer(a[2]), *ws;
-    const int f64 = a[1] == Py_True, alg = (int)number(a[3]);
+    void *fn, *plan, *rp, *col, *val, *B, *C, *ws, *s;
+    const int f64 = a[1] == Py_True;
     size_t ws_bytes;
-    const int32_t m = size32(ask(a[4], s_numel) - 1), nnz = size32(ask(a[5], s_numel)), ncols = size32(number(a[9]));
-    const int64_t ldb = a[12] == Py_None ? ncols : number(a[12]), ldc = a[13] == Py_None ? ncols : number(a[13]);
-    int64_t rows = 0;
-    if (a[14] != Py_None)
-        rows = number(a[14]);
-    else if (ldb != 0)
-        rows = ask(a[7], s_numel) / ldb;
-    else
-        PyErr_SetString(PyExc_ZeroDivisionError, "spmm: ldb = 0");
-    const int32_t k = size32(rows);
-    const int32_t *rp = address(a[4]), *col = address(a[5]);
-    const void *val = address(a[6]), *B = address(a[7]);
-    void *C = address(a[8]);
-    const double alpha = PyFloat_AsDouble(a[10]), beta = PyFloat_AsDouble(a[11]);
-    workspace_of(a[15], &ws, &ws_bytes);
-    void *s = stream();
-    if (PyErr_Occurred()) return NULL;
+    int32_t m, nnz, ncols, k;
+    int64_t alg, ldb, ldc, rows;
+    double alpha, beta;
+    if (!(pointer(a[0], &fn) && pointer(a[2], &plan) && integer(a[3], &alg) && ask32(a[4], s_numel, 1, &m) &&
+          ask32(a[5], s_numel, 0, &nnz) && integer32(a[9], &ncols)))
+        return NULL;
+    ldb = ldc = ncols;
+    if (!((a[12] == Py_None || integer(a[12], &ldb)) && (a[13] == Py_None || integer(a[13], &ldc)))) return NULL;
+    if (a[14] == Py_None && ldb == 0) return PyErr_Format(PyExc_ZeroDivisionError, "spmm: ldb = 0");
+    if (!(a[14] == Py_None ? ask(a[7], s_numel, &rows) && fits32(rows / ldb, &k) : integer32(a[14], &k))) return NULL;
+    if (!(address(a[4], &rp) && address(a[5], &col) && address(a[6], &val) && address(a[7], &B) && address(a[8], &C) &&
+          real(a[10], &alpha) && real(a[11], &beta) && workspace(a[15], &ws, &ws_bytes) && stream(&s)))
+        return NULL;
     int st;
     Py_BEGIN_ALLOW_THREADS;
-    st = f64 ? ((spmm64_t)fn)(plan, alg, m, k, nnz, ncols, alpha, rp, col, val, B, ldb, beta, C, ldc, ws, ws_bytes, s)
-             : ((spmm32_t)fn)(plan, alg, m, k, nnz, ncols, (float)alpha, rp, col, val, B, ldb, (float)beta, C, ldc, ws, ws_bytes, s);
+    st = f64 ? ((spmm64_t)fn)(plan, (int)alg, m, k, nnz, ncols, alpha, rp, col, val, B, ldb, beta, C, ldc, ws, ws_bytes, s)
+             : ((spmm32_t)fn)(plan, (int)alg, m, k, nnz, ncols, (float)alpha, rp, col, val, B, ldb, (float)beta, C, ldc, ws, ws_bytes, s);
     Py_END_ALLOW_THREADS;
     return PyLong_FromLong(st);
 }
@@ -137,8 +178,8 @@ static PyObject *plan_values(PyObject *self, PyObject *const *a, Py_ssize_t n)
 {
     (void)self;
     if (n != 3 || !get_stream) return PyErr_Format(PyExc_TypeError, "plan_values: 3 arguments, after streams_from");
-    void *fn = pointer(a[0]), *plan = pointer(a[1]), *val = address(a[2]), *s = stream();
-    if (PyErr_Occurred()) return NULL;
+    void *fn, *plan, *val, *s;
+    if (!(pointer(a[0], &fn) && pointer(a[1], &plan) && address(a[2], &val) && stream(&s))) return NULL;
     int st;
     Py_BEGIN_ALLOW_THREADS;
     st = ((values_t)fn)(plan, val, s);
@@ -159,6 +200,9 @@ PyMODINIT_FUNC PyInit__calls(void)
     s_data_ptr = PyUnicode_InternFromString("data_ptr");
     s_numel = PyUnicode_InternFromString("numel");
     s_element_size = PyUnicode_InternFromString("element_size");
-    if (!s_data_ptr || !s_numel || !s_element_size) return NULL;
+    PyObject *ctypes = PyImport_ImportModule("ctypes");
+    argument_error = ctypes ? PyObject_GetAttrString(ctypes, "ArgumentError") : NULL;
+    Py_XDECREF(ctypes);
+    if (!s_data_ptr || !s_numel || !s_element_size || !argument_error) return NULL;
     return PyModule_Create(&module);
 }
