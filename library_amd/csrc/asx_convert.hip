@@ -9,6 +9,8 @@
 #include <rocprim/device/device_radix_sort.hpp>
 
 #include <algorithm>
+#include <cstring>
+#include <type_traits>
 
 #include "asx_internal.hpp"
 #include "asx_rank.hpp"
@@ -94,7 +96,7 @@ namespace {
 //      of consecutive places.
 //   3. k_transpose_rows: one workgroup per bucket counts the bucket's columns, writes their row
 //      offsets, and orders the elements by column, up to 4096 at a time, through LDS: a bucket that
-//      fits leaves as one run of consecutive stores.
+//      fits leaves as one run of consecutive stores.  Buckets far above the average follow in pieces.
 // 3.6 M elements, fp32, 250013 columns: 120 us with the CSR multiply that follows it; a radix sort of
 // 64-bit (column, row) keys moved 24 bytes an element five times and took 316 us of kernels alone.
 constexpr int kBuckets = 1024;
@@ -256,36 +258,26 @@ __device__ __forceinline__ void columns_exclusive_sum(int32_t *a, int32_t *wave_
 
 // COLS: columns of a bucket, rounded up to a multiple of kSortThreads
 template <typename T, int COLS>
-__global__ __launch_bounds__(kSortThreads) void k_transpose_rows(const int32_t *__restrict__ offs, int32_t nblocks, int shift,
-                                                                 int nbits, int32_t n, int32_t nnz,
-                                                                 const int32_t *__restrict__ brow,
-                                                                 const uint16_t *__restrict__ bcol, const T *__restrict__ bval,
-                                                                 int32_t *__restrict__ row_ptr_t, int32_t *__restrict__ col_t,
-                                                                 T *__restrict__ val_t)
+struct RowsShared {
+    alignas(16) uint16_t cnt[kSortWaves * COLS];  // per wave and column: count, then first rank of the wave's elements
+    int32_t first[COLS];                          // per column: next free place in A^T
+    int32_t lofs[COLS];                           // per column: count, then first position in column order
+    int32_t wave_tot[kSortWaves];
+    int32_t row_s[kSortElems];
+    uint16_t col_s[kSortElems];
+    T val_s[kSortElems];
+};
+
+// Elements [s0, s1) of a bucket to their places in A^T, sh.first[c] being that of the first one of column c.
+template <typename T, int COLS>
+__device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t s0, int32_t s1, int nbits,
+                                                const int32_t *__restrict__ brow, const uint16_t *__restrict__ bcol,
+                                                const T *__restrict__ bval, int32_t *__restrict__ col_t, T *__restrict__ val_t)
 {
-    __shared__ __align__(16) uint16_t cnt[kSortWaves * COLS];  // per wave and column: count, then first rank of the wave's elements
-    __shared__ int32_t first[COLS];              // per column: next free place in A^T
-    __shared__ int32_t lofs[COLS];               // per column: count, then first position in column order
-    __shared__ int32_t wave_tot[kSortWaves];
-    __shared__ int32_t row_s[kSortElems];
-    __shared__ uint16_t col_s[kSortElems];
-    __shared__ T val_s[kSortElems];
+    uint16_t *cnt = sh.cnt, *col_s = sh.col_s;
+    int32_t *first = sh.first, *lofs = sh.lofs, *row_s = sh.row_s;
+    T *val_s = sh.val_s;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
-    const int32_t b = blockIdx.x;
-    const int32_t s0 = offs[(int64_t)b * nblocks], s1 = offs[(int64_t)(b + 1) * nblocks];
-    // column counts of the whole bucket -> row offsets of A^T
-    for (int i = tid; i < COLS; i += kSortThreads) first[i] = 0;
-    __syncthreads();
-    for (int32_t i = s0 + tid; i < s1; i += kSortThreads) atomicAdd(&first[bcol[i]], 1);
-    __syncthreads();
-    columns_exclusive_sum<COLS>(first, wave_tot);
-    const int64_t c0 = (int64_t)b << shift;
-    for (int i = tid; i < (1 << shift); i += kSortThreads) {
-        const int32_t at = s0 + first[i];
-        first[i] = at;
-        if (c0 + i < n) row_ptr_t[c0 + i] = at;
-    }
-    if (b == (int32_t)gridDim.x - 1 && tid == 0) row_ptr_t[n] = nnz;
     uint16_t *mycnt = cnt + wave * COLS;
     for (int32_t e0 = s0; e0 < s1; e0 += kSortElems) {  // uniform; one turn where the bucket fits
         __syncthreads();
@@ -315,7 +307,7 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_rows(const int32_t *
             lofs[i] = run;
         }
         __syncthreads();
-        columns_exclusive_sum<COLS>(lofs, wave_tot);
+        columns_exclusive_sum<COLS>(lofs, sh.wave_tot);
 #pragma unroll
         for (int k = 0; k < kSortPerLane; ++k) {
             if (wbase + k * kWave + lane < s1) {
@@ -339,11 +331,134 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_rows(const int32_t *
     }
 }
 
+// Buckets of more than kLargeBucket elements - a column that very many rows share - are left to k_transpose_large_*, which
+// cut them into pieces: one workgroup takes 10 us for 4096 elements of one column, so that alone it would keep the device
+// waiting (transpose of 8 M elements fp32, 6 M of them in one column: 14.7 ms, in pieces 0.30; of 400000, 68000 of them in
+// one: 208 us and 153).  large[2 b], large[2 b + 1]: where the
+// elements of such a bucket start and end, for the host (page-locked, cleared).
+constexpr int32_t kLargeBucket = 16 * kSortElems, kLargePiece = 8 * kSortElems;
+
+template <typename T, int COLS>
+__global__ __launch_bounds__(kSortThreads) void k_transpose_rows(const int32_t *__restrict__ offs, int32_t nblocks, int shift,
+                                                                 int nbits, int32_t n, int32_t nnz,
+                                                                 const int32_t *__restrict__ brow,
+                                                                 const uint16_t *__restrict__ bcol, const T *__restrict__ bval,
+                                                                 int32_t *__restrict__ row_ptr_t, int32_t *__restrict__ col_t,
+                                                                 T *__restrict__ val_t, int32_t *__restrict__ large)
+{
+    __shared__ RowsShared<T, COLS> sh;
+    const int tid = threadIdx.x;
+    const int32_t b = blockIdx.x;
+    const int32_t s0 = offs[(int64_t)b * nblocks], s1 = offs[(int64_t)(b + 1) * nblocks];
+    if (b == (int32_t)gridDim.x - 1 && tid == 0) row_ptr_t[n] = nnz;
+    if (s1 - s0 > kLargeBucket) {  // the whole workgroup leaves
+        if (tid == 0) large[2 * b] = s0, large[2 * b + 1] = s1;
+        return;
+    }
+    // column counts of the whole bucket -> row offsets of A^T
+    for (int i = tid; i < COLS; i += kSortThreads) sh.first[i] = 0;
+    __syncthreads();
+    for (int32_t i = s0 + tid; i < s1; i += kSortThreads) atomicAdd(&sh.first[bcol[i]], 1);
+    __syncthreads();
+    columns_exclusive_sum<COLS>(sh.first, sh.wave_tot);
+    const int64_t c0 = (int64_t)b << shift;
+    for (int i = tid; i < (1 << shift); i += kSortThreads) {
+        const int32_t at = s0 + sh.first[i];
+        sh.first[i] = at;
+        if (c0 + i < n) row_ptr_t[c0 + i] = at;
+    }
+    place_by_column<T, COLS>(sh, s0, s1, nbits, brow, bcol, bval, col_t, val_t);
+}
+
+// ---- large buckets: pieces of kLargePiece elements, a workgroup each ----
+// A large bucket: its number, the number of its first piece, its elements.  A call has at most kBuckets of them.
+struct LargeBucket {
+    int32_t bucket, piece, from, to;
+};
+// the bucket of piece p: the last one that starts at or before it (uniform)
+__device__ __forceinline__ LargeBucket bucket_of_piece(const LargeBucket *__restrict__ large, int32_t nlarge, int32_t p)
+{
+    int32_t lo = 0, hi = nlarge - 1;
+    while (lo < hi) {
+        const int32_t mid = lo + (hi - lo + 1) / 2;
+        if (large[mid].piece <= p)
+            lo = mid;
+        else
+            hi = mid - 1;
+    }
+    return large[lo];
+}
+
+// table[p][c] = elements of column c in piece p
+template <int COLS>
+__global__ __launch_bounds__(kSortThreads) void k_transpose_large_count(const LargeBucket *__restrict__ large, int32_t nlarge,
+                                                                        const uint16_t *__restrict__ bcol,
+                                                                        int32_t *__restrict__ table)
+{
+    __shared__ int32_t count[COLS];
+    const LargeBucket q = bucket_of_piece(large, nlarge, blockIdx.x);
+    for (int i = threadIdx.x; i < COLS; i += kSortThreads) count[i] = 0;
+    __syncthreads();
+    const int64_t from = q.from + (int64_t)((int32_t)blockIdx.x - q.piece) * kLargePiece;
+    const int64_t to = from + kLargePiece < q.to ? from + kLargePiece : q.to;
+    for (int64_t i = from + threadIdx.x; i < to; i += kSortThreads) atomicAdd(&count[bcol[i]], 1);
+    __syncthreads();
+    for (int i = threadIdx.x; i < COLS; i += kSortThreads) table[(int64_t)blockIdx.x * COLS + i] = count[i];
+}
+
+// A workgroup per large bucket: row offsets of A^T, and in the table the place of every piece's first element of every column
+template <int COLS>
+__global__ __launch_bounds__(kSortThreads) void k_transpose_large_places(const LargeBucket *__restrict__ large, int shift,
+                                                                         int32_t n, int32_t *__restrict__ table,
+                                                                         int32_t *__restrict__ row_ptr_t)
+{
+    __shared__ int32_t first[COLS];
+    __shared__ int32_t wave_tot[kSortWaves];
+    const LargeBucket q = large[blockIdx.x];
+    const int32_t pieces = (q.to - q.from + kLargePiece - 1) / kLargePiece;
+    int32_t *mine = table + (int64_t)q.piece * COLS;
+    for (int i = threadIdx.x; i < COLS; i += kSortThreads) {
+        int32_t sum = 0;
+#pragma unroll 8
+        for (int32_t p = 0; p < pieces; ++p) sum += mine[(int64_t)p * COLS + i];
+        first[i] = sum;
+    }
+    __syncthreads();
+    columns_exclusive_sum<COLS>(first, wave_tot);
+    const int64_t c0 = (int64_t)q.bucket << shift;
+    for (int i = threadIdx.x; i < COLS; i += kSortThreads) {
+        int32_t at = q.from + first[i];
+        if (i < (1 << shift) && c0 + i < n) row_ptr_t[c0 + i] = at;
+#pragma unroll 8
+        for (int32_t p = 0; p < pieces; ++p) {
+            const int32_t count = mine[(int64_t)p * COLS + i];
+            mine[(int64_t)p * COLS + i] = at;
+            at += count;
+        }
+    }
+}
+
+template <typename T, int COLS>
+__global__ __launch_bounds__(kSortThreads) void k_transpose_large_rows(const LargeBucket *__restrict__ large, int32_t nlarge,
+                                                                       int nbits, const int32_t *__restrict__ brow,
+                                                                       const uint16_t *__restrict__ bcol,
+                                                                       const T *__restrict__ bval,
+                                                                       const int32_t *__restrict__ table,
+                                                                       int32_t *__restrict__ col_t, T *__restrict__ val_t)
+{
+    __shared__ RowsShared<T, COLS> sh;
+    const LargeBucket q = bucket_of_piece(large, nlarge, blockIdx.x);
+    const int64_t from = q.from + (int64_t)((int32_t)blockIdx.x - q.piece) * kLargePiece;
+    const int64_t to = from + kLargePiece < q.to ? from + kLargePiece : q.to;
+    for (int i = threadIdx.x; i < COLS; i += kSortThreads) sh.first[i] = table[(int64_t)blockIdx.x * COLS + i];
+    place_by_column<T, COLS>(sh, (int32_t)from, (int32_t)to, nbits, brow, bcol, bval, col_t, val_t);
+}
+
 // Columns of a bucket, as a power of two: buckets of up to two turns of kSortElems elements (a run of 8 elements per
 // block and bucket in pass 2; 3.6 M elements: 33 us there against 40 with buckets of one turn), fewer where that
-// leaves less than a workgroup per compute unit, more where kBuckets of them are not enough.  -1: the sort by keys takes the matrix, because a bucket would
-// span more than kBucketColumns columns or few columns hold so much that their buckets' workgroups would work in turn
-// (one workgroup takes about 2 us per 4096 elements).
+// leaves less than a workgroup per compute unit, more where kBuckets of them are not enough.  -1: the sort by keys takes the
+// matrix, because a bucket would span more than kBucketColumns columns, or because so few columns hold so much that most
+// buckets would be large ones.
 int bucket_shift(int32_t n, int32_t nnz)
 {
     if (nnz > 0x7fff0000) return -1;  // element numbers past the last one have to fit as well
@@ -392,18 +507,43 @@ int csr_transpose_buckets(int shift, int32_t m, int32_t n, int32_t nnz, int32_t 
     if (st) return st;
     hipLaunchKernelGGL((k_transpose_bucket<T>), dim3((unsigned)(ceil_div64(nblocks, kXcds) * kXcds)), dim3(kSortThreads), 0, s,
                        row_ptr, col, val, seg, nnz, base, shift, nbuckets, bbits, nblocks, counts, brow, bcol, bval);
-#define ASX_ROWS(COLS)                                                                                                   \
-    hipLaunchKernelGGL((k_transpose_rows<T, COLS>), dim3((unsigned)nbuckets), dim3(kSortThreads), 0, s, counts, nblocks, shift, \
-                       shift, n, nnz, brow, bcol, bval, row_ptr_t, col_t, val_t)
-    if (shift <= 9)
-        ASX_ROWS(512);
-    else if (shift == 10)
-        ASX_ROWS(1024);
-    else
-        ASX_ROWS(kBucketColumns);
-#undef ASX_ROWS
-    st = check_launch();
-    if (!st) st = status_of(hipStreamSynchronize(s));
+    int32_t *found = static_cast<int32_t *>(scratch.pinned());
+    static_assert(2 * kBuckets * sizeof(int32_t) <= kPinnedBytes, "large buckets are reported through page-locked memory");
+    if (!found) return ASX_STATUS_ALLOC_FAILED;
+    std::memset(found, 0, 2 * sizeof(int32_t) * (size_t)nbuckets);
+    const auto rows = [&](auto cols_) {
+        constexpr int COLS = decltype(cols_)::value;
+        hipLaunchKernelGGL((k_transpose_rows<T, COLS>), dim3((unsigned)nbuckets), dim3(kSortThreads), 0, s, counts, nblocks, shift,
+                           shift, n, nnz, brow, bcol, bval, row_ptr_t, col_t, val_t, found);
+        int rc = check_launch();
+        if (!rc) rc = status_of(hipStreamSynchronize(s));
+        if (rc) return rc;
+        LargeBucket large[kBuckets];
+        int32_t nlarge = 0, pieces = 0;
+        for (int32_t b = 0; b < nbuckets; ++b) {
+            const int32_t from = found[2 * b], to = found[2 * b + 1];
+            if (to == 0) continue;
+            large[nlarge++] = LargeBucket{b, pieces, from, to};
+            pieces += (int32_t)ceil_div64((int64_t)to - from, kLargePiece);
+        }
+        if (nlarge == 0) return rc;
+        LargeBucket *d_large = nullptr;
+        int32_t *table = nullptr;
+        rc = status_of(scratch.take(&d_large, sizeof(LargeBucket) * (size_t)nlarge));
+        if (!rc) rc = status_of(scratch.take(&table, sizeof(int32_t) * COLS * (size_t)pieces));
+        if (!rc) rc = status_of(hipMemcpyAsync(d_large, large, sizeof(LargeBucket) * (size_t)nlarge, hipMemcpyHostToDevice, s));
+        if (rc) return rc;
+        const dim3 per_piece((unsigned)pieces), threads(kSortThreads);
+        hipLaunchKernelGGL(k_transpose_large_count<COLS>, per_piece, threads, 0, s, d_large, nlarge, bcol, table);
+        hipLaunchKernelGGL(k_transpose_large_places<COLS>, dim3((unsigned)nlarge), threads, 0, s, d_large, shift, n, table, row_ptr_t);
+        hipLaunchKernelGGL((k_transpose_large_rows<T, COLS>), per_piece, threads, 0, s, d_large, nlarge, shift, brow, bcol, bval, table,
+                           col_t, val_t);
+        rc = check_launch();
+        return rc ? rc : status_of(hipStreamSynchronize(s));
+    };
+    st = shift <= 9    ? rows(std::integral_constant<int, 512>{})
+         : shift == 10 ? rows(std::integral_constant<int, 1024>{})
+                       : rows(std::integral_constant<int, kBucketColumns>{});
     scratch.idle = st == ASX_STATUS_SUCCESS;
     return st;
 }
