@@ -45,11 +45,11 @@ __device__ __forceinline__ T spmm_accumulate(T acc, int32_t k_begin, int32_t k_e
                                              const T *__restrict__ val, const T *__restrict__ B,
                                              int64_t ldb)
 {
-    for (int32_t k0 = k_begin; k0 < k_end; k0 += kWave) {
-        const int32_t kk = k0 + lane;
-        const int32_t cl = kk < k_end ? col[kk] : 0;
-        const T vl = kk < k_end ? val[kk] : T(0);
-        const int cnt = k_end - k0 < kWave ? k_end - k0 : kWave;
+    int64_t at = (int64_t)k_begin + lane;
+    for (int32_t left = k_end - k_begin; left > 0; left -= kWave, at += kWave) {  // counted down: k_end may be 2^31 - 1
+        const int32_t cl = lane < left ? col[at] : 0;
+        const T vl = lane < left ? val[at] : T(0);
+        const int cnt = left < kWave ? left : kWave;
         // kSpmmInFlight rows of B at a time
         int j = 0;
         for (; j + kSpmmInFlight <= cnt; j += kSpmmInFlight) {
