@@ -799,7 +799,7 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
     const int64_t ncount = (int64_t)sm.nslices * nblocks + 1;
     const int64_t cap64 = (int64_t)nnz + (int64_t)(kSlicedTile - 1) * sm.nslices;  // the most slots there can be
     const int64_t ncells = ((int64_t)sm.nrb + 1) * sm.nslices;
-    if (cap64 > 0x7fffffff - kSlicedTile || ncount > 0x7fffffff || ncells > 0x7fffffff) return ASX_STATUS_INVALID_SIZE;
+    if (cap64 > 0x7fffffff || ncount > 0x7fffffff || ncells > 0x7fffffff) return ASX_STATUS_INVALID_SIZE;
     const int32_t max_tiles = (int32_t)ceil_div64(cap64, kSlicedTile);
     const size_t max_slots = (size_t)max_tiles * kSlicedTile;
     const size_t max_pieces = (size_t)std::min(target_wgs, kLayoutThreads) + (size_t)sm.nslices;

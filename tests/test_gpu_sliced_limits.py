@@ -1,0 +1,30 @@
+"""Column-sliced plans at the limits of their sizes."""
+import numpy as np
+import pytest
+import torch
+
+from library_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def test_as_many_elements_as_slots_can_be_counted():
+    """2^31 - 1 slots when the 255 that one slice may spare are counted.  Integers: exact in any order."""
+    width, nnz = 32768, 2**31 - 1 - 255
+    m = -(-nnz // width)
+    row_ptr = torch.arange(m + 1, dtype=torch.int64, device="cuda") * width
+    row_ptr[-1] = nnz
+    row_ptr = row_ptr.to(torch.int32)
+    col = torch.arange(width, dtype=torch.int32, device="cuda").repeat(m)[:nnz]
+    val = torch.ones(nnz, dtype=torch.float32, device="cuda")
+    x = (torch.arange(width, device="cuda") % 5).to(torch.float32)
+    plan = capi.Plan(False, capi.SPMV_SLICED, val.dtype, m, width, nnz, row_ptr, col=col, val=val)
+    y = torch.full((m,), -7.0, device="cuda")
+    capi.spmv(row_ptr, col, val, x, y, 1.0, 0.0, plan=plan)
+    torch.cuda.synchronize()
+    plan.destroy()
+    assert bool((y[:-1] == x.sum()).all()) and y[-1].item() == x[:nnz - (m - 1) * width].sum().item()
+    with pytest.raises(capi.AsxError):
+        capi.Plan(False, capi.SPMV_SLICED, val.dtype, m, width + 1, nnz, row_ptr, col=col, val=val)  # two slices
+    capi.lib().asx_release_cached_memory()
+    torch.cuda.empty_cache()
