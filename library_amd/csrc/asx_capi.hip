@@ -688,6 +688,7 @@ static int64_t rows_of_at_least(const asx_plan *p, int32_t len /* a power of two
         if (((int64_t)1 << (b - 1)) >= len) n += p->hist[b];
     return n;
 }
+static int32_t slice_count(const asx_plan *p, size_t sv) { return (int32_t)ceil_div64((int64_t)p->n * (int64_t)sv, kSliceBytes); }
 struct KernelEstimates {
     // seconds; infinity where the kernel does not apply.  window: with one ring of x per block;
     // window_bands: with rings per band of diagonals, window_stacked: with three bands on stacked
@@ -737,7 +738,7 @@ static KernelEstimates estimate_kernels(const asx_plan *p, size_t sv, const Colu
     if (merge < e.rows) e.row_kernel = ASX_SPMV_MERGE, e.rows = merge;
     // Mostly empty rows: only the merge-path kernel counts row ends as work
     if (p->hist[0] > (int64_t)p->m / 2) e.row_kernel = ASX_SPMV_MERGE, e.rows = merge;
-    const int64_t nslices = ceil_div64((int64_t)p->n * (int64_t)sv, kSliceBytes);
+    const int32_t nslices = slice_count(p, sv);
     e.sliced = nslices > kSlicedMaxSlices
                    ? inf
                    : 9.9e-6 + (nnz * (dsv + 2) + cs.pairs * nnz * (2 * dsv + 2) + n * dsv + 2 * m * dsv) / 5.6e12 +
@@ -781,6 +782,21 @@ static int plan_long_rows(asx_plan *p, hipStream_t s)
     return st;
 }
 
+// pass 2: one wave per block of rows, its accumulators (8 bytes a row) in LDS.  Blocks of 256
+// rows, doubled up to 1024 while that leaves more than 8 waves per compute unit and the block's
+// partial sums inside one slice (expected from the column sample) are fewer than 12: a
+// step of pass 2 takes its 64 entries from at most three ranges.  Small blocks mean many waves
+// in flight.  Measured: the power-law matrix (4 per range at 256 rows) 50 / 34.5 / 36.6 us with
+// 512 / 1024 / 2048 rows; 16 per row over 32 slices (100 per range at 256 rows) 17.5 / 20 us
+// with 256 / 512 rows; the same in fp64 over 64 slices 26.5 / 27.5 / 36.8 us with 256 / 512 / 1024.
+static int32_t sliced_rows_per_wave(const asx_plan *p, size_t sv, double pairs_per_element, int cus)
+{
+    const double per_row_slice = pairs_per_element * (double)p->nnz / ((double)p->m * (double)slice_count(p, sv));
+    int32_t rpw = 256;
+    while (rpw < 1024 && (int64_t)rpw * cus * 8 < p->m && per_row_slice * rpw < 12.0) rpw *= 2;
+    return rpw;
+}
+
 // Builds the sliced copy onto a plan that already holds the histogram (`p` takes the slices over;
 // its own split points are dropped).
 template <typename T>
@@ -789,17 +805,7 @@ int plan_add_slices(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
 {
     int cus = 256;
     (void)asx_device_info(&cus, nullptr);
-    // pass 2: one wave per block of rows, its accumulators (8 bytes a row) in LDS.  Blocks of 256
-    // rows, doubled up to 1024 while that leaves more than 8 waves per compute unit and the block's
-    // partial sums inside one slice (expected from the column sample) are fewer than 12: a
-    // step of pass 2 takes its 64 entries from at most three ranges.  Small blocks mean many waves
-    // in flight.  Measured: the power-law matrix (4 per range at 256 rows) 50 / 34.5 / 36.6 us with
-    // 512 / 1024 / 2048 rows; 16 per row over 32 slices (100 per range at 256 rows) 17.5 / 20 us
-    // with 256 / 512 rows; the same in fp64 over 64 slices 26.5 / 27.5 / 36.8 us with 256 / 512 / 1024.
-    const int32_t nslices = (int32_t)ceil_div64((int64_t)p->n * (int64_t)sizeof(T), kSliceBytes);
-    const double per_row_slice = pairs_per_element * (double)p->nnz / ((double)p->m * (double)nslices);
-    int32_t rpw = 256;
-    while (rpw < 1024 && (int64_t)rpw * cus * 8 < p->m && per_row_slice * rpw < 12.0) rpw *= 2;
+    const int32_t rpw = sliced_rows_per_wave(p, sizeof(T), pairs_per_element, cus);
     SlicedMatrix sm{};
     const int st = build_sliced<T>(p->m, p->n, p->nnz, (int32_t)(kSliceBytes / sizeof(T)), rpw, cus, d_row_ptr, d_col,
                                    d_val, &sm, s);
@@ -851,11 +857,19 @@ int plan_add_window(asx_plan *p, const int32_t *d_row_ptr, const int32_t *d_col,
 // the values up to date and a buffer for the partial sums of a call), and its build needs about 4
 // bytes per stored element more for a while.
 // DEFAULT only makes one while twice that is free: a caller who sized the device for one copy of A
-// is not pushed to the edge by an analysis call.
-static bool regrouped_copy_fits(const asx_plan *p, size_t sv, size_t free_bytes)
+// is not pushed to the edge by an analysis call.  Slices also need tables by row block and slice: where the ranges
+// start, and twice, for a while, the steps of pass 2 (512 M rows and 1024 slices: 7.8 GB, whatever the rows hold).
+static bool regrouped_copy_fits(const asx_plan *p, size_t sv, size_t free_bytes, double tables)
 {
     const double copy = (double)p->nnz * (double)(sv + 8) + (double)p->nnz * (double)(sv + 2) + (double)p->nnz * 4.0;
-    return (double)free_bytes >= 2.0 * copy;
+    return (double)free_bytes >= 2.0 * (copy + tables);
+}
+static double sliced_tables(const asx_plan *p, size_t sv, double pairs_per_element)
+{
+    int cus = 256;
+    (void)asx_device_info(&cus, nullptr);
+    const double nslices = (double)slice_count(p, sv), nrb = (double)ceil_div64(p->m, sliced_rows_per_wave(p, sv, pairs_per_element, cus));
+    return 4.0 * nrb * nslices + 32.0 * (double)sliced_steps_most(p->nnz, (int64_t)nrb, (int64_t)nslices);
 }
 
 static bool window_may_pay(const asx_plan *p) { return 2 * p->hist[0] + p->hist[1] <= (int64_t)p->nnz / 4; }
@@ -910,7 +924,7 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
         return f64 ? plan_add_window<double>(p, d_row_ptr, d_col, (const double *)d_val, checked, s)
                    : plan_add_window<float>(p, d_row_ptr, d_col, (const float *)d_val, checked, s);
     };
-    const bool can_regroup = may_regroup && regrouped_copy_fits(p, sv, ps.free_bytes);
+    const bool can_regroup = may_regroup && regrouped_copy_fits(p, sv, ps.free_bytes, 0.0);
     const ColumnSample &cs = ps.sample;
     bool done = false, list_long_rows = false;
     if (alg == ASX_SPMV_WINDOW) {
@@ -932,7 +946,8 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
             const bool large = nnz >= (1 << 22), scattered = cs.spread >= kScatteredMinSpread;
             const double between = large && cs.spread > 0.1 && !scattered ? 1.1 : large ? 0.97 : 0.95;
             const double ahead = (scattered && (large || cs.pairs < 0.15) ? 1.04 : between) * e.rows;
-            const bool sliced_pays = e.sliced < ahead, window_pays = e.window < ahead * (nnz < (1 << 22) ? 0.9 : 1.0);
+            const bool sliced_pays = e.sliced < ahead && regrouped_copy_fits(p, sv, ps.free_bytes, sliced_tables(p, sv, cs.pairs));
+            const bool window_pays = e.window < ahead * (nnz < (1 << 22) ? 0.9 : 1.0);
             const bool in_place = !f64 && p->hist[0] + p->hist[1] == 0 && p->stats[0] <= 16;
             const double slices_for_window = e.sliced * (in_place ? 1.09 : 1 / 1.05);
             if (window_pays && e.window < slices_for_window) done = add_window() == ASX_STATUS_SUCCESS;

@@ -179,6 +179,8 @@ struct SlicedMatrix {
 };
 constexpr int kSlicedStepPad = 64;     // readable step descriptors past the last one
 constexpr int kSlicedReducePad = 256;  // entries of prow / partial that pass 2 may read past the last partial sum
+// the most steps there can be (k_sliced_pack)
+inline int64_t sliced_steps_most(int64_t npartials, int64_t nrb, int64_t nslices) { return npartials / kWave + nrb * (nslices / 3 + 2); }
 template <typename T>
 int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_per_wave, int32_t target_wgs,
                  const int32_t *row_ptr, const int32_t *col, const T *val, SlicedMatrix *out, hipStream_t s);

@@ -25,6 +25,7 @@
 // No global atomics; results are bit-reproducible.  The reference has no counterpart (its CSR
 // kernels gather x from global memory: hip/kernel/level2/alphasparse_spmv_csr_vector.h:99-126).
 #include <algorithm>
+#include <utility>
 
 #include "asx_internal.hpp"
 #include "asx_rank.hpp"
@@ -575,7 +576,6 @@ __device__ __forceinline__ int64_t raw_steps_at(const int32_t *__restrict__ chun
     for (int d = 1; d < kWave; d <<= 1) before += __shfl_xor(before, d, kWave);
     return (int64_t)(before / kWave) + b * (nslices / 3 + 2);
 }
-inline int64_t raw_steps_most(int64_t npartials, int64_t nrb, int64_t nslices) { return npartials / kWave + nrb * (nslices / 3 + 2); }
 
 __global__ __launch_bounds__(kBlock) void k_sliced_pack(const int32_t *__restrict__ chunk_lo, int32_t nrb,
                                                          int32_t nslices, int32_t *__restrict__ count,
@@ -818,6 +818,7 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
     int32_t *lrow = nullptr, *tile_cnt = nullptr, *step_cnt = nullptr;
     int32_t *tmp = nullptr, *info = nullptr;
     i32x4 *raw = nullptr;
+    int64_t most_steps = 0;
 #define ASX_TRY(expr)         \
     do {                      \
         st = status_of(expr); \
@@ -897,8 +898,8 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
     ASX_TRY(hipGetLastError());
     ASX_TRY(hipStreamSynchronize(s));
     sm.ntiles = host[0], sm.nwg = host[1], sm.npieces = host[2], sm.npartials = host[4];
+    most_steps = sliced_steps_most(sm.npartials, sm.nrb, sm.nslices);
     {
-        const int64_t most_steps = raw_steps_most(sm.npartials, sm.nrb, sm.nslices);
         if (most_steps > 0x7fffffff - kSlicedStepPad) {
             st = ASX_STATUS_INVALID_SIZE;
             goto done;
@@ -924,6 +925,17 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
     ASX_TRY(hipGetLastError());
     ASX_TRY(hipStreamSynchronize(s));
     sm.npsteps = host[5];
+    // Few partial sums in many row blocks and slices leave most of the steps' room unused (100000 elements in 16 M rows and
+    // 1024 slices: 90 MB for 2 MB).
+    if (const size_t exact = sizeof(i32x4) * ((size_t)sm.npsteps + kSlicedStepPad), room = sizeof(i32x4) * (size_t)most_steps;
+        room > exact + exact / 4 + ((size_t)4 << 20)) {
+        int32_t *fitting = nullptr;
+        ASX_TRY(pool_malloc(&fitting, exact, false));
+        std::swap(fitting, sm.psteps);
+        st = status_of(hipMemcpyAsync(sm.psteps, fitting, exact, hipMemcpyDeviceToDevice, s));
+        if (!st) st = status_of(hipStreamSynchronize(s));
+        pool_free(fitting, st == ASX_STATUS_SUCCESS);
+    }
 #undef ASX_TRY
 #undef ASX_TRY_ST
 done:

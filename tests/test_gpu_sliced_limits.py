@@ -28,3 +28,27 @@ def test_as_many_elements_as_slots_can_be_counted():
         capi.Plan(False, capi.SPMV_SLICED, val.dtype, m, width + 1, nnz, row_ptr, col=col, val=val)  # two slices
     capi.lib().asx_release_cached_memory()
     torch.cuda.empty_cache()
+
+
+def test_steps_of_many_row_blocks_take_the_room_they_need():
+    """100000 elements in 16 M rows and 1024 slices: tables of 67 MB by row block and slice, 5 MB for the rest, not 90 MB for
+    the most steps that there could be."""
+    m, n, nnz = 1 << 24, 1 << 25, 100000
+    rng = np.random.default_rng(2)
+    rows = np.sort(rng.choice(m, nnz, replace=False))
+    row_ptr = torch.from_numpy(np.searchsorted(rows, np.arange(m + 1)).astype(np.int32)).cuda()
+    col = torch.from_numpy(rng.integers(0, n, nnz).astype(np.int32)).cuda()
+    val, x = torch.ones(nnz, device="cuda"), (torch.arange(n, device="cuda") % 5).to(torch.float32)
+    y = torch.full((m,), -7.0, device="cuda")
+    capi.lib().asx_release_cached_memory()
+    before = torch.cuda.mem_get_info()[0]
+    plan = capi.Plan(False, capi.SPMV_SLICED, val.dtype, m, n, nnz, row_ptr, col=col, val=val)
+    capi.lib().asx_release_cached_memory()
+    held = before - torch.cuda.mem_get_info()[0]
+    capi.spmv(row_ptr, col, val, x, y, 1.0, 0.0, plan=plan)
+    torch.cuda.synchronize()
+    plan.destroy()
+    expect = torch.zeros(m, device="cuda")
+    expect[torch.from_numpy(rows).cuda()] = x[col.long()]
+    assert torch.equal(y, expect)
+    assert held < 110e6, held
