@@ -510,6 +510,17 @@ int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T al
                       bool carry_pass, int tile_bytes, hipStream_t s)
 {
     if (m <= 0 || ncols <= 0) return ASX_STATUS_SUCCESS;
+    // Tiles of columns are blocks along a grid's y, of which there are at most 65535: more columns are walked in slabs of whole
+    // tiles, one after the other in the same workspace.
+    const int64_t slab = (int64_t)65535 * (tile_bytes / (int64_t)sizeof(T));
+    if (ncols > slab) {
+        for (int64_t c = 0; c < ncols; c += slab) {
+            const int st = launch_spmm_merge<T>(m, nnz, items, (int32_t)(ncols - c < slab ? ncols - c : slab), alpha, row_ptr, col, val, B + c,
+                                                ldb, beta, C + c, ldc, xs, ys, carry, carry_row, carry_pass, tile_bytes, s);
+            if (st) return st;
+        }
+        return ASX_STATUS_SUCCESS;
+    }
     const int32_t nseg = spmm_segments(m, nnz, items);
     const SpmmTiling tiling = spmm_tiling(ncols, tile_bytes, sizeof(T));
     if (!carry_pass) carry = nullptr, carry_row = nullptr;  // no row is cut: nothing is left for the pass

@@ -65,3 +65,12 @@ def test_spmm_blocked_widths(oracle, dtype, n):
     rp, col, val = A.indptr.astype(np.int32), A.indices.astype(np.int32), A.data.astype(dtype)
     for ldb, ldc, beta in ((n, n, 0.0), (n, n, 1.0), (n + 1, n + 3, 0.5)):
         _check(oracle, rp, col, val, k, n, ldb, ldc, beta, True, f"blocked n={n} ldb={ldb} beta={beta}", alg=capi.SPMM_BLOCKED)
+
+
+@pytest.mark.parametrize("dtype,n", [(np.float64, 1048561), (np.float32, 2097220)])
+def test_spmm_merge_most_columns(oracle, dtype, n):
+    """More columns than 65535 tiles of 128 bytes hold, rows of B on lines."""
+    rp, col, val = csr_from_lengths(np.array([2, 0, 3]), 4, 9, dtype)
+    ld = (n + 31) // 32 * 32
+    for planned in (False, True):
+        _check(oracle, rp, col, val, 4, n, ld, ld, 0.5, planned, f"n={n} planned={planned}")
