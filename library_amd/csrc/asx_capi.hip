@@ -665,13 +665,13 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
 // With a list of its long rows the vector kernel costs 0.5 more and 0.0004 per element of the longest row instead of the
 // turns, u divided by the turns a wave of the other rows takes.
 // A regrouped kernel is taken when its estimate is 3 % below the row-ordered ones; 5 % (window 15 %, the dearest to build)
-// below 4 M stored elements, where it saves little for what its build costs.  Two exceptions, because what gathers cost the
-// row-ordered kernels is estimated less well than what a copy streams: from 4 M on up to 10 % slower will do where the columns
-// are neither neighbours nor scattered, and up to 4 % where they are scattered (239797 x 47, fp64, values checked in every
-// call: 69 us against 85 with stream) - below 4 M as well where a slice holds seven elements and more of a row, so that the
-// slices have few partial sums to carry (60363 x 37 over 37213 columns, fp64: 14.1 us against 17.2; 246858 x 14 near the
-// diagonal 20.2 against 22.8; where the pairs are more the slices fell behind: 61822 x 34 over 120316 columns 18.0 against
-// 16.6).  Of the two, the sliced one unless the window one is estimated more than 5 % faster - or, in
+// below 4 M stored elements, where it saves little for what its build costs.  Two exceptions from 4 M on, because what gathers
+// cost the row-ordered kernels is estimated less well than what a copy streams: up to 10 % slower will do where the columns
+// are neither neighbours nor scattered, and up to 4 % where they are scattered and the plan is a checked one, which is kept
+// over many calls (239797 x 47, fp64: 69 us a call against 85 with stream).  Other plans may serve one multiply: 300000 x 16
+// over 400000 columns fp64, analysis, multiply and drop take 75 us row-ordered and 236 in slices, which save nothing then
+// (31.0 us a multiply, 30.1 row-ordered); 60363 x 37 over 37213 columns 59 and 166, for 13.5 us a multiply instead of 15.7.
+// Of the two, the sliced one unless the window one is estimated more than 5 % faster - or, in
 // fp32 with rows the tiles do not cut, not more than 9 % slower: its plan reads A's values where the caller keeps them, and a
 // caller who changes them before every multiply has nothing to bring up to date (7 per row, 22 M elements: 48 us against 95;
 // 12 per row, 30 M: 53 against 119).  A caller who never changes them loses a little: those 30 M take 53.5 us, 50.7 in slices.
@@ -945,7 +945,7 @@ static int spmv_plan_create(asx_plan **out, int alg, int value_type, int32_t m, 
         if (can_regroup && cs.ok) {
             const bool large = nnz >= (1 << 22), scattered = cs.spread >= kScatteredMinSpread;
             const double between = large && cs.spread > 0.1 && !scattered ? 1.1 : large ? 0.97 : 0.95;
-            const double ahead = (scattered && (large || cs.pairs < 0.15) ? 1.04 : between) * e.rows;
+            const double ahead = (large && scattered && checked ? 1.04 : between) * e.rows;
             const bool sliced_pays = e.sliced < ahead && regrouped_copy_fits(p, sv, ps.free_bytes, sliced_tables(p, sv, cs.pairs));
             const bool window_pays = e.window < ahead * (nnz < (1 << 22) ? 0.9 : 1.0);
             const bool in_place = !f64 && p->hist[0] + p->hist[1] == 0 && p->stats[0] <= 16;
