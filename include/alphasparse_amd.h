@@ -202,8 +202,8 @@ int asx_spmm_plan_create(asx_plan **plan, int alg, int value_type, int32_t m, in
  * must not overlap.  alg = ASX_SPMV_DEFAULT estimates every kernel's time from the sizes, the row-length
  * histogram and a sample of the columns (64 tiles of 1024 stored elements) and picks the lowest: a row-ordered
  * kernel, or for nnz >= 2^21 that kernel where it is far enough ahead to be worth building; the choice depends on
- * the matrix alone, not on timings.  A plan for the vector kernel also lists the long rows where a few rows are much longer than the rest.  Other algorithms as
- * asx_plan_create.  No counterpart in the reference (its
+ * the matrix alone, not on timings.  A plan for the vector kernel also lists the long rows where a few rows are
+ * much longer than the rest.  Other algorithms as asx_plan_create.  No counterpart in the reference (its
  * alphasparseSpMV_analysis is a stub).  alg = ASX_SPMV_WINDOW builds the row-block copy for the
  * kernel that keeps sliding windows of x in LDS (again a COPY of columns and values, and the
  * carry slots of a call; a matrix without rows of fewer than two stored elements needs no copy of

@@ -4,8 +4,9 @@
 //
 // It pays only where blocks are dense: per stored element it streams 4/fill bytes of A (fp32)
 // instead of 8, and reads 4 rows of B per block instead of one row per stored element
-// (16/fill vs 256 bytes per element at N = 64).  fill = nnz / (64 * blocks); below about 1/8
-// the merge kernel moves fewer bytes, so DEFAULT picks this variant only above that.
+// (16/fill vs 256 bytes per element at N = 64).  fill = nnz / (64 * blocks); below about 1/8 (0.2, 0.3
+// and 0.4 where rows of B are down to 128, 64 and fewer bytes) the merge kernel is ahead, so DEFAULT
+// picks this variant only above that.
 //
 // The reference's counterpart (hip/kernel/level3/alphasparse_spmm_tc4csr.h:38-256) builds the
 // blocks on the host through a dense ceil(M/16) x ceil(K/4) bitmap, keeps them in a global, and
@@ -14,7 +15,8 @@
 //
 // The zero fill of a block is multiplied with real rows of B: a non-finite value in a row of B
 // that some row of the block does not reference reaches that row of C as NaN (0 * Inf), where a
-// row-wise kernel would not have read it.  As for any padded block format, B must be finite.
+// row-wise kernel would not have read it.  As for any padded block format, B must be finite.  (What
+// a batch fetches past the last block or past B's last row counts as zeros and is not multiplied.)
 #include <rocprim/device/device_radix_sort.hpp>
 #include <rocprim/device/device_scan.hpp>
 

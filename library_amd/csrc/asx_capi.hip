@@ -119,10 +119,11 @@ ColumnSample sample_columns(const int32_t *d_col, int32_t nnz, size_t sv, hipStr
 constexpr int32_t kSmallNnz = 1 << 18;
 constexpr int64_t kSmallMaxRow = 2048;
 
-// DEFAULT with a plan: the flat kernel, except for matrices with very long rows, where the
-// merge-path kernel measured about 1 % faster (power-law: 569 vs 576 us).  Elsewhere flat is the
-// fastest of the four or within 1 % of it (5-point stencil 300 us vs stream 305; uniform 16/row
-// 95 vs stream 96), and it has no bad case: work per tile is bounded whatever the row lengths.
+// DEFAULT with a plan made without columns and values (with them estimate_kernels decides): the flat
+// kernel, except for matrices with very long rows, where the merge-path kernel measured about 1 %
+// faster (power-law: 569 vs 576 us).  Elsewhere flat is within a few per cent of the fastest
+// (5-point stencil 300 us vs stream 305), and it has no bad case: work per tile is bounded whatever
+// the row lengths.
 // Matrices small enough to be bound by launch overhead take the vector kernel, the only one that
 // is a single launch with no metadata (1280 x 1280 banded: 13.4 us against 16.2 us).
 // Mostly-empty matrices (more than half of the rows hold nothing) take the merge-path kernel,
@@ -265,9 +266,9 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         } else {
             xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
-        return launch_spmm_merge<T>(m, nnz, plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T)), ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
-                                    ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
-                                    plan ? plan->carry_pass != 0 : true,
+        const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
+        return launch_spmm_merge<T>(m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
+                                    (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off), plan ? plan->carry_pass != 0 : true,
                                     spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
     }
     case ASX_SPMM_BLOCKED:

@@ -334,8 +334,8 @@ __device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t
 // Buckets of more than kLargeBucket elements - a column that very many rows share - are left to k_transpose_large_*, which
 // cut them into pieces: one workgroup takes 10 us for 4096 elements of one column, so that alone it would keep the device
 // waiting (transpose of 8 M elements fp32, 6 M of them in one column: 14.7 ms, in pieces 0.30; of 400000, 68000 of them in
-// one: 208 us and 153).  large[2 b], large[2 b + 1]: where the
-// elements of such a bucket start and end, for the host (page-locked, cleared).
+// one: 208 us and 153).  large[2 b], large[2 b + 1]: where the elements of such a bucket start and end, for the host
+// (page-locked, cleared).
 constexpr int32_t kLargeBucket = 16 * kSortElems, kLargePiece = 8 * kSortElems;
 
 template <typename T, int COLS>

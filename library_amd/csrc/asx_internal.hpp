@@ -16,7 +16,9 @@ constexpr int kMergeItemsPerThread = 8;
 constexpr int kMergeTile = kBlock * kMergeItemsPerThread;  // rows + stored elements per tile
 constexpr int kStreamTile = 1024;                          // stored elements per row block
 constexpr int kFlatTile = 1024;                            // stored elements per flat tile
-constexpr int kLongRow = 8192;  // DEFAULT (with a plan) switches to the merge-path kernel above this row length
+// Plans made without columns and values go from the flat to the merge-path kernel above this row length; with them the
+// estimates (estimate_kernels) leave the flat kernel out there.
+constexpr int kLongRow = 8192;
 // SpMM: merge items (rows + stored elements) per wave
 constexpr int kSpmmSegmentSmall = 128, kSpmmSegmentMedium = 256, kSpmmSegmentLarge = 512;
 constexpr double kScatteredMinSpread = 0.5;  // of a column sample: from here on the columns count as scattered
@@ -66,8 +68,8 @@ int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const
 // the counters set to zero, then launch_row_histogram and launch_sample_columns in one launch (samples = 0: no sample);
 // d_row_blocks: the nb row blocks of launch_stream_row_blocks too (null: not wanted)
 int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int64_t *d_hist, int64_t *d_stats,
-                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample, int32_t nb, int32_t *d_row_blocks,
-                      hipStream_t s);
+                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample, int32_t nb,
+                      int32_t *d_row_blocks, hipStream_t s);
 int launch_gather_lines(const void *d_buf, size_t bytes, int group_lanes, int per_lane, void *d_out, int *nthreads,
                         hipStream_t s);
 
@@ -338,8 +340,9 @@ struct asx_plan {
     int value_type;
     int32_t m, n, nnz, ncols;
     const int32_t *row_ptr;  // the device array the plan was built from (identity check only)
-    int64_t *d_counters;     // kPlanCounters words on the device: histogram (33), stats (4), a flag (40), counts of long rows (41), checksums of the values:
-                             // of this call (44, 45) and of the copy the plan holds (46, 47), 64 sample counts (64..95)
+    int64_t *d_counters;     // kPlanCounters words on the device: histogram (33), stats (4), a flag (40), counts of long rows (41),
+                             // checksums of the values: of this call (44, 45) and of the copy the plan holds (46, 47),
+                             // 64 sample counts (64..95)
     int checked;             // the plan holds a copy of A's values and a checksum of them (asx_spmv_plan_create_checked)
     unsigned long long *d_checksum_parts;  // checked plans: the workgroups' partial sums of one checksum run
     int32_t nmarked;         // row blocks of the stream kernel behind the counters (0: none)

@@ -168,7 +168,8 @@ __global__ __launch_bounds__(kBlock) void k_spmm_splits(int32_t m, int32_t nnz, 
 }
 
 // Boundaries seg and seg + 1 by the wave that owns the segment, for calls without a plan (a launch of k_spmm_splits
-// before it: 13.9 us against 10.0 with 85000 elements and 8 columns, 271 against 266 with 3.8 M and 100): four groups of 16 lanes search the points seg - 1 .. seg + 2 side by side, 16 probes at a time.
+// before it: 13.9 us against 10.0 with 85000 elements and 8 columns, 271 against 266 with 3.8 M and 100): four groups of 16
+// lanes search the points seg - 1 .. seg + 2 side by side, 16 probes at a time.
 __device__ __forceinline__ void segment_ends(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nnz, int32_t items,
                                              int32_t nseg, int64_t seg, int32_t &x0, int32_t &y0, int32_t &x1, int32_t &y1)
 {
@@ -466,9 +467,9 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge_fixup(int32_t m, int32_t 
 // N is cut into equal tiles of at most tile_bytes of a row of B (every tile at least VEC wide); lanes per row of B: the
 // smallest power of two that spans a tile at VEC columns each.
 template <typename T, int VEC, int SEG>
-static void launch_merge_width(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
-                               const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
-                               T *carry, int32_t *carry_row, hipStream_t s)
+static void launch_merge_width(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
+                               const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                               const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, hipStream_t s)
 {
     const dim3 grid((unsigned)(ceil_div64(ceil_div64(nseg, kBlock / kWave), kXcds) * kXcds), (unsigned)tiling.tiles);
 #define ASX_WIDTH(LOGG)                                                                                              \
@@ -490,17 +491,20 @@ static void launch_merge_width(const SpmmTiling &tiling, int32_t m, int32_t nnz,
 }
 
 template <typename T, int SEG>
-static void launch_merge_seg(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
-                             const T *B, int64_t ldb, T beta, T *C, int64_t ldc, const int32_t *xs, const int32_t *ys,
-                             T *carry, int32_t *carry_row, hipStream_t s)
+static void launch_merge_seg(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
+                             const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                             const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, hipStream_t s)
 {
     constexpr int kFull = 16 / sizeof(T);
     if (tiling.vec == kFull)
-        launch_merge_width<T, kFull, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_merge_width<T, kFull, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
+                                         xs, ys, carry, carry_row, s);
     else if (tiling.vec == 2)
-        launch_merge_width<T, 2, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_merge_width<T, 2, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
+                                     xs, ys, carry, carry_row, s);
     else
-        launch_merge_width<T, 1, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_merge_width<T, 1, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
+                                     xs, ys, carry, carry_row, s);
 }
 
 template <typename T>
