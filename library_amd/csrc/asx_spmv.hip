@@ -56,6 +56,28 @@ inline bool use_nontemporal(int64_t nnz, size_t sv)
     return nnz * (int64_t)(sv + 4) > kNonTemporalAboveBytes;
 }
 
+// A workgroup's gathers start when all its stored elements have arrived.  A compute unit's L1 returns what it was asked for in
+// order: gathers that an L2 could serve wait behind every stored element still on its way from memory, so the fewer times
+// the two meet the better (gathers of 64-byte rows from an L2 beside a stream from memory: 175 G/s wave by wave, 217 behind
+// barriers, 259 without the stream).  8.4 M elements within 50000 of the diagonal, fp64, stream kernel: 58.3 us without the
+// barrier, 50.9 with it; 12 M scattered ones 72.1 and 59.6 (x of 1.8 MB), 95.7 and 93.9 (x of 6 MB).  Up to
+// one round of workgroups (eight on each of 256 compute units) all of them load and then gather anyway, and the
+// barrier costs 0.1 us.
+constexpr unsigned kBunchedTiles = 2048;
+template <int N, typename T>
+__device__ __forceinline__ void wait_for_elements(const int32_t (&c)[N], const T (&v)[N])
+{
+    if (gridDim.x <= kBunchedTiles) return;  // uniform
+#pragma unroll
+    for (int i = 0; i < N; ++i) asm volatile("" ::"v"(c[i]), "v"(v[i]));  // a use: the loads have to be back
+    __syncthreads();
+}
+
+// Entry i of count > 0; those behind the last one repeat it.  Loads of lanes past the end are clamped and not branched around:
+// behind a branch each gather is waited for before the next is issued (7.5 M elements of a stencil, fp64, stream kernel 26.2 ->
+// 21.9 us; 30 per row within 1000 of the diagonal 23.8 -> 18.7, flat 27.1 -> 22.3, merge 30.2 -> 21.4).
+__device__ __forceinline__ int32_t clamped(int32_t i, int32_t count) { return i < count ? i : count - 1; }
+
 template <typename T>
 __device__ __forceinline__ T axpby_out(T alpha, T sum, T beta, const T *y, int64_t r)
 {
@@ -290,16 +312,12 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream(int32_t m, int32_t nbloc
     // ---- issue every load of the block up front: stored elements, row pointers, y ----
     constexpr int IPT = kStreamTile / kBlock;
     int32_t cj[IPT];
-    T vj[IPT];
+    T vj[IPT], xj[IPT];
+    if (n1 > 0) {  // uniform
 #pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int j = tid + i * kBlock;
-        cj[i] = j < n1 ? stream_load<NT>(col + (int64_t)a + j) : 0;
-    }
+        for (int i = 0; i < IPT; ++i) cj[i] = stream_load<NT>(col + (int64_t)a + clamped(tid + i * kBlock, n1));
 #pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int j = tid + i * kBlock;
-        vj[i] = j < n1 ? stream_load<NT>(val + (int64_t)a + j) : T(0);
+        for (int i = 0; i < IPT; ++i) vj[i] = stream_load<NT>(val + (int64_t)a + clamped(tid + i * kBlock, n1));
     }
     constexpr int RPI = (kStreamRowCap + 1 + kBlock - 1) / kBlock;
     const int32_t rp_n = nrows < kStreamRowCap ? nrows : kStreamRowCap;  // pointers 0..rp_n
@@ -317,10 +335,12 @@ __global__ __launch_bounds__(kBlock) void k_spmv_stream(int32_t m, int32_t nbloc
     const bool y_first_ok = beta != T(0) && my_g < nrows && (tid & ((1 << g_shift) - 1)) == 0;
     const T y_first = y_first_ok ? y[(int64_t)r0 + my_g] : T(0);
 
+    if (n1 > 0) {
+        wait_for_elements(cj, vj);
 #pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int j = tid + i * kBlock;
-        if (j < n1) s_prod[pad32(j)] = vj[i] * x[cj[i]];
+        for (int i = 0; i < IPT; ++i) xj[i] = x[cj[i]];
+#pragma unroll
+        for (int i = 0; i < IPT; ++i) s_prod[pad32(clamped(tid + i * kBlock, n1))] = vj[i] * xj[i];
     }
 #pragma unroll
     for (int i = 0; i < RPI; ++i) {
@@ -440,20 +460,27 @@ __global__ __launch_bounds__(kBlock) void k_spmv_merge(int32_t m, int32_t nnz, i
     // ---- stage: stored elements first (the long-latency part), then row ends ----
     int32_t cj[IPT];
     T vj[IPT];
+    if (nz > 0) {  // uniform
 #pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int j = tid + i * kBlock;
-        cj[i] = j < nz ? stream_load<NT>(col + (int64_t)y0 + j) : 0;
-        vj[i] = j < nz ? stream_load<NT>(val + (int64_t)y0 + j) : T(0);
+        for (int i = 0; i < IPT; ++i) {
+            const int64_t at = (int64_t)y0 + clamped(tid + i * kBlock, nz);
+            cj[i] = stream_load<NT>(col + at);
+            vj[i] = stream_load<NT>(val + at);
+        }
+    }
+    T xj[IPT];
+    if (nz > 0) {
+        wait_for_elements(cj, vj);
+#pragma unroll
+        for (int i = 0; i < IPT; ++i) xj[i] = x[cj[i]];
     }
     for (int i = tid; i <= nr; i += kBlock) {
         const int32_t r = x0 + i;
         s_rend[i] = (r < m ? row_ptr[r + 1] : nnz) - y0;
     }
+    if (nz > 0) {
 #pragma unroll
-    for (int i = 0; i < IPT; ++i) {
-        const int j = tid + i * kBlock;
-        if (j < nz) s_val[j] = vj[i] * x[cj[i]];
+        for (int i = 0; i < IPT; ++i) s_val[clamped(tid + i * kBlock, nz)] = vj[i] * xj[i];
     }
     __syncthreads();
 
@@ -741,6 +768,11 @@ __device__ __forceinline__ void flat_tile(FlatShared<T> &sh, int t, int32_t m, i
     const int32_t nwritten = re - rs;                   // rows that end inside this tile
     const int32_t rcount = nwritten + (re < m ? 1 : 0);  // plus the one left open
     const bool fits = rcount <= kFlatRowCap + 1;  // 1024 one-element rows plus the open row still fit
+    T g[4];
+    if (n1 > 0) {  // uniform; all gathers at once, ahead of the row ends (past the last element c is 0)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) g[j] = x[c[j]];
+    }
     int has_long = 0;
     if (fits) {
         for (int i = tid; i < rcount; i += kBlock) {
@@ -750,9 +782,10 @@ __device__ __forceinline__ void flat_tile(FlatShared<T> &sh, int t, int32_t m, i
             has_long |= (hi - lo) > kFlatRowModeMaxLen;
         }
     }
+    if (n1 > 0) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j)
-        if (k0 + j < n1) p[j] *= x[c[j]];
+        for (int j = 0; j < 4; ++j) p[j] *= g[j];
+    }
 #pragma unroll
     for (int j = 0; j < 4; ++j) s_prod[k0 + j + ((k0 + j) >> 5)] = k0 + j < n1 ? p[j] : T(0);
     const bool walk = fits && __syncthreads_or(has_long);  // also the barrier after staging
@@ -896,6 +929,7 @@ __global__ __launch_bounds__(kBlock) void k_spmv_flat(int32_t m, int32_t nnz, in
         rs = t == 0 ? 0 : seg_row[t];
         re = seg_row[t + 1];
     }
+    wait_for_elements(c, p);
     flat_tile<T, NT>(sh, t, m, nnz, alpha, row_ptr, c, p, x, beta, y, rs, re, carry);
 }
 
