@@ -267,7 +267,7 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
             xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
         const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
-        return launch_spmm_merge<T>(m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
+        return launch_spmm_merge<T>(plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T)), m, k, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
                                     (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off), plan ? plan->carry_pass != 0 : true,
                                     spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
     }
@@ -491,7 +491,9 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv).bytes;
         // B's rows one after the other, from the start of a line on, as nearly every caller has them
         const int tile_bytes = spmm_tile_bytes(p->columns, p->n, nullptr, (size_t)p->ncols * sv);
-        p->items = spmm_plan_items(usual, p->columns, spmm_tiling(p->ncols, tile_bytes, sv).groups, m, nnz, p->stats[0]);
+        p->chunked = spmm_plan_chunked(m, nnz, p->ncols, sv, p->stats[0]);
+        p->items = spmm_plan_items(usual, p->columns, spmm_tiling(p->ncols, tile_bytes, sv).groups, m, nnz, p->stats[0],
+                                   p->chunked != 0);
         for (;; p->items = usual) {
             const size_t ns = (size_t)spmm_segments(m, nnz, p->items);
             p->nunits = (int32_t)ns;
@@ -504,6 +506,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             if (st || p->items == usual || !p->carry_pass) return st;
             pool_free(p->d_meta, true);  // read_flag has waited; the flag stays set, so that the carry pass runs
             p->d_meta = nullptr;
+            p->chunked = spmm_chunked(m, nnz, p->ncols, sv);
         }
     }
     if (!st) st = status_of(hipStreamSynchronize(s));

@@ -21,6 +21,32 @@ constexpr int kFlatTile = 1024;                            // stored elements pe
 constexpr int kLongRow = 8192;
 // SpMM: merge items (rows + stored elements) per wave
 constexpr int kSpmmSegmentSmall = 128, kSpmmSegmentMedium = 256, kSpmmSegmentLarge = 512;
+// SpMM chunk kernel: threads of a workgroup, what it can stage, and merge items per segment - where rows may be cut (a segment
+// then holds up to twice as many elements) and where none is longer than kChunkLongest.
+constexpr int kChunkThreads = 512, kChunkElems = 2880, kChunkRows = 2689;
+constexpr int kChunkItems = 1344, kChunkItemsMost = 2688, kChunkLongest = kChunkElems - kChunkItemsMost;
+static_assert(2 * kChunkItems <= kChunkElems && kChunkItemsMost < kChunkRows, "a segment fits what is staged");
+// Which calls it takes.  Rows of B of up to 32 bytes, planned or not, unless rows of A are short: 66 such cases of all families 9 %
+// faster on average (3 columns fp64, 56 per row 16.7 -> 7.4 us; 2 columns fp32, 5 per row 21.0 -> 16.0), but with 4 per row,
+// 2 columns fp32 8.2 -> 10.1, with 7, 3 columns fp64 4.7 -> 5.1.  Rows of B of 33 to 64 bytes only where a plan knows that no
+// row of A is long and there are several rounds of workgroups (16 columns fp32, 23 per row, 8 M elements 60.9 -> 52.2 us; 9 per
+// row, 5 M 50.5 and 50.5; but 14 columns, 27 per row, 2.2 M 23.3 -> 24.3; rows of up to 1510 57.4 -> 73.5).  Wider ones gain
+// and lose alike (18 columns fp32 27.3 -> 29.6, 12 columns fp64 86.8 -> 83.0).
+inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
+{
+    return ncols * (int64_t)sv <= 32 && 2 * (int64_t)nnz >= (sv == 4 ? 9 : 16) * (int64_t)m;
+}
+inline bool spmm_plan_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv, int64_t longest)
+{
+    return spmm_chunked(m, nnz, ncols, sv) || (ncols * (int64_t)sv <= 64 && longest <= kChunkLongest && (int64_t)m + nnz >= 4000000);
+}
+// One round of three workgroups on each of 256 compute units, if its segments are neither short (448 to 896 items are alike up
+// to 500000 items; at 1 M 896 take 20 % longer than 1344) nor more than a workgroup can stage.
+inline int32_t spmm_chunk_items(int64_t items, int32_t most = kChunkItems)
+{
+    const int64_t round = ceil_div64(items, 768);
+    return (int32_t)(round < kChunkItems / 2 ? kChunkItems / 2 : round > most ? most : round);
+}
 constexpr double kScatteredMinSpread = 0.5;  // of a column sample: from here on the columns count as scattered
 
 inline int status_of(hipError_t e)
@@ -105,7 +131,7 @@ template <typename T>
 int launch_spmm_row(int32_t m, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col,
                     const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s);
 template <typename T>
-int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
+int launch_spmm_merge(bool chunked, int32_t m, int32_t k, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
                       bool carry_pass, int tile_bytes, hipStream_t s);
@@ -289,6 +315,7 @@ inline int spmm_columns(double spread, double span, double mean, size_t sv)
 inline int32_t spmm_segment_items(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
 {
     const int64_t items = (int64_t)m + nnz;
+    if (spmm_chunked(m, nnz, ncols, sv)) return spmm_chunk_items(items);
     if (items < (int64_t)kSpmmSegmentMedium * 4096) return kSpmmSegmentSmall;
     return sv == 4 && ncols > 32 && items >= (int64_t)kSpmmSegmentLarge * 4096 ? kSpmmSegmentLarge : kSpmmSegmentMedium;
 }
@@ -319,8 +346,17 @@ constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 
 // of one length (the longest at most a quarter above the mean) they hold as many as the wave's groups take in full turns.
 // 64 columns fp32, 20 per row within 1000 of the diagonal: 94.9 us with segments of 512 items, 54.2 with two turns of 84;
 // 7-point stencil 78.7 -> 59.7, 5-point stencil 128.7 -> 85.7; 13 per row 50.2 -> 42.3.
-inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest)
+// Chunk kernel: where rows are too long for the longest segments, but none for one of the usual length, no row is cut (a carry
+// pass is a launch more: longest row 913 of 82000 elements 8.8 -> 5.9 us); even rows fill its groups' last turn.
+inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest, bool chunked)
 {
+    if (chunked) {
+        if (longest > kChunkLongest) return longest > kChunkItems || longest <= usual ? usual : (int32_t)longest;  // usual <= kChunkItems
+        const int32_t items = spmm_chunk_items((int64_t)m + nnz, kChunkItemsMost);
+        const int64_t turn = (int64_t)groups * (kChunkThreads / kWave) * (longest + 1);
+        const int64_t turns = ceil_div64(items, turn) * turn;  // all groups of a workgroup at work to the end
+        return turns > kChunkItemsMost || 4 * (longest + 1) * m > 5 * ((int64_t)m + nnz) ? items : (int32_t)turns;
+    }
     if (columns != kColumnsNear && columns != kColumnsSpread) return usual;
     const int32_t least = usual == kSpmmSegmentLarge ? kSpmmSegmentSmall : usual;
     const int64_t turn = groups * (longest + 1);
@@ -352,7 +388,8 @@ struct asx_plan {
     int carry_pass;  // flat and SpMM merge kernel: 0 when no row is cut between units of work
     int32_t nwide, nlong, long_len;  // vector kernel: d_meta lists the long rows (asx::LongRows)
     int columns;     // SpMM merge kernel: kColumns*
-    int32_t items;   // SpMM merge kernel: merge items per segment
+    int32_t items;   // SpMM merge and chunk kernels: merge items per segment
+    int chunked;     // SpMM: the chunk kernel
     int64_t hist[33];
     int64_t stats[4];
     size_t workspace_bytes;

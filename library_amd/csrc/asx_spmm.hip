@@ -2,7 +2,7 @@
 //
 // Every access to a row of B or C covers consecutive columns: 64 lanes of one element in the row kernel, whose stored elements
 // are read 64 at a time and broadcast through v_readlane (the address of the row of B is then wave-uniform), 16 bytes a lane
-// in the merge kernel, whose lane groups work on different rows of A.
+// in the merge and chunk kernels, whose lane groups work on different rows of A.
 //
 //   row   : one wave per (row, column tile).  Simple; long rows serialise.
 //   merge : one wave per segment of consecutive items of the merge path over
@@ -12,6 +12,7 @@
 //           a segment end is kept as a carry row and added by an ordered pass afterwards.  No atomics (the reference's default SpMM,
 //           hip/kernel/level3/alphasparse_spmm_csr_nnz_split.h:283-409, scales C in a
 //           separate pass and joins segments with atomicAdd).
+//   chunk : the same with a workgroup per (longer) segment, for rows of B of up to 64 bytes.
 #include <algorithm>
 
 #include "asx_internal.hpp"
@@ -224,11 +225,11 @@ struct Int {
     static constexpr int value = N;
 };
 
-// Sum over staged elements i0, i0 + ST, ... below e: a * B[col, lane's columns].  Bc: B plus the lane's
-// first column.  Batches of U, then at most one of U / 2, then one of U / 2 that is not full.
-template <typename T, int VEC, int ST, int U, bool UNIFORM>
-__device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, int32_t e, const int32_t *s_col,
-                                                                    const T *s_val, const char *Bc, uint64_t ldb_bytes)
+// Sum over staged elements i0, i0 + ST, ... below e: a * (the lane's columns of the row of B that row_of_b fetches for what is
+// staged of the element's column).  Batches of U, then at most one of U / 2, then one of U / 2 that is not full.
+template <typename T, int VEC, int ST, int U, typename F>
+__device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, int32_t e, const int32_t *s_col, const T *s_val,
+                                                                    const F &row_of_b)
 {
     typedef typename VecOf<T, VEC>::type V;
     V acc = T(0);
@@ -241,9 +242,7 @@ __device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, 
 #pragma unroll
         for (int u = 0; u < N; ++u) {
             const int32_t iu = !PARTIAL || i + u * ST < e ? i + u * ST : i;
-            uint32_t c = (uint32_t)s_col[iu];
-            if (UNIFORM) c = (uint32_t)__builtin_amdgcn_readfirstlane((int)c);
-            b[u] = *(const V *)(Bc + c * ldb_bytes);
+            b[u] = row_of_b(s_col[iu]);
             a[u] = s_val[iu];
         }
 #pragma unroll
@@ -352,8 +351,12 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
+    const auto row_of_b = [&](int32_t column) -> V {
+        const uint32_t at = (uint32_t)(NG == 1 ? __builtin_amdgcn_readfirstlane(column) : column);
+        return *(const V *)(Bc + at * ldb_bytes);
+    };
     const auto together = [&](int32_t k, int32_t e) {  // the row's sum over all groups, in every group
-        V acc = spmm_staged<T, VEC, NG, U, NG == 1>(k + grp, e, s_col, s_val, Bc, ldb_bytes);
+        V acc = spmm_staged<T, VEC, NG, U>(k + grp, e, s_col, s_val, row_of_b);
 #pragma unroll
         for (int d = G; d < kWave; d <<= 1)
 #pragma unroll
@@ -369,7 +372,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
             V *out = (V *)(C + (int64_t)(x0 + r) * ldc + c);
             V c_old = T(0);
             if (beta != T(0)) c_old = *out;  // requested before the row's loads of B
-            const V acc = spmm_staged<T, VEC, 1, U, NG == 1>(k, e, s_col, s_val, Bc, ldb_bytes);
+            const V acc = spmm_staged<T, VEC, 1, U>(k, e, s_col, s_val, row_of_b);
             const V y = beta == T(0) ? (V)(alpha * acc) : __builtin_elementwise_fma((V)alpha, acc, (V)(beta * c_old));
             if (active) *out = y;
         }
@@ -397,6 +400,154 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
         if (stores) *(V *)(carry + seg * ncols + c) = acc;
     }
     if (carry_row && lane == 0 && blockIdx.y == 0) carry_row[seg] = has_tail ? x1 : -1;
+}
+
+// ===========================================================================================
+// chunk: one workgroup per segment, for narrow rows of B
+// ===========================================================================================
+// Where a row of B takes four lanes or fewer, rows of B that the L2s could serve wait for stored elements of A on their way from
+// memory: a compute unit's L1 answers in order (64-byte rows from an L2 beside a stream from memory 175 G/s wave by wave,
+// 217 behind barriers, 259 alone).  So a workgroup of 512 stages one long segment, all of it requested at once, and no wave
+// fetches a row of B before the barrier: three workgroups a compute unit that each meet memory once a segment, where the
+// merge kernel's twenty waves meet it every 256 items.  Longer segments also give narrow rows enough rows of A to deal out.  Eight
+// rows of B in flight a group (four, and the four workgroups that then fit: 103.5 us where eight take 91.9).  Merge kernel and
+// this one, three matrices in turn: 8 columns fp64, 20 per row within 3000 of the diagonal 65.4 -> 56.5 us, 2 columns
+// 54.1 -> 39.8; 16 columns fp32, 50 per row within 20000 122 -> 91.9; 4 columns fp32, 8 per row within 300 29.3 -> 20.2; band of
+// 11, 2 columns fp64 24.3 -> 16.7.
+//
+// NARROW: B spans at most 4 GB, and what is staged is the byte offset of its row: a 32-bit add per row of B and lane instead of
+// a 64-bit multiplication.
+template <typename T, int VEC, int LOGG, bool NARROW>
+__global__ __launch_bounds__(kChunkThreads, NARROW ? 6 : 4) void k_spmm_chunk(
+    int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
+    const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ B, int64_t ldb, T beta, T *__restrict__ C, int64_t ldc,
+    const int32_t *__restrict__ xs, const int32_t *__restrict__ ys, T *__restrict__ carry, int32_t *__restrict__ carry_row)
+{
+    typedef typename VecOf<T, VEC>::type V;
+    constexpr int G = 1 << LOGG, NG = kWave / G;
+    constexpr int U = 8;  // rows of B a lane has in flight
+    constexpr int kDealt = spmm_dealt(NG);
+    constexpr int kWide = 256;  // longer rows are taken by all waves (elements)
+    constexpr int kWaves = kChunkThreads / kWave, NE = (kChunkElems + kChunkThreads - 1) / kChunkThreads;
+    __shared__ int32_t s_col[kChunkElems];
+    __shared__ T s_val[kChunkElems];
+    __shared__ uint16_t s_end[kChunkRows + 1];  // s_end[r + 1]: end of row x0 + r, relative to y0
+    __shared__ int32_t s_cut[4], s_wide[kChunkElems / kWide], s_nwide;
+    __shared__ V s_part[kWaves][G];
+    const int tid = threadIdx.x, lane = tid & (kWave - 1);
+    const int w = __builtin_amdgcn_readfirstlane(tid / kWave);
+    const uint32_t per_xcd = gridDim.x / kXcds;  // consecutive segments on one XCD, as in the merge kernel
+    const int64_t seg = (int64_t)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
+    if (seg >= nseg) return;  // the whole workgroup leaves
+    const int grp = lane >> LOGG, gl = lane & (G - 1);
+    const bool active = gl * VEC < ncols;
+    const int32_t c = gl * VEC < ncols - VEC ? gl * VEC : ncols - VEC;  // as in the merge kernel
+    const uint64_t ldb_bytes = (uint64_t)ldb * sizeof(T);
+    int32_t x0, y0, x1, y1;
+    if (xs) {  // uniform
+        x0 = xs[seg], y0 = ys[seg], x1 = xs[seg + 1], y1 = ys[seg + 1];
+    } else {
+        if (w == 0) {
+            segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1);
+            if (lane == 0) s_cut[0] = x0, s_cut[1] = y0, s_cut[2] = x1, s_cut[3] = y1;
+        }
+        __syncthreads();
+        x0 = s_cut[0], y0 = s_cut[1], x1 = s_cut[2], y1 = s_cut[3];
+    }
+    x0 = __builtin_amdgcn_readfirstlane(x0), y0 = __builtin_amdgcn_readfirstlane(y0);
+    const int32_t nel = __builtin_amdgcn_readfirstlane(y1 - y0 < kChunkElems ? y1 - y0 : kChunkElems);
+    const int32_t nrow = __builtin_amdgcn_readfirstlane(x1 - x0 < kChunkRows ? x1 - x0 : kChunkRows);
+    {
+        int32_t tc[NE];
+        T tv[NE];
+#pragma unroll
+        for (int j = 0; j < NE; ++j)
+            if (j * kChunkThreads < nel) {  // uniform; lanes past the end repeat the last element
+                const int i = j * kChunkThreads + tid;
+                const int64_t k = (int64_t)y0 + (i < nel ? i : nel - 1);
+                tc[j] = col[k];
+                tv[j] = val[k];
+            }
+        if (tid == 0) s_end[0] = 0, s_nwide = 0;
+        for (int i = tid; i < nrow; i += kChunkThreads) s_end[i + 1] = (uint16_t)(row_ptr[x0 + i + 1] - y0);
+#pragma unroll
+        for (int j = 0; j < NE; ++j)
+            if (j * kChunkThreads < nel) {
+                const int i = j * kChunkThreads + tid;
+                if (i < kChunkElems) {
+                    s_col[i] = NARROW ? (int32_t)((uint32_t)tc[j] * (uint32_t)ldb_bytes) : tc[j];
+                    s_val[i] = tv[j];
+                }
+            }
+    }
+    __syncthreads();
+
+    const uint32_t c_bytes = (uint32_t)c * (uint32_t)sizeof(T);
+    const auto row_of_b = [&](int32_t staged) -> V {
+        return *(const V *)((const char *)B + (NARROW ? (uint64_t)((uint32_t)staged + c_bytes) : (uint32_t)staged * ldb_bytes + c_bytes));
+    };
+    const auto together = [&](int32_t k, int32_t e) {  // the sum over the wave's groups, in every group
+        V acc = spmm_staged<T, VEC, NG, U / 2>(k + grp, e, s_col, s_val, row_of_b);
+#pragma unroll
+        for (int d = G; d < kWave; d <<= 1)
+#pragma unroll
+            for (int v = 0; v < VEC; ++v) acc[v] += __shfl_xor(acc[v], d, kWave);
+        return acc;
+    };
+    const bool stores = active && grp == 0;
+    for (int32_t r0 = w * NG; r0 < nrow; r0 += kWaves * NG) {
+        const int32_t r = r0 + grp;
+        const int32_t k = r < nrow ? s_end[r] : 0, e = r < nrow ? s_end[r + 1] : 0;
+        const bool dealt = e - k <= kDealt;
+        if (r < nrow && dealt) {
+            V *out = (V *)(C + (int64_t)(x0 + r) * ldc + c);
+            V c_old = T(0);
+            if (beta != T(0)) c_old = *out;  // requested before the row's loads of B
+            const V acc = spmm_staged<T, VEC, 1, U>(k, e, s_col, s_val, row_of_b);
+            const V y = beta == T(0) ? (V)(alpha * acc) : __builtin_elementwise_fma((V)alpha, acc, (V)(beta * c_old));
+            if (active) *out = y;
+        }
+        if (e - k > kWide && gl == 0) s_wide[atomicAdd(&s_nwide, 1)] = r;  // in any order: each is a sum of its own
+        unsigned long long todo = __ballot(!dealt && e - k <= kWide && gl == 0);
+        while (todo) {  // wave-uniform
+            const int src = __builtin_ctzll(todo);
+            todo &= todo - 1;
+            const int32_t rr = r0 + (src >> LOGG);
+            const int32_t kk = __builtin_amdgcn_readlane(k, src), ee = __builtin_amdgcn_readlane(e, src);
+            V *out = (V *)(C + (int64_t)(x0 + rr) * ldc + c);
+            V c_old = T(0);
+            if (beta != T(0) && stores) c_old = *out;
+            const V acc = together(kk, ee);
+            const V y = beta == T(0) ? (V)(alpha * acc) : __builtin_elementwise_fma((V)alpha, acc, (V)(beta * c_old));
+            if (stores) *out = y;
+        }
+    }
+    __syncthreads();
+    // Rows wider than kWide, and what the segment holds of a row that goes on past its end: a stretch a wave, added up in the
+    // order of the waves.
+    const int32_t last = s_end[nrow], nwide = s_nwide;
+    const bool tail = carry_row && nel > last;
+    for (int32_t i = 0; i < nwide + (tail ? 1 : 0); ++i) {  // uniform
+        const int32_t r = i < nwide ? s_wide[i] : nrow;
+        const int32_t from = s_end[r], to = i < nwide ? s_end[r + 1] : nel, share = (to - from + kWaves - 1) / kWaves;
+        const int32_t k = from + w * share, e = k + share < to ? k + share : to;
+        const V acc = together(k, e);
+        if (grp == 0) s_part[w][gl] = acc;
+        __syncthreads();
+        if (w == 0 && stores) {
+            V sum = s_part[0][gl];
+#pragma unroll
+            for (int q = 1; q < kWaves; ++q) sum += s_part[q][gl];
+            if (i < nwide) {
+                V *out = (V *)(C + (int64_t)(x0 + r) * ldc + c);
+                *out = beta == T(0) ? (V)(alpha * sum) : __builtin_elementwise_fma((V)alpha, sum, (V)(beta * *out));
+            } else {
+                *(V *)(carry + seg * ncols + c) = sum;
+            }
+        }
+        __syncthreads();
+    }
+    if (carry_row && tid == 0) carry_row[seg] = tail ? x1 : -1;
 }
 
 // Every wave looks at kFixupSegs consecutive segments (one lane each) for the first segment of a run
@@ -507,8 +658,44 @@ static void launch_merge_seg(const SpmmTiling &tiling, int32_t m, int32_t nnz, i
                                      xs, ys, carry, carry_row, s);
 }
 
+// As many lanes a group as span the columns.
 template <typename T>
-int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
+static void launch_chunk(const SpmmTiling &tiling, int32_t m, int32_t k, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
+                         const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                         const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, hipStream_t s)
+{
+    constexpr int kFull = 16 / sizeof(T);
+    const bool narrow = (uint64_t)k * (uint64_t)ldb <= 0xffffffffull / sizeof(T);
+    const auto launch = [&](auto vec_, auto log_) {
+        const auto with = [&](auto narrow_) {
+            hipLaunchKernelGGL((k_spmm_chunk<T, decltype(vec_)::value, decltype(log_)::value, decltype(narrow_)::value != 0>),
+                               dim3((unsigned)(ceil_div64(nseg, kXcds) * kXcds)), dim3(kChunkThreads), 0, s, m, nnz, items, nseg, ncols, alpha,
+                               row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);
+        };
+        if (narrow)
+            with(Int<1>{});
+        else
+            with(Int<0>{});
+    };
+    if (tiling.vec == kFull) {
+        if (tiling.log_lanes == 0)
+            launch(Int<kFull>{}, Int<0>{});
+        else if (tiling.log_lanes == 1)
+            launch(Int<kFull>{}, Int<1>{});
+        else
+            launch(Int<kFull>{}, Int<2>{});
+    } else if (tiling.vec == 1) {
+        launch(Int<1>{}, Int<0>{});
+    } else if constexpr (kFull > 2) {  // two or three columns of fp32
+        if (tiling.log_lanes == 0)
+            launch(Int<2>{}, Int<0>{});
+        else
+            launch(Int<2>{}, Int<1>{});
+    }
+}
+
+template <typename T>
+int launch_spmm_merge(bool chunked, int32_t m, int32_t k, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
                       bool carry_pass, int tile_bytes, hipStream_t s)
@@ -519,7 +706,7 @@ int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T al
     const int64_t slab = (int64_t)65535 * (tile_bytes / (int64_t)sizeof(T));
     if (ncols > slab) {
         for (int64_t c = 0; c < ncols; c += slab) {
-            const int st = launch_spmm_merge<T>(m, nnz, items, (int32_t)(ncols - c < slab ? ncols - c : slab), alpha, row_ptr, col, val, B + c,
+            const int st = launch_spmm_merge<T>(chunked, m, k, nnz, items, (int32_t)(ncols - c < slab ? ncols - c : slab), alpha, row_ptr, col, val, B + c,
                                                 ldb, beta, C + c, ldc, xs, ys, carry, carry_row, carry_pass, tile_bytes, s);
             if (st) return st;
         }
@@ -528,16 +715,20 @@ int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T al
     const int32_t nseg = spmm_segments(m, nnz, items);
     const SpmmTiling tiling = spmm_tiling(ncols, tile_bytes, sizeof(T));
     if (!carry_pass) carry = nullptr, carry_row = nullptr;  // no row is cut: nothing is left for the pass
-    const auto launch = [&](auto seg_) {
-        launch_merge_seg<T, decltype(seg_)::value>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
-                                                   carry_row, s);
-    };
-    if (items <= kSpmmSegmentSmall)
-        launch(Int<kSpmmSegmentSmall>{});
-    else if (items <= kSpmmSegmentMedium)
-        launch(Int<kSpmmSegmentMedium>{});
-    else if constexpr (sizeof(T) == 4)
-        launch(Int<kSpmmSegmentLarge>{});
+    if (chunked) {
+        launch_chunk<T>(tiling, m, k, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+    } else {
+        const auto launch = [&](auto seg_) {
+            launch_merge_seg<T, decltype(seg_)::value>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
+                                                       carry_row, s);
+        };
+        if (items <= kSpmmSegmentSmall)
+            launch(Int<kSpmmSegmentSmall>{});
+        else if (items <= kSpmmSegmentMedium)
+            launch(Int<kSpmmSegmentMedium>{});
+        else if constexpr (sizeof(T) == 4)
+            launch(Int<kSpmmSegmentLarge>{});
+    }
     if (carry_pass)
         hipLaunchKernelGGL((k_spmm_merge_fixup<T>), dim3((unsigned)ceil_div64(ceil_div64(nseg, kFixupSegs), kBlock / kWave)),
                            dim3(kBlock), 0, s, m, nseg, ncols, alpha, carry, carry_row, C, ldc);
@@ -547,7 +738,7 @@ int launch_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t ncols, T al
 #define ASX_INST(T)                                                                                  \
     template int launch_spmm_row<T>(int32_t, int32_t, T, const int32_t *, const int32_t *, const T *, \
                                     const T *, int64_t, T, T *, int64_t, hipStream_t);               \
-    template int launch_spmm_merge<T>(int32_t, int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
+    template int launch_spmm_merge<T>(bool, int32_t, int32_t, int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
                                       const T *, const T *, int64_t, T, T *, int64_t, const int32_t *, \
                                       const int32_t *, T *, int32_t *, bool, int, hipStream_t);
 ASX_INST(float)

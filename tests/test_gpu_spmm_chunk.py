@@ -1,0 +1,64 @@
+"""The SpMM kernel for narrow rows of B, which stages a long segment a workgroup: every width it takes and the ones beside them,
+rows around what a lane group, a wave and a segment take, segments of one row and of empty rows only, sizes at which its segments
+are shortest, one round, longest and full turns, and a B that 32-bit offsets do not span.  Products of small integers, whose sums
+are exact in both types and in any order, against integer sums."""
+import numpy as np
+import pytest
+import torch
+
+from library_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(lens, k, ncols, dtype, planned, pad=0, beta=0.5):
+    rng = np.random.default_rng(len(lens) + ncols)
+    m, rp = len(lens), np.r_[0, np.cumsum(lens)].astype(np.int32)
+    ldb, ldc = ncols + pad, ncols + 2 * pad
+    col, val = rng.integers(0, k, rp[-1]).astype(np.int32), rng.integers(-3, 4, rp[-1]).astype(dtype)
+    B, C0 = rng.integers(-3, 4, (k, ldb)).astype(dtype), 2 * rng.integers(-3, 4, (m, ldc)).astype(dtype)
+    d = [torch.from_numpy(a).cuda() for a in (rp, col, val, B, C0)]
+    plan = capi.Plan(True, capi.SPMM_MERGE, val.dtype, m, k, col.size, d[0], ncols=ncols, col=d[1], val=d[2]) if planned else None
+    capi.spmm(*d, ncols, 2.0, beta, alg=capi.SPMM_MERGE, plan=plan, ldb=ldb, ldc=ldc, k=k)
+    # one column at a time: cumulative sums of integers, exact in float64
+    ref = C0.copy()
+    for c in range(ncols):
+        s = np.r_[0.0, np.cumsum(val.astype(np.float64) * B[col, c])]
+        ref[:, c] = 2.0 * (s[rp[1:]] - s[rp[:-1]]) + beta * C0[:, c]
+    assert np.array_equal(d[4].cpu().numpy(), ref), (ncols, planned, pad)
+    if plan is not None:
+        plan.destroy()
+
+
+@pytest.mark.parametrize("dtype", [np.float32, np.float64])
+@pytest.mark.parametrize("ncols", [1, 2, 3, 4, 5, 7, 8, 9, 16])
+@pytest.mark.parametrize("planned", [False, True])
+def test_rows_of_every_kind(dtype, ncols, planned):
+    rng = np.random.default_rng(1)
+    edges = [0, 1, 7, 8, 9, 63, 64, 65, 255, 256, 257, 511, 671, 672, 673, 1343, 1344, 1345, 2687, 2688, 2689, 6001]
+    lens = np.r_[rng.integers(0, 30, 700), np.repeat(edges, 2), np.zeros(4000, int), rng.permutation(edges), 3000, 1]
+    _check(lens, 500, ncols, dtype, planned, pad=3, beta=0.0)
+    _check(rng.integers(5, 40, 900), 333, ncols, dtype, planned)
+
+
+@pytest.mark.parametrize("dtype,ncols", [(np.float32, 2), (np.float32, 16), (np.float64, 2), (np.float64, 8)])
+@pytest.mark.parametrize("m,per,ragged", [(1, 9, 0), (300, 20, 0), (40000, 20, 5), (61000, 20, 0), (205000, 20, 0), (200000, 20, 9), (21000, 192, 0),
+                                          (3000, 1344, 0), (1500, 1440, 0), (600, 2000, 700)])
+def test_segment_sizes(dtype, ncols, m, per, ragged):
+    lens = np.full(m, per) + (np.random.default_rng(m).integers(-ragged, ragged + 1, m) if ragged else 0)
+    for planned in (False, True):
+        _check(lens, 4000, ncols, dtype, planned)
+
+
+def test_wide_b():
+    k, ldb, m = 9, 1 << 27, 3000  # 4.8 GB of B
+    gen = torch.Generator(device="cuda").manual_seed(5)
+    B = torch.zeros((k, ldb), device="cuda")
+    B[:, :8] = torch.randint(-3, 4, (k, 8), device="cuda", generator=gen).float()
+    rp = (torch.arange(m + 1, device="cuda") * 12).to(torch.int32)
+    col = torch.randint(0, k, (m * 12,), device="cuda", generator=gen, dtype=torch.int32)
+    val = torch.randint(-3, 4, (m * 12,), device="cuda", generator=gen).float()
+    C = torch.zeros((m, 8), device="cuda")
+    capi.spmm(rp, col, val, B, C, 8, 1.0, 0.0, ldb=ldb, ldc=8, k=k)
+    ref = (val[:, None] * B[:, :8][col.long()]).reshape(m, 12, 8).sum(1)
+    assert torch.equal(C, ref)
