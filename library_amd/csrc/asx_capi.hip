@@ -491,9 +491,9 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv).bytes;
         // B's rows one after the other, from the start of a line on, as nearly every caller has them
         const int tile_bytes = spmm_tile_bytes(p->columns, p->n, nullptr, (size_t)p->ncols * sv);
-        p->chunked = spmm_plan_chunked(m, nnz, p->ncols, sv, p->stats[0]);
-        p->items = spmm_plan_items(usual, p->columns, spmm_tiling(p->ncols, tile_bytes, sv).groups, m, nnz, p->stats[0],
-                                   p->chunked != 0);
+        const int groups = spmm_tiling(p->ncols, tile_bytes, sv).groups;
+        p->chunked = spmm_plan_chunked(m, nnz, p->ncols, sv, p->stats[0], p->columns == kColumnsScattered, kWave / groups);
+        p->items = spmm_plan_items(usual, p->columns, groups, m, nnz, p->stats[0], p->chunked != 0, p->ncols * (int64_t)sv);
         for (;; p->items = usual) {
             const size_t ns = (size_t)spmm_segments(m, nnz, p->items);
             p->nunits = (int32_t)ns;
@@ -503,7 +503,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             // does any row stay cut?  (one int read back; creation syncs anyway)
             if (!st) st = launch_spmm_splits(m, nnz, p->items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
             if (!st) st = read_flag();
-            if (st || p->items == usual || !p->carry_pass) return st;
+            if (st || p->items >= usual || !p->carry_pass) return st;
             pool_free(p->d_meta, true);  // read_flag has waited; the flag stays set, so that the carry pass runs
             p->d_meta = nullptr;
             p->chunked = spmm_chunked(m, nnz, p->ncols, sv);

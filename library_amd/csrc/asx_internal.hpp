@@ -1,5 +1,6 @@
 // Internal declarations shared by the HIP translation units of libalphasparse_amd.so.
 #pragma once
+#include <algorithm>
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
@@ -25,26 +26,57 @@ constexpr int kSpmmSegmentSmall = 128, kSpmmSegmentMedium = 256, kSpmmSegmentLar
 // then holds up to twice as many elements) and where none is longer than kChunkLongest.
 constexpr int kChunkThreads = 512, kChunkElems = 2880, kChunkRows = 2689;
 constexpr int kChunkItems = 1344, kChunkItemsMost = 2688, kChunkLongest = kChunkElems - kChunkItemsMost;
+constexpr int kChunkItemsWide = 640;      // the most where rows of B are wide
+constexpr int64_t kChunkRound = 768;      // three workgroups on each of 256 compute units
 static_assert(2 * kChunkItems <= kChunkElems && kChunkItemsMost < kChunkRows, "a segment fits what is staged");
 // Which calls it takes.  Rows of B of up to 32 bytes, planned or not, unless rows of A are short: 66 such cases of all families 9 %
 // faster on average (3 columns fp64, 56 per row 16.7 -> 7.4 us; 2 columns fp32, 5 per row 21.0 -> 16.0), but with 4 per row,
 // 2 columns fp32 8.2 -> 10.1, with 7, 3 columns fp64 4.7 -> 5.1.  Rows of B of 33 to 64 bytes only where a plan knows that no
 // row of A is long and there are several rounds of workgroups (16 columns fp32, 23 per row, 8 M elements 60.9 -> 52.2 us; 9 per
-// row, 5 M 50.5 and 50.5; but 14 columns, 27 per row, 2.2 M 23.3 -> 24.3; rows of up to 1510 57.4 -> 73.5).  Wider ones gain
-// and lose alike (18 columns fp32 27.3 -> 29.6, 12 columns fp64 86.8 -> 83.0).
-inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
+// row, 5 M 50.5 and 50.5; but 14 columns, 27 per row, 2.2 M 23.3 -> 24.3; rows of up to 1510 57.4 -> 73.5).  Rows of 65 to 128
+// bytes gain and lose alike (18 columns fp32 27.3 -> 29.6, 12 columns fp64 86.8 -> 83.0).
+inline bool spmm_chunked_narrow(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
     return ncols * (int64_t)sv <= 32 && 2 * (int64_t)nnz >= (sv == 4 ? 9 : 16) * (int64_t)m;
 }
-inline bool spmm_plan_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv, int64_t longest)
+// Wider rows of B while one round of workgroups takes all of A: the merge kernel's few waves then walk 128 items each, one or two
+// rows of A at a time, where eight waves share them here.  40 such cases of all families, planned or not, take 0.7 of their time
+// (37 columns fp64, 5-point stencil of 26353 elements 12.3 -> 5.6 us; 80 columns fp32, power-law rows of 77812 37.6 -> 18.5; 57,
+// 12543 rows of 5 16.4 -> 8.3); none is slower, except where four groups share rows of more than 32 elements (20 columns fp64, 64
+// per row 8.6 -> 9.6).  Rows of B that start on lines are cut into tiles that keep the merge kernel's groups at work.
+inline int64_t spmm_chunk_wide_work(int32_t m, int32_t nnz, int64_t row_bytes) { return ((int64_t)m + nnz) * ceil_div64(row_bytes, 512); }
+inline bool spmm_chunked_wide(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
-    return spmm_chunked(m, nnz, ncols, sv) || (ncols * (int64_t)sv <= 64 && longest <= kChunkLongest && (int64_t)m + nnz >= 4000000);
+    const int64_t bytes = ncols * (int64_t)sv;
+    return bytes > 128 && bytes % 128 != 0 && (bytes > 256 || nnz <= 32 * (int64_t)m) &&
+           spmm_chunk_wide_work(m, nnz, bytes) <= kChunkRound * kChunkItemsWide;
 }
-// One round of three workgroups on each of 256 compute units, if its segments are neither short (448 to 896 items are alike up
+inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
+{
+    return spmm_chunked_narrow(m, nnz, ncols, sv) || spmm_chunked_wide(m, nnz, ncols, sv);
+}
+// tile_lanes: lanes that take a row of B.  Where they are 32 or more and columns are scattered, the merge kernel's waves, whose
+// LDS leaves room for 20 a compute unit, wait for one or two rows of B at a time, and its short segments leave more carries: 36 such
+// cases of 0.5 to 13 M items 3 % faster, none more than 1 % slower (91 columns fp64, power-law rows of 5 178 -> 155 us; 34,
+// 6 per row 264 -> 240; 113 fp32, rows of up to 75394 127 -> 113).  Near columns gain and lose alike (199 fp32 29.6 -> 27.7,
+// 248 49.1 -> 50.5).
+inline bool spmm_plan_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv, int64_t longest, bool scattered, int tile_lanes)
+{
+    if (spmm_chunked(m, nnz, ncols, sv)) return true;
+    if (ncols * (int64_t)sv <= 64) return longest <= kChunkLongest && (int64_t)m + nnz >= 4000000;
+    return scattered && tile_lanes >= 32;
+}
+// Segments of wide rows of B fill whole rounds (527000 items, rows of B of 520 bytes: in 1030 workgroups, a round and a third, 70 us, in 687 59).
+inline int32_t spmm_chunk_wide_items(int64_t work)
+{
+    const int64_t rounds = ceil_div64(work, kChunkRound * kChunkItemsWide), items = ceil_div64(work, kChunkRound * rounds);
+    return (int32_t)(items < kSpmmSegmentSmall ? kSpmmSegmentSmall : items);
+}
+// One round, if its segments are neither short (448 to 896 items are alike up
 // to 500000 items; at 1 M 896 take 20 % longer than 1344) nor more than a workgroup can stage.
 inline int32_t spmm_chunk_items(int64_t items, int32_t most = kChunkItems)
 {
-    const int64_t round = ceil_div64(items, 768);
+    const int64_t round = ceil_div64(items, kChunkRound);
     return (int32_t)(round < kChunkItems / 2 ? kChunkItems / 2 : round > most ? most : round);
 }
 constexpr double kScatteredMinSpread = 0.5;  // of a column sample: from here on the columns count as scattered
@@ -315,7 +347,8 @@ inline int spmm_columns(double spread, double span, double mean, size_t sv)
 inline int32_t spmm_segment_items(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
 {
     const int64_t items = (int64_t)m + nnz;
-    if (spmm_chunked(m, nnz, ncols, sv)) return spmm_chunk_items(items);
+    if (spmm_chunked_narrow(m, nnz, ncols, sv)) return spmm_chunk_items(items);
+    if (spmm_chunked_wide(m, nnz, ncols, sv)) return spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, ncols * (int64_t)sv));
     if (items < (int64_t)kSpmmSegmentMedium * 4096) return kSpmmSegmentSmall;
     return sv == 4 && ncols > 32 && items >= (int64_t)kSpmmSegmentLarge * 4096 ? kSpmmSegmentLarge : kSpmmSegmentMedium;
 }
@@ -347,9 +380,12 @@ constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 
 // 64 columns fp32, 20 per row within 1000 of the diagonal: 94.9 us with segments of 512 items, 54.2 with two turns of 84;
 // 7-point stencil 78.7 -> 59.7, 5-point stencil 128.7 -> 85.7; 13 per row 50.2 -> 42.3.
 // Chunk kernel: where rows are too long for the longest segments, but none for one of the usual length, no row is cut (a carry
-// pass is a launch more: longest row 913 of 82000 elements 8.8 -> 5.9 us); even rows fill its groups' last turn.
-inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest, bool chunked)
+// pass is a launch more: longest row 913 of 82000 elements 8.8 -> 5.9 us); even rows fill its groups' last turn.  Wide rows of B
+// (row_bytes): never more segments than usual, so that their carries fit.
+inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest, bool chunked,
+                               int64_t row_bytes)
 {
+    if (chunked && row_bytes > 64) return std::max(usual, spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, row_bytes)));
     if (chunked) {
         if (longest > kChunkLongest) return longest > kChunkItems || longest <= usual ? usual : (int32_t)longest;  // usual <= kChunkItems
         const int32_t items = spmm_chunk_items((int64_t)m + nnz, kChunkItemsMost);

@@ -12,7 +12,7 @@
 //           a segment end is kept as a carry row and added by an ordered pass afterwards.  No atomics (the reference's default SpMM,
 //           hip/kernel/level3/alphasparse_spmm_csr_nnz_split.h:283-409, scales C in a
 //           separate pass and joins segments with atomicAdd).
-//   chunk : the same with a workgroup per (longer) segment, for rows of B of up to 64 bytes.
+//   chunk : the same with a workgroup per (longer) segment, for narrow rows of B, and for wide ones of small or scattered matrices.
 #include <algorithm>
 
 #include "asx_internal.hpp"
@@ -403,7 +403,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
 }
 
 // ===========================================================================================
-// chunk: one workgroup per segment, for narrow rows of B
+// chunk: one workgroup per segment
 // ===========================================================================================
 // Where a row of B takes four lanes or fewer, rows of B that the L2s could serve wait for stored elements of A on their way from
 // memory: a compute unit's L1 answers in order (64-byte rows from an L2 beside a stream from memory 175 G/s wave by wave,
@@ -414,6 +414,9 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
 // this one, three matrices in turn: 8 columns fp64, 20 per row within 3000 of the diagonal 65.4 -> 56.5 us, 2 columns
 // 54.1 -> 39.8; 16 columns fp32, 50 per row within 20000 122 -> 91.9; 4 columns fp32, 8 per row within 300 29.3 -> 20.2; band of
 // 11, 2 columns fp64 24.3 -> 16.7.
+//
+// Rows of B of more than 128 bytes (spmm_chunked_wide says which) come here for another reason: too few waves.  Eight waves deal the
+// segment's rows out, and one of more than 64 elements is cut between them, in which eight rows of B are then in flight a group.
 //
 // NARROW: B spans at most 4 GB, and what is staged is the byte offset of its row: a 32-bit add per row of B and lane instead of
 // a 64-bit multiplication.
@@ -426,8 +429,8 @@ __global__ __launch_bounds__(kChunkThreads, NARROW ? 6 : 4) void k_spmm_chunk(
     typedef typename VecOf<T, VEC>::type V;
     constexpr int G = 1 << LOGG, NG = kWave / G;
     constexpr int U = 8;  // rows of B a lane has in flight
-    constexpr int kDealt = spmm_dealt(NG);
-    constexpr int kWide = 256;  // longer rows are taken by all waves (elements)
+    constexpr int kWide = NG > 4 ? 256 : 64;  // longer rows are taken by all waves (elements)
+    constexpr int kDealt = spmm_dealt(NG) < kWide ? spmm_dealt(NG) : kWide;
     constexpr int kWaves = kChunkThreads / kWave, NE = (kChunkElems + kChunkThreads - 1) / kChunkThreads;
     __shared__ int32_t s_col[kChunkElems];
     __shared__ T s_val[kChunkElems];
@@ -440,8 +443,10 @@ __global__ __launch_bounds__(kChunkThreads, NARROW ? 6 : 4) void k_spmm_chunk(
     const int64_t seg = (int64_t)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
     if (seg >= nseg) return;  // the whole workgroup leaves
     const int grp = lane >> LOGG, gl = lane & (G - 1);
-    const bool active = gl * VEC < ncols;
-    const int32_t c = gl * VEC < ncols - VEC ? gl * VEC : ncols - VEC;  // as in the merge kernel
+    const int32_t t0 = (int32_t)((int64_t)blockIdx.y * ncols / gridDim.y), t1 = (int32_t)((int64_t)(blockIdx.y + 1) * ncols / gridDim.y);
+    int32_t c = t0 + gl * VEC;  // as in the merge kernel
+    const bool active = c < t1;
+    c = c < t1 - VEC ? c : t1 - VEC;
     const uint64_t ldb_bytes = (uint64_t)ldb * sizeof(T);
     int32_t x0, y0, x1, y1;
     if (xs) {  // uniform
@@ -487,7 +492,7 @@ __global__ __launch_bounds__(kChunkThreads, NARROW ? 6 : 4) void k_spmm_chunk(
         return *(const V *)((const char *)B + (NARROW ? (uint64_t)((uint32_t)staged + c_bytes) : (uint32_t)staged * ldb_bytes + c_bytes));
     };
     const auto together = [&](int32_t k, int32_t e) {  // the sum over the wave's groups, in every group
-        V acc = spmm_staged<T, VEC, NG, U / 2>(k + grp, e, s_col, s_val, row_of_b);
+        V acc = spmm_staged<T, VEC, NG, (NG > 4 ? U / 2 : U)>(k + grp, e, s_col, s_val, row_of_b);
 #pragma unroll
         for (int d = G; d < kWave; d <<= 1)
 #pragma unroll
@@ -547,7 +552,7 @@ __global__ __launch_bounds__(kChunkThreads, NARROW ? 6 : 4) void k_spmm_chunk(
         }
         __syncthreads();
     }
-    if (carry_row && tid == 0) carry_row[seg] = tail ? x1 : -1;
+    if (carry_row && tid == 0 && blockIdx.y == 0) carry_row[seg] = tail ? x1 : -1;
 }
 
 // Every wave looks at kFixupSegs consecutive segments (one lane each) for the first segment of a run
@@ -669,7 +674,7 @@ static void launch_chunk(const SpmmTiling &tiling, int32_t m, int32_t k, int32_t
     const auto launch = [&](auto vec_, auto log_) {
         const auto with = [&](auto narrow_) {
             hipLaunchKernelGGL((k_spmm_chunk<T, decltype(vec_)::value, decltype(log_)::value, decltype(narrow_)::value != 0>),
-                               dim3((unsigned)(ceil_div64(nseg, kXcds) * kXcds)), dim3(kChunkThreads), 0, s, m, nnz, items, nseg, ncols, alpha,
+                               dim3((unsigned)(ceil_div64(nseg, kXcds) * kXcds), (unsigned)tiling.tiles), dim3(kChunkThreads), 0, s, m, nnz, items, nseg, ncols, alpha,
                                row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);
         };
         if (narrow)
@@ -682,8 +687,16 @@ static void launch_chunk(const SpmmTiling &tiling, int32_t m, int32_t k, int32_t
             launch(Int<kFull>{}, Int<0>{});
         else if (tiling.log_lanes == 1)
             launch(Int<kFull>{}, Int<1>{});
-        else
+        else if (tiling.log_lanes == 2)
             launch(Int<kFull>{}, Int<2>{});
+        else if (tiling.log_lanes == 3)
+            launch(Int<kFull>{}, Int<3>{});
+        else if (tiling.log_lanes == 4)
+            launch(Int<kFull>{}, Int<4>{});
+        else if (tiling.log_lanes == 5)
+            launch(Int<kFull>{}, Int<5>{});
+        else
+            launch(Int<kFull>{}, Int<6>{});
     } else if (tiling.vec == 1) {
         launch(Int<1>{}, Int<0>{});
     } else if constexpr (kFull > 2) {  // two or three columns of fp32

@@ -62,3 +62,18 @@ def test_wide_b():
     capi.spmm(rp, col, val, B, C, 8, 1.0, 0.0, ldb=ldb, ldc=8, k=k)
     ref = (val[:, None] * B[:, :8][col.long()]).reshape(m, 12, 8).sum(1)
     assert torch.equal(C, ref)
+
+
+@pytest.mark.parametrize("dtype,ncols", [(np.float32, n) for n in (33, 57, 65, 101, 129, 257, 300)] + [(np.float64, n) for n in (17, 33, 65, 129, 301)])
+@pytest.mark.parametrize("planned", [False, True])
+def test_wide_rows_of_b(dtype, ncols, planned):
+    """Every number of lanes a row and one or more tiles of them; rows around what a group, a wave and a segment take, each added to
+    C once; the fewest items a segment holds, the most of one round, and more than a round (where scattered columns still come here)."""
+    rng = np.random.default_rng(ncols)
+    edges = [0, 1, 7, 8, 9, 31, 32, 33, 63, 64, 65, 127, 128, 129, 639, 640, 641, 1279, 1281]
+    _check(np.r_[rng.integers(0, 12, 300), edges, np.zeros(900, int), rng.permutation(edges), 1500, 1], 500, ncols, dtype, planned, pad=3)
+    _check([3], 5, ncols, dtype, planned, beta=0.0)
+    turns = -(-ncols * np.dtype(dtype).itemsize // 512)
+    for work in (768 * 128 + 5, 768 * 640 - 9, 768 * 640 + 4000):
+        per = 11
+        _check(np.r_[np.full(work // turns // (per + 1), per), 700], 3000, ncols, dtype, planned)
