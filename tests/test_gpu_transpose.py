@@ -85,3 +85,20 @@ def test_transpose_with_a_column_that_many_rows_share_takes_no_longer_than_a_few
             times.append(a.elapsed_time(b))
         best.append(min(times))
     assert best[1] < 4 * best[0], best
+
+
+@pytest.mark.parametrize("dtype,n,nnz", [(np.float32, 60000, 700001), (np.float64, 500001, 2000003), (np.float32, 1000001, 4290 * 4096),
+                                         (np.float32, 1000001, 4300 * 4096)])
+def test_transpose_where_the_counts_take_a_scan_of_blocks(dtype, n, nnz):
+    """A few blocks of 4096 counts, some hundred, and as few and as many as lie either side of 1024, from where on their sums
+    are scanned first."""
+    rng = np.random.default_rng(n)
+    col = rng.integers(0, n, nnz).astype(np.int32)
+    val = rng.uniform(-1, 1, nnz).astype(dtype)
+    d, rows = _transposed(nnz // 9, n, col, val)
+    got = capi.csr_transpose(*d, n)
+    order = torch.sort(d[1], stable=True)[1]
+    assert torch.equal(got[0][1:], torch.cumsum(torch.bincount(d[1], minlength=n), 0).to(torch.int32))
+    assert int(got[0][0]) == 0
+    assert torch.equal(got[1], torch.from_numpy(rows).cuda()[order])
+    assert torch.equal(got[2], d[2][order])
