@@ -786,18 +786,24 @@ static int plan_long_rows(asx_plan *p, hipStream_t s)
     return st;
 }
 
-// pass 2: one wave per block of rows, its accumulators (8 bytes a row) in LDS.  Blocks of 256
-// rows, doubled up to 1024 while that leaves more than 8 waves per compute unit and the block's
-// partial sums inside one slice (expected from the column sample) are fewer than 12: a
-// step of pass 2 takes its 64 entries from at most three ranges.  Small blocks mean many waves
-// in flight.  Measured: the power-law matrix (4 per range at 256 rows) 50 / 34.5 / 36.6 us with
-// 512 / 1024 / 2048 rows; 16 per row over 32 slices (100 per range at 256 rows) 17.5 / 20 us
-// with 256 / 512 rows; the same in fp64 over 64 slices 26.5 / 27.5 / 36.8 us with 256 / 512 / 1024.
+// pass 2: one wave per block of rows, its accumulators (8 bytes a row) in LDS.  Small blocks mean many waves in flight, large
+// ones long ranges of partial sums inside a slice, fewer lines of which only a part is wanted, and full steps (a step
+// takes its 64 entries from at most three ranges).  Blocks of 256 rows, doubled while either holds:
+//   up to 1024, if that leaves more than 4 waves a compute unit and the ranges (expected from the column sample) are
+//     shorter than 12 entries;
+//   up to 2048, if it leaves 8 waves a compute unit in fp64, 11 in fp32, and the ranges are shorter than 48 entries.
+// Four matrices in turn, whole multiply: power-law rows, 4.2 M x 4.2 M, 33 M elements, fp64 163 us with 1024 rows, 152 with 2048,
+// 170 with 4096; 7 per row, 4.2 M fp64 254 / 204 / 182 / 172 / 200 us with 256 / 512 / 1024 / 2048 / 4096, fp32 125 / 109 /
+// 100 / 109 with 256 / 512 / 1024 / 2048; 1.5 M fp64 73 / 69 / 72 / 87, fp32 46 / 45 / 52; 16 per row of 1 M, fp32 51 / 57.
 static int32_t sliced_rows_per_wave(const asx_plan *p, size_t sv, double pairs_per_element, int cus)
 {
     const double per_row_slice = pairs_per_element * (double)p->nnz / ((double)p->m * (double)slice_count(p, sv));
     int32_t rpw = 256;
-    while (rpw < 1024 && (int64_t)rpw * cus * 8 < p->m && per_row_slice * rpw < 12.0) rpw *= 2;
+    for (; rpw < 2048; rpw *= 2) {
+        const int64_t waves = ceil_div64(p->m, (int64_t)rpw) / cus;  // a compute unit, now
+        const double range = per_row_slice * rpw;
+        if (!(rpw < 1024 && waves >= 8 && range < 12.0) && !(waves >= (sv == 8 ? 16 : 22) && range < 48.0)) break;
+    }
     return rpw;
 }
 

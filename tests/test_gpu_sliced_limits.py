@@ -52,3 +52,24 @@ def test_steps_of_many_row_blocks_take_the_room_they_need():
     expect[torch.from_numpy(rows).cuda()] = x[col.long()]
     assert torch.equal(y, expect)
     assert held < 110e6, held
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float64])
+@pytest.mark.parametrize("m", [524289, 1048576, 1441793, 2097153, 2883585, 4194305, 5767169])
+def test_row_blocks_of_every_size(m, dtype):
+    """Matrices on which row blocks of 256 to 2048 rows begin, the last one of a single row.  Integers: exact in any order."""
+    gen = torch.Generator(device="cuda").manual_seed(m)
+    lens = torch.randint(0, 5, (m,), device="cuda", generator=gen)
+    lens[-1], lens[m // 2] = 2, 70000
+    row_ptr = torch.zeros(m + 1, dtype=torch.int32, device="cuda")
+    row_ptr[1:] = torch.cumsum(lens, 0)
+    nnz = int(row_ptr[-1])
+    col = torch.randint(0, m, (nnz,), device="cuda", generator=gen, dtype=torch.int32)
+    draw = lambda k: torch.randint(-3, 4, (k,), device="cuda", generator=gen).to(dtype)
+    val, x, y = draw(nnz), draw(m), 2 * draw(m)
+    rows = torch.repeat_interleave(torch.arange(m, device="cuda"), lens)
+    ref = (2 * torch.zeros(m, dtype=torch.float64, device="cuda").index_add_(0, rows, (val * x[col.long()]).double()) + 0.5 * y).to(dtype)
+    plan = capi.Plan(False, capi.SPMV_SLICED, dtype, m, m, nnz, row_ptr, col=col, val=val)
+    capi.spmv(row_ptr, col, val, x, y, 2.0, 0.5, plan=plan)
+    assert torch.equal(y, ref)
+    plan.destroy()
