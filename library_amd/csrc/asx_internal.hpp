@@ -33,11 +33,18 @@ static_assert(2 * kChunkItems <= kChunkElems && kChunkItemsMost < kChunkRows, "a
 // faster on average (3 columns fp64, 56 per row 16.7 -> 7.4 us; 2 columns fp32, 5 per row 21.0 -> 16.0), but with 4 per row,
 // 2 columns fp32 8.2 -> 10.1, with 7, 3 columns fp64 4.7 -> 5.1.  Rows of B of 33 to 64 bytes only where a plan knows that no
 // row of A is long and there are several rounds of workgroups (16 columns fp32, 23 per row, 8 M elements 60.9 -> 52.2 us; 9 per
-// row, 5 M 50.5 and 50.5; but 14 columns, 27 per row, 2.2 M 23.3 -> 24.3; rows of up to 1510 57.4 -> 73.5).  Rows of 65 to 128
-// bytes gain and lose alike (18 columns fp32 27.3 -> 29.6, 12 columns fp64 86.8 -> 83.0).
+// row, 5 M 50.5 and 50.5; but 14 columns, 27 per row, 2.2 M 23.3 -> 24.3; rows of up to 1510 57.4 -> 73.5).
 inline bool spmm_chunked_narrow(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
     return ncols * (int64_t)sv <= 32 && 2 * (int64_t)nnz >= (sv == 4 ? 9 : 16) * (int64_t)m;
+}
+// Rows of B of 33 to 128 bytes while one round of workgroups takes all of A, planned or not: 57 such cases of all families 6 %
+// faster on average (7 columns fp64, 61 per row, 462624 elements 12.1 -> 8.1 us; 31 fp32, 5-point stencil of 642649 14.4 -> 11.9;
+// 24 fp32, power-law rows of 699314 19.3 -> 17.0), none slower by more than calls of 6 us differ; with several rounds they gain and lose
+// alike (18 columns fp32 27.3 -> 29.6, 12 columns fp64 86.8 -> 83.0).
+inline bool spmm_chunked_mid(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
+{
+    return ncols * (int64_t)sv > 32 && ncols * (int64_t)sv <= 128 && (int64_t)m + nnz <= kChunkRound * kChunkItems;
 }
 // Wider rows of B while one round of workgroups takes all of A: the merge kernel's few waves then walk 128 items each, one or two
 // rows of A at a time, where eight waves share them here.  40 such cases of all families, planned or not, take 0.7 of their time
@@ -53,7 +60,7 @@ inline bool spmm_chunked_wide(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 }
 inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
-    return spmm_chunked_narrow(m, nnz, ncols, sv) || spmm_chunked_wide(m, nnz, ncols, sv);
+    return spmm_chunked_narrow(m, nnz, ncols, sv) || spmm_chunked_mid(m, nnz, ncols, sv) || spmm_chunked_wide(m, nnz, ncols, sv);
 }
 // tile_lanes: lanes that take a row of B.  Where they are 32 or more and columns are scattered, the merge kernel's waves, whose
 // LDS leaves room for 20 a compute unit, wait for one or two rows of B at a time, and its short segments leave more carries: 36 such
@@ -348,6 +355,7 @@ inline int32_t spmm_segment_items(int32_t m, int32_t nnz, int32_t ncols, size_t 
 {
     const int64_t items = (int64_t)m + nnz;
     if (spmm_chunked_narrow(m, nnz, ncols, sv)) return spmm_chunk_items(items);
+    if (spmm_chunked_mid(m, nnz, ncols, sv)) return (int32_t)std::max<int64_t>(kSpmmSegmentMedium, ceil_div64(items, kChunkRound));
     if (spmm_chunked_wide(m, nnz, ncols, sv)) return spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, ncols * (int64_t)sv));
     if (items < (int64_t)kSpmmSegmentMedium * 4096) return kSpmmSegmentSmall;
     return sv == 4 && ncols > 32 && items >= (int64_t)kSpmmSegmentLarge * 4096 ? kSpmmSegmentLarge : kSpmmSegmentMedium;
@@ -385,6 +393,7 @@ constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 
 inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest, bool chunked,
                                int64_t row_bytes)
 {
+    if (chunked && spmm_chunked_mid(m, nnz, row_bytes, 1)) return usual;
     if (chunked && row_bytes > 64) return std::max(usual, spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, row_bytes)));
     if (chunked) {
         if (longest > kChunkLongest) return longest > kChunkItems || longest <= usual ? usual : (int32_t)longest;  // usual <= kChunkItems

@@ -77,3 +77,12 @@ def test_wide_rows_of_b(dtype, ncols, planned):
     for work in (768 * 128 + 5, 768 * 640 - 9, 768 * 640 + 4000):
         per = 11
         _check(np.r_[np.full(work // turns // (per + 1), per), 700], 3000, ncols, dtype, planned)
+
+
+@pytest.mark.parametrize("dtype,ncols", [(np.float32, n) for n in (9, 12, 17, 25, 32)] + [(np.float64, n) for n in (5, 6, 10, 13, 16)])
+@pytest.mark.parametrize("planned", [False, True])
+def test_rows_of_b_between_narrow_and_wide(dtype, ncols, planned):
+    """The fewest items a segment holds, the most, and more than one round of segments; rows that are cut and rows that are not."""
+    for work in (768 * 256 - 3, 768 * 256 + 900, 768 * 1344 - 9, 768 * 1344 + 4000):
+        _check(np.full(work // 15, 14), 3000, ncols, dtype, planned)
+    _check(np.r_[np.full(3000, 11), 5000, np.zeros(700, int), 255, 256, 257, 511, 512, 513], 700, ncols, dtype, planned, pad=1)
