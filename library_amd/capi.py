@@ -159,6 +159,9 @@ def _handle(h):
 
 def _stream():
     import torch
+    raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)
+    if raw is not None and torch.cuda.is_initialized():  # 0.4 us, a Stream object 3.2
+        return C.c_void_p(raw(torch._C._cuda_getDevice()))
     return C.c_void_p(torch.cuda.current_stream().cuda_stream)
 
 
