@@ -108,18 +108,20 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_count(const int32_t 
                                                                   int32_t *__restrict__ counts, int32_t *__restrict__ seg_row)
 {
     __shared__ int32_t hist[kBuckets];
+    const int32_t b = block_of_xcd();
+    if (b >= nblocks) return;  // the whole workgroup leaves
+    int32_t c[kSortPerLane];
+    load_columns(col, nnz, b, c);
     for (int s = threadIdx.x; s < nbuckets; s += kSortThreads) hist[s] = 0;
     __syncthreads();
-    const int64_t first = (int64_t)blockIdx.x * kSortElems;
 #pragma unroll
-    for (int k = 0; k < kSortPerLane; ++k) {
-        const int64_t i = first + k * kSortThreads + threadIdx.x;
-        if (i < nnz) atomicAdd(&hist[(col[i] - base) >> shift], 1);  // integer counts: the order does not matter
-    }
-    block_seg_rows(row_ptr, m, nnz, base, seg_row);
+    for (int k = 0; k < kSortPerLane; ++k)
+        if ((int64_t)b * kSortElems + k * kSortThreads + threadIdx.x < nnz)
+            atomicAdd(&hist[(c[k] - base) >> shift], 1);  // integer counts: the order does not matter
+    block_seg_rows(row_ptr, m, nnz, base, b, nblocks, seg_row);
     __syncthreads();
-    for (int s = threadIdx.x; s < nbuckets; s += kSortThreads) counts[(int64_t)s * nblocks + blockIdx.x] = hist[s];
-    if (blockIdx.x == 0 && threadIdx.x == 0) counts[(int64_t)nbuckets * nblocks] = 0;
+    for (int s = threadIdx.x; s < nbuckets; s += kSortThreads) counts[(int64_t)s * nblocks + b] = hist[s];
+    if (b == 0 && threadIdx.x == 0) counts[(int64_t)nbuckets * nblocks] = 0;
 }
 
 // Four workgroups a compute unit in fp32 (37 KB of LDS, 64 registers), three in fp64 (53 KB): its chain of dependent steps
@@ -358,7 +360,17 @@ __global__ __launch_bounds__(kSortThreads) void k_transpose_rows(const int32_t *
     // column counts of the whole bucket -> row offsets of A^T
     for (int i = tid; i < COLS; i += kSortThreads) sh.first[i] = 0;
     __syncthreads();
-    for (int32_t i = s0 + tid; i < s1; i += kSortThreads) atomicAdd(&sh.first[bcol[i]], 1);
+    for (int32_t i0 = s0; i0 < s1; i0 += kSortElems) {  // uniform; a turn's loads together (28.0 -> 26.1 us), past the end the last one
+        int32_t c[kSortPerLane];
+#pragma unroll
+        for (int k = 0; k < kSortPerLane; ++k) {
+            const int32_t i = i0 + k * kSortThreads + tid;
+            c[k] = bcol[i < s1 ? i : s1 - 1];
+        }
+#pragma unroll
+        for (int k = 0; k < kSortPerLane; ++k)
+            if (i0 + k * kSortThreads + tid < s1) atomicAdd(&sh.first[c[k]], 1);
+    }
     __syncthreads();
     columns_exclusive_sum<COLS>(sh.first, sh.wave_tot);
     const int64_t c0 = (int64_t)b << shift;
@@ -501,7 +513,7 @@ int csr_transpose_buckets(int shift, int32_t m, int32_t n, int32_t nnz, int32_t 
     uint16_t *bcol = (uint16_t *)(arena + o_col);
     T *bval = (T *)(arena + o_val);
     const int bbits = nbuckets > 1 ? bits_for(nbuckets) : 0;
-    hipLaunchKernelGGL(k_transpose_count, dim3((unsigned)nblocks), dim3(kSortThreads), 0, s, row_ptr, col, m, nnz, base, shift,
+    hipLaunchKernelGGL(k_transpose_count, dim3(count_grid(nblocks)), dim3(kSortThreads), 0, s, row_ptr, col, m, nnz, base, shift,
                        nbuckets, nblocks, counts, seg);
     st = launch_exclusive_scan_i32(counts, counts, ncount, (int32_t *)(arena + o_tmp), s);
     if (st) return st;

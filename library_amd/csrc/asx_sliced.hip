@@ -52,18 +52,20 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_count(const int32_t *__
                                                                 int32_t *__restrict__ counts, int32_t *__restrict__ seg_row)
 {
     __shared__ int32_t hist[kSlicedMaxSlices];
+    const int32_t b = block_of_xcd();
+    if (b >= nblocks) return;  // the whole workgroup leaves
+    int32_t c[kSortPerLane];
+    load_columns(col, nnz, b, c);
     for (int s = threadIdx.x; s < nslices; s += kSortThreads) hist[s] = 0;
     __syncthreads();
-    const int64_t base = (int64_t)blockIdx.x * kSortElems;
 #pragma unroll
-    for (int k = 0; k < kSortPerLane; ++k) {
-        const int64_t i = base + k * kSortThreads + threadIdx.x;
-        if (i < nnz) atomicAdd(&hist[col[i] / width], 1);  // integer counts: the order does not matter
-    }
-    block_seg_rows(row_ptr, m, nnz, 0, seg_row);
+    for (int k = 0; k < kSortPerLane; ++k)
+        if ((int64_t)b * kSortElems + k * kSortThreads + threadIdx.x < nnz)
+            atomicAdd(&hist[c[k] / width], 1);  // integer counts: the order does not matter
+    block_seg_rows(row_ptr, m, nnz, 0, b, nblocks, seg_row);
     __syncthreads();
-    for (int s = threadIdx.x; s < nslices; s += kSortThreads) counts[(int64_t)s * nblocks + blockIdx.x] = hist[s];
-    if (blockIdx.x == 0 && threadIdx.x == 0) counts[(int64_t)nslices * nblocks] = 0;
+    for (int s = threadIdx.x; s < nslices; s += kSortThreads) counts[(int64_t)s * nblocks + b] = hist[s];
+    if (b == 0 && threadIdx.x == 0) counts[(int64_t)nslices * nblocks] = 0;
 }
 
 // exclusive sum of one value per thread over a workgroup of kLayoutThreads; *total: of all (barriers inside)
@@ -869,7 +871,7 @@ int build_sliced(int32_t m, int32_t n, int32_t nnz, int32_t width, int32_t rows_
     }
 
     // 1. every block's stored elements per slice, and from their scan the block's place in each slice
-    hipLaunchKernelGGL(k_sliced_count, dim3((unsigned)nblocks), dim3(kSortThreads), 0, s, row_ptr, m, col, nnz, width, sm.nslices,
+    hipLaunchKernelGGL(k_sliced_count, dim3(count_grid(nblocks)), dim3(kSortThreads), 0, s, row_ptr, m, col, nnz, width, sm.nslices,
                        nblocks, counts, seg_row);
     ASX_TRY_ST(launch_exclusive_scan_i32(counts, offs, ncount, tmp, s));
     // 2. tiles, and the workgroups of pass 1

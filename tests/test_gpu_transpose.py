@@ -102,3 +102,19 @@ def test_transpose_where_the_counts_take_a_scan_of_blocks(dtype, n, nnz):
     assert int(got[0][0]) == 0
     assert torch.equal(got[1], torch.from_numpy(rows).cuda()[order])
     assert torch.equal(got[2], d[2][order])
+
+
+@pytest.mark.parametrize("nnz", [7 * 4096, 8 * 4096 - 1, 8 * 4096, 8 * 4096 + 1, 9 * 4096 + 511, 17 * 4096 + 513])
+@pytest.mark.parametrize("n", [64, 5000])
+def test_transpose_of_blocks_that_fill_the_xcds_or_not(n, nnz):
+    """Blocks of 4096 elements are counted XCD by XCD: a multiple of eight blocks and others, last blocks that are full and not;
+    buckets whose columns are counted in one turn and in several."""
+    rng = np.random.default_rng(nnz)
+    col = rng.integers(0, n, nnz).astype(np.int32)
+    val = rng.uniform(-1, 1, nnz).astype(np.float32)
+    d, rows = _transposed(nnz // 9, n, col, val)
+    got = capi.csr_transpose(*d, n)
+    order = np.argsort(col, kind="stable")
+    assert np.array_equal(got[0].cpu().numpy(), np.concatenate([[0], np.cumsum(np.bincount(col, minlength=n))]))
+    assert np.array_equal(got[1].cpu().numpy(), rows[order])
+    assert np.array_equal(got[2].cpu().numpy(), val[order])
