@@ -267,7 +267,8 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
             xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
         const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
-        return launch_spmm_merge<T>(plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T)), m, k, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
+        const bool chunked = plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T));
+        return launch_spmm_merge<T>(chunked, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
                                     (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off), plan ? plan->carry_pass != 0 : true,
                                     spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
     }

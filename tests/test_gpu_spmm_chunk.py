@@ -64,6 +64,28 @@ def test_wide_b():
     assert torch.equal(C, ref)
 
 
+@pytest.mark.parametrize("planned", [False, True])
+@pytest.mark.parametrize("k", [None, 1])
+def test_view_of_a_matrix_beyond_4_gb(planned, k):
+    """Eight of 64 columns of 20 M rows, 5.1 GB from the first row to the last, by calls that do not say how many rows there are
+    and by calls that say too few."""
+    rows, m = 20_000_000, 30000
+    gen = torch.Generator(device="cuda").manual_seed(6)
+    B = torch.empty((rows, 64), device="cuda")[:, :8]
+    B.copy_(torch.randint(-3, 4, B.shape, device="cuda", generator=gen, dtype=torch.int8))
+    rp = (torch.arange(m + 1, device="cuda") * 12).to(torch.int32)
+    col = torch.randint(0, rows, (m * 12,), device="cuda", generator=gen, dtype=torch.int32)
+    col[-1] = rows - 1
+    val = torch.randint(-3, 4, (m * 12,), device="cuda", generator=gen).float()
+    C = torch.zeros((m, 8), device="cuda")
+    plan = capi.Plan(True, capi.SPMM_DEFAULT, val.dtype, m, rows, col.numel(), rp, ncols=8, col=col, val=val) if planned else None
+    capi.spmm(rp, col, val, B, C, 8, 1.0, 0.0, plan=plan, ldb=64, ldc=8, k=k)
+    ref = (val[:, None] * B[col.long()]).reshape(m, 12, 8).sum(1)
+    assert torch.equal(C, ref)
+    if plan is not None:
+        plan.destroy()
+
+
 @pytest.mark.parametrize("dtype,ncols", [(np.float32, n) for n in (33, 57, 65, 101, 129, 257, 300)] + [(np.float64, n) for n in (17, 33, 65, 129, 301)])
 @pytest.mark.parametrize("planned", [False, True])
 def test_wide_rows_of_b(dtype, ncols, planned):
