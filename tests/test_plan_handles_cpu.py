@@ -53,3 +53,24 @@ def test_values_of_a_plan_that_are_no_tensor():
     for call in (plan.update_values, plan.refresh_if_changed):
         with pytest.raises(AttributeError):
             call(3)
+
+
+@pytest.mark.parametrize("B, ncols, ldb, rows", [
+    (torch.empty(1000, 64)[:, :8], 8, 64, 1000), (torch.empty(1000, 64)[:, 56:], 8, 64, 1000), (torch.empty(3, 64)[:, :8], 8, 64, 3),
+    (torch.empty(1000, 64), 8, 64, 1000), (torch.empty(64000), 8, 64, 1000), (torch.empty(64000 - 56), 8, 64, 1000),
+    (torch.empty(1000, 8), 8, None, 1000), (torch.empty(8000), 8, None, 1000), (torch.empty(7), 8, 64, 0), (torch.empty(0, 8), 8, 64, 0)])
+def test_rows_of_b_when_the_caller_does_not_say(B, ncols, ldb, rows):
+    seen = []
+    signature = C.CFUNCTYPE(C.c_int, C.c_void_p, C.c_int, C.c_int32, C.c_int32, C.c_int32, C.c_int32, C.c_float, C.c_void_p,
+                            C.c_void_p, C.c_void_p, C.c_void_p, C.c_int64, C.c_float, C.c_void_p, C.c_int64, C.c_void_p, C.c_size_t, C.c_void_p)
+    fn = signature(lambda plan, alg, m, k, *rest: seen.append(k) or 0)
+    calls = capi._loaded()
+    from library_amd import _calls
+    _calls.streams_from(lambda: 0, lambda device: 0)
+    try:
+        for k in (None, 17):
+            assert calls.spmm(C.cast(fn, C.c_void_p).value, False, None, 0, torch.zeros(2, dtype=torch.int32), torch.zeros(1, dtype=torch.int32),
+                              torch.zeros(1), B, torch.zeros(8), ncols, 1.0, 0.0, ldb, None, k, None) == 0
+    finally:
+        capi._fast = None  # the next call asks torch for its streams again
+    assert seen == [rows, 17]
