@@ -108,3 +108,36 @@ def test_rows_of_b_between_narrow_and_wide(dtype, ncols, planned):
     for work in (768 * 256 - 3, 768 * 256 + 900, 768 * 1344 - 9, 768 * 1344 + 4000):
         _check(np.full(work // 15, 14), 3000, ncols, dtype, planned)
     _check(np.r_[np.full(3000, 11), 5000, np.zeros(700, int), 255, 256, 257, 511, 512, 513], 700, ncols, dtype, planned, pad=1)
+
+
+def _microseconds(per, ncols, dtype, elements=6_000_000):
+    """Of a planned multiply with even rows of `per` elements within 2 * per of the diagonal, the least of several."""
+    m, k = elements // per, 100000
+    gen = torch.Generator(device="cuda").manual_seed(per)
+    rp = (torch.arange(m + 1, device="cuda") * per).to(torch.int32)
+    low = (torch.arange(m, device="cuda") * k // m - 2 * per).clamp(0, k - 4 * per)
+    col = (low[:, None] + 4 * torch.arange(per, device="cuda")[None, :]).reshape(-1).to(torch.int32)
+    val = torch.rand(m * per, device="cuda", generator=gen, dtype=dtype)
+    B, C = torch.rand((k, ncols), device="cuda", generator=gen, dtype=dtype), torch.empty((m, ncols), device="cuda", dtype=dtype)
+    plan = capi.Plan(True, capi.SPMM_DEFAULT, dtype, m, k, m * per, rp, ncols=ncols, col=col, val=val)
+    ws = torch.empty(max(plan.workspace_bytes, 256), dtype=torch.uint8, device="cuda")
+    best = 1e9
+    for _ in range(8):
+        a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        a.record()
+        for _ in range(10):
+            capi.spmm(rp, col, val, B, C, ncols, 1.0, 0.0, plan=plan, workspace=ws)
+        b.record()
+        b.synchronize()
+        best = min(best, a.elapsed_time(b) * 100)
+    plan.destroy()
+    return best
+
+
+@pytest.mark.parametrize("dtype,ncols", [(torch.float64, 2), (torch.float64, 5), (torch.float32, 3), (torch.float32, 11)])
+@pytest.mark.parametrize("per", [90, 180])
+def test_as_many_elements_in_rows_that_a_wave_takes(dtype, ncols, per):
+    """Little longer than in rows that a lane group takes: the waves of a workgroup share them.  Where the wave that dealt rows out
+    took the long ones of its own, seven of eight had nothing to do and it took 2.3 to 4.3 times as long.  The bound: up to 64 lane
+    groups of a wave have four rows of B in flight each, 256 places for 180 elements, 1.42, and then add up over six shuffles."""
+    assert _microseconds(per, ncols, dtype) < 1.8 * _microseconds(60, ncols, dtype)
