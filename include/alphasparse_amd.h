@@ -260,8 +260,8 @@ const char *asx_kernel_name(int is_spmm, int kernel);
  * read). */
 int asx_plan_alg(const asx_plan *plan);
 size_t asx_plan_workspace_bytes(const asx_plan *plan);
-/* What a plan that holds a regrouped copy of A looks like (for logs and tests; -1 where the
- * figure does not apply to the plan's kernel).  No counterpart in the reference. */
+/* What a plan looks like: one that holds a regrouped copy of A, or one for SpMM (for logs and tests; -1 where
+ * the figure does not apply to the plan's kernel).  No counterpart in the reference. */
 enum {
     ASX_PLAN_INFO_TILES = 0,          /* tiles of 256 slots (sliced, window) */
     ASX_PLAN_INFO_SLICES = 1,         /* column slices (sliced) */
@@ -278,9 +278,11 @@ enum {
     ASX_PLAN_INFO_PIECES = 12,        /* pieces of x fetched over all blocks (window) */
     ASX_PLAN_INFO_STACKED_ROWS = 13,  /* rows of a plane when the three bands share rotating regions of LDS and the
                                          blocks are stored plane above plane (window; 0 otherwise) */
-    ASX_PLAN_INFO_BY_REFERENCE = 14   /* 1 when the plan keeps no copy of A's values (window: no row of A holds fewer than two
+    ASX_PLAN_INFO_BY_REFERENCE = 14,  /* 1 when the plan keeps no copy of A's values (window: no row of A holds fewer than two
                                          stored elements, so the stored elements of a tile are consecutive in A's val, which
                                          every call reads in place; asx_plan_holds_values is 0 then) */
+    ASX_PLAN_INFO_SEGMENT_ITEMS = 15,   /* rows and stored elements, added up, of a segment (SpMM, row-ordered) */
+    ASX_PLAN_INFO_SHARED_SEGMENTS = 16  /* 1 when a workgroup shares a segment, 0 when a wave takes it (SpMM, row-ordered) */
 };
 int64_t asx_plan_info(const asx_plan *plan, int what);
 /* Frees the buffer a sliced or window plan keeps for the partial sums / carries of a call.  Calls

@@ -1179,7 +1179,11 @@ const char *asx_kernel_name(int is_spmm, int kernel)
 size_t asx_plan_workspace_bytes(const asx_plan *plan) { return plan ? plan->workspace_bytes : 0; }
 int64_t asx_plan_info(const asx_plan *plan, int what)
 {
-    if (!plan || plan->is_spmm) return -1;
+    if (!plan) return -1;
+    if (plan->is_spmm) {
+        if (plan->alg != ASX_SPMM_MERGE) return -1;
+        return what == ASX_PLAN_INFO_SEGMENT_ITEMS ? plan->items : what == ASX_PLAN_INFO_SHARED_SEGMENTS ? plan->chunked : -1;
+    }
     const bool sliced = plan->alg == ASX_SPMV_SLICED, window = plan->alg == ASX_SPMV_WINDOW;
     switch (what) {
     case ASX_PLAN_INFO_TILES: return sliced ? plan->sliced.ntiles : window ? plan->window.ntiles : -1;

@@ -31,9 +31,8 @@ constexpr int64_t kChunkRound = 768;      // three workgroups on each of 256 com
 static_assert(2 * kChunkItems <= kChunkElems && kChunkItemsMost < kChunkRows, "a segment fits what is staged");
 // Which calls it takes.  Rows of B of up to 32 bytes, planned or not, unless rows of A are short: 66 such cases of all families 9 %
 // faster on average (3 columns fp64, 56 per row 16.7 -> 7.4 us; 2 columns fp32, 5 per row 21.0 -> 16.0), but with 4 per row,
-// 2 columns fp32 8.2 -> 10.1, with 7, 3 columns fp64 4.7 -> 5.1.  Rows of B of 33 to 64 bytes only where a plan knows that no
-// row of A is long and there are several rounds of workgroups (16 columns fp32, 23 per row, 8 M elements 60.9 -> 52.2 us; 9 per
-// row, 5 M 50.5 and 50.5; but 14 columns, 27 per row, 2.2 M 23.3 -> 24.3; rows of up to 1510 57.4 -> 73.5).
+// 2 columns fp32 8.2 -> 10.1, with 7, 3 columns fp64 4.7 -> 5.1.  What it takes beside these: spmm_chunked_mid, spmm_chunked_wide
+// and, under plans only, spmm_plan_chunked.
 inline bool spmm_chunked_narrow(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
     return ncols * (int64_t)sv <= 32 && 2 * (int64_t)nnz >= (sv == 4 ? 9 : 16) * (int64_t)m;
@@ -62,7 +61,13 @@ inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
     return spmm_chunked_narrow(m, nnz, ncols, sv) || spmm_chunked_mid(m, nnz, ncols, sv) || spmm_chunked_wide(m, nnz, ncols, sv);
 }
-// tile_lanes: lanes that take a row of B.  Where they are 32 or more and columns are scattered, the merge kernel's waves, whose
+// Under a plan also rows of B of up to 64 bytes (those of up to 32 that spmm_chunked_narrow leaves out among them) where no row of A
+// is long, rows hold 3.5 elements or more on average, and there are several rounds of workgroups (16 columns fp32, 23 per row,
+// 8 M elements 60.9 -> 52.2 us; 9 per row, 5 M 50.5 and 50.5; but 14 columns, 27 per row, 2.2 M 23.3 -> 24.3; rows of up to
+// 1510 57.4 -> 73.5).  With 3 per row, 2 to 16 columns, both types, near and scattered, merge is 5 % ahead on average (2 columns
+// fp32 15.5 against 14.5, 6 columns 68.8 against 61.9, 16 columns 61.2 against 55.8); from 4 on they differ by 1 % on average.
+//
+// And scattered columns where 32 lanes or more (tile_lanes) take a row of B: the merge kernel's waves, whose
 // LDS leaves room for 20 a compute unit, wait for one or two rows of B at a time, and its short segments leave more carries: 36 such
 // cases of 0.5 to 13 M items 3 % faster, none more than 1 % slower (91 columns fp64, power-law rows of 5 178 -> 155 us; 34,
 // 6 per row 264 -> 240; 113 fp32, rows of up to 75394 127 -> 113).  Near columns gain and lose alike (199 fp32 29.6 -> 27.7,
@@ -70,7 +75,8 @@ inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 inline bool spmm_plan_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv, int64_t longest, bool scattered, int tile_lanes)
 {
     if (spmm_chunked(m, nnz, ncols, sv)) return true;
-    if (ncols * (int64_t)sv <= 64) return longest <= kChunkLongest && (int64_t)m + nnz >= 4000000;
+    if (ncols * (int64_t)sv <= 64)
+        return longest <= kChunkLongest && 2 * (int64_t)nnz >= 7 * (int64_t)m && (int64_t)m + nnz >= 4000000;
     return scattered && tile_lanes >= 32;
 }
 // Segments of wide rows of B fill whole rounds (527000 items, rows of B of 520 bytes: in 1030 workgroups, a round and a third, 70 us, in 687 59).
