@@ -23,7 +23,10 @@ constexpr int kLongRow = 8192;
 // SpMM: merge items (rows + stored elements) per wave
 constexpr int kSpmmSegmentSmall = 128, kSpmmSegmentMedium = 256, kSpmmSegmentLarge = 512;
 // SpMM chunk kernel: threads of a workgroup, what it can stage, and merge items per segment - where rows may be cut (a segment
-// then holds up to twice as many elements) and where none is longer than kChunkLongest.
+// then holds up to twice as many elements) and where none is longer than kChunkLongest.  kChunkItemsMost: the shortest segments
+// that are within 1 % of the fastest (8 M elements, 5 to 48 per row within 3000 of the diagonal, 4 and 8 columns fp64, 4 and 16
+// fp32, on average: 1664 items 8 % behind, 2048 3 %, 2368 1.5 %, 3008 and 3392 alike; 24 per row, 8 columns fp64 58.0, 55.5, 55.4, 2688
+// items 55.5, 53.3, 53.3; 20 per row 59.9, 57.1, 56.1, 54.7, 55.2, 55.1).
 constexpr int kChunkThreads = 512, kChunkElems = 2880, kChunkRows = 2689;
 constexpr int kChunkItems = 1344, kChunkItemsMost = 2688, kChunkLongest = kChunkElems - kChunkItemsMost;
 constexpr int kChunkItemsWide = 640;      // the most where rows of B are wide
@@ -394,8 +397,11 @@ constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 
 // 64 columns fp32, 20 per row within 1000 of the diagonal: 94.9 us with segments of 512 items, 54.2 with two turns of 84;
 // 7-point stencil 78.7 -> 59.7, 5-point stencil 128.7 -> 85.7; 13 per row 50.2 -> 42.3.
 // Chunk kernel: where rows are too long for the longest segments, but none for one of the usual length, no row is cut (a carry
-// pass is a launch more: longest row 913 of 82000 elements 8.8 -> 5.9 us); even rows fill its groups' last turn.  Wide rows of B
-// (row_bytes): never more segments than usual, so that their carries fit.
+// pass is a launch more: longest row 913 of 82000 elements 8.8 -> 5.9 us).  Even rows fill whole turns of all groups of a workgroup:
+// one more where it fits, else without a last turn that would not be half full (8 columns fp64 within 3000 of the diagonal, 8 M
+// elements, full turns against segments of 2688 items: 15 per row 62.1 against 66.5 us, 17 59.5 and 64.3, 19 57.7 and 61.7, 20
+// alike, as 2688 is one turn; 16 columns fp32, 19 per row 54.2 and 56.0; last turns that are half full or more are kept: 10 per
+// row 71.9 without and 68.7 with).  Wide rows of B (row_bytes): never more segments than usual, so that their carries fit.
 inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest, bool chunked,
                                int64_t row_bytes)
 {
@@ -404,9 +410,11 @@ inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m
     if (chunked) {
         if (longest > kChunkLongest) return longest > kChunkItems || longest <= usual ? usual : (int32_t)longest;  // usual <= kChunkItems
         const int32_t items = spmm_chunk_items((int64_t)m + nnz, kChunkItemsMost);
-        const int64_t turn = (int64_t)groups * (kChunkThreads / kWave) * (longest + 1);
-        const int64_t turns = ceil_div64(items, turn) * turn;  // all groups of a workgroup at work to the end
-        return turns > kChunkItemsMost || 4 * (longest + 1) * m > 5 * ((int64_t)m + nnz) ? items : (int32_t)turns;
+        if (4 * (longest + 1) * m > 5 * ((int64_t)m + nnz)) return items;
+        const int64_t turn = (int64_t)groups * (kChunkThreads / kWave) * (longest + 1), over = items % turn;
+        const int64_t more = ceil_div64(items, turn) * turn;
+        if (more <= kChunkItemsMost) return (int32_t)more;
+        return items == kChunkItemsMost && turn <= items && 2 * over <= turn ? (int32_t)(items - over) : items;
     }
     if (columns != kColumnsNear && columns != kColumnsSpread) return usual;
     const int32_t least = usual == kSpmmSegmentLarge ? kSpmmSegmentSmall : usual;

@@ -159,3 +159,24 @@ def test_short_rows_of_large_matrices(dtype, ncols, per, shared):
     assert torch.equal(C, (val[:, None] * B[col.long()]).reshape(m, per, ncols).sum(1))
     assert plan.info("shared_segments") == shared
     plan.destroy()
+
+
+@pytest.mark.parametrize("ncols,dtype,groups", [(8, np.float64, 16), (16, np.float32, 16), (4, np.float64, 32), (2, np.float64, 64)])
+@pytest.mark.parametrize("per", [5, 10, 15, 19, 20, 21])
+def test_even_rows_fill_whole_turns(ncols, dtype, groups, per):
+    """Segments of several rounds end with a turn of all lane groups that is full or more than half full."""
+    m = 8_000_000 // (per + 1)
+    rp = (torch.arange(m + 1, device="cuda") * per).to(torch.int32)
+    gen = torch.Generator(device="cuda").manual_seed(per)
+    t = torch.float64 if dtype == np.float64 else torch.float32
+    col = ((torch.arange(m, device="cuda")[:, None] + torch.arange(per, device="cuda")) % m).reshape(-1).to(torch.int32)
+    val = torch.randint(-3, 4, (m * per,), device="cuda", generator=gen).to(t)
+    B = torch.randint(-3, 4, (m, ncols), device="cuda", generator=gen).to(t)
+    C = torch.zeros((m, ncols), device="cuda", dtype=t)
+    plan = capi.Plan(True, capi.SPMM_MERGE, t, m, m, m * per, rp, ncols=ncols, col=col, val=val)
+    capi.spmm(rp, col, val, B, C, ncols, 1.0, 0.0, alg=capi.SPMM_MERGE, plan=plan)
+    assert torch.equal(C, (val[:, None] * B[col.long()]).reshape(m, per, ncols).sum(1))
+    turn = groups * 8 * (per + 1)
+    rest = plan.info("segment_items") % turn
+    assert plan.info("shared_segments") == 1 and (rest == 0 or 2 * rest > min(turn, 2688)), (plan.info("segment_items"), turn)
+    plan.destroy()
