@@ -182,7 +182,8 @@ typedef struct asx_plan asx_plan;
 
 /* Builds a plan for SpMV (ncols_dense = 1) or SpMM (ncols_dense = N > 1).  `alg` is one of
  * the ASX_SPMV_* / ASX_SPMM_* values; DEFAULT reads the row-length histogram back (one small
- * synchronous copy) and picks a kernel.  Synchronises `stream` before returning. */
+ * synchronous copy) and picks a kernel.  n: A's columns, which the offsets that planned calls compute with are sized by.
+ * Synchronises `stream` before returning. */
 int asx_plan_create(asx_plan **plan, int is_spmm, int alg, int value_type, int32_t m, int32_t n,
                     int32_t nnz, const int32_t *d_row_ptr, int32_t ncols_dense, void *stream);
 /* SpMM plan that may look at A's columns and values.  alg = ASX_SPMM_BLOCKED re-tiles A into

@@ -268,7 +268,7 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         }
         const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
         const bool chunked = plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T));
-        return launch_spmm_merge<T>(chunked, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
+        return launch_spmm_merge<T>(chunked, plan ? std::max(plan->n, k) : 0, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
                                     (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off), plan ? plan->carry_pass != 0 : true,
                                     spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
     }

@@ -179,7 +179,7 @@ template <typename T>
 int launch_spmm_row(int32_t m, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col,
                     const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s);
 template <typename T>
-int launch_spmm_merge(bool chunked, int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
+int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
                       bool carry_pass, int tile_bytes, hipStream_t s);

@@ -418,12 +418,14 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
 // Rows of B of more than 128 bytes (spmm_chunked_wide says which) come here for another reason: too few waves.  Eight waves deal the
 // segment's rows out, and one of more than 64 elements is cut between them, in which eight rows of B are then in flight a group.
 //
-// NARROW: a row of B is shorter than 4 GB, so that one 32-bit multiply-add into 64 bits finds it, however many rows there are.
-// Offsets of 32 bits, staged in place of columns, would take the same time within 1 % (8 columns fp64, 20 per row within 3000 of
-// the diagonal 54.8 us, 55.3 like this; 25 other cases 0.4 % on average) and could only be right where a caller's k says how far
-// B reaches: no kernel here that works row by row takes k for more than the width of a tile.
-template <typename T, int VEC, int LOGG, bool NARROW>
-__global__ __launch_bounds__(kChunkThreads, NARROW ? 6 : 4) void k_spmm_chunk(
+// How a row of B is found (REACH).  kOffsets: its byte offset is staged in place of the column and fits 32 bits, an add a lane and
+// row of B; a plan says so, whose number of columns is the matrix's own.  kRowsNear: a 32-bit pitch, a multiply-add into 64 bits,
+// however many rows there are: without a plan a caller's k is no more than the width of a tile to the kernels that work
+// row by row.  kRowsFar: rows of B of 4 GB and more.  Planned, 8 M elements within 3000 of the diagonal, kRowsNear and kOffsets: 4
+// columns fp32, 20 per row 27.1 and 25.9 us, 60 24.9 and 22.6; 8 columns fp64, 16 columns fp32 within 1 % of each other.
+enum { kRowsFar = 0, kRowsNear = 1, kOffsets = 2 };
+template <typename T, int VEC, int LOGG, int REACH>
+__global__ __launch_bounds__(kChunkThreads, REACH == kRowsFar ? 4 : 6) void k_spmm_chunk(
     int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
     const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ B, int64_t ldb, T beta, T *__restrict__ C, int64_t ldc,
     const int32_t *__restrict__ xs, const int32_t *__restrict__ ys, T *__restrict__ carry, int32_t *__restrict__ carry_row)
@@ -482,16 +484,18 @@ __global__ __launch_bounds__(kChunkThreads, NARROW ? 6 : 4) void k_spmm_chunk(
             if (j * kChunkThreads < nel) {
                 const int i = j * kChunkThreads + tid;
                 if (i < kChunkElems) {
-                    s_col[i] = tc[j];
+                    s_col[i] = REACH == kOffsets ? (int32_t)((uint32_t)tc[j] * (uint32_t)ldb_bytes) : tc[j];
                     s_val[i] = tv[j];
                 }
             }
     }
     __syncthreads();
 
-    const char *Bc = (const char *)(B + c);
-    const auto row_of_b = [&](int32_t column) -> V {
-        return *(const V *)(Bc + (uint32_t)column * (NARROW ? (uint64_t)(uint32_t)ldb_bytes : ldb_bytes));
+    const uint64_t pitch = REACH == kRowsFar ? ldb_bytes : (uint32_t)ldb_bytes;
+    const uint32_t c_bytes = (uint32_t)c * (uint32_t)sizeof(T);
+    const auto row_of_b = [&](int32_t staged) -> V {
+        return REACH == kOffsets ? *(const V *)((const char *)B + ((uint32_t)staged + c_bytes))
+                                 : *(const V *)((const char *)(B + c) + (uint32_t)staged * pitch);
     };
     const auto together = [&](int32_t k, int32_t e) {  // the sum over the wave's groups, in every group
         V acc = spmm_staged<T, VEC, NG, (NG > 4 ? U / 2 : U)>(k + grp, e, s_col, s_val, row_of_b);
@@ -670,24 +674,26 @@ static void launch_merge_seg(const SpmmTiling &tiling, int32_t m, int32_t nnz, i
                                      xs, ys, carry, carry_row, s);
 }
 
-// As many lanes a group as span the columns.
+// As many lanes a group as span the columns.  rows: of B where a plan knows them, else 0.
 template <typename T>
-static void launch_chunk(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
-                         const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+static void launch_chunk(const SpmmTiling &tiling, int32_t rows, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols,
+                         T alpha, const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
                          const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, hipStream_t s)
 {
     constexpr int kFull = 16 / sizeof(T);
-    const bool narrow = (uint64_t)ldb <= 0xffffffffull / sizeof(T);
+    const dim3 grid((unsigned)(ceil_div64(nseg, kXcds) * kXcds), (unsigned)tiling.tiles);
     const auto launch = [&](auto vec_, auto log_) {
-        const auto with = [&](auto narrow_) {
-            hipLaunchKernelGGL((k_spmm_chunk<T, decltype(vec_)::value, decltype(log_)::value, decltype(narrow_)::value != 0>),
-                               dim3((unsigned)(ceil_div64(nseg, kXcds) * kXcds), (unsigned)tiling.tiles), dim3(kChunkThreads), 0, s, m, nnz, items, nseg, ncols, alpha,
-                               row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);
+        const auto with = [&](auto reach_) {
+            hipLaunchKernelGGL((k_spmm_chunk<T, decltype(vec_)::value, decltype(log_)::value, decltype(reach_)::value>), grid,
+                               dim3(kChunkThreads), 0, s, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
+                               ys, carry, carry_row);
         };
-        if (narrow)
-            with(Int<1>{});
+        if ((uint64_t)ldb > 0xffffffffull / sizeof(T))
+            with(Int<kRowsFar>{});
+        else if (rows > 0 && (uint64_t)rows * (uint64_t)ldb <= 0xffffffffull / sizeof(T))
+            with(Int<kOffsets>{});
         else
-            with(Int<0>{});
+            with(Int<kRowsNear>{});
     };
     if (tiling.vec == kFull) {
         if (tiling.log_lanes == 0)
@@ -715,7 +721,7 @@ static void launch_chunk(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32
 }
 
 template <typename T>
-int launch_spmm_merge(bool chunked, int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
+int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
                       bool carry_pass, int tile_bytes, hipStream_t s)
@@ -726,7 +732,7 @@ int launch_spmm_merge(bool chunked, int32_t m, int32_t nnz, int32_t items, int32
     const int64_t slab = (int64_t)65535 * (tile_bytes / (int64_t)sizeof(T));
     if (ncols > slab) {
         for (int64_t c = 0; c < ncols; c += slab) {
-            const int st = launch_spmm_merge<T>(chunked, m, nnz, items, (int32_t)(ncols - c < slab ? ncols - c : slab), alpha, row_ptr, col, val, B + c,
+            const int st = launch_spmm_merge<T>(chunked, rows, m, nnz, items, (int32_t)(ncols - c < slab ? ncols - c : slab), alpha, row_ptr, col, val, B + c,
                                                 ldb, beta, C + c, ldc, xs, ys, carry, carry_row, carry_pass, tile_bytes, s);
             if (st) return st;
         }
@@ -736,7 +742,7 @@ int launch_spmm_merge(bool chunked, int32_t m, int32_t nnz, int32_t items, int32
     const SpmmTiling tiling = spmm_tiling(ncols, tile_bytes, sizeof(T));
     if (!carry_pass) carry = nullptr, carry_row = nullptr;  // no row is cut: nothing is left for the pass
     if (chunked) {
-        launch_chunk<T>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
+        launch_chunk<T>(tiling, rows, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
     } else {
         const auto launch = [&](auto seg_) {
             launch_merge_seg<T, decltype(seg_)::value>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
@@ -758,7 +764,7 @@ int launch_spmm_merge(bool chunked, int32_t m, int32_t nnz, int32_t items, int32
 #define ASX_INST(T)                                                                                  \
     template int launch_spmm_row<T>(int32_t, int32_t, T, const int32_t *, const int32_t *, const T *, \
                                     const T *, int64_t, T, T *, int64_t, hipStream_t);               \
-    template int launch_spmm_merge<T>(bool, int32_t, int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
+    template int launch_spmm_merge<T>(bool, int32_t, int32_t, int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
                                       const T *, const T *, int64_t, T, T *, int64_t, const int32_t *, \
                                       const int32_t *, T *, int32_t *, bool, int, hipStream_t);
 ASX_INST(float)
