@@ -25,6 +25,7 @@
 // No global atomics; results are bit-reproducible.  The reference has no counterpart (its CSR
 // kernels gather x from global memory: hip/kernel/level2/alphasparse_spmv_csr_vector.h:99-126).
 #include <algorithm>
+#include <type_traits>
 #include <utility>
 
 #include "asx_internal.hpp"
@@ -988,15 +989,24 @@ int launch_spmv_sliced(int32_t m, int32_t n, T alpha, const SlicedMatrix *sm, co
             return ASX_STATUS_INVALID_VALUE;
     }
 #undef ASX_PROD
-    // steps per batch and batches in flight: 4 x 2 measured best (8 x 2, 4 x 4: the same or 1-3 % slower)
-    constexpr int kSteps = 4, kBatches = 2;
-    static_assert((kBatches + 1) * kSteps <= kSlicedStepPad, "descriptors are read this far past a block's last step");
     const int32_t rw = sm->rows_per_wave;
     const size_t lds = align_up(((size_t)rw + kWave) * sizeof(double), 16);
     if (rw < 1 || rw > 32767 || lds > 65536) return ASX_STATUS_INVALID_VALUE;
     const unsigned rgrid = (unsigned)(ceil_div64(sm->nrb, kXcds) * kXcds);
-    hipLaunchKernelGGL((k_sliced_reduce<T, kSteps, kBatches>), dim3(rgrid), dim3(kWave), lds, s, m, sm->nrb, rw, alpha, beta,
-                       sm->pstep_ptr, reinterpret_cast<const i32x4 *>(sm->psteps), sm->prow, partial, y);
+    const auto reduce = [&](auto steps_) {
+        constexpr int kSteps = decltype(steps_)::value, kBatches = 2;
+        static_assert((kBatches + 1) * kSteps <= kSlicedStepPad, "descriptors are read this far past a block's last step");
+        hipLaunchKernelGGL((k_sliced_reduce<T, kSteps, kBatches>), dim3(rgrid), dim3(kWave), lds, s, m, sm->nrb, rw, alpha, beta,
+                           sm->pstep_ptr, reinterpret_cast<const i32x4 *>(sm->psteps), sm->prow, partial, y);
+    };
+    // Steps a batch, two batches in flight.  Blocks of 2048 rows leave 8 waves a compute unit or little more, and each has twice
+    // as many loads in flight for it; of up to 1024 rows 4 x 2 is best (8 x 2 the same or up to 2.5 % slower).  Whole multiply, fp64,
+    // blocks of 2048 rows with 4 and 8 steps, power-law rows of 8, 4.2 M: three matrices in turn 144.0 and 143.1 us, one again
+    // and again 124.9 and 123.4; 7 per row, 4.2 M 176.0 and 175.1, 3.7 M 154.0 and 151.0; 4 per row, 4.2 M 113.4 and 114.2.
+    if (rw > 1024)
+        reduce(std::integral_constant<int, 8>{});
+    else
+        reduce(std::integral_constant<int, 4>{});
     return check_launch();
 }
 

@@ -72,4 +72,8 @@ def test_row_blocks_of_every_size(m, dtype):
     plan = capi.Plan(False, capi.SPMV_SLICED, dtype, m, m, nnz, row_ptr, col=col, val=val)
     capi.spmv(row_ptr, col, val, x, y, 2.0, 0.5, plan=plan)
     assert torch.equal(y, ref)
+    if torch.cuda.get_device_properties(0).multi_processor_count == 256:
+        sizes = {524289: (256, 256), 1048576: (256, 512), 1441793: (512, 1024), 2097153: (512, 1024), 2883585: (1024, 1024),
+                 4194305: (1024, 2048), 5767169: (2048, 2048)}
+        assert plan.info("rows_per_wave") == sizes[m][dtype == torch.float64]
     plan.destroy()
