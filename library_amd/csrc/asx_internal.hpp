@@ -52,7 +52,10 @@ inline bool spmm_chunked_mid(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 // rows of A at a time, where eight waves share them here.  40 such cases of all families, planned or not, take 0.7 of their time
 // (37 columns fp64, 5-point stencil of 26353 elements 12.3 -> 5.6 us; 80 columns fp32, power-law rows of 77812 37.6 -> 18.5; 57,
 // 12543 rows of 5 16.4 -> 8.3); none is slower, except where four groups share rows of more than 32 elements (20 columns fp64, 64
-// per row 8.6 -> 9.6).  Rows of B that start on lines are cut into tiles that keep the merge kernel's groups at work.
+// per row 8.6 -> 9.6).  Not rows of B that end on lines, which are cut into tiles that keep the merge kernel's groups at work: 120 such
+// calls (256, 512 and 1024 bytes, 2000 to 30000 rows of 8 to 20) would take 1.13 times as long on average (128 columns fp32, 6000
+// uniform rows of 12 without a plan 10.7 -> 19.0 us, 12000 planned rows of 20 11.3 -> 12.9), though 18 of power-law rows up to 0.3
+// less (64 columns fp32, 2000 rows of 8 13.2 -> 9.4).
 inline int64_t spmm_chunk_wide_work(int32_t m, int32_t nnz, int64_t row_bytes) { return ((int64_t)m + nnz) * ceil_div64(row_bytes, 512); }
 inline bool spmm_chunked_wide(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
@@ -319,9 +322,11 @@ inline int vector_lanes(int32_t m, int32_t nnz)
 }
 inline int32_t merge_tiles(int32_t m, int32_t nnz) { return (int32_t)ceil_div64((int64_t)m + nnz, kMergeTile); }
 // Without a plan the flat kernel's tiles look up their own rows up to this many tiles; beyond it the search's latency at the
-// start of every workgroup costs more than a launch of its own (4700 tiles 32 us against 35, 16400 104 against 98, 78000 412
-// against 333).
-constexpr int32_t kFlatSelfSearchMost = 8192;
+// start of every workgroup costs more than a launch of its own (12 per row, within 3000 of the diagonal, tiles' own search and the
+// launch: 2000 tiles fp64 16.8 and 17.8 us, fp32 13.3 and 14.7; 4700 28.1 and 28.3, 22.8 and 22.0; 6500 37.7 and 36.4, 28.3 and
+// 27.2; 8192 47.9 and 46.8, 33.3 and 30.8; 16400 91.5 and 87.0, 65.3 and 59.1; scattered columns, fp32 2000 18.3 and 19.1, 8192
+// 53.7 and 50.3).
+constexpr int32_t kFlatSelfSearchMost = 4096;
 inline int32_t flat_tiles(int32_t nnz) { int32_t t = (int32_t)ceil_div64(nnz, kFlatTile); return t < 1 ? 1 : t; }
 inline int32_t stream_blocks(int32_t nnz) { return (int32_t)ceil_div64(nnz, kStreamTile); }
 // What an SpMM plan knows of A's columns: nothing; that neighbouring rows share most of them (stencils, narrow bands); that
