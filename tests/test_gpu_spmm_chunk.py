@@ -109,7 +109,8 @@ def test_offsets_up_to_4_gb(rows):
 @pytest.mark.parametrize("planned", [False, True])
 def test_wide_rows_of_b(dtype, ncols, planned):
     """Every number of lanes a row and one or more tiles of them; rows around what a group, a wave and a segment take, each added to
-    C once; the fewest items a segment holds, the most of one round, and more than a round (where scattered columns still come here)."""
+    C once; the fewest items a segment holds, the most of one round, and more than a round (where only scattered columns come here,
+    so that these run the merge kernel)."""
     rng = np.random.default_rng(ncols)
     edges = [0, 1, 7, 8, 9, 31, 32, 33, 63, 64, 65, 127, 128, 129, 639, 640, 641, 1279, 1281]
     _check(np.r_[rng.integers(0, 12, 300), edges, np.zeros(900, int), rng.permutation(edges), 1500, 1], 500, ncols, dtype, planned, pad=3)
@@ -118,6 +119,29 @@ def test_wide_rows_of_b(dtype, ncols, planned):
     for work in (768 * 128 + 5, 768 * 640 - 9, 768 * 640 + 4000):
         per = 11
         _check(np.r_[np.full(work // turns // (per + 1), per), 700], 3000, ncols, dtype, planned)
+
+
+@pytest.mark.parametrize("dtype,ncols", [(torch.float32, n) for n in (65, 129, 257, 300)] + [(torch.float64, n) for n in (33, 65, 129, 301)])
+@pytest.mark.parametrize("rows", [3000, 60000])
+def test_scattered_columns(dtype, ncols, rows):
+    """DEFAULT's plan for columns that lie all over B: tiles of up to 1 KB, 32 and 64 lanes a row of B, where several rounds of
+    workgroups (60000 rows) come here for the columns alone; rows around what a wave and a segment take, cut ones among them."""
+    k, gen = 200000, torch.Generator(device="cuda").manual_seed(ncols)
+    edges = torch.tensor([0, 1, 7, 8, 9, 63, 64, 65, 127, 128, 129, 511, 512, 513, 639, 640, 641, 1281, 5000])
+    lens = torch.cat([torch.randint(4, 15, (rows,), generator=torch.Generator().manual_seed(rows)), edges, torch.zeros(700, dtype=torch.int64), edges])
+    rp = torch.cat([torch.zeros(1, dtype=torch.int64), lens.cumsum(0)]).to(torch.int32).cuda()
+    m, nnz = lens.numel(), int(lens.sum())
+    col = torch.randint(0, k, (nnz,), device="cuda", generator=gen, dtype=torch.int32)
+    draw = lambda *shape: torch.randint(-3, 4, shape, device="cuda", generator=gen).to(dtype)
+    val, B, C = draw(nnz), draw(k, ncols), 2 * draw(m, ncols)
+    row = torch.repeat_interleave(torch.arange(m, device="cuda"), lens.cuda())
+    ref = 2 * torch.zeros_like(C).index_add_(0, row, val[:, None] * B[col.long()]) + 0.5 * C
+    plan = capi.Plan(True, capi.SPMM_DEFAULT, dtype, m, k, nnz, rp, ncols=ncols, col=col, val=val)
+    capi.spmm(rp, col, val, B, C, ncols, 2.0, 0.5, plan=plan)
+    assert torch.equal(C, ref)
+    several = (m + nnz) * -(-ncols * val.element_size() // 512) > 768 * 640
+    assert plan.info("shared_segments") == 1 and several == (rows == 60000)
+    plan.destroy()
 
 
 @pytest.mark.parametrize("dtype,ncols", [(np.float32, n) for n in (9, 12, 17, 25, 32)] + [(np.float64, n) for n in (5, 6, 10, 13, 16)])
