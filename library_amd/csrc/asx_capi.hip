@@ -268,8 +268,9 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         }
         const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
         const bool chunked = plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T));
-        return launch_spmm_merge<T>(chunked, plan ? std::max(plan->n, k) : 0, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys,
-                                    (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off), plan ? plan->carry_pass != 0 : true,
+        return launch_spmm_merge<T>(chunked, plan ? std::max(plan->n, k) : 0, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb,
+                                    beta, C, ldc, xs, ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
+                                    plan ? plan->carry_pass != 0 : true,
                                     spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
     }
     case ASX_SPMM_BLOCKED:
@@ -504,10 +505,9 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             // does any row stay cut?  (one int read back; creation syncs anyway)
             if (!st) st = launch_spmm_splits(m, nnz, p->items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
             if (!st) st = read_flag();
-            if (st || p->items >= usual || !p->carry_pass) return st;
+            if (st || p->items >= usual || !p->carry_pass) return st;  // the chunk kernel's segments hold usual or more
             pool_free(p->d_meta, true);  // read_flag has waited; the flag stays set, so that the carry pass runs
             p->d_meta = nullptr;
-            p->chunked = spmm_chunked(m, nnz, p->ncols, sv);
         }
     }
     if (!st) st = status_of(hipStreamSynchronize(s));
@@ -647,7 +647,11 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
 // histogram, the sizes, the column sample), never from timings: two analyses of one matrix keep the
 // same kernel.  Estimated times, fitted to 306 matrices timed with every kernel on MI355X, three copies
 // of each in turn (uniform, power-law, banded, near-diagonal rows and stencils of 60 000 to 32 M stored
-// elements in both types; the kernel chosen is on average 2.4 % behind the fastest).  In microseconds, with
+// elements in both types).  The rates are of kernels whose gathers were not yet issued together behind a barrier (stream, flat
+// and merge take 0.7 to 0.9 of these times on some matrices since); of 100 matrices drawn from the same families and timed
+// with the kernels as they are, the one chosen is the fastest, or within 3 %, for 89, and on average 2.3 % behind it: six of
+// the others have a stream kernel that is faster than estimated (12 per row within 324 of the diagonal, 4.4 M, fp64: window 20.4
+// us, stream 15.3; 25 per row within 3592, 1.1 M, fp32: vector 7.0, stream 5.7).  In microseconds, with
 //   gathers(r) = nnz spread' / r thousand, r falling to 62 while x grows from 3 to 6 MB (an L2 holds 4);
 //                spread' = the sample's spread, at least 0.05 (neighbouring columns share a line)
 //   bytes      = nnz (sv + 4) + n sv + m (sv + 4)
@@ -790,12 +794,16 @@ static int plan_long_rows(asx_plan *p, hipStream_t s)
 // pass 2: one wave per block of rows, its accumulators (8 bytes a row) in LDS.  Small blocks mean many waves in flight, large
 // ones long ranges of partial sums inside a slice, fewer lines of which only a part is wanted, and full steps (a step
 // takes its 64 entries from at most three ranges).  Blocks of 256 rows, doubled while either holds:
-//   up to 1024, if that leaves more than 4 waves a compute unit and the ranges (expected from the column sample) are
+//   up to 1024, if that leaves at least 4 waves a compute unit and the ranges (expected from the column sample) are
 //     shorter than 12 entries;
 //   up to 2048, if it leaves 8 waves a compute unit in fp64, 11 in fp32, and the ranges are shorter than 48 entries.
 // Four matrices in turn, whole multiply: power-law rows, 4.2 M x 4.2 M, 33 M elements, fp64 163 us with 1024 rows, 152 with 2048,
 // 170 with 4096; 7 per row, 4.2 M fp64 254 / 204 / 182 / 172 / 200 us with 256 / 512 / 1024 / 2048 / 4096, fp32 125 / 109 /
 // 100 / 109 with 256 / 512 / 1024 / 2048; 1.5 M fp64 73 / 69 / 72 / 87, fp32 46 / 45 / 52; 16 per row of 1 M, fp32 51 / 57.
+// Around the line in fp64 (4.19 M rows; steps as launch_spmv_sliced takes them), 1024 and 2048 rows, three matrices in turn and
+// one again and again: power-law rows of 8, 3.3 M 118.3 and 115.0, 100.5 and 103.2; 3.7 M 134.3 and 128.8, 113.0 and 116.1; 4.19 M
+// 153.8 and 143.1, 121.8 and 123.4; 7 per row, 3.3 M 143.1 and 136.0, 130.5 and 126.6; 3.7 M 159.8 and 151.0, 150.7 and 141.3; 4.19 M
+// 186.0 and 175.1, 181.1 and 169.2; 5 per row, 3.0 M 99.9 and 95.2, 83.5 and 85.7.
 static int32_t sliced_rows_per_wave(const asx_plan *p, size_t sv, double pairs_per_element, int cus)
 {
     const double per_row_slice = pairs_per_element * (double)p->nnz / ((double)p->m * (double)slice_count(p, sv));

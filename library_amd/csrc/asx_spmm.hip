@@ -732,8 +732,9 @@ int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_
     const int64_t slab = (int64_t)65535 * (tile_bytes / (int64_t)sizeof(T));
     if (ncols > slab) {
         for (int64_t c = 0; c < ncols; c += slab) {
-            const int st = launch_spmm_merge<T>(chunked, rows, m, nnz, items, (int32_t)(ncols - c < slab ? ncols - c : slab), alpha, row_ptr, col, val, B + c,
-                                                ldb, beta, C + c, ldc, xs, ys, carry, carry_row, carry_pass, tile_bytes, s);
+            const int32_t wide = (int32_t)(ncols - c < slab ? ncols - c : slab);
+            const int st = launch_spmm_merge<T>(chunked, rows, m, nnz, items, wide, alpha, row_ptr, col, val, B + c, ldb, beta, C + c,
+                                                ldc, xs, ys, carry, carry_row, carry_pass, tile_bytes, s);
             if (st) return st;
         }
         return ASX_STATUS_SUCCESS;
@@ -745,8 +746,8 @@ int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_
         launch_chunk<T>(tiling, rows, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, s);
     } else {
         const auto launch = [&](auto seg_) {
-            launch_merge_seg<T, decltype(seg_)::value>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
-                                                       carry_row, s);
+            launch_merge_seg<T, decltype(seg_)::value>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
+                                                       xs, ys, carry, carry_row, s);
         };
         if (items <= kSpmmSegmentSmall)
             launch(Int<kSpmmSegmentSmall>{});

@@ -60,9 +60,12 @@ inline bool use_nontemporal(int64_t nnz, size_t sv)
 // order: gathers that an L2 could serve wait behind every stored element still on its way from memory, so the fewer times
 // the two meet the better (gathers of 64-byte rows from an L2 beside a stream from memory: 175 G/s wave by wave, 217 behind
 // barriers, 259 without the stream).  8.4 M elements within 50000 of the diagonal, fp64, stream kernel: 58.3 us without the
-// barrier, 50.9 with it; 12 M scattered ones 72.1 and 59.6 (x of 1.8 MB), 95.7 and 93.9 (x of 6 MB).  Up to
-// one round of workgroups (eight on each of 256 compute units) all of them load and then gather anyway, and the
-// barrier costs 0.1 us.
+// barrier, 50.9 with it; 12 M scattered ones 72.1 and 59.6 (x of 1.8 MB), 95.7 and 93.9 (x of 6 MB).  With few workgroups
+// most load and then gather at the same time anyway.  The line is a measured one for all three kernels, of which six to eight
+// workgroups fit a compute unit (16 per row within 20000 of the diagonal, without the barrier and with it: stream fp32 1200
+// workgroups 7.83 and 7.82, 2040 11.59 and 11.57, 2300 12.93 and 12.48, 3400 17.31 and 16.83 us; fp64 1200 9.08 and 9.31, 2300
+// 14.86 and 14.60; flat within 1 % up to 3400; merge fp64 1200 19.1 and 19.5, 2300 29.3 and 29.9, 2800 33.9 and 34.5, 3400 43.4 and
+// 40.7).
 constexpr unsigned kBunchedTiles = 2048;
 template <int N, typename T>
 __device__ __forceinline__ void wait_for_elements(const int32_t (&c)[N], const T (&v)[N])
