@@ -418,11 +418,13 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
 // Rows of B of more than 128 bytes (spmm_chunked_wide says which) come here for another reason: too few waves.  Eight waves deal the
 // segment's rows out, and one of more than 64 elements is cut between them, in which eight rows of B are then in flight a group.
 //
-// How a row of B is found (REACH).  kOffsets: its byte offset is staged in place of the column and fits 32 bits, an add a lane and
-// row of B; a plan says so, whose number of columns is the matrix's own.  kRowsNear: a 32-bit pitch, a multiply-add into 64 bits,
-// however many rows there are: without a plan a caller's k is no more than the width of a tile to the kernels that work
-// row by row.  kRowsFar: rows of B of 4 GB and more.  Planned, 8 M elements within 3000 of the diagonal, kRowsNear and kOffsets: 4
-// columns fp32, 20 per row 27.1 and 25.9 us, 60 24.9 and 22.6; 8 columns fp64, 16 columns fp32 within 1 % of each other.
+// How a row of B is found (REACH).  kRowsNear: a 32-bit pitch, a multiply-add into 64 bits, however many rows there are: without a
+// plan a caller's k is no more than the width of a tile to the kernels that work row by row.  kRowsFar: rows of B of 4 GB and
+// more.  kOffsets: where a lane takes a whole row of B, its byte offset is staged in place of the column and fits 32 bits; a
+// plan says so, whose number of columns is the matrix's own.  Registers for eight of them in flight then leave room for
+// four workgroups a compute unit in fp32.  Planned, 8 M elements within 3000 of the diagonal, kRowsNear and kOffsets: 4 columns fp32, 8 per
+// row 40.9 and 37.4 us, 16 29.8 and 28.0, 60 23.7 and 22.8; 2 columns fp64 within 2 %; wider rows of B no faster (8 columns fp64, 20 per
+// row 53.7 and 54.9, 40 53.7 and 54.7).
 enum { kRowsFar = 0, kRowsNear = 1, kOffsets = 2 };
 template <typename T, int VEC, int LOGG, int REACH>
 __global__ __launch_bounds__(kChunkThreads, REACH == kRowsFar ? 4 : 6) void k_spmm_chunk(
@@ -432,7 +434,10 @@ __global__ __launch_bounds__(kChunkThreads, REACH == kRowsFar ? 4 : 6) void k_sp
 {
     typedef typename VecOf<T, VEC>::type V;
     constexpr int G = 1 << LOGG, NG = kWave / G;
-    constexpr int U = 8;  // rows of B a lane has in flight
+    // Rows of B a lane has in flight.  Where a lane takes a whole one, fp32, six of them and their 64-bit addresses leave room for the
+    // registers of four workgroups a compute unit, eight of three (no plan, 4 columns, 20 per row 49.7 us with eight, 44.1 with six,
+    // 43.9 with four; 40 per row 50.1, 47.2, 47.1; 60 52.9, 48.2, 50.9).
+    constexpr int U = REACH == kRowsNear && sizeof(T) == 4 && VEC == 4 && LOGG == 0 ? 6 : 8;
     constexpr int kWide = NG > 4 ? 256 : 64;  // longer rows are taken by all waves (elements)
     constexpr int kDealt = spmm_dealt(NG) < kWide ? spmm_dealt(NG) : kWide;
     constexpr int kWaves = kChunkThreads / kWave, NE = (kChunkElems + kChunkThreads - 1) / kChunkThreads;
@@ -688,10 +693,10 @@ static void launch_chunk(const SpmmTiling &tiling, int32_t rows, int32_t m, int3
                                dim3(kChunkThreads), 0, s, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs,
                                ys, carry, carry_row);
         };
+        if constexpr (decltype(log_)::value == 0)
+            if (rows > 0 && (uint64_t)rows * (uint64_t)ldb <= 0xffffffffull / sizeof(T)) return with(Int<kOffsets>{});
         if ((uint64_t)ldb > 0xffffffffull / sizeof(T))
             with(Int<kRowsFar>{});
-        else if (rows > 0 && (uint64_t)rows * (uint64_t)ldb <= 0xffffffffull / sizeof(T))
-            with(Int<kOffsets>{});
         else
             with(Int<kRowsNear>{});
     };

@@ -86,22 +86,24 @@ def test_view_of_a_matrix_beyond_4_gb(planned, k):
         plan.destroy()
 
 
+@pytest.mark.parametrize("ncols", [4, 8])
 @pytest.mark.parametrize("rows", [(1 << 24) - 1, 1 << 24])
-def test_offsets_up_to_4_gb(rows):
-    """Rows of 256 bytes up to 2^32 - 256 bytes, whose offsets a planned call holds in 32 bits, and one row more."""
+def test_offsets_up_to_4_gb(rows, ncols):
+    """Rows of 256 bytes up to 2^32 - 256 bytes, whose offsets a planned call holds in 32 bits where a lane takes 4 columns, and one
+    row more; the same with 8 columns, which it multiplies out."""
     m = 30000
     gen = torch.Generator(device="cuda").manual_seed(7)
     B = torch.empty((rows, 64), device="cuda")
-    B[:, 56:].copy_(torch.randint(-3, 4, (rows, 8), device="cuda", generator=gen, dtype=torch.int8))
+    B[:, -ncols:].copy_(torch.randint(-3, 4, (rows, ncols), device="cuda", generator=gen, dtype=torch.int8))
     rp = (torch.arange(m + 1, device="cuda") * 12).to(torch.int32)
     col = torch.randint(0, rows, (m * 12,), device="cuda", generator=gen, dtype=torch.int32)
     col[::7] = rows - 1
     val = torch.randint(-3, 4, (m * 12,), device="cuda", generator=gen).float()
-    C = torch.zeros((m, 8), device="cuda")
-    plan = capi.Plan(True, capi.SPMM_DEFAULT, val.dtype, m, rows, col.numel(), rp, ncols=8, col=col, val=val)
-    capi.spmm(rp, col, val, B[:, 56:], C, 8, 1.0, 0.0, plan=plan, ldb=64, ldc=8)
+    C = torch.zeros((m, ncols), device="cuda")
+    plan = capi.Plan(True, capi.SPMM_DEFAULT, val.dtype, m, rows, col.numel(), rp, ncols=ncols, col=col, val=val)
+    capi.spmm(rp, col, val, B[:, -ncols:], C, ncols, 1.0, 0.0, plan=plan, ldb=64, ldc=ncols)
     assert plan.info("shared_segments") == 1
-    assert torch.equal(C, (val[:, None] * B[:, 56:][col.long()]).reshape(m, 12, 8).sum(1))
+    assert torch.equal(C, (val[:, None] * B[:, -ncols:][col.long()]).reshape(m, 12, ncols).sum(1))
     plan.destroy()
 
 
