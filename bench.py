@@ -56,7 +56,7 @@ MEASURED_TRAFFIC_BYTES = {
     "banded_f64": 457_318,  # profiles/spmv_vector_banded_f64.md
     "uniform16_f32": 256_479_642,  # profiles/spmv_sliced_uniform16_f32.md
     "uniform16_f64": 478_002_995,  # profiles/spmv_sliced_uniform16_f64.md
-    "powerlaw_f64": 730_648_883,  # profiles/spmv_sliced_powerlaw_f64.md
+    "powerlaw_f64": 729_508_659,  # profiles/spmv_sliced_powerlaw_f64.md
     "stencil5_f64": 1_142_514_688,  # profiles/spmv_window_stencil5_f64.md
     "spmm_zipf_f32": 4_923_132_211,  # profiles/spmm_merge_spmm_zipf_f32.md
     "spmm_banded_f32": 1_277_375_283,  # profiles/spmm_blocked_spmm_banded_f32.md
