@@ -91,12 +91,21 @@ inline int32_t spmm_chunk_wide_items(int64_t work)
     const int64_t rounds = ceil_div64(work, kChunkRound * kChunkItemsWide), items = ceil_div64(work, kChunkRound * rounds);
     return (int32_t)(items < kSpmmSegmentSmall ? kSpmmSegmentSmall : items);
 }
-// One round, if its segments are neither short (448 to 896 items are alike up
+// Where rows may be cut: one round, if its segments are neither short (448 to 896 items are alike up
 // to 500000 items; at 1 M 896 take 20 % longer than 1344) nor more than a workgroup can stage.
-inline int32_t spmm_chunk_items(int64_t items, int32_t most = kChunkItems)
+inline int32_t spmm_chunk_items(int64_t items)
 {
-    const int64_t round = ceil_div64(items, kChunkRound);
-    return (int32_t)(round < kChunkItems / 2 ? kChunkItems / 2 : round > most ? most : round);
+    return (int32_t)std::min<int64_t>(std::max<int64_t>(ceil_div64(items, kChunkRound), kChunkItems / 2), kChunkItems);
+}
+// Where a plan knows that none is: segments that fill one round of workgroups or two, with more rounds the longest.  A round that is
+// only begun leaves the chip idle: 16 per row, 2.0 M elements within 20000 of the diagonal, in 800 workgroups and in 1536 (3 columns
+// fp64 17.3 and 15.2 us, 8 fp32 15.7 and 14.0); 12 per row, 2.6 M (4 columns fp64 19.6 and 18.3); 66 such cases of 2 and 2.6 M
+// elements 3 % faster on average, of 4 M and more alike.
+inline int32_t spmm_chunk_uncut_items(int64_t items)
+{
+    const int64_t rounds = std::max<int64_t>(ceil_div64(items, kChunkRound * kChunkItemsMost), 1);
+    if (rounds > 2) return kChunkItemsMost;
+    return (int32_t)std::max<int64_t>(ceil_div64(items, kChunkRound * rounds), kChunkItems / 2);
 }
 constexpr double kScatteredMinSpread = 0.5;  // of a column sample: from here on the columns count as scattered
 
@@ -402,11 +411,13 @@ constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 
 // 64 columns fp32, 20 per row within 1000 of the diagonal: 94.9 us with segments of 512 items, 54.2 with two turns of 84;
 // 7-point stencil 78.7 -> 59.7, 5-point stencil 128.7 -> 85.7; 13 per row 50.2 -> 42.3.
 // Chunk kernel: where rows are too long for the longest segments, but none for one of the usual length, no row is cut (a carry
-// pass is a launch more: longest row 913 of 82000 elements 8.8 -> 5.9 us).  Even rows fill whole turns of all groups of a workgroup:
-// one more where it fits, else without a last turn that would not be half full (8 columns fp64 within 3000 of the diagonal, 8 M
-// elements, full turns against segments of 2688 items: 15 per row 62.1 against 66.5 us, 17 59.5 and 64.3, 19 57.7 and 61.7, 20
-// alike, as 2688 is one turn; 16 columns fp32, 19 per row 54.2 and 56.0; last turns that are half full or more are kept: 10 per
-// row 71.9 without and 68.7 with).  Wide rows of B (row_bytes): never more segments than usual, so that their carries fit.
+// pass is a launch more: longest row 913 of 82000 elements 8.8 -> 5.9 us).  In more than two rounds even rows do without a last turn
+// of a workgroup's groups that would not be half full (8 columns fp64 within 3000 of the diagonal, 8 M elements, whole turns against
+// segments of 2688 items: 15 per row 62.1 against 66.5 us, 17 59.5 and 64.3, 19 57.7 and 61.7; 16 columns fp32, 19 per row 54.2
+// and 56.0; a last turn that is half full is kept: 10 per row 71.9 without and 68.7 with), in one or two without one of a sixteenth
+// (5 per row, 6 columns fp32, 2 M 20.0 -> 18.1).  Rounding up would make fewer and longer segments: 9 per row, 350000 elements, 3
+// columns fp64 152 workgroups 7.0 us, 579 6.2; 5 per row, 8 fp32 7.6 and 6.5; 9 per row, 3 columns fp64, 800000 10.3 and 8.9, 1.4 M
+// 14.2 and 13.0.  Wide rows of B (row_bytes): never more segments than usual, so that their carries fit.
 inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest, bool chunked,
                                int64_t row_bytes)
 {
@@ -414,12 +425,10 @@ inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m
     if (chunked && row_bytes > 64) return std::max(usual, spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, row_bytes)));
     if (chunked) {
         if (longest > kChunkLongest) return longest > kChunkItems || longest <= usual ? usual : (int32_t)longest;  // usual <= kChunkItems
-        const int32_t items = spmm_chunk_items((int64_t)m + nnz, kChunkItemsMost);
+        const int32_t items = spmm_chunk_uncut_items((int64_t)m + nnz);
         if (4 * (longest + 1) * m > 5 * ((int64_t)m + nnz)) return items;
         const int64_t turn = (int64_t)groups * (kChunkThreads / kWave) * (longest + 1), over = items % turn;
-        const int64_t more = ceil_div64(items, turn) * turn;
-        if (more <= kChunkItemsMost) return (int32_t)more;
-        return items == kChunkItemsMost && turn <= items && 2 * over <= turn ? (int32_t)(items - over) : items;
+        return turn <= items && (items < kChunkItemsMost ? 16 : 2) * over <= turn ? (int32_t)(items - over) : items;
     }
     if (columns != kColumnsNear && columns != kColumnsSpread) return usual;
     const int32_t least = usual == kSpmmSegmentLarge ? kSpmmSegmentSmall : usual;

@@ -225,3 +225,26 @@ def test_even_rows_fill_whole_turns(ncols, dtype, groups, per):
     rest = plan.info("segment_items") % turn
     assert plan.info("shared_segments") == 1 and (rest == 0 or 2 * rest > min(turn, 2688)), (plan.info("segment_items"), turn)
     plan.destroy()
+
+
+@pytest.mark.parametrize("dtype,ncols", [(torch.float64, 3), (torch.float32, 8)])
+@pytest.mark.parametrize("per,rows,rounds", [(9, 38904, 1), (8, 62000, 1), (16, 121000, 1), (16, 125000, 2), (9, 412000, 2)])
+def test_segments_fill_whole_rounds(dtype, ncols, per, rows, rounds):
+    """One round of workgroups or two, three a compute unit, whatever whole turns of their lane groups take of even rows."""
+    rp = (torch.arange(rows + 1, device="cuda") * per).to(torch.int32)
+    gen = torch.Generator(device="cuda").manual_seed(per)
+    col = torch.randint(0, rows, (rows * per,), device="cuda", generator=gen, dtype=torch.int32)
+    val = torch.randint(-3, 4, (rows * per,), device="cuda", generator=gen).to(dtype)
+    B = torch.randint(-3, 4, (rows, ncols), device="cuda", generator=gen).to(dtype)
+    C = torch.zeros((rows, ncols), device="cuda", dtype=dtype)
+    plan = capi.Plan(True, capi.SPMM_DEFAULT, dtype, rows, rows, rows * per, rp, ncols=ncols, col=col, val=val)
+    ref = (val[:, None] * B[col.long()]).reshape(rows, per, ncols).sum(1)
+    for p in (plan, None):
+        C.fill_(-1)
+        capi.spmm(rp, col, val, B, C, ncols, 1.0, 0.0, plan=p)
+        assert torch.equal(C, ref)
+    total = rows * (per + 1)
+    assert plan.info("shared_segments") == 1
+    filled = max(672, -(-total // (768 * rounds)))
+    assert 15 * filled <= 16 * plan.info("segment_items") <= 16 * filled  # without a last turn of a sixteenth
+    plan.destroy()
