@@ -32,13 +32,25 @@ constexpr int kChunkItems = 1344, kChunkItemsMost = 2688, kChunkLongest = kChunk
 constexpr int kChunkItemsWide = 640;      // the most where rows of B are wide
 constexpr int64_t kChunkRound = 768;      // three workgroups on each of 256 compute units
 static_assert(2 * kChunkItems <= kChunkElems && kChunkItemsMost < kChunkRows, "a segment fits what is staged");
-// Which calls it takes.  Rows of B of up to 32 bytes, planned or not, unless rows of A are short: 66 such cases of all families 9 %
+// Which calls it takes.  Rows of B of up to 32 bytes unless rows of A are short: 66 such cases of all families 9 %
 // faster on average (3 columns fp64, 56 per row 16.7 -> 7.4 us; 2 columns fp32, 5 per row 21.0 -> 16.0), but with 4 per row,
-// 2 columns fp32 8.2 -> 10.1, with 7, 3 columns fp64 4.7 -> 5.1.  What it takes beside these: spmm_chunked_mid, spmm_chunked_wide
-// and, under plans only, spmm_plan_chunked.
+// 2 columns fp32 8.2 -> 10.1, with 7, 3 columns fp64 4.7 -> 5.1.  spmm_chunked_unplanned and spmm_plan_chunked say when; what it
+// takes beside these: spmm_chunked_mid, spmm_chunked_wide.
 inline bool spmm_chunked_narrow(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
     return ncols * (int64_t)sv <= 32 && 2 * (int64_t)nnz >= (sv == 4 ? 9 : 16) * (int64_t)m;
+}
+// One round of workgroups takes all of A: then in any case (8 to 50 per row, 0.5 to 1 M items, both types: merge takes 1 to 2.2 times
+// as long).  With more rounds only where a plan knows that no row of A is long: rows that are cut leave carries, and segments
+// of few long rows have no work for most lane groups (planned, power-law rows of up to 4000: 4 columns fp64, 14 per row, 3 M items
+// 39.6 us with merge, 43.4 here; 45 per row, 5 M 50.7 and 66.3; 8 fp32 44.6 and 62.0; 2 fp64, 25 per row, 8 M 86.7 and 109.8), and
+// without a plan every workgroup looks its segment up before it loads any of it (1.1 to 5 M items, 8 to 20 per row: merge takes
+// 0.84 to 1.01 of the time for 3 columns fp64, 0.81 to 1.01 for 8 fp32, 0.82 to 1.03 for 2 fp64).  Rows of B of up to 16 bytes in fp32
+// come here all the same: merge takes 0.9 to 1.4 of the time with 8 to 30 per row, 1.2 to 1.7 with 50, 0.9 to 1.3 with power-law rows.
+inline bool spmm_chunk_one_round(int32_t m, int32_t nnz) { return (int64_t)m + nnz <= kChunkRound * kChunkItems; }
+inline bool spmm_chunked_unplanned(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
+{
+    return spmm_chunked_narrow(m, nnz, ncols, sv) && (spmm_chunk_one_round(m, nnz) || (sv == 4 && ncols <= 4));
 }
 // Rows of B of 33 to 128 bytes while one round of workgroups takes all of A, planned or not: 57 such cases of all families 6 %
 // faster on average (7 columns fp64, 61 per row, 462624 elements 12.1 -> 8.1 us; 31 fp32, 5-point stencil of 642649 14.4 -> 11.9;
@@ -46,7 +58,7 @@ inline bool spmm_chunked_narrow(int32_t m, int32_t nnz, int64_t ncols, size_t sv
 // alike (18 columns fp32 27.3 -> 29.6, 12 columns fp64 86.8 -> 83.0).
 inline bool spmm_chunked_mid(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
-    return ncols * (int64_t)sv > 32 && ncols * (int64_t)sv <= 128 && (int64_t)m + nnz <= kChunkRound * kChunkItems;
+    return ncols * (int64_t)sv > 32 && ncols * (int64_t)sv <= 128 && spmm_chunk_one_round(m, nnz);
 }
 // Wider rows of B while one round of workgroups takes all of A: the merge kernel's few waves then walk 128 items each, one or two
 // rows of A at a time, where eight waves share them here.  40 such cases of all families, planned or not, take 0.7 of their time
@@ -63,9 +75,9 @@ inline bool spmm_chunked_wide(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
     return bytes > 128 && bytes % 128 != 0 && (bytes > 256 || nnz <= 32 * (int64_t)m) &&
            spmm_chunk_wide_work(m, nnz, bytes) <= kChunkRound * kChunkItemsWide;
 }
-inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
+inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)  // without a plan
 {
-    return spmm_chunked_narrow(m, nnz, ncols, sv) || spmm_chunked_mid(m, nnz, ncols, sv) || spmm_chunked_wide(m, nnz, ncols, sv);
+    return spmm_chunked_unplanned(m, nnz, ncols, sv) || spmm_chunked_mid(m, nnz, ncols, sv) || spmm_chunked_wide(m, nnz, ncols, sv);
 }
 // Under a plan also rows of B of up to 64 bytes (those of up to 32 that spmm_chunked_narrow leaves out among them) where no row of A
 // is long, rows hold 3.5 elements or more on average, and there are several rounds of workgroups (16 columns fp32, 23 per row,
@@ -80,7 +92,8 @@ inline bool spmm_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 // 248 49.1 -> 50.5).
 inline bool spmm_plan_chunked(int32_t m, int32_t nnz, int64_t ncols, size_t sv, int64_t longest, bool scattered, int tile_lanes)
 {
-    if (spmm_chunked(m, nnz, ncols, sv)) return true;
+    if (spmm_chunked(m, nnz, ncols, sv)) return true;  // a plan's segments are never more than a call's without one
+    if (spmm_chunked_narrow(m, nnz, ncols, sv)) return longest <= kChunkLongest;
     if (ncols * (int64_t)sv <= 64)
         return longest <= kChunkLongest && 2 * (int64_t)nnz >= 7 * (int64_t)m && (int64_t)m + nnz >= 4000000;
     return scattered && tile_lanes >= 32;
@@ -377,7 +390,7 @@ inline int spmm_columns(double spread, double span, double mean, size_t sv)
 inline int32_t spmm_segment_items(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
 {
     const int64_t items = (int64_t)m + nnz;
-    if (spmm_chunked_narrow(m, nnz, ncols, sv)) return spmm_chunk_items(items);
+    if (spmm_chunked_unplanned(m, nnz, ncols, sv)) return spmm_chunk_items(items);
     if (spmm_chunked_mid(m, nnz, ncols, sv)) return (int32_t)std::max<int64_t>(kSpmmSegmentMedium, ceil_div64(items, kChunkRound));
     if (spmm_chunked_wide(m, nnz, ncols, sv)) return spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, ncols * (int64_t)sv));
     if (items < (int64_t)kSpmmSegmentMedium * 4096) return kSpmmSegmentSmall;
@@ -424,7 +437,8 @@ inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m
     if (chunked && spmm_chunked_mid(m, nnz, row_bytes, 1)) return usual;
     if (chunked && row_bytes > 64) return std::max(usual, spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, row_bytes)));
     if (chunked) {
-        if (longest > kChunkLongest) return longest > kChunkItems || longest <= usual ? usual : (int32_t)longest;  // usual <= kChunkItems
+        const int32_t cut = spmm_chunk_items((int64_t)m + nnz);  // usual or more
+        if (longest > kChunkLongest) return longest > kChunkItems || longest <= cut ? cut : (int32_t)longest;
         const int32_t items = spmm_chunk_uncut_items((int64_t)m + nnz);
         if (4 * (longest + 1) * m > 5 * ((int64_t)m + nnz)) return items;
         const int64_t turn = (int64_t)groups * (kChunkThreads / kWave) * (longest + 1), over = items % turn;

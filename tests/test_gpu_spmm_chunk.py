@@ -248,3 +248,22 @@ def test_segments_fill_whole_rounds(dtype, ncols, per, rows, rounds):
     filled = max(672, -(-total // (768 * rounds)))
     assert 15 * filled <= 16 * plan.info("segment_items") <= 16 * filled  # without a last turn of a sixteenth
     plan.destroy()
+
+
+@pytest.mark.parametrize("ncols,dtype", [(2, np.float64), (4, np.float64), (8, np.float32), (4, np.float32)])
+@pytest.mark.parametrize("rows,per", [(60000, 16), (62000, 16), (130000, 16), (30000, 45)])
+def test_long_rows_and_no_plan_around_one_round(ncols, dtype, rows, per):
+    """Rows that are cut, with a plan and without: one round of workgroups goes to whole workgroups, more to the waves unless rows of B
+    hold 4 columns fp32 at most."""
+    lens = np.full(rows, per)
+    lens[::997] = 4000
+    total = rows + int(lens.sum())
+    for planned in (True, False):
+        _check(lens, 5000, ncols, dtype, planned)
+    rp = torch.from_numpy(np.r_[0, np.cumsum(lens)].astype(np.int32)).cuda()
+    col = torch.zeros(int(lens.sum()), dtype=torch.int32, device="cuda")
+    val = torch.zeros(col.numel(), dtype=torch.float64 if dtype == np.float64 else torch.float32, device="cuda")
+    plan = capi.Plan(True, capi.SPMM_MERGE, val.dtype, rows, 5000, col.numel(), rp, ncols=ncols, col=col, val=val)
+    assert plan.info("shared_segments") == int(total <= 768 * 1344 or (dtype == np.float32 and ncols <= 4))
+    assert plan.info("shared_segments") or plan.info("segment_items") <= 512
+    plan.destroy()
