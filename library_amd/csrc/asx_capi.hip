@@ -505,7 +505,7 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
             // does any row stay cut?  (one int read back; creation syncs anyway)
             if (!st) st = launch_spmm_splits(m, nnz, p->items, d_row_ptr, p->d_meta, p->d_meta + (ns + 1), d_flag, s);
             if (!st) st = read_flag();
-            if (st || p->items >= usual || !p->carry_pass) return st;  // the chunk kernel's segments hold usual or more
+            if (st || p->items >= usual || !p->carry_pass) return st;  // the chunk kernel's hold usual or more, or cut no row
             pool_free(p->d_meta, true);  // read_flag has waited; the flag stays set, so that the carry pass runs
             p->d_meta = nullptr;
         }
