@@ -283,7 +283,8 @@ enum {
                                          stored elements, so the stored elements of a tile are consecutive in A's val, which
                                          every call reads in place; asx_plan_holds_values is 0 then) */
     ASX_PLAN_INFO_SEGMENT_ITEMS = 15,   /* rows and stored elements, added up, of a segment (SpMM, row-ordered) */
-    ASX_PLAN_INFO_SHARED_SEGMENTS = 16  /* 1 when a workgroup shares a segment, 0 when a wave takes it (SpMM, row-ordered) */
+    ASX_PLAN_INFO_SHARED_SEGMENTS = 16, /* 1 when a workgroup shares a segment, 0 when a wave takes it (SpMM, row-ordered) */
+    ASX_PLAN_INFO_SWEEP = 17            /* 1 when all waves go through the columns of A together (SpMM, row-ordered) */
 };
 int64_t asx_plan_info(const asx_plan *plan, int what);
 /* Frees the buffer a sliced or window plan keeps for the partial sums / carries of a call.  Calls

@@ -313,7 +313,9 @@ __global__ __launch_bounds__(256) void k_copy16(const u32x4 *__restrict__ src, u
 // touch (col >> shift entered into a hash table in LDS: 4096 slots, linear probing).  With
 // row_ptr given also out[64 + t] = number of (row, slice) pairs among the tile's elements, slices
 // of `width` columns: an element opens a pair when it is the first of its row (or of the tile) or
-// lies in another slice than the element before it (columns ascend inside a row).
+// lies in another slice than the element before it (columns ascend inside a row); without row_ptr
+// out[64 + t] = columns between the tile's lowest and highest, out[128 + t] = elements whose column
+// is lower than the one before them: one a row or fewer where columns ascend.
 struct SampleArgs {
     const int32_t *col;
     int64_t stride;
@@ -370,6 +372,8 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
         }
         if (q.row_ptr)
             mine_pairs += i == 0 || c[u] / q.width != left[u] / q.width || (starts[i >> 5] >> (i & 31) & 1u) != 0;
+        else
+            mine_pairs += c[u] < left[u];
     }
     if (!q.row_ptr) {
         int32_t lo = c[0], hi = c[0];
@@ -384,6 +388,7 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
     if (threadIdx.x == 0) {
         q.out[t] = count;
         q.out[64 + t] = q.row_ptr ? pairs : highest - lowest;
+        if (!q.row_ptr) q.out[128 + t] = pairs;
     }
 }
 __global__ __launch_bounds__(kBlock) void k_sample_columns(SampleArgs q) { sample_columns_tile(q, blockIdx.x); }

@@ -82,30 +82,31 @@ SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
 //           sums the column-sliced kernel would carry through memory.  16 random columns per row
 //           over 32 slices give 0.8, a band matrix about 1 / (row length).
 //   span    columns between a tile's first and last, on average (instead of the pairs, for SpMM).
+//   falls   elements of a tile, on average, whose column is lower than the one before (for SpMM).
 struct ColumnSample {
     bool ok;
-    double spread, pairs, span;
+    double spread, pairs, span, falls;
 };
 constexpr int32_t kSliceBytes = 131072;  // of x per slice: one workgroup of 16 waves per compute unit
 int sample_tiles(int32_t nnz) { return (int)std::min<int64_t>(64, nnz / kFlatTile); }
 int64_t sample_stride(int32_t nnz) { return (int64_t)(nnz / kFlatTile) / std::max(sample_tiles(nnz), 1) * kFlatTile; }
 int line_shift(size_t sv) { return sv == 8 ? 4 : 5; }  // columns per 128-byte line of x
-// h: distinct lines of every tile, then (with row offsets) the pairs, as counted on the device
-ColumnSample sample_result(const int32_t h[128], int32_t nnz, bool with_pairs)
+// h: distinct lines of every tile, then the pairs (with row offsets) or the span and the falls, as counted on the device
+ColumnSample sample_result(const int32_t *h, int32_t nnz, bool with_pairs)
 {
     const int samples = sample_tiles(nnz);
-    int64_t distinct = 0, pairs = 0;
-    for (int t = 0; t < samples; ++t) distinct += h[t], pairs += h[64 + t];
-    ColumnSample cs{samples > 0, 0.0, 1.0, 0.0};
+    int64_t distinct = 0, pairs = 0, falls = 0;
+    for (int t = 0; t < samples; ++t) distinct += h[t], pairs += h[64 + t], falls += with_pairs ? 0 : h[128 + t];
+    ColumnSample cs{samples > 0, 0.0, 1.0, 0.0, 0.0};
     if (samples > 0) cs.spread = (double)distinct / ((double)samples * kFlatTile);
     if (samples > 0 && with_pairs) cs.pairs = (double)pairs / ((double)samples * kFlatTile);
-    if (samples > 0 && !with_pairs) cs.span = (double)pairs / (double)samples;
+    if (samples > 0 && !with_pairs) cs.span = (double)pairs / (double)samples, cs.falls = (double)falls / (double)samples;
     return cs;
 }
 // the spread and the span, counted now
 ColumnSample sample_columns(const int32_t *d_col, int32_t nnz, size_t sv, hipStream_t s)
 {
-    const ColumnSample none{false, 0.0, 1.0, 0.0};
+    const ColumnSample none{false, 0.0, 1.0, 0.0, 0.0};
     Scratch scratch(s);
     int32_t *h = static_cast<int32_t *>(scratch.pinned());
     if (sample_tiles(nnz) < 1 || !h) return none;
@@ -266,6 +267,9 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         } else {
             xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
+        if (plan && plan->sweep && (uint64_t)ldb <= 0xffffffffull / sizeof(T))
+            return launch_spmm_sweep<T>(spmm_sweep(m, plan->n, nnz, ncols, sizeof(T)), m, plan->n, ncols, alpha, row_ptr, col, val, B, ldb,
+                                        beta, C, ldc, s);
         const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
         const bool chunked = plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T));
         return launch_spmm_merge<T>(chunked, plan ? std::max(plan->n, k) : 0, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb,
@@ -430,7 +434,7 @@ int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n
     scratch.idle = true;
     std::memcpy(p->hist, h, sizeof(p->hist));
     std::memcpy(p->stats, h + 33, sizeof(p->stats));
-    if (more) more->sample = samples > 0 ? sample_result(reinterpret_cast<const int32_t *>(h + 64), nnz, true) : ColumnSample{false, 0.0, 1.0, 0.0};
+    if (more) more->sample = samples > 0 ? sample_result(reinterpret_cast<const int32_t *>(h + 64), nnz, true) : ColumnSample{false, 0.0, 1.0, 0.0, 0.0};
     *out = p;
     return ASX_STATUS_SUCCESS;
 }
@@ -514,9 +518,9 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
     return st;
 }
 
-// columns: kColumns* of an SpMM plan
+// columns: kColumns* of an SpMM plan; everywhere: they ascend in a row and lie all over B
 int plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m, int32_t n, int32_t nnz,
-                const int32_t *d_row_ptr, int32_t ncols_dense, int columns, void *stream)
+                const int32_t *d_row_ptr, int32_t ncols_dense, int columns, bool everywhere, void *stream)
 {
     if (!out) return ASX_STATUS_INVALID_POINTER;
     *out = nullptr;
@@ -536,7 +540,11 @@ int plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m,
         asx_plan_destroy(p);
         return ASX_STATUS_NOT_SUPPORTED;
     }
-    if (kernel == ASX_SPMM_MERGE && is_spmm) p->columns = columns;
+    if (kernel == ASX_SPMM_MERGE && is_spmm) {
+        p->columns = columns;
+        p->sweep = everywhere && p->stats[0] <= spmm_sweep_longest(m, nnz) &&
+                   spmm_sweep(m, n, nnz, ncols_dense, vsize(value_type)).slots > 0;
+    }
     st = plan_row_ordered(p, kernel, s);
     if (st) {
         asx_plan_destroy(p);
@@ -553,7 +561,7 @@ extern "C" {
 int asx_plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m, int32_t n,
                     int32_t nnz, const int32_t *d_row_ptr, int32_t ncols_dense, void *stream)
 {
-    return plan_create(out, is_spmm, alg, value_type, m, n, nnz, d_row_ptr, ncols_dense, kColumnsUnknown, stream);
+    return plan_create(out, is_spmm, alg, value_type, m, n, nnz, d_row_ptr, ncols_dense, kColumnsUnknown, false, stream);
 }
 
 int asx_plan_destroy(asx_plan *plan)
@@ -594,15 +602,18 @@ int asx_spmm_plan_create(asx_plan **out, int alg, int value_type, int32_t m, int
     // scattered columns (a sample of tiles of 1024 stored elements touches mostly distinct
     // 128-byte lines) cannot fill 16x4 blocks: the blocks are not even built then
     int columns = kColumnsUnknown;
+    bool everywhere = false;
     bool probe_blocked = alg == ASX_SPMM_DEFAULT && nnz > 0 && nnz <= kBlockedProbeMaxNnz && d_col &&
                          (value_type == ASX_R_32F || value_type == ASX_R_64F);
     if (probe_blocked) {
         const ColumnSample cs = sample_columns(d_col, nnz, vsize(value_type), (hipStream_t)stream);
         probe_blocked = cs.ok && cs.spread < kScatteredMinSpread;
-        if (cs.ok) columns = spmm_columns(cs.spread, cs.span, (double)nnz / std::max(m, 1), vsize(value_type));
+        const double mean = (double)nnz / std::max(m, 1);
+        if (cs.ok) columns = spmm_columns(cs.spread, cs.span, mean, vsize(value_type));
+        everywhere = cs.ok && spmm_everywhere(cs.spread, cs.span, cs.falls, mean, k, vsize(value_type));
     }
     const auto row_ordered = [&]() {
-        return plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, columns, stream);
+        return plan_create(out, 1, alg, value_type, m, k, nnz, d_row_ptr, ncols, columns, everywhere, stream);
     };
     if (!want_blocked && !probe_blocked) return row_ordered();
     if (m < 0 || k < 0 || nnz < 0 || ncols < 1) return ASX_STATUS_INVALID_SIZE;
@@ -1190,7 +1201,12 @@ int64_t asx_plan_info(const asx_plan *plan, int what)
     if (!plan) return -1;
     if (plan->is_spmm) {
         if (plan->alg != ASX_SPMM_MERGE) return -1;
-        return what == ASX_PLAN_INFO_SEGMENT_ITEMS ? plan->items : what == ASX_PLAN_INFO_SHARED_SEGMENTS ? plan->chunked : -1;
+        switch (what) {
+        case ASX_PLAN_INFO_SEGMENT_ITEMS: return plan->items;
+        case ASX_PLAN_INFO_SHARED_SEGMENTS: return plan->chunked;
+        case ASX_PLAN_INFO_SWEEP: return plan->sweep;
+        default: return -1;
+        }
     }
     const bool sliced = plan->alg == ASX_SPMV_SLICED, window = plan->alg == ASX_SPMV_WINDOW;
     switch (what) {

@@ -1,6 +1,7 @@
 // Internal declarations shared by the HIP translation units of libalphasparse_amd.so.
 #pragma once
 #include <algorithm>
+#include <cmath>
 #include <hip/hip_runtime.h>
 #include <stddef.h>
 #include <stdint.h>
@@ -13,6 +14,7 @@ namespace asx {
 
 // Tile geometry of the SpMV kernels (one workgroup of 256 threads per tile).
 constexpr int kBlock = 256;
+constexpr int kXcds = 8;  // workgroups are dealt to the 8 XCDs round-robin (workgroup b runs on XCD b % 8)
 constexpr int kMergeItemsPerThread = 8;
 constexpr int kMergeTile = kBlock * kMergeItemsPerThread;  // rows + stored elements per tile
 constexpr int kStreamTile = 1024;                          // stored elements per row block
@@ -209,6 +211,19 @@ int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
                       bool carry_pass, int tile_bytes, hipStream_t s);
 
+// ---- SpMM of columns that lie all over B (asx_spmm_sweep.hip) ----
+struct SpmmSweep {
+    int32_t slots;   // rows of C a lane group has registers for (0: not taken)
+    int32_t rows;    // and how many it is given
+    int32_t cap;     // elements of A a wave stages at once
+    uint32_t width;  // columns a window
+    int log_lanes;   // of a group
+    int64_t tiles;   // of columns of B
+};
+template <typename T>
+int launch_spmm_sweep(const SpmmSweep &sw, int32_t m, int32_t n, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col,
+                      const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s);
+
 // merge-path split points of SpMM, `items` apart, moved to the ends of the short rows they cut; *has_carry (may be null)
 // is set to 1 if a row stays cut
 int launch_spmm_splits(int32_t m, int32_t nnz, int32_t items, const int32_t *row_ptr, int32_t *xs, int32_t *ys,
@@ -235,7 +250,6 @@ template <typename T>
 int launch_spmm_blocked(int32_t m, int32_t k, int32_t ncols, T alpha, const BlockedMatrix *bm, const T *B,
                         int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s);
 
-constexpr int kXcds = 8;  // workgroups are dealt to the 8 XCDs round-robin (workgroup b runs on XCD b % 8)
 // out[r] = first i with sorted[i] >= r, r in [0, n]
 int launch_offsets_from_sorted(const int32_t *sorted, int32_t count, int32_t n, int32_t *out, hipStream_t s);
 
@@ -451,6 +465,56 @@ inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m
     if (longest > spmm_dealt(groups) || turn > most || 4 * (longest + 1) * m > 5 * ((int64_t)m + nnz)) return least;
     return (int32_t)(most / turn * turn);
 }
+// Columns lie all over B and ascend in a row, as a sample's tiles of 1024 elements tell: first and last column of a tile nearly as
+// far apart as B has rows (uniform columns: 0.998 of them); about as many different lines as uniform columns would touch, of
+// `lines` on average lines (1 - exp(-1024 / lines)); and about one fall a row (unsorted rows: one every other element, two a row and
+// more from four elements on).
+inline bool spmm_everywhere(double spread, double span, double falls, double mean, int64_t k, size_t sv)
+{
+    const double lines = (double)k * (double)sv / 128.0 + 1.0;
+    return span >= 0.9 * (double)k && spread * kFlatTile >= 0.7 * lines * (1.0 - exp(-kFlatTile / lines)) && falls * mean <= 1.25 * kFlatTile;
+}
+// The sweep kernel, where its sizes suit it (slots 0: not).  What its caller has to know beside these: that columns ascend in a row
+// and lie all over B, and that no row is longer than spmm_sweep_longest.
+//   Sixteen waves a compute unit share 160 KB of LDS, in which a wave stages its part of A; a group takes as many rows as that and
+//   its registers allow, evened out over the rounds of waves.
+//   Windows: the more, the less of B a window needs (a wave ahead or behind does less harm), but every window costs its
+//   instructions whether rows have an element in it or not: 1.24 MB(B)^0.35 mean^-0.3 windows an element of a mean row, between 1
+//   and 2.5, fitted to 110 uniform matrices (both types, rows of B of 72 to 2000 bytes, 4 to 64 per row, B of 14 to 317 MB)
+//   timed with 1 to 6: 0.5 % behind the best of these on average.
+//   On those 110 it takes 0.78 of the row-ordered kernels' time on average (100 columns fp32, 160000 rows of 25 270 us against
+//   130; 96, 94796 of 49 316 and 136; 64, 573065 of 9 204 and 191; 22, 1 M of 4 138 and 133).  Not taken: a B that the L2s keep
+//   between them (9 MB, 14 where rows of A are short) - where rows of B start on lines the row-ordered kernels work through it
+//   in tiles of one line, which they can keep up to 40000 rows or 20 MB (192 columns fp32, 27903 rows of 8 22.6 us there, 23.4 here;
+//   32, 101110 of 8 17.3 and 18.4; 448, 28456 of 9 52.3 and 59.8) -; rows of fewer than 4; and where an XCD's waves meet a row of B
+//   only every fourth round or less (kSweepSharedLeast; 74 columns fp32, 525797 x 1032224, 13 per row 406 and 429).
+constexpr int kSweepWaves = 16;
+constexpr double kSweepSharedLeast = 0.25;
+inline int64_t spmm_sweep_longest(int32_t m, int32_t nnz) { return 2 * ((int64_t)nnz / (m > 0 ? m : 1)) + 8; }
+inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, size_t sv)
+{
+    SpmmSweep sw{};
+    const int64_t bytes = ncols * (int64_t)sv;
+    if (m <= 0 || n <= 0 || bytes <= 64 || nnz / m < 4) return sw;
+    const double mean = (double)nnz / m, mb = 1e-6 * (double)bytes * n;
+    if (bytes % 128 == 0 ? mb < 20.0 || n < 40000 : mb < (mean < 14.0 ? 14.0 : 9.0)) return sw;
+    const SpmmTiling t = spmm_tiling(ncols, 1024, sv);
+    const int groups = t.groups;
+    const int32_t cap = (int32_t)(160 * 1024 / kSweepWaves / (4 + sv)) & ~1;
+    int64_t rows = std::min<int64_t>(t.log_lanes < 5 ? 1 << t.log_lanes : 20, (int64_t)(cap / (1.05 * mean * groups)));
+    if (t.log_lanes < 3 || rows < 1 || t.tiles > 65535) return sw;
+    const int64_t round = (int64_t)kSweepWaves * 256 * groups, rounds = ceil_div64(m, round * rows);
+    rows = ceil_div64(m, round * rounds);
+    if ((double)std::min<int64_t>(round * rows, m) * mean / kXcds < kSweepSharedLeast * n) return sw;
+    sw.rows = (int32_t)rows;
+    sw.slots = rows <= 4 ? 4 : rows <= 8 ? 8 : rows <= 12 ? 12 : rows <= 16 ? 16 : 20;
+    sw.cap = std::min(cap, ((int32_t)(1.1 * mean * (double)(rows * groups)) + 2) & ~1);
+    const double windows = mean * std::min(std::max(1.24 * pow(mb, 0.35) * pow(mean, -0.3), 1.0), 2.5);
+    sw.width = (uint32_t)std::max((double)n / windows, 1.0) + 1;
+    sw.log_lanes = t.log_lanes;
+    sw.tiles = t.tiles;
+    return sw;
+}
 inline int32_t spmm_segments(int32_t m, int32_t nnz, int32_t items) { return (int32_t)ceil_div64((int64_t)m + nnz, items); }
 
 }  // namespace asx
@@ -477,6 +541,7 @@ struct asx_plan {
     int columns;     // SpMM merge kernel: kColumns*
     int32_t items;   // SpMM merge and chunk kernels: merge items per segment
     int chunked;     // SpMM: the chunk kernel
+    int sweep;       // SpMM: rows and columns of A suit the sweep kernel
     int64_t hist[33];
     int64_t stats[4];
     size_t workspace_bytes;

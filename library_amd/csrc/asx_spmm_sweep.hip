@@ -1,0 +1,236 @@
+// CSR x dense SpMM for gfx950 where the columns of A lie all over B: C = alpha*A*B + beta*C, B and C row-major.
+//
+// The row-ordered kernels (asx_spmm.hip) fetch a row of B for every stored element, and where B is larger than an L2 nearly each
+// fetch goes past it, at 56 to 59 G lines/s whatever the kernel does.  An XCD's registers, though, hold the rows of C that its
+// share of A makes (32 compute units with 512 KB each), so here every wave keeps its rows of C in registers, and all waves go
+// through the columns of A together, in windows: while a window lasts, its part of B stays in the XCD's L2 and serves the
+// elements of all rows.  Nothing orders the waves but that they do the same work a window; those ahead wait for memory, those
+// behind find their rows of B in the L2.
+//
+// Uniform columns, 25 per row, 100 columns fp32 of 150001 rows: 258 us with the merge kernel, 15.4 M lines past the L2s; 124 here.
+// 49 per row, 96 columns of 94796 rows 316 and 136; 24 per row, 103 columns fp64 of 97486 337 and 215.
+#include "asx_internal.hpp"
+
+namespace asx {
+
+namespace {
+
+template <typename T>
+struct Vec16 {  // 16 bytes of a row, aligned as an element is
+    static constexpr int N = 16 / sizeof(T);
+    typedef T type __attribute__((ext_vector_type(16 / sizeof(T)), aligned(sizeof(T))));
+};
+
+template <int I>
+struct Const {
+    static constexpr int value = I;
+};
+template <int I, int N, typename F>
+__device__ __forceinline__ void static_for(const F &f)
+{
+    if constexpr (I < N) {
+        f(Const<I>{});
+        static_for<I + 1, N>(f);
+    }
+}
+
+// what lane J of every group of 2^LOGL lanes holds, in all lanes of the group
+template <int LOGL, int J>
+__device__ __forceinline__ uint32_t group_lane(uint32_t v)
+{
+    if constexpr (LOGL == 6)
+        return (uint32_t)__builtin_amdgcn_readlane((int)v, J);
+    else
+        return (uint32_t)__builtin_amdgcn_ds_swizzle((int)v, ((32 - (1 << LOGL)) & 31) | J << 5);
+}
+template <int LOGL, int J>
+__device__ __forceinline__ float group_lane(float v)
+{
+    return __builtin_bit_cast(float, group_lane<LOGL, J>(__builtin_bit_cast(uint32_t, v)));
+}
+template <int LOGL, int J>
+__device__ __forceinline__ double group_lane(double v)
+{
+    return __hiloint2double((int)group_lane<LOGL, J>((uint32_t)__double2hiint(v)), (int)group_lane<LOGL, J>((uint32_t)__double2loint(v)));
+}
+
+}  // namespace
+
+// lanes j0 .. j0 + n - 1 of every group of l
+constexpr uint64_t lanes_of_groups(int l, int j0, int n)
+{
+    uint64_t mask = 0;
+    for (int g = 0; g < kWave; g += l) mask |= ((1ull << n) - 1) << (g + j0);
+    return mask;
+}
+constexpr uint32_t kNoColumn = 0xffffffffu, kAllColumns = 0x80000000u;
+constexpr int sweep_batch(int slots) { return slots == 20 ? 5 : slots == 12 ? 6 : slots == 4 ? 4 : 8; }
+
+// A group of L = 2^LOGL lanes, 16 bytes a lane, spans a tile of a row of B; the wave's NG groups have `rows` rows of C each, in S
+// slots of registers (a slot is an array element by a constant: registers indexed at run time gave wrong sums where an indexed
+// write is followed closely by an indexed read).  Lane j of a group knows where its slot j is in the row of A, which the wave has
+// staged in LDS.  A step is a window: slots whose next element lies in it fetch a row of B, one element a slot and step, so
+// that loads and sums need no more than a broadcast of slot j's column and value over the group; a slot that has several elements
+// in a window is late for a step or two.  What bounds it: a step costs a slot ~10 instructions whether it has an element or not,
+// and a load 16 cycles of a compute unit's L1 where all lanes take part, none where none does - slots without an element are
+// masked out, not sent past a buffer's end (119 us against 157 for the first example above) -; and lines past the L2s for what
+// waves are apart.  Batches of G slots, all loads of a batch ahead of its sums.
+template <typename T, int LOGL, int S>
+__global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
+    int32_t m, int32_t rows, int32_t cap, uint32_t width, uint32_t last, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
+    const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ B, int64_t ldb, T beta, T *__restrict__ C, int64_t ldc)
+{
+    typedef typename Vec16<T>::type V;
+    constexpr int VEC = Vec16<T>::N, L = 1 << LOGL, NG = kWave / L, G = sweep_batch(S);
+    static_assert(S <= L && S % G == 0, "a lane knows where one row of its group is");
+    extern __shared__ char s_all[];
+    const int lane = threadIdx.x & (kWave - 1);
+    const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+    const uint32_t per_xcd = gridDim.x / kXcds;
+    const int64_t wave = ((int64_t)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds) * (kBlock / kWave) + w;
+    const int64_t x0 = wave * rows * NG;
+    if (x0 >= m) return;
+    const int32_t nrow = (int32_t)(m - x0 < rows * NG ? m - x0 : rows * NG);
+    const int grp = lane >> LOGL, gl = lane & (L - 1);
+    const int32_t t0 = (int32_t)((int64_t)blockIdx.y * ncols / gridDim.y), t1 = (int32_t)((int64_t)(blockIdx.y + 1) * ncols / gridDim.y);
+    int32_t c = t0 + gl * VEC;
+    const bool active = c < t1;
+    c = c < t1 - VEC ? c : t1 - VEC;
+    uint32_t *s_col = (uint32_t *)(s_all + (size_t)w * cap * (sizeof(T) + 4) + (size_t)cap * sizeof(T));
+    T *s_val = (T *)(s_all + (size_t)w * cap * (sizeof(T) + 4));
+    const char *Bc = (const char *)(B + c);
+    const uint32_t pitch = (uint32_t)((uint64_t)ldb * sizeof(T));
+
+    // the lane's row: element s up to e
+    const int32_t mine = grp * rows + gl;
+    const bool has_row = gl < rows && mine < nrow;
+    const int32_t s = has_row ? row_ptr[x0 + mine] : 0, e = has_row ? row_ptr[x0 + mine + 1] : 0;
+    const int32_t begin = __builtin_amdgcn_readfirstlane(row_ptr[x0]), end = __builtin_amdgcn_readfirstlane(row_ptr[x0 + nrow]);
+
+    V acc[S];
+#pragma unroll
+    for (int j = 0; j < S; ++j) acc[j] = T(0);
+    for (int32_t from = begin; from < end;) {  // once, unless rows are longer than usual
+        const int32_t nel = end - from < cap ? end - from : cap;
+        for (int i0 = 0; i0 < nel; i0 += 4 * kWave) {
+            int32_t tc[4];
+            T tv[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = i0 + j * kWave + lane;
+                const int64_t k = (int64_t)from + (i < nel ? i : nel - 1);
+                tc[j] = __builtin_nontemporal_load(col + k);
+                tv[j] = __builtin_nontemporal_load(val + k);
+            }
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int i = i0 + j * kWave + lane;
+                if (i < nel) s_col[i] = (uint32_t)tc[j], s_val[i] = tv[j];
+            }
+        }
+        // the staged data is private to this wave: order its LDS writes before its LDS reads
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        int32_t p = s < from ? 0 : s - from < nel ? s - from : nel;
+        const int32_t pe = e < from ? 0 : e - from < nel ? e - from : nel;
+        uint32_t next = p < pe ? s_col[p] : kNoColumn;
+        T a_next = p < pe ? s_val[p] : T(0);
+        uint32_t wend = width;
+        bool more;
+        do {
+            const bool go = next < wend;
+            wend = wend < last ? wend + width : kAllColumns;
+            const uint32_t at = go ? next : kNoColumn;
+            const T a = go ? a_next : T(0);
+            p += go ? 1 : 0;
+            if (go) next = kNoColumn;
+            more = __ballot(p < pe) != 0;
+            const uint64_t now = __ballot(go);
+            if (now == 0) continue;
+            if (go && p < pe) next = s_col[p], a_next = s_val[p];
+            static_for<0, S / G>([&](auto g_) {
+                constexpr int j0 = decltype(g_)::value * G;
+                if ((now & lanes_of_groups(L, j0, G)) == 0) return;
+                V b[G];
+                uint32_t o[G];
+                __builtin_amdgcn_sched_barrier(0);
+                static_for<0, G>([&](auto u_) { o[decltype(u_)::value] = group_lane<LOGL, j0 + decltype(u_)::value>(at); });
+                static_for<0, G>([&](auto u_) {
+                    constexpr int u = decltype(u_)::value;
+                    b[u] = T(0);
+                    if (o[u] != kNoColumn) b[u] = *(const V *)(Bc + (uint64_t)o[u] * pitch);
+                });
+                __builtin_amdgcn_sched_barrier(0);
+                static_for<0, G>([&](auto u_) {
+                    constexpr int u = decltype(u_)::value;
+                    V t = __builtin_elementwise_fma((V)group_lane<LOGL, j0 + u>(a), b[u], acc[j0 + u]);
+                    static_for<0, VEC>([&](auto v_) {  // keeps the sum here: left alone, all of a step's move behind its last load
+                        T x = t[decltype(v_)::value];
+                        asm volatile("" : "+v"(x));
+                        acc[j0 + u][decltype(v_)::value] = x;
+                    });
+                });
+                __builtin_amdgcn_sched_barrier(0);
+            });
+        } while (more);
+        from += nel;
+        if (from < end) __builtin_amdgcn_wave_barrier();
+    }
+    static_for<0, S / G>([&](auto g_) {
+        constexpr int j0 = decltype(g_)::value * G;
+        V c_old[G];
+        static_for<0, G>([&](auto u_) {
+            constexpr int j = j0 + decltype(u_)::value;
+            c_old[decltype(u_)::value] = T(0);
+            if (beta != T(0) && j < rows && grp * rows + j < nrow)
+                c_old[decltype(u_)::value] = *(const V *)(C + (x0 + grp * rows + j) * ldc + c);
+        });
+        static_for<0, G>([&](auto u_) {
+            constexpr int j = j0 + decltype(u_)::value;
+            const V y = beta == T(0) ? (V)(alpha * acc[j]) : __builtin_elementwise_fma((V)alpha, acc[j], (V)(beta * c_old[decltype(u_)::value]));
+            if (active && j < rows && grp * rows + j < nrow) *(V *)(C + (x0 + grp * rows + j) * ldc + c) = y;
+        });
+    });
+}
+
+template <typename T>
+int launch_spmm_sweep(const SpmmSweep &sw, int32_t m, int32_t n, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
+                      const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s)
+{
+    const int64_t waves = ceil_div64(m, (int64_t)sw.rows * (kWave >> sw.log_lanes));
+    const dim3 grid((unsigned)(ceil_div64(ceil_div64(waves, kBlock / kWave), kXcds) * kXcds), (unsigned)sw.tiles);
+    const size_t lds = (size_t)sw.cap * (sizeof(T) + 4) * (kBlock / kWave);
+    const uint32_t last = (uint32_t)n > sw.width ? (uint32_t)n - sw.width : 0;
+#define ASX_SWEEP(LOGL, S)                                                                                                              \
+    if (sw.log_lanes == LOGL && sw.slots == S) {                                                                                        \
+        hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S>), grid, dim3(kBlock), lds, s, m, sw.rows, sw.cap, sw.width, last, ncols, alpha, \
+                           row_ptr, col, val, B, ldb, beta, C, ldc);                                                                    \
+        return check_launch();                                                                                                          \
+    }
+    ASX_SWEEP(3, 4)
+    ASX_SWEEP(3, 8)
+    ASX_SWEEP(4, 4)
+    ASX_SWEEP(4, 8)
+    ASX_SWEEP(4, 12)
+    ASX_SWEEP(4, 16)
+    ASX_SWEEP(5, 4)
+    ASX_SWEEP(5, 8)
+    ASX_SWEEP(5, 12)
+    ASX_SWEEP(5, 16)
+    ASX_SWEEP(5, 20)
+    ASX_SWEEP(6, 4)
+    ASX_SWEEP(6, 8)
+    ASX_SWEEP(6, 12)
+    ASX_SWEEP(6, 16)
+    ASX_SWEEP(6, 20)
+#undef ASX_SWEEP
+    return ASX_STATUS_INTERNAL_ERROR;
+}
+
+template int launch_spmm_sweep<float>(const SpmmSweep &, int32_t, int32_t, int32_t, float, const int32_t *, const int32_t *, const float *,
+                                      const float *, int64_t, float, float *, int64_t, hipStream_t);
+template int launch_spmm_sweep<double>(const SpmmSweep &, int32_t, int32_t, int32_t, double, const int32_t *, const int32_t *, const double *,
+                                       const double *, int64_t, double, double *, int64_t, hipStream_t);
+
+}  // namespace asx
