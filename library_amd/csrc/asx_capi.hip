@@ -58,8 +58,8 @@ FlatLayout spmv_flat_layout(int32_t nnz, size_t sv, bool with_split)
     return L;
 }
 
-struct SpmmLayout {  // [carry_row | carry]
-    size_t crow_off, carry_off, bytes;
+struct SpmmLayout {  // [carry_row | carry | what the device says of the columns]
+    size_t crow_off, carry_off, bytes, ask_off, asked_bytes;  // bytes: without the last
 };
 SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
 {
@@ -70,7 +70,10 @@ SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
     off = align_up(off + std::max<size_t>(ns, 1) * 4, kAlign);
     L.carry_off = off;
     off = align_up(off + std::max<size_t>(ns, 1) * (size_t)ncols * sv, kAlign);
-    L.bytes = off;
+    L.bytes = L.ask_off = L.asked_bytes = off;
+    const SpmmSweep sw = spmm_sweep_shape(m, nnz, ncols, sv);
+    if (spmm_sweep_askable(sw, m, nnz, ncols, sv, spmm_segment_items(m, nnz, ncols, sv)))
+        L.asked_bytes = align_up(off + 8 + (size_t)spmm_sweep_blocks(sw, m), kAlign);
     return L;
 }
 
@@ -268,14 +271,29 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
             xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
         if (plan && plan->sweep && (uint64_t)ldb <= 0xffffffffull / sizeof(T))
-            return launch_spmm_sweep<T>(spmm_sweep(m, plan->n, nnz, ncols, sizeof(T)), m, plan->n, ncols, alpha, row_ptr, col, val, B, ldb,
-                                        beta, C, ldc, s);
+            return launch_spmm_sweep<T>(spmm_sweep(m, plan->n, nnz, ncols, sizeof(T)), nullptr, m, plan->n, nnz, ncols, alpha, row_ptr, col,
+                                        val, B, ldb, beta, C, ldc, s);
         const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
         const bool chunked = plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T));
+        SweepAsk ask{};
+        if ((plan ? plan->asks != 0 : alg == ASX_SPMM_DEFAULT) && !chunked && L.asked_bytes > L.bytes && ws_bytes >= L.asked_bytes &&
+            items == spmm_segment_items(m, nnz, ncols, sizeof(T)) && (uint64_t)ldb <= 0xffffffffull / sizeof(T)) {
+            const int32_t n = plan ? plan->n : k;
+            const SpmmSweep sw = spmm_sweep(m, n, nnz, ncols, sizeof(T));
+            if (sw.slots > 0 && spmm_sweep_shared(sw, m, n, nnz) >= kSweepAskShared) {
+                ask.n = n;
+                ask.longest = (int32_t)spmm_sweep_longest(m, nnz);
+                ask.blocks = (int32_t)spmm_sweep_blocks(sw, m);
+                ask.answer = (int32_t *)(w + L.ask_off);
+                ask.too_long = (uint8_t *)(w + L.ask_off + 8);
+                const int st = launch_spmm_sweep<T>(sw, &ask, m, n, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, s);
+                if (st) return st;
+            }
+        }
         return launch_spmm_merge<T>(chunked, plan ? std::max(plan->n, k) : 0, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb,
                                     beta, C, ldc, xs, ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
                                     plan ? plan->carry_pass != 0 : true,
-                                    spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), s);
+                                    spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), ask, s);
     }
     case ASX_SPMM_BLOCKED:
         // the blocks hold a copy of A's values and are built by asx_spmm_plan_create
@@ -494,7 +512,8 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         }
     } else if (kernel == ASX_SPMM_MERGE) {
         const int32_t usual = spmm_segment_items(m, nnz, p->ncols, sv);
-        p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv).bytes;
+        const SpmmLayout layout = spmm_merge_layout(m, nnz, p->ncols, sv);
+        p->workspace_bytes = p->asks ? layout.asked_bytes : layout.bytes;
         // B's rows one after the other, from the start of a line on, as nearly every caller has them
         const int tile_bytes = spmm_tile_bytes(p->columns, p->n, nullptr, (size_t)p->ncols * sv);
         const int groups = spmm_tiling(p->ncols, tile_bytes, sv).groups;
@@ -542,6 +561,7 @@ int plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m,
     }
     if (kernel == ASX_SPMM_MERGE && is_spmm) {
         p->columns = columns;
+        p->asks = alg == ASX_SPMM_DEFAULT && columns == kColumnsUnknown;
         p->sweep = everywhere && p->stats[0] <= spmm_sweep_longest(m, nnz) &&
                    spmm_sweep(m, n, nnz, ncols_dense, vsize(value_type)).slots > 0;
     }
@@ -1374,7 +1394,10 @@ int asx_spmm_resolve_alg(int alg, int32_t m, int32_t nnz, int32_t ncols)
 size_t asx_spmm_workspace_bytes(int alg, int value_type, int32_t m, int32_t nnz, int32_t ncols)
 {
     const int kernel = asx_spmm_resolve_alg(alg, m, nnz, ncols);
-    if (kernel == ASX_SPMM_MERGE) return spmm_merge_layout(m, nnz, ncols, vsize(value_type)).bytes;
+    if (kernel == ASX_SPMM_MERGE) {
+        const SpmmLayout layout = spmm_merge_layout(m, nnz, ncols, vsize(value_type));
+        return alg == ASX_SPMM_DEFAULT ? layout.asked_bytes : layout.bytes;
+    }
     return 0;
 }
 

@@ -205,11 +205,19 @@ int launch_flat_has_carry(const int32_t *d_row_ptr, int32_t m, int32_t nnz, cons
 template <typename T>
 int launch_spmm_row(int32_t m, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col,
                     const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s);
+// Where the device decides whether the sweep kernel takes a call: what it has to know, and where it leaves its answer.
+struct SweepAsk {
+    int32_t n;          // columns of A
+    int32_t longest;    // row the sweep takes
+    int32_t blocks;     // its workgroups
+    int32_t *answer;    // 1: taken (null: nobody asks)
+    uint8_t *too_long;  // of each workgroup: it left rows of more than `longest` elements out
+};
 template <typename T>
 int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
-                      bool carry_pass, int tile_bytes, hipStream_t s);
+                      bool carry_pass, int tile_bytes, const SweepAsk &ask, hipStream_t s);
 
 // ---- SpMM of columns that lie all over B (asx_spmm_sweep.hip) ----
 struct SpmmSweep {
@@ -221,8 +229,9 @@ struct SpmmSweep {
     int64_t tiles;   // of columns of B
 };
 template <typename T>
-int launch_spmm_sweep(const SpmmSweep &sw, int32_t m, int32_t n, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col,
-                      const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s);
+int launch_spmm_sweep(const SpmmSweep &sw, const SweepAsk *ask, int32_t m, int32_t n, int32_t nnz, int32_t ncols, T alpha,
+                      const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
+                      hipStream_t s);
 
 // merge-path split points of SpMM, `items` apart, moved to the ends of the short rows they cut; *has_carry (may be null)
 // is set to 1 if a row stays cut
@@ -491,29 +500,64 @@ inline bool spmm_everywhere(double spread, double span, double falls, double mea
 constexpr int kSweepWaves = 16;
 constexpr double kSweepSharedLeast = 0.25;
 inline int64_t spmm_sweep_longest(int32_t m, int32_t nnz) { return 2 * ((int64_t)nnz / (m > 0 ? m : 1)) + 8; }
-inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, size_t sv)
+constexpr int32_t spmm_sweep_cap(size_t sv) { return (int32_t)(160 * 1024 / kSweepWaves / (4 + sv)) & ~1; }
+// what does not depend on the number of columns
+inline SpmmSweep spmm_sweep_shape(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
 {
     SpmmSweep sw{};
-    const int64_t bytes = ncols * (int64_t)sv;
-    if (m <= 0 || n <= 0 || bytes <= 64 || nnz / m < 4) return sw;
-    const double mean = (double)nnz / m, mb = 1e-6 * (double)bytes * n;
-    if (bytes % 128 == 0 ? mb < 20.0 || n < 40000 : mb < (mean < 14.0 ? 14.0 : 9.0)) return sw;
+    if (m <= 0 || ncols * (int64_t)sv <= 64 || nnz / m < 4) return sw;
+    const double mean = (double)nnz / m;
     const SpmmTiling t = spmm_tiling(ncols, 1024, sv);
-    const int groups = t.groups;
-    const int32_t cap = (int32_t)(160 * 1024 / kSweepWaves / (4 + sv)) & ~1;
-    int64_t rows = std::min<int64_t>(t.log_lanes < 5 ? 1 << t.log_lanes : 20, (int64_t)(cap / (1.05 * mean * groups)));
+    const int32_t cap = spmm_sweep_cap(sv);
+    int64_t rows = std::min<int64_t>(t.log_lanes < 5 ? 1 << t.log_lanes : 20, (int64_t)(cap / (1.05 * mean * t.groups)));
     if (t.log_lanes < 3 || rows < 1 || t.tiles > 65535) return sw;
-    const int64_t round = (int64_t)kSweepWaves * 256 * groups, rounds = ceil_div64(m, round * rows);
-    rows = ceil_div64(m, round * rounds);
-    if ((double)std::min<int64_t>(round * rows, m) * mean / kXcds < kSweepSharedLeast * n) return sw;
+    const int64_t round = (int64_t)kSweepWaves * 256 * t.groups;
+    rows = ceil_div64(m, round * ceil_div64(m, round * rows));
     sw.rows = (int32_t)rows;
     sw.slots = rows <= 4 ? 4 : rows <= 8 ? 8 : rows <= 12 ? 12 : rows <= 16 ? 16 : 20;
-    sw.cap = std::min(cap, ((int32_t)(1.1 * mean * (double)(rows * groups)) + 2) & ~1);
-    const double windows = mean * std::min(std::max(1.24 * pow(mb, 0.35) * pow(mean, -0.3), 1.0), 2.5);
-    sw.width = (uint32_t)std::max((double)n / windows, 1.0) + 1;
+    sw.cap = std::min(cap, ((int32_t)(1.1 * mean * (double)(rows * t.groups)) + 2) & ~1);
     sw.log_lanes = t.log_lanes;
     sw.tiles = t.tiles;
     return sw;
+}
+inline int64_t spmm_sweep_blocks(const SpmmSweep &sw, int32_t m)
+{
+    const int64_t waves = ceil_div64(m, (int64_t)sw.rows * (kWave >> sw.log_lanes));
+    return ceil_div64(ceil_div64(waves, kBlock / kWave), kXcds) * kXcds;
+}
+// elements an XCD's waves hold at a time for each row of B
+inline double spmm_sweep_shared(const SpmmSweep &sw, int32_t m, int32_t n, int32_t nnz)
+{
+    const int64_t round = (int64_t)kSweepWaves * 256 * (kWave >> sw.log_lanes);
+    return (double)std::min<int64_t>(round * sw.rows, m) * ((double)nnz / m) / kXcds / n;
+}
+inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, size_t sv)
+{
+    const int64_t bytes = ncols * (int64_t)sv;
+    SpmmSweep sw = spmm_sweep_shape(m, nnz, ncols, sv);
+    if (sw.slots == 0 || n <= 0) return SpmmSweep{};
+    const double mean = (double)nnz / m, mb = 1e-6 * (double)bytes * n;
+    if (bytes % 128 == 0 ? mb < 20.0 || n < 40000 : mb < (mean < 14.0 ? 14.0 : 9.0)) return SpmmSweep{};
+    if (spmm_sweep_shared(sw, m, n, nnz) < kSweepSharedLeast) return SpmmSweep{};
+    const double windows = mean * std::min(std::max(1.24 * pow(mb, 0.35) * pow(mean, -0.3), 1.0), 2.5);
+    sw.width = (uint32_t)std::max((double)n / windows, 1.0) + 1;
+    return sw;
+}
+// Calls whose columns nobody has looked at: whether asking pays (slots 0: not).  Where the answer is no, the launch is spent: 4.6 us with
+// one round of workgroups (100 columns fp32, 160001 power-law rows of 20: 264 us before), 5.8 with two, 9 with five.  So it is for calls
+// whose rows of B, each fetched by itself, take 240 us and more, for two rounds at most, and where an XCD's waves meet a row of B often
+// (100 columns fp32, 150001 uniform rows of 25, 1.6: 257 us without, 157 with). Rows of B that start on lines, which the merge kernel
+// takes a line or two at a time, gain less (256 columns fp32, 60001 uniform rows of 30, 173 us without and 157 with; 128 fp64, 20 per row
+// within 3000 of the diagonal 165 and 171): from twice as many lines on.  Rows that the merge kernel cuts have to be longer than
+// the sweep takes: it looks at whole rows only.
+constexpr double kSweepAskLines = 240e-6 * 58e9, kSweepAskShared = 0.6;
+constexpr int64_t kSweepAskBlocks = 2048;
+inline bool spmm_sweep_askable(const SpmmSweep &sw, int32_t m, int32_t nnz, int64_t ncols, size_t sv, int32_t items)
+{
+    const int64_t bytes = ncols * (int64_t)sv;
+    return sw.slots > 0 && (double)nnz * ((double)bytes / 128.0 + (bytes % 128 ? 1.0 : 0.0)) >= kSweepAskLines &&
+           (bytes % 128 || (double)nnz * (double)bytes / 128.0 >= 2.0 * kSweepAskLines) &&
+           spmm_sweep_longest(m, nnz) <= items && spmm_sweep_blocks(sw, m) <= kSweepAskBlocks;
 }
 inline int32_t spmm_segments(int32_t m, int32_t nnz, int32_t items) { return (int32_t)ceil_div64((int64_t)m + nnz, items); }
 
@@ -542,6 +586,7 @@ struct asx_plan {
     int32_t items;   // SpMM merge and chunk kernels: merge items per segment
     int chunked;     // SpMM: the chunk kernel
     int sweep;       // SpMM: rows and columns of A suit the sweep kernel
+    int asks;        // SpMM: DEFAULT without a look at the columns
     int64_t hist[33];
     int64_t stats[4];
     size_t workspace_bytes;

@@ -170,22 +170,30 @@ __global__ __launch_bounds__(kBlock) void k_spmm_splits(int32_t m, int32_t nnz, 
 
 // Boundaries seg and seg + 1 by the wave that owns the segment, for calls without a plan (a launch of k_spmm_splits
 // before it: 13.9 us against 10.0 with 85000 elements and 8 columns, 271 against 266 with 3.8 M and 100): four groups of 16
-// lanes search the points seg - 1 .. seg + 2 side by side, 16 probes at a time.
-__device__ __forceinline__ void segment_ends(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nnz, int32_t items,
-                                             int32_t nseg, int64_t seg, int32_t &x0, int32_t &y0, int32_t &x1, int32_t &y1)
+// lanes search the points seg - 1 .. seg + 2 side by side, 16 probes at a time.  rest() runs behind the first probes' requests; where it
+// says that nothing is left to do, false comes back.
+template <typename F>
+__device__ __forceinline__ bool segment_ends(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nnz, int32_t items,
+                                             int32_t nseg, int64_t seg, int32_t &x0, int32_t &y0, int32_t &x1, int32_t &y1,
+                                             const F &rest)
 {
     const int lane = threadIdx.x & (kWave - 1), q = lane >> 4, l = lane & 15;
     const int64_t total = (int64_t)m + nnz;
     int64_t d = (seg - 1 + q) * items;
     d = d < 0 ? 0 : d > total ? total : d;
     int64_t lo = d > nnz ? d - nnz : 0, hi = d < m ? d : m;
+    bool first = true;
     while (__ballot(lo < hi)) {  // uniform; a group that is done repeats its answer
         const int64_t step = (hi - lo + 15) / 16, p = lo + l * step;
-        const bool before = lo < hi && p < hi && (int64_t)row_ptr[p + 1] < d - p;  // the point lies behind p
+        const bool in = lo < hi && p < hi;
+        const int32_t end = row_ptr[in ? p + 1 : 0];
+        if (first && !rest()) return false;
+        first = false;
+        const bool before = in && (int64_t)end < d - p;  // the point lies behind p
         const int n = __popc((unsigned)(__ballot(before) >> (q * 16)) & 0xffffu);
-        const int64_t at = lo + (n > 0 ? (n - 1) * step + 1 : 0), end = lo + n * step;
+        const int64_t at = lo + (n > 0 ? (n - 1) * step + 1 : 0), to = lo + n * step;
         lo = lo < hi ? at : lo;
-        hi = end < hi ? end : hi;
+        hi = to < hi ? to : hi;
     }
     int32_t x[4], y[4];
 #pragma unroll
@@ -202,6 +210,7 @@ __device__ __forceinline__ void segment_ends(const int32_t *__restrict__ row_ptr
     };
     snap(seg, 1, x0, y0);
     snap(seg + 1, 2, x1, y1);
+    return true;
 }
 
 int launch_spmm_splits(int32_t m, int32_t nnz, int32_t items, const int32_t *row_ptr, int32_t *xs, int32_t *ys,
@@ -272,6 +281,7 @@ __device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, 
 // bits from the same old values of C, in one wave).
 // Consecutive segments run on one XCD, whose L2 then fetches the rows of B that neighbouring rows
 // of A share once.
+// ask: where the sweep kernel has been launched ahead and answered that it takes the call, what is left are rows longer than it takes.
 template <typename T, int VEC, int LOGG, int SEG>
 __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
                                                        const int32_t *__restrict__ row_ptr,
@@ -279,7 +289,7 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
                                                        const T *__restrict__ B, int64_t ldb, T beta,
                                                        T *__restrict__ C, int64_t ldc,
                                                        const int32_t *__restrict__ xs, const int32_t *__restrict__ ys,
-                                                       T *__restrict__ carry, int32_t *__restrict__ carry_row)
+                                                       T *__restrict__ carry, int32_t *__restrict__ carry_row, SweepAsk ask)
 {
     typedef typename VecOf<T, VEC>::type V;
     constexpr int G = 1 << LOGG, NG = kWave / G;
@@ -295,6 +305,16 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     const int64_t blk = (int64_t)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds;
     const int64_t seg = blk * (kBlock / kWave) + w;
     if (seg >= nseg) return;  // wave-uniform
+    int32_t least = -1;  // only rows of more elements are left to do
+    const int32_t swept = ask.answer ? *ask.answer : 0;
+    const auto rest = [&]() {
+        if (!swept) return true;
+        bool any = false;
+        for (int i = lane * 8; i < ask.blocks; i += kWave * 8) any |= *(const uint64_t *)(ask.too_long + i) != 0;
+        if (__ballot(any) == 0) return false;
+        least = ask.longest;
+        return true;
+    };
     const int grp = lane >> LOGG, gl = lane & (G - 1);
     const int64_t t0 = (int64_t)blockIdx.y * ncols / gridDim.y, t1 = (int64_t)(blockIdx.y + 1) * ncols / gridDim.y;
     int64_t c = t0 + gl * VEC;
@@ -303,10 +323,16 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     const char *Bc = (const char *)(B + c);
     const uint64_t ldb_bytes = (uint64_t)ldb * sizeof(T);
     int32_t x0, y0, x1, y1;
-    if (xs)  // uniform
+    if (xs) {  // uniform
         x0 = xs[seg], y0 = ys[seg], x1 = xs[seg + 1], y1 = ys[seg + 1];
-    else
-        segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1);
+        if (!rest()) {
+            if (carry_row && lane == 0 && blockIdx.y == 0) carry_row[seg] = -1;
+            return;
+        }
+    } else if (!segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1, rest)) {
+        if (carry_row && lane == 0 && blockIdx.y == 0) carry_row[seg] = -1;
+        return;
+    }
     const int32_t nel = y1 - y0 < kElems ? y1 - y0 : kElems, nrow = x1 - x0 < kEnds ? x1 - x0 : kEnds;
     int32_t *s_col = s_col_all[w];
     T *s_val = s_val_all[w];
@@ -364,11 +390,14 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
         return acc;
     };
     const bool stores = active && grp == 0;
+    // a row that is cut covers a segment, which holds `least` elements or more
+    const bool first_cut = least >= 0 && row_ptr[x0] != y0;
     for (int32_t r0 = 0; r0 < nrow; r0 += NG) {
         const int32_t r = r0 + grp;
         const int32_t k = r < nrow ? s_end[r] : 0, e = r < nrow ? s_end[r + 1] : 0;
-        const bool dealt = e - k <= kDealt;
-        if (r < nrow && dealt) {
+        const bool wanted = r < nrow && (e - k > least || (first_cut && r == 0));
+        const bool dealt = !wanted || e - k <= kDealt;
+        if (wanted && dealt) {
             V *out = (V *)(C + (int64_t)(x0 + r) * ldc + c);
             V c_old = T(0);
             if (beta != T(0)) c_old = *out;  // requested before the row's loads of B
@@ -462,7 +491,7 @@ __global__ __launch_bounds__(kChunkThreads, REACH == kRowsFar ? 4 : 6) void k_sp
         x0 = xs[seg], y0 = ys[seg], x1 = xs[seg + 1], y1 = ys[seg + 1];
     } else {
         if (w == 0) {
-            segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1);
+            segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1, [] { return true; });
             if (lane == 0) s_cut[0] = x0, s_cut[1] = y0, s_cut[2] = x1, s_cut[3] = y1;
         }
         __syncthreads();
@@ -641,13 +670,13 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge_fixup(int32_t m, int32_t 
 template <typename T, int VEC, int SEG>
 static void launch_merge_width(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
                                const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
-                               const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, hipStream_t s)
+                               const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, const SweepAsk &ask, hipStream_t s)
 {
     const dim3 grid((unsigned)(ceil_div64(ceil_div64(nseg, kBlock / kWave), kXcds) * kXcds), (unsigned)tiling.tiles);
 #define ASX_WIDTH(LOGG)                                                                                              \
     if (tiling.log_lanes <= LOGG) {                                                                                      \
         hipLaunchKernelGGL((k_spmm_merge<T, VEC, LOGG, SEG>), grid, dim3(kBlock), 0, s, m, nnz, items, nseg, ncols, alpha, row_ptr, col, \
-                           val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);                                     \
+                           val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, ask);                                \
         return;                                                                                                      \
     }
     ASX_WIDTH(0)
@@ -665,18 +694,18 @@ static void launch_merge_width(const SpmmTiling &tiling, int32_t m, int32_t nnz,
 template <typename T, int SEG>
 static void launch_merge_seg(const SpmmTiling &tiling, int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
                              const int32_t *row_ptr, const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc,
-                             const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, hipStream_t s)
+                             const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row, const SweepAsk &ask, hipStream_t s)
 {
     constexpr int kFull = 16 / sizeof(T);
     if (tiling.vec == kFull)
         launch_merge_width<T, kFull, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
-                                         xs, ys, carry, carry_row, s);
+                                         xs, ys, carry, carry_row, ask, s);
     else if (tiling.vec == 2)
         launch_merge_width<T, 2, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
-                                     xs, ys, carry, carry_row, s);
+                                     xs, ys, carry, carry_row, ask, s);
     else
         launch_merge_width<T, 1, SEG>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
-                                     xs, ys, carry, carry_row, s);
+                                     xs, ys, carry, carry_row, ask, s);
 }
 
 // As many lanes a group as span the columns.  rows: of B where a plan knows them, else 0.
@@ -729,7 +758,7 @@ template <typename T>
 int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_t items, int32_t ncols, T alpha, const int32_t *row_ptr,
                       const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C,
                       int64_t ldc, const int32_t *xs, const int32_t *ys, T *carry, int32_t *carry_row,
-                      bool carry_pass, int tile_bytes, hipStream_t s)
+                      bool carry_pass, int tile_bytes, const SweepAsk &ask, hipStream_t s)
 {
     if (m <= 0 || ncols <= 0) return ASX_STATUS_SUCCESS;
     // Tiles of columns are blocks along a grid's y, of which there are at most 65535: more columns are walked in slabs of whole
@@ -739,7 +768,7 @@ int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_
         for (int64_t c = 0; c < ncols; c += slab) {
             const int32_t wide = (int32_t)(ncols - c < slab ? ncols - c : slab);
             const int st = launch_spmm_merge<T>(chunked, rows, m, nnz, items, wide, alpha, row_ptr, col, val, B + c, ldb, beta, C + c,
-                                                ldc, xs, ys, carry, carry_row, carry_pass, tile_bytes, s);
+                                                ldc, xs, ys, carry, carry_row, carry_pass, tile_bytes, ask, s);
             if (st) return st;
         }
         return ASX_STATUS_SUCCESS;
@@ -752,7 +781,7 @@ int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_
     } else {
         const auto launch = [&](auto seg_) {
             launch_merge_seg<T, decltype(seg_)::value>(tiling, m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc,
-                                                       xs, ys, carry, carry_row, s);
+                                                       xs, ys, carry, carry_row, ask, s);
         };
         if (items <= kSpmmSegmentSmall)
             launch(Int<kSpmmSegmentSmall>{});
@@ -772,7 +801,7 @@ int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_
                                     const T *, int64_t, T, T *, int64_t, hipStream_t);               \
     template int launch_spmm_merge<T>(bool, int32_t, int32_t, int32_t, int32_t, int32_t, T, const int32_t *, const int32_t *, \
                                       const T *, const T *, int64_t, T, T *, int64_t, const int32_t *, \
-                                      const int32_t *, T *, int32_t *, bool, int, hipStream_t);
+                                      const int32_t *, T *, int32_t *, bool, int, const SweepAsk &, hipStream_t);
 ASX_INST(float)
 ASX_INST(double)
 #undef ASX_INST

@@ -7,6 +7,10 @@
 // elements of all rows.  Nothing orders the waves but that they do the same work a window; those ahead wait for memory, those
 // behind find their rows of B in the L2.
 //
+// Calls whose columns nobody has looked at ask the device (sweep_asks): the first wave of every workgroup looks at 64 rows spread over
+// A, all workgroups come to the same answer, and where it is no they end; the merge kernel, launched behind them, finds the
+// answer in the call's workspace and does what is left: everything, or the rows that are too long to be walked by one lane group.
+//
 // Uniform columns, 25 per row, 100 columns fp32 of 150001 rows: 258 us with the merge kernel, 15.4 M lines past the L2s; 124 here.
 // 49 per row, 96 columns of 94796 rows 316 and 136; 24 per row, 103 columns fp64 of 97486 337 and 215.
 #include "asx_internal.hpp"
@@ -64,6 +68,30 @@ constexpr uint64_t lanes_of_groups(int l, int j0, int n)
     return mask;
 }
 constexpr uint32_t kNoColumn = 0xffffffffu, kAllColumns = 0x80000000u;
+
+// Whether A looks as if its columns lay all over B and ascended in a row, and its rows were of one length: by the first and last
+// column and one between of 64 rows spread over A, one a lane, of which most have to say so (counted with ballots: every workgroup
+// looks, and sums over the lanes took half a microsecond of the 4 to 5 that asking costs).
+//   No row is longer than the sweep takes (some 4 of 64 power-law rows with exponents of up to 2.6 and a mean of 16 are), 48 have half of
+//   the mean or more (power-law rows with an exponent of 2.2 some 30).
+//   Columns ascend; 44 rows reach three quarters as far as uniform columns do on average, (len - 1) / (len + 1) of B (of uniform rows
+//   of 4 51 do, of longer ones more); and in 44 a column is a tenth of B or more from one of the next row (uniform columns 52, matrices near a
+//   diagonal, whose next row is a 64th of B away, none).
+__device__ __forceinline__ bool sweep_suits(const SweepAsk &ask, int32_t m, int32_t nnz, int lane, const int32_t *__restrict__ row_ptr,
+                                            const int32_t *__restrict__ col)
+{
+    const int64_t r = (int64_t)m * (2 * lane + 1) / (2 * kWave);
+    const int32_t s = row_ptr[r], len = row_ptr[r + 1] - s;
+    const int64_t last = (int64_t)nnz - 1, l = len > 0 ? len : 1;
+    const int64_t k0 = s < last ? s : last, k1 = k0 + l - 1 < last ? k0 + l - 1 : last;
+    const int64_t kx = k0 + ((int64_t)(lane * 0x9e3779b1u >> 8) * l >> 24);
+    const int32_t c0 = col[k0], cx = col[kx < last ? kx : last], c1 = col[k1];
+    const float n = (float)ask.n, apart = fabsf((float)cx - (float)__shfl(cx, (lane + 1) & (kWave - 1), kWave));
+    const uint64_t far = __ballot(len > ask.longest), half = __ballot(2.0f * (float)len * (float)m >= (float)nnz);
+    const uint64_t falls = __ballot(cx < c0 || c1 < cx);
+    const uint64_t reach = __ballot(((float)c1 - (float)c0) * (float)(l + 1) >= 0.75f * n * (float)(l - 1)), across = __ballot(apart >= 0.1f * n);
+    return far == 0 && falls == 0 && __popcll(half) >= 48 && __popcll(reach) >= 44 && __popcll(across) >= 44;
+}
 constexpr int sweep_batch(int slots) { return slots == 20 ? 5 : slots == 12 ? 6 : slots == 4 ? 4 : 8; }
 
 // A group of L = 2^LOGL lanes, 16 bytes a lane, spans a tile of a row of B; the wave's NG groups have `rows` rows of C each, in S
@@ -75,9 +103,11 @@ constexpr int sweep_batch(int slots) { return slots == 20 ? 5 : slots == 12 ? 6 
 // and a load 16 cycles of a compute unit's L1 where all lanes take part, none where none does - slots without an element are
 // masked out, not sent past a buffer's end (119 us against 157 for the first example above) -; and lines past the L2s for what
 // waves are apart.  Batches of G slots, all loads of a batch ahead of its sums.
-template <typename T, int LOGL, int S>
+//
+// ASK: the call does not know its columns (above).  Rows longer than ask.longest are left to the merge kernel.
+template <typename T, int LOGL, int S, bool ASK>
 __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
-    int32_t m, int32_t rows, int32_t cap, uint32_t width, uint32_t last, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
+    SweepAsk ask, int32_t m, int32_t nnz, int32_t rows, int32_t cap, uint32_t width, uint32_t last, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
     const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ B, int64_t ldb, T beta, T *__restrict__ C, int64_t ldc)
 {
     typedef typename Vec16<T>::type V;
@@ -89,8 +119,8 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
     const uint32_t per_xcd = gridDim.x / kXcds;
     const int64_t wave = ((int64_t)(blockIdx.x % kXcds) * per_xcd + blockIdx.x / kXcds) * (kBlock / kWave) + w;
     const int64_t x0 = wave * rows * NG;
-    if (x0 >= m) return;
-    const int32_t nrow = (int32_t)(m - x0 < rows * NG ? m - x0 : rows * NG);
+    if (!ASK && x0 >= m) return;
+    const int32_t nrow = (int32_t)(x0 >= m ? 0 : m - x0 < rows * NG ? m - x0 : rows * NG);
     const int grp = lane >> LOGL, gl = lane & (L - 1);
     const int32_t t0 = (int32_t)((int64_t)blockIdx.y * ncols / gridDim.y), t1 = (int32_t)((int64_t)(blockIdx.y + 1) * ncols / gridDim.y);
     int32_t c = t0 + gl * VEC;
@@ -103,8 +133,28 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
 
     // the lane's row: element s up to e
     const int32_t mine = grp * rows + gl;
-    const bool has_row = gl < rows && mine < nrow;
-    const int32_t s = has_row ? row_ptr[x0 + mine] : 0, e = has_row ? row_ptr[x0 + mine + 1] : 0;
+    bool has_row = gl < rows && mine < nrow;
+    int32_t s = has_row ? row_ptr[x0 + mine] : 0, e = has_row ? row_ptr[x0 + mine + 1] : 0;
+    if constexpr (ASK) {
+        __shared__ int s_yes, s_long[kBlock / kWave];
+        const bool too_long = e - s > ask.longest;
+        const bool some = __ballot(too_long) != 0;
+        if (lane == 0) s_long[w] = some;
+        if (w == 0) {
+            const bool yes = sweep_suits(ask, m, nnz, lane, row_ptr, col);
+            if (lane == 0) s_yes = yes;
+        }
+        __syncthreads();
+        if (threadIdx.x == 0) {
+            int any = 0;
+            for (int i = 0; i < kBlock / kWave; ++i) any |= s_long[i];
+            ask.too_long[blockIdx.x] = (uint8_t)any;
+            if (blockIdx.x == 0) *ask.answer = s_yes;
+        }
+        if (!s_yes || x0 >= m) return;
+        if (too_long) has_row = false, s = e = 0;
+    }
+    const uint64_t kept = __ballot(has_row);
     const int32_t begin = __builtin_amdgcn_readfirstlane(row_ptr[x0]), end = __builtin_amdgcn_readfirstlane(row_ptr[x0 + nrow]);
 
     V acc[S];
@@ -125,7 +175,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
                 const int i = i0 + j * kWave + lane;
-                if (i < nel) s_col[i] = (uint32_t)tc[j], s_val[i] = tv[j];
+                if (i < nel) s_col[i] = (uint32_t)tc[j] & ~kAllColumns, s_val[i] = tv[j];  // 31 bits: every column comes up in a window
             }
         }
         // the staged data is private to this wave: order its LDS writes before its LDS reads
@@ -175,7 +225,18 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
             });
         } while (more);
         from += nel;
-        if (from < end) __builtin_amdgcn_wave_barrier();
+        if (from < end) {
+            __builtin_amdgcn_wave_barrier();
+            if constexpr (ASK) {  // past rows that are left out
+                int32_t at = e > from ? (s > from ? s : from) : end;
+#pragma unroll
+                for (int d = 1; d < kWave; d <<= 1) {
+                    const int32_t other = __shfl_xor(at, d, kWave);
+                    at = other < at ? other : at;
+                }
+                from = __builtin_amdgcn_readfirstlane(at);
+            }
+        }
     }
     static_for<0, S / G>([&](auto g_) {
         constexpr int j0 = decltype(g_)::value * G;
@@ -183,29 +244,29 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
         static_for<0, G>([&](auto u_) {
             constexpr int j = j0 + decltype(u_)::value;
             c_old[decltype(u_)::value] = T(0);
-            if (beta != T(0) && j < rows && grp * rows + j < nrow)
+            if (beta != T(0) && (kept >> (grp * L + j) & 1))
                 c_old[decltype(u_)::value] = *(const V *)(C + (x0 + grp * rows + j) * ldc + c);
         });
         static_for<0, G>([&](auto u_) {
             constexpr int j = j0 + decltype(u_)::value;
             const V y = beta == T(0) ? (V)(alpha * acc[j]) : __builtin_elementwise_fma((V)alpha, acc[j], (V)(beta * c_old[decltype(u_)::value]));
-            if (active && j < rows && grp * rows + j < nrow) *(V *)(C + (x0 + grp * rows + j) * ldc + c) = y;
+            if (active && (kept >> (grp * L + j) & 1)) *(V *)(C + (x0 + grp * rows + j) * ldc + c) = y;
         });
     });
 }
 
-template <typename T>
-int launch_spmm_sweep(const SpmmSweep &sw, int32_t m, int32_t n, int32_t ncols, T alpha, const int32_t *row_ptr, const int32_t *col, const T *val,
-                      const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s)
+template <typename T, bool ASK>
+static int launch_sweep(const SpmmSweep &sw, const SweepAsk &ask, int32_t m, int32_t n, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
+                        const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s)
 {
-    const int64_t waves = ceil_div64(m, (int64_t)sw.rows * (kWave >> sw.log_lanes));
-    const dim3 grid((unsigned)(ceil_div64(ceil_div64(waves, kBlock / kWave), kXcds) * kXcds), (unsigned)sw.tiles);
-    const size_t lds = (size_t)sw.cap * (sizeof(T) + 4) * (kBlock / kWave);
+    const dim3 grid((unsigned)spmm_sweep_blocks(sw, m), (unsigned)sw.tiles);
+    const int32_t cap = ASK ? std::min(sw.cap, spmm_sweep_cap(sizeof(T)) - 2) : sw.cap;  // asking takes 20 bytes of LDS
+    const size_t lds = (size_t)cap * (sizeof(T) + 4) * (kBlock / kWave);
     const uint32_t last = (uint32_t)n > sw.width ? (uint32_t)n - sw.width : 0;
 #define ASX_SWEEP(LOGL, S)                                                                                                              \
     if (sw.log_lanes == LOGL && sw.slots == S) {                                                                                        \
-        hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S>), grid, dim3(kBlock), lds, s, m, sw.rows, sw.cap, sw.width, last, ncols, alpha, \
-                           row_ptr, col, val, B, ldb, beta, C, ldc);                                                                    \
+        hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S, ASK>), grid, dim3(kBlock), lds, s, ask, m, nnz, sw.rows, cap, sw.width, last,      \
+                           ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc);                                                      \
         return check_launch();                                                                                                          \
     }
     ASX_SWEEP(3, 4)
@@ -228,9 +289,19 @@ int launch_spmm_sweep(const SpmmSweep &sw, int32_t m, int32_t n, int32_t ncols, 
     return ASX_STATUS_INTERNAL_ERROR;
 }
 
-template int launch_spmm_sweep<float>(const SpmmSweep &, int32_t, int32_t, int32_t, float, const int32_t *, const int32_t *, const float *,
-                                      const float *, int64_t, float, float *, int64_t, hipStream_t);
-template int launch_spmm_sweep<double>(const SpmmSweep &, int32_t, int32_t, int32_t, double, const int32_t *, const int32_t *, const double *,
-                                       const double *, int64_t, double, double *, int64_t, hipStream_t);
+template <typename T>
+int launch_spmm_sweep(const SpmmSweep &sw, const SweepAsk *ask, int32_t m, int32_t n, int32_t nnz, int32_t ncols, T alpha, const int32_t *row_ptr,
+                      const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s)
+{
+    if (ask) return launch_sweep<T, true>(sw, *ask, m, n, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, s);
+    return launch_sweep<T, false>(sw, SweepAsk{}, m, n, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, s);
+}
+
+#define ASX_INST(T)                                                                                                                      \
+    template int launch_spmm_sweep<T>(const SpmmSweep &, const SweepAsk *, int32_t, int32_t, int32_t, int32_t, T, const int32_t *,       \
+                                      const int32_t *, const T *, const T *, int64_t, T, T *, int64_t, hipStream_t);
+ASX_INST(float)
+ASX_INST(double)
+#undef ASX_INST
 
 }  // namespace asx
