@@ -490,7 +490,9 @@ inline bool spmm_everywhere(double spread, double span, double falls, double mea
 //   Windows: the more, the less of B a window needs (a wave ahead or behind does less harm), but every window costs its
 //   instructions whether rows have an element in it or not: 1.24 MB(B)^0.35 mean^-0.3 windows an element of a mean row, between 1
 //   and 2.5, fitted to 110 uniform matrices (both types, rows of B of 72 to 2000 bytes, 4 to 64 per row, B of 14 to 317 MB)
-//   timed with 1 to 6: 0.5 % behind the best of these on average.
+//   timed with 1 to 6: 0.5 % behind the best of these on average; a tenth less where a group has 16 lanes or more, which inputs that
+//   are not in the Infinity Cache want (74 such matrices, three sets of inputs in turn: 0.986 of the time with the tenth; 100
+//   columns fp32, 150001 rows of 25 150 us and 141).
 //   On those 110 it takes 0.78 of the row-ordered kernels' time on average (100 columns fp32, 160000 rows of 25 270 us against
 //   130; 96, 94796 of 49 316 and 136; 64, 573065 of 9 204 and 191; 22, 1 M of 4 138 and 133).  Not taken: a B that the L2s keep
 //   between them (9 MB, 14 where rows of A are short) - where rows of B start on lines the row-ordered kernels work through it
@@ -539,7 +541,7 @@ inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, si
     const double mean = (double)nnz / m, mb = 1e-6 * (double)bytes * n;
     if (bytes % 128 == 0 ? mb < 20.0 || n < 40000 : mb < (mean < 14.0 ? 14.0 : 9.0)) return SpmmSweep{};
     if (spmm_sweep_shared(sw, m, n, nnz) < kSweepSharedLeast) return SpmmSweep{};
-    const double windows = mean * std::min(std::max(1.24 * pow(mb, 0.35) * pow(mean, -0.3), 1.0), 2.5);
+    const double windows = (sw.log_lanes >= 4 ? 0.9 : 1.0) * mean * std::min(std::max(1.24 * pow(mb, 0.35) * pow(mean, -0.3), 1.0), 2.5);
     sw.width = (uint32_t)std::max((double)n / windows, 1.0) + 1;
     return sw;
 }
