@@ -35,10 +35,13 @@ __device__ __forceinline__ void mark_blocks(int64_t r, int32_t m, int32_t s, int
     }
 }
 
+// parts: the workgroup's own counts, 37 words a workgroup (bin, longest and classes one behind the other, `blocks` of each), instead
+// of atomics on hist and stats.
+constexpr int kHistogramTurns = 8;  // of 256 rows, whose offsets a workgroup requests together
 template <bool MARK = false>
 __device__ __forceinline__ void row_histogram(const int32_t *__restrict__ row_ptr, int32_t m, int64_t block, int64_t blocks,
                                               unsigned long long *hist /*33*/, unsigned long long *stats /*4*/,
-                                              int32_t nb = 0, int2 *__restrict__ row_blocks = nullptr)
+                                              int32_t nb = 0, int2 *__restrict__ row_blocks = nullptr, uint32_t *__restrict__ parts = nullptr)
 {
     __shared__ unsigned int s_hist[33];
     __shared__ unsigned int s_bins[3];
@@ -49,34 +52,49 @@ __device__ __forceinline__ void row_histogram(const int32_t *__restrict__ row_pt
     __syncthreads();
     int local_max = 0;
     const int lane = threadIdx.x & (kWave - 1);
-    for (int64_t r0 = block * 256; r0 < m; r0 += blocks * 256) {  // uniform
-        const int64_t r = r0 + threadIdx.x;
-        const bool valid = r < m;
-        const int32_t from = valid ? row_ptr[r] : 0, to = valid ? row_ptr[r + 1] : 0;
-        const int len = to - from;
-        if (MARK && valid) mark_blocks(r, m, from, to, nb, row_blocks);
-        const int bin = len <= 0 ? 0 : 32 - __clz(len);
-        // one LDS atomic per distinct bin among the wave's 64 rows (rows of one length would
-        // otherwise serialise 64 atomics on one address)
-        unsigned long long todo = __ballot(valid);
-        while (todo) {  // uniform
-            const int first = __builtin_ctzll(todo);
-            const int b = __builtin_amdgcn_readlane(bin, first);
-            const unsigned long long same = __ballot(valid && bin == b);
-            if (lane == first) atomicAdd(&s_hist[b], (unsigned int)__popcll(same));
-            todo &= ~same;
+    for (int64_t r00 = block * 256; r00 < m; r00 += blocks * 256 * kHistogramTurns) {  // uniform
+        int32_t starts[kHistogramTurns], ends[kHistogramTurns];
+#pragma unroll
+        for (int u = 0; u < kHistogramTurns; ++u) {
+            const int64_t r = r00 + u * blocks * 256 + threadIdx.x;
+            starts[u] = row_ptr[r < m ? r : 0], ends[u] = row_ptr[r < m ? r + 1 : 0];
         }
-        const unsigned int c0 = __popcll(__ballot(valid && len < 2)), c1 = __popcll(__ballot(valid && len >= 2 && len < 1024));
-        const unsigned int c2 = __popcll(__ballot(valid && len >= 1024));
-        if (lane == 0) {
-            if (c0) atomicAdd(&s_bins[0], c0);
-            if (c1) atomicAdd(&s_bins[1], c1);
-            if (c2) atomicAdd(&s_bins[2], c2);
+#pragma unroll
+        for (int u = 0; u < kHistogramTurns; ++u) {
+            const int64_t r = r00 + u * blocks * 256 + threadIdx.x;
+            const bool valid = r < m;
+            const int32_t from = valid ? starts[u] : 0, to = valid ? ends[u] : 0;
+            const int len = to - from;
+            if (MARK && valid) mark_blocks(r, m, from, to, nb, row_blocks);
+            const int bin = len <= 0 ? 0 : 32 - __clz(len);
+            // one LDS atomic per distinct bin among the wave's 64 rows (rows of one length would
+            // otherwise serialise 64 atomics on one address)
+            unsigned long long todo = __ballot(valid);
+            while (todo) {  // uniform
+                const int first = __builtin_ctzll(todo);
+                const int b = __builtin_amdgcn_readlane(bin, first);
+                const unsigned long long same = __ballot(valid && bin == b);
+                if (lane == first) atomicAdd(&s_hist[b], (unsigned int)__popcll(same));
+                todo &= ~same;
+            }
+            const unsigned int c0 = __popcll(__ballot(valid && len < 2)), c1 = __popcll(__ballot(valid && len >= 2 && len < 1024));
+            const unsigned int c2 = __popcll(__ballot(valid && len >= 1024));
+            if (lane == 0) {
+                if (c0) atomicAdd(&s_bins[0], c0);
+                if (c1) atomicAdd(&s_bins[1], c1);
+                if (c2) atomicAdd(&s_bins[2], c2);
+            }
+            local_max = len > local_max ? len : local_max;
         }
-        local_max = len > local_max ? len : local_max;
     }
     atomicMax(&s_max, local_max);
     __syncthreads();
+    if (parts) {
+        if (threadIdx.x < 33) parts[threadIdx.x * blocks + block] = s_hist[threadIdx.x];
+        if (threadIdx.x == 33) parts[33 * blocks + block] = (uint32_t)s_max;
+        if (threadIdx.x >= 34 && threadIdx.x < 37) parts[threadIdx.x * blocks + block] = s_bins[threadIdx.x - 34];
+        return;
+    }
     if (threadIdx.x < 33 && s_hist[threadIdx.x])
         atomicAdd(&hist[threadIdx.x], (unsigned long long)s_hist[threadIdx.x]);
     if (threadIdx.x < 3 && s_bins[threadIdx.x])
@@ -92,9 +110,10 @@ __global__ __launch_bounds__(256) void k_row_histogram(const int32_t *__restrict
 
 static unsigned histogram_blocks(int32_t m)
 {
-    const int64_t grid = ceil_div64(m, 256 * 8);
+    const int64_t grid = ceil_div64(m, 256 * kHistogramTurns);
     return (unsigned)(grid > 4096 ? 4096 : grid);
 }
+static unsigned histogram_parts(int32_t m) { return std::min(histogram_blocks(m), 1024u); }  // whose counts one workgroup adds up
 
 int launch_row_histogram(const int32_t *d_row_ptr, int32_t m, int64_t *d_hist, int64_t *d_stats,
                          hipStream_t s)
@@ -329,7 +348,7 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
     constexpr int kSlots = 4096;
     __shared__ int32_t table[kSlots];
     __shared__ uint32_t starts[kFlatTile / 32];  // bit i: element i of the tile is the first of its row
-    __shared__ int32_t count, pairs, lowest, highest;
+    __shared__ int32_t count, pairs, lowest, highest, rows[2];
     for (int i = threadIdx.x; i < kSlots; i += kBlock) table[i] = -1;
     if (threadIdx.x < kFlatTile / 32) starts[threadIdx.x] = 0;
     if (threadIdx.x == 0) count = 0, pairs = 0, lowest = 0x7fffffff, highest = 0;
@@ -347,8 +366,11 @@ __device__ __forceinline__ void sample_columns_tile(const SampleArgs &q, int t)
     if (q.row_ptr) {
         // the rows that start in the tile: found by two searches, marked by one read each (a search
         // per element was a chain of twenty reads, 23 us for the whole sample)
-        const int32_t lo = wave_row_holding(q.row_ptr, 0, q.m, (int32_t)first),
-                      hi = wave_row_holding(q.row_ptr, lo, q.m, (int32_t)(first + kFlatTile - 1));
+        const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
+        const int32_t r = wave_row_holding(q.row_ptr, 0, q.m, (int32_t)(w & 1 ? first + kFlatTile - 1 : first));
+        if (threadIdx.x < 2 * kWave && threadIdx.x % kWave == 0) rows[w] = r;
+        __syncthreads();
+        const int32_t lo = rows[0], hi = rows[1];
         for (int64_t r = (int64_t)lo + threadIdx.x; r <= hi && r < q.m; r += kBlock) {
             const int64_t at = (int64_t)q.row_ptr[r] - first;
             if (at >= 0 && at < kFlatTile) atomicOr(&starts[at >> 5], 1u << (at & 31));
@@ -405,29 +427,65 @@ int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const
 // What an analysis looks at first, in one launch: the sample (its workgroups first, they take longest) and the
 // histogram of the row lengths; with row_blocks also the row blocks of the stream kernel, which come with the row offsets
 // that are read anyway (searched for afterwards they took a kernel of 7 us and a second wait for the device).
+// Every workgroup leaves its own counts, and k_plan_totals adds them up into the plan's counters and into page-locked memory of the
+// host: counters set to zero ahead and copied to the host behind were a launch and a copy more.
 __global__ __launch_bounds__(kBlock) void k_plan_stats(SampleArgs q, const int32_t *__restrict__ row_ptr, int32_t m,
-                                                       unsigned long long *hist, unsigned long long *stats, int32_t nb,
-                                                       int2 *__restrict__ row_blocks)
+                                                       uint32_t *__restrict__ parts, int32_t nb, int2 *__restrict__ row_blocks)
 {
     if ((int)blockIdx.x < q.samples)
         sample_columns_tile(q, blockIdx.x);
     else if (row_blocks)
-        row_histogram<true>(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, hist, stats, nb, row_blocks);
+        row_histogram<true>(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, nullptr, nullptr, nb, row_blocks, parts);
     else
-        row_histogram(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, hist, stats);
+        row_histogram(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, nullptr, nullptr, 0, nullptr, parts);
 }
 
-int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int64_t *d_hist, int64_t *d_stats,
-                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample,
-                      int32_t nb, int32_t *d_row_blocks, hipStream_t s)
+// counters[0 .. 36] = what k_plan_stats counted, the sample at `sampled`, 0 elsewhere; the same to the host.  A wave a count.
+__global__ __launch_bounds__(1024) void k_plan_totals(const uint32_t *__restrict__ parts, int blocks, const int32_t *__restrict__ sample, int samples,
+                                                      int64_t *__restrict__ counters, int ncounters, int sampled, int64_t *__restrict__ host)
+{
+    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
+    for (int i = 37 + threadIdx.x; i < ncounters; i += 1024) {
+        const int t = 2 * (i - sampled);  // two words of the sample a counter
+        uint64_t v = 0;
+        if (i >= sampled && t < 2 * 64) {
+            const uint32_t lo = (t & 63) < samples ? (uint32_t)sample[t] : 0u, hi = (t & 63) + 1 < samples ? (uint32_t)sample[t + 1] : 0u;
+            v = (uint64_t)hi << 32 | lo;
+        }
+        counters[i] = (int64_t)v;
+        host[i] = (int64_t)v;
+    }
+    for (int c = w; c < 37; c += 1024 / kWave) {
+        uint64_t total = 0;
+        for (int b = lane; b < blocks; b += kWave) {
+            const uint32_t v = parts[(int64_t)c * blocks + b];
+            total = c == 33 ? (v > total ? v : total) : total + v;
+        }
+#pragma unroll
+        for (int d = 1; d < kWave; d <<= 1) {
+            const uint64_t other = __shfl_xor((unsigned long long)total, d, kWave);
+            total = c == 33 ? (other > total ? other : total) : total + other;
+        }
+        if (lane == 0) counters[c] = (int64_t)total, host[c] = (int64_t)total;
+    }
+}
+
+size_t plan_stats_bytes(int32_t m) { return (size_t)histogram_parts(m) * 37 * sizeof(uint32_t) + 128 * sizeof(int32_t); }
+
+int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int sampled, int64_t *h_counters,
+                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, void *d_scratch, int32_t nb,
+                      int32_t *d_row_blocks, hipStream_t s)
 {
     if (samples < 0 || samples > 64) return ASX_STATUS_INVALID_VALUE;
-    hipLaunchKernelGGL(k_zero_i64, dim3(1), dim3(256), 0, s, d_counters, ncounters);
+    int32_t *d_sample = static_cast<int32_t *>(d_scratch);
+    uint32_t *d_parts = reinterpret_cast<uint32_t *>(d_sample + 128);
+    const unsigned blocks = histogram_parts(m);
     if (m > 0) {
         const SampleArgs q{d_col, stride, shift, d_row_ptr, m, width, samples, d_sample};
-        hipLaunchKernelGGL(k_plan_stats, dim3(histogram_blocks(m) + (unsigned)samples), dim3(kBlock), 0, s, q, d_row_ptr, m,
-                           (unsigned long long *)d_hist, (unsigned long long *)d_stats, nb, reinterpret_cast<int2 *>(d_row_blocks));
+        hipLaunchKernelGGL(k_plan_stats, dim3(blocks + (unsigned)samples), dim3(kBlock), 0, s, q, d_row_ptr, m, d_parts, nb,
+                           reinterpret_cast<int2 *>(d_row_blocks));
     }
+    hipLaunchKernelGGL(k_plan_totals, dim3(1), dim3(1024), 0, s, d_parts, (int)blocks, d_sample, (int)samples, d_counters, ncounters, sampled, h_counters);
     return check_launch();
 }
 

@@ -432,13 +432,13 @@ int plan_begin(asx_plan **out, int is_spmm, int value_type, int32_t m, int32_t n
     const int32_t nb = std::max(stream_blocks(nnz), 1);
     p->nmarked = mark_blocks && samples > 0 && nb <= kMarkedBlocksMost ? nb : 0;
     const size_t marked_bytes = p->nmarked > 0 ? ((size_t)nb + 1) * sizeof(int2) : 0;
+    void *d_parts = nullptr;
     int st = h ? status_of(pool_malloc(&p->d_counters, kPlanCounters * sizeof(int64_t) + marked_bytes, false)) : ASX_STATUS_ALLOC_FAILED;
+    if (!st) st = status_of(scratch.take(&d_parts, plan_stats_bytes(m)));
     if (!st)
-        st = launch_plan_stats(d_row_ptr, m, p->d_counters, kPlanCounters, p->d_counters, p->d_counters + 33, d_col, sample_stride(nnz),
-                               line_shift(sv), (int32_t)(kSliceBytes / sv), samples,
-                               reinterpret_cast<int32_t *>(p->d_counters + 64), nb,
+        st = launch_plan_stats(d_row_ptr, m, p->d_counters, kPlanCounters, 64, h, d_col, sample_stride(nnz),
+                               line_shift(sv), (int32_t)(kSliceBytes / sv), samples, d_parts, nb,
                                p->nmarked > 0 ? reinterpret_cast<int32_t *>(p->d_counters + kPlanCounters) : nullptr, s);
-    if (!st) st = status_of(hipMemcpyAsync(h, p->d_counters, kPlanCounters * sizeof(int64_t), hipMemcpyDeviceToHost, s));
     if (ask_memory) {  // while the device counts
         size_t total = 0;
         if (hipMemGetInfo(&more->free_bytes, &total) != hipSuccess) more->free_bytes = 0;

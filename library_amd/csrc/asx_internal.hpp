@@ -166,10 +166,12 @@ int launch_checksum(const void *d_data, size_t bytes, unsigned long long *d_part
 int launch_checksum_commit(const unsigned long long *d_now, unsigned long long *d_kept, hipStream_t s);
 int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const int32_t *d_row_ptr, int32_t m,
                           int32_t width, int32_t samples, int32_t *d_out, hipStream_t s);
-// the counters set to zero, then launch_row_histogram and launch_sample_columns in one launch (samples = 0: no sample);
-// d_row_blocks: the nb row blocks of launch_stream_row_blocks too (null: not wanted)
-int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int64_t *d_hist, int64_t *d_stats,
-                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, int32_t *d_sample, int32_t nb,
+// what launch_row_histogram and launch_sample_columns count (samples = 0: no sample), in one launch and one that adds up: the histogram,
+// the stats and, from word `sampled` on, the sample, in d_counters, the other words 0, and the same in h_counters (page-locked);
+// d_scratch: plan_stats_bytes; d_row_blocks: the nb row blocks of launch_stream_row_blocks too (null: not wanted)
+size_t plan_stats_bytes(int32_t m);
+int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, int ncounters, int sampled, int64_t *h_counters,
+                      const int32_t *d_col, int64_t stride, int shift, int32_t width, int32_t samples, void *d_scratch, int32_t nb,
                       int32_t *d_row_blocks, hipStream_t s);
 int launch_gather_lines(const void *d_buf, size_t bytes, int group_lanes, int per_lane, void *d_out, int *nthreads,
                         hipStream_t s);
