@@ -94,10 +94,10 @@ namespace {
 //   2. k_transpose_bucket: the block's elements are ranked inside their buckets (stable: row order
 //      survives), ordered by bucket in LDS and written - row, column inside the bucket, value - in runs
 //      of consecutive places.
-//   3. k_transpose_rows: one workgroup per bucket counts the bucket's columns, writes their row
-//      offsets, and orders the elements by column, up to 4096 at a time, through LDS: a bucket that
-//      fits leaves as one run of consecutive stores.  Buckets far above the average follow in pieces.
-// 3.6 M elements, fp32, 250013 columns: 120 us with the CSR multiply that follows it; a radix sort of
+//   3. k_transpose_rows: one workgroup per bucket orders its elements by column through LDS and writes the columns' row
+//      offsets: up to 8 elements a thread in one turn, larger buckets 4096 elements at a time behind a
+//      count of their columns.  Buckets far above the average follow in pieces.
+// 3.6 M elements, fp32, 250013 columns: 97 us with the CSR multiply that follows it; a radix sort of
 // 64-bit (column, row) keys moved 24 bytes an element five times and took 316 us of kernels alone.
 constexpr int kBuckets = 1024;
 constexpr int kBucketColumns = 4096;  // the most columns a bucket may span: 16-bit counters per wave in LDS
@@ -228,16 +228,17 @@ __global__ __launch_bounds__(kSortThreads, sizeof(T) == 4 ? 8 : 6) void k_transp
     for (int j = tid; j < count; j += kSortThreads) bval[to[col_s[j] >> shift] + j] = val_s[j];
 }
 
-// in-place exclusive sum of a[0 .. COLS) by the whole workgroup, COLS a multiple of kSortThreads (barriers inside)
-template <int COLS>
+// in-place exclusive sum of a[0 .. COLS) by the whole workgroup, COLS a multiple of THREADS or the other way round (barriers inside)
+template <int COLS, int THREADS = kSortThreads>
 __device__ __forceinline__ void columns_exclusive_sum(int32_t *a, int32_t *wave_tot)
 {
-    constexpr int Q = COLS / kSortThreads;
+    constexpr int Q = COLS > THREADS ? COLS / THREADS : 1;
+    const bool has = (int)threadIdx.x * Q < COLS;
     const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = tid / kWave;
     int32_t v[Q], mine = 0;
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        v[q] = a[tid * Q + q];
+        v[q] = has ? a[tid * Q + q] : 0;
         mine += v[q];
     }
     int32_t incl = mine;
@@ -252,30 +253,31 @@ __device__ __forceinline__ void columns_exclusive_sum(int32_t *a, int32_t *wave_
     for (int w = 0; w < wave; ++w) run += wave_tot[w];
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
-        a[tid * Q + q] = run;
+        if (has) a[tid * Q + q] = run;
         run += v[q];
     }
     __syncthreads();
 }
 
 // COLS: columns of a bucket, rounded up to a multiple of kSortThreads
-template <typename T, int COLS>
+template <typename T, int COLS, int THREADS = kSortThreads>
 struct RowsShared {
-    alignas(16) uint16_t cnt[kSortWaves * COLS];  // per wave and column: count, then first rank of the wave's elements
+    alignas(16) uint16_t cnt[THREADS / kWave * COLS];  // per wave and column: count, then first rank of the wave's elements
     int32_t first[COLS];                          // per column: next free place in A^T
     int32_t lofs[COLS];                           // per column: count, then first position in column order
-    int32_t wave_tot[kSortWaves];
+    int32_t wave_tot[THREADS / kWave];
     int32_t row_s[kSortElems];
     uint16_t col_s[kSortElems];
     T val_s[kSortElems];
 };
 
 // Elements [s0, s1) of a bucket to their places in A^T, sh.first[c] being that of the first one of column c.
-template <typename T, int COLS>
-__device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t s0, int32_t s1, int nbits,
+template <typename T, int COLS, int THREADS = kSortThreads>
+__device__ __forceinline__ void place_by_column(RowsShared<T, COLS, THREADS> &sh, int32_t s0, int32_t s1, int nbits,
                                                 const int32_t *__restrict__ brow, const uint16_t *__restrict__ bcol,
                                                 const T *__restrict__ bval, int32_t *__restrict__ col_t, T *__restrict__ val_t)
 {
+    constexpr int WAVES = THREADS / kWave, PER = kSortElems / THREADS;
     uint16_t *cnt = sh.cnt, *col_s = sh.col_s;
     int32_t *first = sh.first, *lofs = sh.lofs, *row_s = sh.row_s;
     T *val_s = sh.val_s;
@@ -283,12 +285,12 @@ __device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t
     uint16_t *mycnt = cnt + wave * COLS;
     for (int32_t e0 = s0; e0 < s1; e0 += kSortElems) {  // uniform; one turn where the bucket fits
         __syncthreads();
-        for (int i = tid; i < kSortWaves * COLS / 2; i += kSortThreads) reinterpret_cast<uint32_t *>(cnt)[i] = 0;
-        const int32_t wbase = e0 + wave * kSortWaveElems;
-        int32_t c[kSortPerLane], p[kSortPerLane], r[kSortPerLane];
-        T v[kSortPerLane];
+        for (int i = tid; i < WAVES * COLS / 2; i += THREADS) reinterpret_cast<uint32_t *>(cnt)[i] = 0;
+        const int32_t wbase = e0 + wave * (kSortElems / WAVES);
+        int32_t c[PER], p[PER], r[PER];
+        T v[PER];
 #pragma unroll
-        for (int k = 0; k < kSortPerLane; ++k) {
+        for (int k = 0; k < PER; ++k) {
             const int32_t i = wbase + k * kWave + lane, at = i < s1 ? i : s1 - 1;
             c[k] = bcol[at];
             r[k] = brow[at];
@@ -296,12 +298,12 @@ __device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t
         }
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < kSortPerLane; ++k) p[k] = wave_rank(c[k], wbase + k * kWave + lane < s1, nbits, mycnt);
+        for (int k = 0; k < PER; ++k) p[k] = wave_rank(c[k], wbase + k * kWave + lane < s1, nbits, mycnt);
         __syncthreads();
-        for (int i = tid; i < COLS; i += kSortThreads) {
+        for (int i = tid; i < COLS; i += THREADS) {
             int32_t run = 0;
 #pragma unroll
-            for (int w = 0; w < kSortWaves; ++w) {
+            for (int w = 0; w < WAVES; ++w) {
                 const int32_t t = cnt[w * COLS + i];
                 cnt[w * COLS + i] = (uint16_t)run;
                 run += t;
@@ -309,9 +311,9 @@ __device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t
             lofs[i] = run;
         }
         __syncthreads();
-        columns_exclusive_sum<COLS>(lofs, sh.wave_tot);
+        columns_exclusive_sum<COLS, THREADS>(lofs, sh.wave_tot);
 #pragma unroll
-        for (int k = 0; k < kSortPerLane; ++k) {
+        for (int k = 0; k < PER; ++k) {
             if (wbase + k * kWave + lane < s1) {
                 const int32_t q = lofs[c[k]] + mycnt[c[k]] + p[k];
                 col_s[q] = (uint16_t)c[k];
@@ -321,14 +323,14 @@ __device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t
         }
         __syncthreads();
         const int32_t count = s1 - e0 < kSortElems ? s1 - e0 : kSortElems;
-        for (int j = tid; j < count; j += kSortThreads) {
+        for (int j = tid; j < count; j += THREADS) {
             const int32_t q = col_s[j], d = first[q] + (j - lofs[q]);
             col_t[d] = row_s[j];
             val_t[d] = val_s[j];
         }
         if (e0 + kSortElems < s1) {  // uniform: where the next elements of every column go
             __syncthreads();
-            for (int i = tid; i < COLS; i += kSortThreads) first[i] += (i + 1 < COLS ? lofs[i + 1] : count) - lofs[i];
+            for (int i = tid; i < COLS; i += THREADS) first[i] += (i + 1 < COLS ? lofs[i + 1] : count) - lofs[i];
         }
     }
 }
@@ -340,46 +342,137 @@ __device__ __forceinline__ void place_by_column(RowsShared<T, COLS> &sh, int32_t
 // (page-locked, cleared).
 constexpr int32_t kLargeBucket = 16 * kSortElems, kLargePiece = 8 * kSortElems;
 
-template <typename T, int COLS>
-__global__ __launch_bounds__(kSortThreads) void k_transpose_rows(const int32_t *__restrict__ offs, int32_t nblocks, int shift,
-                                                                 int nbits, int32_t n, int32_t nnz,
-                                                                 const int32_t *__restrict__ brow,
-                                                                 const uint16_t *__restrict__ bcol, const T *__restrict__ bval,
-                                                                 int32_t *__restrict__ row_ptr_t, int32_t *__restrict__ col_t,
-                                                                 T *__restrict__ val_t, int32_t *__restrict__ large)
+// A bucket of up to PER elements a thread is sorted in one turn: its elements are loaded once, ranked, and what the waves have counted
+// per column gives the row offsets of A^T as well as the places, which are consecutive then.  Buckets of 4096 to 8192 elements take
+// 1024 threads instead of a count and two turns of 512, one workgroup behind the other on a compute unit being what bounds the kernel;
+// counters and staged elements share LDS and values are loaded late, so that two such workgroups fit (64 registers).
+// 3.6 M elements of 489 buckets, fp32: 25.9 -> 19.6 us.  Transpose and multiply, 4 M uniform elements into 200013 rows: fp32 127 -> 112
+// us, fp64 149 -> 134; 1 M in one turn of 512 threads 62 -> 59.
+template <typename T, int COLS, int THREADS>
+struct OneTurn {
+    static constexpr int PER = 8, WAVES = THREADS / kWave;
+    static constexpr size_t kCounters = sizeof(uint16_t) * WAVES * COLS, kStage = sizeof(T) * PER * THREADS;
+    alignas(16) unsigned char lds[kCounters > kStage ? kCounters : kStage];
+    int32_t lofs[COLS];  // per column: count, then first position in column order
+    int32_t wave_tot[WAVES];
+};
+template <typename T, int COLS, int THREADS>
+__device__ __forceinline__ void rows_in_one_turn(OneTurn<T, COLS, THREADS> &sh, int32_t s0, int32_t s1, int nbits, int64_t c0, int32_t ncols,
+                                                 const int32_t *__restrict__ brow, const uint16_t *__restrict__ bcol, const T *__restrict__ bval,
+                                                 int32_t *__restrict__ row_ptr_t, int32_t *__restrict__ col_t, T *__restrict__ val_t)
 {
-    __shared__ RowsShared<T, COLS> sh;
+    constexpr int PER = OneTurn<T, COLS, THREADS>::PER, WAVES = THREADS / kWave;
+    const int tid = threadIdx.x, lane = tid & (kWave - 1), wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+    uint16_t *cnt = reinterpret_cast<uint16_t *>(sh.lds), *mycnt = cnt + wave * COLS;
+    int32_t *lofs = sh.lofs;
+    const int32_t count = s1 - s0, wbase = s0 + wave * (PER * kWave);
+    const int32_t from = wbase < s1 ? wbase : s1 - 1;  // uniform; elements past the bucket's last repeat it
+    const uint32_t most = (uint32_t)(s1 - 1 - from);
+    const auto at = [&](int k) { return (uint32_t)(k * kWave + lane) < most ? (uint32_t)(k * kWave + lane) : most; };
+    brow += from, bcol += from, bval += from;
+    int32_t c[PER], p[PER], r[PER];
+    T v[PER];
+#pragma unroll
+    for (int k = 0; k < PER; ++k) {
+        c[k] = bcol[at(k)];
+        r[k] = brow[at(k)];
+    }
+    for (int i = tid; i < WAVES * COLS / 2; i += THREADS) reinterpret_cast<uint32_t *>(cnt)[i] = 0;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k) p[k] = wave_rank(c[k], wbase + k * kWave + lane < s1, nbits, mycnt);
+    // ahead of the ranks the values would take the registers of a second workgroup, 64-bit ones ahead of the rows' places as well
+    const auto values = [&]() {
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int k = 0; k < PER; ++k) v[k] = bval[at(k)];
+    };
+    if constexpr (sizeof(T) == 4) values();
+    __syncthreads();
+    for (int i = tid; i < COLS; i += THREADS) {
+        int32_t run = 0;
+#pragma unroll
+        for (int w = 0; w < WAVES; ++w) {
+            const int32_t t = cnt[w * COLS + i];
+            cnt[w * COLS + i] = (uint16_t)run;
+            run += t;
+        }
+        lofs[i] = run;
+    }
+    __syncthreads();
+    columns_exclusive_sum<COLS, THREADS>(lofs, sh.wave_tot);
+    for (int i = tid; i < ncols; i += THREADS) row_ptr_t[c0 + i] = s0 + lofs[i];
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+        if (wbase + k * kWave + lane < s1) p[k] += lofs[c[k]] + mycnt[c[k]];
+    __syncthreads();
+    int32_t *row_s = reinterpret_cast<int32_t *>(sh.lds);
+    T *val_s = reinterpret_cast<T *>(sh.lds);
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+        if (wbase + k * kWave + lane < s1) row_s[p[k]] = r[k];
+    if constexpr (sizeof(T) == 8) values();
+    __syncthreads();
+    for (int j = tid; j < count; j += THREADS) col_t[s0 + j] = row_s[j];
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < PER; ++k)
+        if (wbase + k * kWave + lane < s1) val_s[p[k]] = v[k];
+    __syncthreads();
+    for (int j = tid; j < count; j += THREADS) val_t[s0 + j] = val_s[j];
+}
+
+template <typename T, int COLS, int THREADS>
+__global__ __launch_bounds__(THREADS, THREADS > kSortThreads ? 8 : 1) void k_transpose_rows(const int32_t *__restrict__ offs, int32_t nblocks, int shift,
+                                                            int nbits, int32_t n, int32_t nnz,
+                                                            const int32_t *__restrict__ brow,
+                                                            const uint16_t *__restrict__ bcol, const T *__restrict__ bval,
+                                                            int32_t *__restrict__ row_ptr_t, int32_t *__restrict__ col_t,
+                                                            T *__restrict__ val_t, int32_t *__restrict__ large)
+{
+    __shared__ union Lds {
+        RowsShared<T, COLS, THREADS> turns;
+        OneTurn<T, COLS, THREADS> one;
+        __device__ Lds() {}
+    } lds;
+    RowsShared<T, COLS, THREADS> &sh = lds.turns;
     const int tid = threadIdx.x;
     const int32_t b = blockIdx.x;
     const int32_t s0 = offs[(int64_t)b * nblocks], s1 = offs[(int64_t)(b + 1) * nblocks];
+    const int64_t c0 = (int64_t)b << shift;
     if (b == (int32_t)gridDim.x - 1 && tid == 0) row_ptr_t[n] = nnz;
     if (s1 - s0 > kLargeBucket) {  // the whole workgroup leaves
         if (tid == 0) large[2 * b] = s0, large[2 * b + 1] = s1;
         return;
     }
+    if (s1 > s0 && s1 - s0 <= OneTurn<T, COLS, THREADS>::PER * THREADS) {  // uniform
+        const int64_t ncols = n - c0 < (int64_t)1 << shift ? n - c0 : (int64_t)1 << shift;
+        rows_in_one_turn<T, COLS, THREADS>(lds.one, s0, s1, nbits, c0, (int32_t)ncols, brow, bcol, bval, row_ptr_t, col_t, val_t);
+        return;
+    }
     // column counts of the whole bucket -> row offsets of A^T
-    for (int i = tid; i < COLS; i += kSortThreads) sh.first[i] = 0;
+    constexpr int PER = kSortElems / THREADS;
+    for (int i = tid; i < COLS; i += THREADS) sh.first[i] = 0;
     __syncthreads();
     for (int32_t i0 = s0; i0 < s1; i0 += kSortElems) {  // uniform; a turn's loads together (28.0 -> 26.1 us), past the end the last one
-        int32_t c[kSortPerLane];
+        int32_t c[PER];
 #pragma unroll
-        for (int k = 0; k < kSortPerLane; ++k) {
-            const int32_t i = i0 + k * kSortThreads + tid;
+        for (int k = 0; k < PER; ++k) {
+            const int32_t i = i0 + k * THREADS + tid;
             c[k] = bcol[i < s1 ? i : s1 - 1];
         }
 #pragma unroll
-        for (int k = 0; k < kSortPerLane; ++k)
-            if (i0 + k * kSortThreads + tid < s1) atomicAdd(&sh.first[c[k]], 1);
+        for (int k = 0; k < PER; ++k)
+            if (i0 + k * THREADS + tid < s1) atomicAdd(&sh.first[c[k]], 1);
     }
     __syncthreads();
-    columns_exclusive_sum<COLS>(sh.first, sh.wave_tot);
-    const int64_t c0 = (int64_t)b << shift;
-    for (int i = tid; i < (1 << shift); i += kSortThreads) {
+    columns_exclusive_sum<COLS, THREADS>(sh.first, sh.wave_tot);
+    for (int i = tid; i < (1 << shift); i += THREADS) {
         const int32_t at = s0 + sh.first[i];
         sh.first[i] = at;
         if (c0 + i < n) row_ptr_t[c0 + i] = at;
     }
-    place_by_column<T, COLS>(sh, s0, s1, nbits, brow, bcol, bval, col_t, val_t);
+    place_by_column<T, COLS, THREADS>(sh, s0, s1, nbits, brow, bcol, bval, col_t, val_t);
 }
 
 // ---- large buckets: pieces of kLargePiece elements, a workgroup each ----
@@ -523,9 +616,9 @@ int csr_transpose_buckets(int shift, int32_t m, int32_t n, int32_t nnz, int32_t 
     static_assert(2 * kBuckets * sizeof(int32_t) <= kPinnedBytes, "large buckets are reported through page-locked memory");
     if (!found) return ASX_STATUS_ALLOC_FAILED;
     std::memset(found, 0, 2 * sizeof(int32_t) * (size_t)nbuckets);
-    const auto rows = [&](auto cols_) {
-        constexpr int COLS = decltype(cols_)::value;
-        hipLaunchKernelGGL((k_transpose_rows<T, COLS>), dim3((unsigned)nbuckets), dim3(kSortThreads), 0, s, counts, nblocks, shift,
+    const auto rows = [&](auto cols_, auto threads_) {
+        constexpr int COLS = decltype(cols_)::value, THREADS = decltype(threads_)::value;
+        hipLaunchKernelGGL((k_transpose_rows<T, COLS, THREADS>), dim3((unsigned)nbuckets), dim3(THREADS), 0, s, counts, nblocks, shift,
                            shift, n, nnz, brow, bcol, bval, row_ptr_t, col_t, val_t, found);
         int rc = check_launch();
         if (!rc) rc = status_of(hipStreamSynchronize(s));
@@ -553,9 +646,12 @@ int csr_transpose_buckets(int shift, int32_t m, int32_t n, int32_t nnz, int32_t 
         rc = check_launch();
         return rc ? rc : status_of(hipStreamSynchronize(s));
     };
-    st = shift <= 9    ? rows(std::integral_constant<int, 512>{})
-         : shift == 10 ? rows(std::integral_constant<int, 1024>{})
-                       : rows(std::integral_constant<int, kBucketColumns>{});
+    const std::integral_constant<int, kSortThreads> usual;
+    const bool wide = nnz / nbuckets > kSortElems;  // most buckets would take a second turn of 512 threads
+    st = shift <= 9    ? wide ? rows(std::integral_constant<int, 512>{}, std::integral_constant<int, 2 * kSortThreads>{})
+                              : rows(std::integral_constant<int, 512>{}, usual)
+         : shift == 10 ? rows(std::integral_constant<int, 1024>{}, usual)
+                       : rows(std::integral_constant<int, kBucketColumns>{}, usual);
     scratch.idle = st == ASX_STATUS_SUCCESS;
     return st;
 }
