@@ -273,8 +273,10 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         if (plan && plan->sweep && (uint64_t)ldb <= 0xffffffffull / sizeof(T))
             return launch_spmm_sweep<T>(spmm_sweep(m, plan->n, nnz, ncols, sizeof(T)), nullptr, m, plan->n, nnz, ncols, alpha, row_ptr, col,
                                         val, B, ldb, beta, C, ldc, s);
-        const int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
         const bool chunked = plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T));
+        const int tile_bytes = spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T));
+        int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
+        if (!plan && !chunked) items = spmm_filled_items(items, spmm_tiling(ncols, tile_bytes, sizeof(T)), m, nnz, sizeof(T));
         SweepAsk ask{};
         if ((plan ? plan->asks != 0 : alg == ASX_SPMM_DEFAULT) && !chunked && L.asked_bytes > L.bytes && ws_bytes >= L.asked_bytes &&
             items == spmm_segment_items(m, nnz, ncols, sizeof(T)) && (uint64_t)ldb <= 0xffffffffull / sizeof(T)) {
@@ -293,7 +295,7 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         return launch_spmm_merge<T>(chunked, plan ? std::max(plan->n, k) : 0, m, nnz, items, ncols, alpha, row_ptr, col, val, B, ldb,
                                     beta, C, ldc, xs, ys, (T *)(w + L.carry_off), (int32_t *)(w + L.crow_off),
                                     plan ? plan->carry_pass != 0 : true,
-                                    spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T)), ask, s);
+                                    tile_bytes, ask, s);
     }
     case ASX_SPMM_BLOCKED:
         // the blocks hold a copy of A's values and are built by asx_spmm_plan_create
@@ -516,9 +518,9 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         p->workspace_bytes = p->asks ? layout.asked_bytes : layout.bytes;
         // B's rows one after the other, from the start of a line on, as nearly every caller has them
         const int tile_bytes = spmm_tile_bytes(p->columns, p->n, nullptr, (size_t)p->ncols * sv);
-        const int groups = spmm_tiling(p->ncols, tile_bytes, sv).groups;
-        p->chunked = spmm_plan_chunked(m, nnz, p->ncols, sv, p->stats[0], p->columns == kColumnsScattered, kWave / groups);
-        p->items = spmm_plan_items(usual, p->columns, groups, m, nnz, p->stats[0], p->chunked != 0, p->ncols * (int64_t)sv);
+        const SpmmTiling tiling = spmm_tiling(p->ncols, tile_bytes, sv);
+        p->chunked = spmm_plan_chunked(m, nnz, p->ncols, sv, p->stats[0], p->columns == kColumnsScattered, kWave / tiling.groups);
+        p->items = spmm_plan_items(usual, p->columns, tiling, m, nnz, p->stats[0], p->chunked != 0, p->ncols * (int64_t)sv, sv);
         for (;; p->items = usual) {
             const size_t ns = (size_t)spmm_segments(m, nnz, p->items);
             p->nunits = (int32_t)ns;

@@ -443,6 +443,21 @@ inline SpmmTiling spmm_tiling(int64_t ncols, int tile_bytes, size_t sv)
 // up to 4 groups: 40 columns fp64, 20 per row within 2000 of the diagonal 170 -> 148 us, 64 columns fp32 over scattered rows
 // of 25 141 -> 135 us, power-law rows 207.7 -> 204.1 us.
 constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 4 ? 32 : 64; }
+// Where a wave's groups take a row each and its segment holds fewer than five eighths as many, most groups have nothing to do: then the
+// segment is twice as long, up to 256 items, or 512 of fp32 that several tiles of columns read (one tile: 21 columns, 55 per row 29.5 us with 256
+// and 35.3 with 512).  Never shorter than usual, so that the carries fit.  The merge kernel with
+// rows of B on lines, 128 bytes of them at a time, 0.9 M elements, uniform columns and within 1500 of the diagonal, segments of 128 items
+// against 256 and 512: 28 per row 256 columns fp32 91.8 and 78.5, 83.0 and 60.1; 48 88.3 and 61.5, 83.6 and 56.9; 61 94.8, 78.1 and 66.1, 91.7,
+// 76.1 and 57.7; 96 columns fp64, 36 per row 34.9 and 25.2; but 20 per row, 6 of 8 groups, 60.0 and 64.0, 34.2 and 36.8.  Twelve
+// waves a compute unit have to be left (27 columns fp64, 3144 rows of 62 17.4 us in 1550 waves, 20.4 in 775).
+inline int32_t spmm_filled_items(int32_t usual, const SpmmTiling &tiling, int32_t m, int32_t nnz, size_t sv)
+{
+    const int32_t most = sv == 4 && tiling.tiles > 1 ? kSpmmSegmentLarge : kSpmmSegmentMedium;
+    const int64_t all = (int64_t)m + nnz;
+    int32_t items = usual;
+    while (items < most && 8 * (int64_t)items * m < 5 * tiling.groups * all && all / (2 * items) * tiling.tiles >= 12 * 256) items *= 2;
+    return items;
+}
 // Segments of a plan whose columns are near or spread, where they leave no row cut (carries of more segments would not fit the
 // workspace that callers size without a plan).  They are short, so that fewer rows of B are in use at a time, and where rows are
 // of one length (the longest at most a quarter above the mean) they hold as many as the wave's groups take in full turns.
@@ -456,9 +471,10 @@ constexpr int spmm_dealt(int groups) { return groups == 1 ? 1 << 30 : groups <= 
 // (5 per row, 6 columns fp32, 2 M 20.0 -> 18.1).  Rounding up would make fewer and longer segments: 9 per row, 350000 elements, 3
 // columns fp64 152 workgroups 7.0 us, 579 6.2; 5 per row, 8 fp32 7.6 and 6.5; 9 per row, 3 columns fp64, 800000 10.3 and 8.9, 1.4 M
 // 14.2 and 13.0.  Wide rows of B (row_bytes): never more segments than usual, so that their carries fit.
-inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m, int32_t nnz, int64_t longest, bool chunked,
-                               int64_t row_bytes)
+inline int32_t spmm_plan_items(int32_t usual, int columns, const SpmmTiling &tiling, int32_t m, int32_t nnz, int64_t longest, bool chunked,
+                               int64_t row_bytes, size_t sv)
 {
+    const int groups = tiling.groups;
     if (chunked && spmm_chunked_mid(m, nnz, row_bytes, 1)) return usual;
     if (chunked && row_bytes > 64) return std::max(usual, spmm_chunk_wide_items(spmm_chunk_wide_work(m, nnz, row_bytes)));
     if (chunked) {
@@ -469,7 +485,7 @@ inline int32_t spmm_plan_items(int32_t usual, int columns, int groups, int32_t m
         const int64_t turn = (int64_t)groups * (kChunkThreads / kWave) * (longest + 1), over = items % turn;
         return turn <= items && (items < kChunkItemsMost ? 16 : 2) * over <= turn ? (int32_t)(items - over) : items;
     }
-    if (columns != kColumnsNear && columns != kColumnsSpread) return usual;
+    if (columns != kColumnsNear && columns != kColumnsSpread) return spmm_filled_items(usual, tiling, m, nnz, sv);
     const int32_t least = usual == kSpmmSegmentLarge ? kSpmmSegmentSmall : usual;
     const int64_t turn = groups * (longest + 1);
     const int32_t most = usual == kSpmmSegmentLarge && turn > kSpmmSegmentSmall ? kSpmmSegmentMedium : least;
