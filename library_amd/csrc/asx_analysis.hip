@@ -428,7 +428,7 @@ int launch_sample_columns(const int32_t *d_col, int64_t stride, int shift, const
 // histogram of the row lengths; with row_blocks also the row blocks of the stream kernel, which come with the row offsets
 // that are read anyway (searched for afterwards they took a kernel of 7 us and a second wait for the device).
 // Every workgroup leaves its own counts, and k_plan_totals adds them up into the plan's counters and into page-locked memory of the
-// host: counters set to zero ahead and copied to the host behind were a launch and a copy more.
+// host (a workgroup a count; one for all took 4.8 us with 147 parts and 8 with 342): counters set to zero ahead and copied to the host behind were a launch and a copy more.
 __global__ __launch_bounds__(kBlock) void k_plan_stats(SampleArgs q, const int32_t *__restrict__ row_ptr, int32_t m,
                                                        uint32_t *__restrict__ parts, int32_t nb, int2 *__restrict__ row_blocks)
 {
@@ -440,34 +440,41 @@ __global__ __launch_bounds__(kBlock) void k_plan_stats(SampleArgs q, const int32
         row_histogram(row_ptr, m, (int64_t)blockIdx.x - q.samples, (int64_t)gridDim.x - q.samples, nullptr, nullptr, 0, nullptr, parts);
 }
 
-// counters[0 .. 36] = what k_plan_stats counted, the sample at `sampled`, 0 elsewhere; the same to the host.  A wave a count.
-__global__ __launch_bounds__(1024) void k_plan_totals(const uint32_t *__restrict__ parts, int blocks, const int32_t *__restrict__ sample, int samples,
-                                                      int64_t *__restrict__ counters, int ncounters, int sampled, int64_t *__restrict__ host)
+// counters[0 .. 36] = what k_plan_stats counted, a workgroup each, and by one more the sample at `sampled` and 0 elsewhere; the same to
+// the host.
+__global__ __launch_bounds__(kBlock) void k_plan_totals(const uint32_t *__restrict__ parts, int blocks, const int32_t *__restrict__ sample, int samples,
+                                                        int64_t *__restrict__ counters, int ncounters, int sampled, int64_t *__restrict__ host)
 {
-    const int lane = threadIdx.x & (kWave - 1), w = threadIdx.x / kWave;
-    for (int i = 37 + threadIdx.x; i < ncounters; i += 1024) {
-        const int t = 2 * (i - sampled);  // two words of the sample a counter
-        uint64_t v = 0;
-        if (i >= sampled && t < 2 * 64) {
-            const uint32_t lo = (t & 63) < samples ? (uint32_t)sample[t] : 0u, hi = (t & 63) + 1 < samples ? (uint32_t)sample[t + 1] : 0u;
-            v = (uint64_t)hi << 32 | lo;
+    __shared__ uint64_t wave_total[kBlock / kWave];
+    const int c = blockIdx.x;
+    if (c == 37) {
+        for (int i = 37 + threadIdx.x; i < ncounters; i += kBlock) {
+            const int t = 2 * (i - sampled);  // two words of the sample a counter
+            uint64_t v = 0;
+            if (i >= sampled && t < 2 * 64) {
+                const uint32_t lo = (t & 63) < samples ? (uint32_t)sample[t] : 0u, hi = (t & 63) + 1 < samples ? (uint32_t)sample[t + 1] : 0u;
+                v = (uint64_t)hi << 32 | lo;
+            }
+            counters[i] = (int64_t)v;
+            host[i] = (int64_t)v;
         }
-        counters[i] = (int64_t)v;
-        host[i] = (int64_t)v;
+        return;
     }
-    for (int c = w; c < 37; c += 1024 / kWave) {
-        uint64_t total = 0;
-        for (int b = lane; b < blocks; b += kWave) {
-            const uint32_t v = parts[(int64_t)c * blocks + b];
-            total = c == 33 ? (v > total ? v : total) : total + v;
-        }
+    const bool longest = c == 33;
+    uint64_t total = 0;
+    for (int b = threadIdx.x; b < blocks; b += kBlock) {
+        const uint32_t v = parts[(int64_t)c * blocks + b];
+        total = longest ? (v > total ? v : total) : total + v;
+    }
+    const auto join = [&](uint64_t x, uint64_t y) { return longest ? (x > y ? x : y) : x + y; };
 #pragma unroll
-        for (int d = 1; d < kWave; d <<= 1) {
-            const uint64_t other = __shfl_xor((unsigned long long)total, d, kWave);
-            total = c == 33 ? (other > total ? other : total) : total + other;
-        }
-        if (lane == 0) counters[c] = (int64_t)total, host[c] = (int64_t)total;
-    }
+    for (int d = 1; d < kWave; d <<= 1) total = join(total, __shfl_xor((unsigned long long)total, d, kWave));
+    if (threadIdx.x % kWave == 0) wave_total[threadIdx.x / kWave] = total;
+    __syncthreads();
+    if (threadIdx.x > 0) return;
+    for (int w = 1; w < kBlock / kWave; ++w) total = join(total, wave_total[w]);
+    counters[c] = (int64_t)total;
+    host[c] = (int64_t)total;
 }
 
 size_t plan_stats_bytes(int32_t m) { return (size_t)histogram_parts(m) * 37 * sizeof(uint32_t) + 128 * sizeof(int32_t); }
@@ -485,7 +492,7 @@ int launch_plan_stats(const int32_t *d_row_ptr, int32_t m, int64_t *d_counters, 
         hipLaunchKernelGGL(k_plan_stats, dim3(blocks + (unsigned)samples), dim3(kBlock), 0, s, q, d_row_ptr, m, d_parts, nb,
                            reinterpret_cast<int2 *>(d_row_blocks));
     }
-    hipLaunchKernelGGL(k_plan_totals, dim3(1), dim3(1024), 0, s, d_parts, (int)blocks, d_sample, (int)samples, d_counters, ncounters, sampled, h_counters);
+    hipLaunchKernelGGL(k_plan_totals, dim3(38), dim3(kBlock), 0, s, d_parts, (int)blocks, d_sample, (int)samples, d_counters, ncounters, sampled, h_counters);
     return check_launch();
 }
 

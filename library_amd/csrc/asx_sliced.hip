@@ -454,9 +454,9 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_rescatter(const T *__re
     uint16_t p[kSortPerLane];
 #pragma unroll
     for (int k = 0; k < kSortPerLane; ++k) {
-        const int32_t j = k * kSortThreads + tid;
-        v[k] = j < count ? val[base + j] : T(0);
-        p[k] = j < count ? pos[base + j] : (uint16_t)0;
+        const int32_t j = k * kSortThreads + tid, at = j < count ? j : count - 1;  // no branch: all loads are in flight together
+        v[k] = val[base + at];
+        p[k] = pos[base + at];
     }
     for (int s = tid; s < nslices; s += kSortThreads) {
         const int32_t g = block_base[(int64_t)b * nslices + s];
@@ -469,16 +469,13 @@ __global__ __launch_bounds__(kSortThreads) void k_sliced_rescatter(const T *__re
     for (int k = 0; k < kSortPerLane; ++k)
         if (k * kSortThreads + tid < count) val_s[p[k]] = v[k];
     __syncthreads();
-    for (int j = tid; j < count; j += kSortThreads) {
-        int lo = 0, hi = nslices - 1;  // the slice of position j: the last one that starts at or before j
-        while (lo < hi) {
-            const int mid = lo + (hi - lo + 1) / 2;
-            if (lofs[mid] <= j)
-                lo = mid;
-            else
-                hi = mid - 1;
-        }
-        val_out[slot_val_pos<T>((int64_t)gbase[lo] + (j - lofs[lo]))] = val_s[j];
+    // A group of lanes a run, as many as an average one holds: a search for the slice of every position was six dependent reads of LDS.
+    const int shift = count > 32 * nslices ? 6 : 4;  // uniform
+    const int lane = tid & ((1 << shift) - 1);
+    for (int s = tid >> shift; s < nslices; s += kSortThreads >> shift) {
+        const int32_t from = lofs[s], to = s + 1 < nslices ? lofs[s + 1] : count;
+        const int64_t out = (int64_t)gbase[s] - from;
+        for (int32_t j = from + lane; j < to; j += 1 << shift) val_out[slot_val_pos<T>(out + j)] = val_s[j];
     }
 }
 
