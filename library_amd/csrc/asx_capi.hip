@@ -514,8 +514,8 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         }
     } else if (kernel == ASX_SPMM_MERGE) {
         const int32_t usual = spmm_segment_items(m, nnz, p->ncols, sv);
-        const SpmmLayout layout = spmm_merge_layout(m, nnz, p->ncols, sv);
-        p->workspace_bytes = p->asks ? layout.asked_bytes : layout.bytes;
+        // with room for an answer also where none is asked for: a buffer sized for one algorithm id or plan does for another
+        p->workspace_bytes = spmm_merge_layout(m, nnz, p->ncols, sv).asked_bytes;
         // B's rows one after the other, from the start of a line on, as nearly every caller has them
         const int tile_bytes = spmm_tile_bytes(p->columns, p->n, nullptr, (size_t)p->ncols * sv);
         const SpmmTiling tiling = spmm_tiling(p->ncols, tile_bytes, sv);
@@ -1396,10 +1396,7 @@ int asx_spmm_resolve_alg(int alg, int32_t m, int32_t nnz, int32_t ncols)
 size_t asx_spmm_workspace_bytes(int alg, int value_type, int32_t m, int32_t nnz, int32_t ncols)
 {
     const int kernel = asx_spmm_resolve_alg(alg, m, nnz, ncols);
-    if (kernel == ASX_SPMM_MERGE) {
-        const SpmmLayout layout = spmm_merge_layout(m, nnz, ncols, vsize(value_type));
-        return alg == ASX_SPMM_DEFAULT ? layout.asked_bytes : layout.bytes;
-    }
+    if (kernel == ASX_SPMM_MERGE) return spmm_merge_layout(m, nnz, ncols, vsize(value_type)).asked_bytes;
     return 0;
 }
 

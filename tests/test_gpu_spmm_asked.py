@@ -11,8 +11,14 @@ from test_gpu_spmm_sweep import _matrix
 pytestmark = pytest.mark.gpu
 
 
-def _bytes(alg, vt, m, nnz, ncols):
-    return capi.lib().asx_spmm_workspace_bytes(alg, vt, m, nnz, ncols)
+def _answer(ws):
+    """Where the answer lies in a workspace that was filled with 0x55, and what it says.  Behind it are four bytes that nobody writes, a
+    byte for every workgroup of the sweep, 0 or 1, and what rounds the size up."""
+    w = ws.cpu().numpy()
+    i = int(np.flatnonzero(w != 0x55)[-1]) + 1
+    i = int(np.flatnonzero(w[:i] > 1)[-1]) + 1
+    assert (w[i - 4:i] == 0x55).all()
+    return i - 8, int(w[i - 8:i - 4].view(np.int32)[0])
 
 
 def _run(lens, n, ncols, dtype, taken, beta=0.5, pad=0, reach=None, room=True, ascending=True):
@@ -31,14 +37,18 @@ def _run(lens, n, ncols, dtype, taken, beta=0.5, pad=0, reach=None, room=True, a
         s = torch.cumsum(torch.cat([torch.zeros(1, device="cuda", dtype=torch.float64), val.double() * B[:, c].double()[col.long()]]), 0)
         y = 2.0 * (s[ends[1:]] - s[ends[:-1]]).to(dtype)
         ref[:, c] = y if beta == 0.0 else y + beta * C[:, c]
-    vt = capi.value_type(dtype)
-    at, need = _bytes(capi.SPMM_MERGE, vt, m, nnz, ncols), _bytes(capi.SPMM_DEFAULT, vt, m, nnz, ncols)
-    assert need > at
-    ws = torch.full((need if room else at,), 0x55, dtype=torch.uint8, device="cuda")
+    need = [capi.lib().asx_spmm_workspace_bytes(alg, capi.value_type(dtype), m, nnz, ncols) for alg in (capi.SPMM_DEFAULT, capi.SPMM_MERGE)]
+    assert need[0] == need[1]  # a buffer for one does for the other
+    ws = torch.full((need[0],), 0x55, dtype=torch.uint8, device="cuda")
     start = C.clone()
     capi.spmm(rp, col, val, B, C, ncols, 2.0, beta, workspace=ws, ldb=ncols + pad, ldc=ncols + pad, k=n)
-    if room:
-        assert int(ws[at:at + 4].view(torch.int32)) == taken
+    at, answer = _answer(ws)
+    assert answer == taken
+    if not room:  # a workspace without the answer's place, and nothing behind it is written
+        ws.fill_(0x55)
+        C.copy_(start)
+        capi.spmm(rp, col, val, B, C, ncols, 2.0, beta, workspace=ws[:at], ldb=ncols + pad, ldc=ncols + pad, k=n)
+        assert bool((ws[at:] == 0x55).all())
     assert torch.equal(C[:, :ncols], ref[:, :ncols]) and (not pad or beta == 0.0 or torch.equal(C[:, ncols:], ref[:, ncols:]))
     # a plan that has not seen the columns takes the same way
     plan = capi.Plan(True, capi.SPMM_DEFAULT, dtype, m, n, nnz, rp, ncols=ncols)
@@ -80,4 +90,4 @@ def test_other_matrices_stay_with_the_merge_kernel(dtype, ncols, m, per):
     uneven = np.minimum((rng.pareto(1.3, m) * per * 0.24 + per * 0.24).astype(int), 20000)
     uneven[rng.integers(0, m, m // 50)] += max(0, per * m - int(uneven.sum())) // (m // 50) + 1
     _run(uneven, m, ncols, dtype, 0)
-    _run(_even(m, per), m, ncols, dtype, 0, room=False)  # a workspace sized for the merge kernel
+    _run(_even(m, per), m, ncols, dtype, 1, room=False)  # then without room for an answer
