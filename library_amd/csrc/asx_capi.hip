@@ -71,9 +71,8 @@ SpmmLayout spmm_merge_layout(int32_t m, int32_t nnz, int32_t ncols, size_t sv)
     L.carry_off = off;
     off = align_up(off + std::max<size_t>(ns, 1) * (size_t)ncols * sv, kAlign);
     L.bytes = L.ask_off = L.asked_bytes = off;
-    const SpmmSweep sw = spmm_sweep_shape(m, nnz, ncols, sv);
-    if (spmm_sweep_askable(sw, m, nnz, ncols, sv, spmm_segment_items(m, nnz, ncols, sv)))
-        L.asked_bytes = align_up(off + 8 + (size_t)spmm_sweep_blocks(sw, m), kAlign);
+    if (spmm_sweep_askable(spmm_sweep_shape(m, nnz, ncols, sv, 1), m, nnz, ncols, sv, spmm_segment_items(m, nnz, ncols, sv)))
+        L.asked_bytes = align_up(off + 8 + (size_t)kSweepAskBlocks, kAlign);  // sums a row, and with them workgroups, depend on where B lies
     return L;
 }
 
@@ -270,21 +269,26 @@ int spmm_impl(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, 
         } else {
             xs = ys = nullptr;  // the kernel's waves look their own segments up
         }
-        if (plan && plan->sweep && (uint64_t)ldb <= 0xffffffffull / sizeof(T))
-            return launch_spmm_sweep<T>(spmm_sweep(m, plan->n, nnz, ncols, sizeof(T)), nullptr, m, plan->n, nnz, ncols, alpha, row_ptr, col,
-                                        val, B, ldb, beta, C, ldc, s);
         const bool chunked = plan ? plan->chunked != 0 : spmm_chunked(m, nnz, ncols, sizeof(T));
         const int tile_bytes = spmm_tile_bytes(plan ? plan->columns : kColumnsUnknown, k, B, (size_t)ldb * sizeof(T));
+        const SpmmTiling tiling = spmm_tiling(ncols, tile_bytes, sizeof(T));
+        if (plan && plan->sweep && (uint64_t)ldb <= 0xffffffffull / sizeof(T)) {
+            const SpmmSweep sw = spmm_sweep(m, plan->n, nnz, ncols, sizeof(T), spmm_sweep_chains(plan->stats[0], tiling.groups, chunked));
+            if (sw.slots > 0)  // 0: B lies otherwise than the plan had it
+                return launch_spmm_sweep<T>(sw, nullptr, m, plan->n, nnz, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, s);
+        }
         int32_t items = plan ? plan->items : spmm_segment_items(m, nnz, ncols, sizeof(T));
-        if (!plan && !chunked) items = spmm_filled_items(items, spmm_tiling(ncols, tile_bytes, sizeof(T)), m, nnz, sizeof(T));
+        if (!plan && !chunked) items = spmm_filled_items(items, tiling, m, nnz, sizeof(T));
         SweepAsk ask{};
         if ((plan ? plan->asks != 0 : alg == ASX_SPMM_DEFAULT) && !chunked && L.asked_bytes > L.bytes && ws_bytes >= L.asked_bytes &&
             items == spmm_segment_items(m, nnz, ncols, sizeof(T)) && (uint64_t)ldb <= 0xffffffffull / sizeof(T)) {
             const int32_t n = plan ? plan->n : k;
-            const SpmmSweep sw = spmm_sweep(m, n, nnz, ncols, sizeof(T));
-            if (sw.slots > 0 && spmm_sweep_shared(sw, m, n, nnz) >= kSweepAskShared) {
+            const int32_t longest = spmm_sweep_ask_longest(m, nnz, tiling.groups);
+            const SpmmSweep sw = spmm_sweep(m, n, nnz, ncols, sizeof(T), spmm_sweep_chains(longest, tiling.groups, false));
+            if (sw.slots > 0 && (int64_t)longest * m >= nnz && spmm_sweep_blocks(sw, m) <= spmm_sweep_ask_blocks(sw.chains) &&
+                spmm_sweep_shared(sw, m, n, nnz) >= kSweepAskShared) {
                 ask.n = n;
-                ask.longest = (int32_t)spmm_sweep_longest(m, nnz);
+                ask.longest = longest;
                 ask.blocks = (int32_t)spmm_sweep_blocks(sw, m);
                 ask.answer = (int32_t *)(w + L.ask_off);
                 ask.too_long = (uint8_t *)(w + L.ask_off + 8);
@@ -521,6 +525,8 @@ int plan_row_ordered(asx_plan *p, int kernel, hipStream_t s)
         const SpmmTiling tiling = spmm_tiling(p->ncols, tile_bytes, sv);
         p->chunked = spmm_plan_chunked(m, nnz, p->ncols, sv, p->stats[0], p->columns == kColumnsScattered, kWave / tiling.groups);
         p->items = spmm_plan_items(usual, p->columns, tiling, m, nnz, p->stats[0], p->chunked != 0, p->ncols * (int64_t)sv, sv);
+        p->sweep = p->sweep && p->stats[0] <= std::min<int64_t>(spmm_sweep_longest(m, nnz), usual) &&
+                   spmm_sweep(m, p->n, nnz, p->ncols, sv, spmm_sweep_chains(p->stats[0], tiling.groups, p->chunked != 0)).slots > 0;
         for (;; p->items = usual) {
             const size_t ns = (size_t)spmm_segments(m, nnz, p->items);
             p->nunits = (int32_t)ns;
@@ -564,8 +570,7 @@ int plan_create(asx_plan **out, int is_spmm, int alg, int value_type, int32_t m,
     if (kernel == ASX_SPMM_MERGE && is_spmm) {
         p->columns = columns;
         p->asks = alg == ASX_SPMM_DEFAULT && columns == kColumnsUnknown;
-        p->sweep = everywhere && p->stats[0] <= spmm_sweep_longest(m, nnz) &&
-                   spmm_sweep(m, n, nnz, ncols_dense, vsize(value_type)).slots > 0;
+        p->sweep = everywhere;
     }
     st = plan_row_ordered(p, kernel, s);
     if (st) {

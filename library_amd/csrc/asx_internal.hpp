@@ -30,6 +30,7 @@ constexpr int kSpmmSegmentSmall = 128, kSpmmSegmentMedium = 256, kSpmmSegmentLar
 // fp32, on average: 1664 items 8 % behind, 2048 3 %, 2368 1.5 %, 3008 and 3392 alike; 24 per row, 8 columns fp64 58.0, 55.5, 55.4, 2688
 // items 55.5, 53.3, 53.3; 20 per row 59.9, 57.1, 56.1, 54.7, 55.2, 55.1).
 constexpr int kChunkThreads = 512, kChunkElems = 2880, kChunkRows = 2689;
+constexpr int kChunkWideLeast = 64;  // longer rows are taken by all waves where a wave has four groups or fewer
 constexpr int kChunkItems = 1344, kChunkItemsMost = 2688, kChunkLongest = kChunkElems - kChunkItemsMost;
 constexpr int kChunkItemsWide = 640;      // the most where rows of B are wide
 constexpr int64_t kChunkRound = 768;      // three workgroups on each of 256 compute units
@@ -223,12 +224,14 @@ int launch_spmm_merge(bool chunked, int32_t rows, int32_t m, int32_t nnz, int32_
 
 // ---- SpMM of columns that lie all over B (asx_spmm_sweep.hip) ----
 struct SpmmSweep {
-    int32_t slots;   // rows of C a lane group has registers for (0: not taken)
-    int32_t rows;    // and how many it is given
+    int32_t slots;   // sums of rows of C a lane group has registers for (0: not taken)
+    int32_t rows;    // rows it is given, `chains` sums each
     int32_t cap;     // elements of A a wave stages at once
     uint32_t width;  // columns a window
     int log_lanes;   // of a group
     int64_t tiles;   // of columns of B
+    int32_t chains;  // sums of stretches that a row of more than `dealt` elements is made of: 1, 2 or 4
+    int32_t dealt;
 };
 template <typename T>
 int launch_spmm_sweep(const SpmmSweep &sw, const SweepAsk *ask, int32_t m, int32_t n, int32_t nnz, int32_t ncols, T alpha,
@@ -517,24 +520,37 @@ inline bool spmm_everywhere(double spread, double span, double falls, double mea
 //   in tiles of one line, which they can keep up to 40000 rows or 20 MB (192 columns fp32, 27903 rows of 8 22.6 us there, 23.4 here;
 //   32, 101110 of 8 17.3 and 18.4; 448, 28456 of 9 52.3 and 59.8) -; rows of fewer than 4; and where an XCD's waves meet a row of B
 //   only every fourth round or less (kSweepSharedLeast; 74 columns fp32, 525797 x 1032224, 13 per row 406 and 429).
+//   Long rows: in fp32 a row's error grows with the elements that one sum runs over, and the row-ordered kernels sum rows of more than
+//   spmm_dealt elements in as many sums as a wave has groups.  So does the sweep (chains), and a group then has registers for
+//   1 / chains of the rows; rows that those kernels cut, or give to a whole workgroup, are not taken.  49 per row, 100 columns: rms error 1.34
+//   times theirs with one sum, as theirs with two.
 constexpr int kSweepWaves = 16;
 constexpr double kSweepSharedLeast = 0.25;
+// sums a row for rows of up to `longest` elements, none of which is cut; 0: more than the sweep has
+inline int spmm_sweep_chains(int64_t longest, int groups, bool chunked)
+{
+    if (longest <= (chunked ? std::min(spmm_dealt(groups), kChunkWideLeast) : spmm_dealt(groups))) return 1;
+    return groups > 1 && groups <= 4 && (!chunked || longest <= kChunkWideLeast) ? groups : 0;
+}
 inline int64_t spmm_sweep_longest(int32_t m, int32_t nnz) { return 2 * ((int64_t)nnz / (m > 0 ? m : 1)) + 8; }
 constexpr int32_t spmm_sweep_cap(size_t sv) { return (int32_t)(160 * 1024 / kSweepWaves / (4 + sv)) & ~1; }
 // what does not depend on the number of columns
-inline SpmmSweep spmm_sweep_shape(int32_t m, int32_t nnz, int64_t ncols, size_t sv)
+inline SpmmSweep spmm_sweep_shape(int32_t m, int32_t nnz, int64_t ncols, size_t sv, int chains)
 {
     SpmmSweep sw{};
-    if (m <= 0 || ncols * (int64_t)sv <= 64 || nnz / m < 4) return sw;
+    if (m <= 0 || ncols * (int64_t)sv <= 64 || nnz / m < 4 || chains < 1) return sw;
     const double mean = (double)nnz / m;
     const SpmmTiling t = spmm_tiling(ncols, 1024, sv);
     const int32_t cap = spmm_sweep_cap(sv);
-    int64_t rows = std::min<int64_t>(t.log_lanes < 5 ? 1 << t.log_lanes : 20, (int64_t)(cap / (1.05 * mean * t.groups)));
+    int64_t rows = std::min<int64_t>((t.log_lanes < 5 ? 1 << t.log_lanes : 20) / chains, (int64_t)(cap / (1.05 * mean * t.groups)));
     if (t.log_lanes < 3 || rows < 1 || t.tiles > 65535) return sw;
     const int64_t round = (int64_t)kSweepWaves * 256 * t.groups;
     rows = ceil_div64(m, round * ceil_div64(m, round * rows));
     sw.rows = (int32_t)rows;
-    sw.slots = rows <= 4 ? 4 : rows <= 8 ? 8 : rows <= 12 ? 12 : rows <= 16 ? 16 : 20;
+    sw.chains = chains;
+    sw.dealt = chains == 1 ? 0x7fffffff : spmm_dealt(chains);
+    const int64_t slots = rows * chains;
+    sw.slots = slots <= 4 ? 4 : slots <= 8 ? 8 : slots <= 12 ? 12 : slots <= 16 ? 16 : 20;
     sw.cap = std::min(cap, ((int32_t)(1.1 * mean * (double)(rows * t.groups)) + 2) & ~1);
     sw.log_lanes = t.log_lanes;
     sw.tiles = t.tiles;
@@ -551,10 +567,10 @@ inline double spmm_sweep_shared(const SpmmSweep &sw, int32_t m, int32_t n, int32
     const int64_t round = (int64_t)kSweepWaves * 256 * (kWave >> sw.log_lanes);
     return (double)std::min<int64_t>(round * sw.rows, m) * ((double)nnz / m) / kXcds / n;
 }
-inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, size_t sv)
+inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, size_t sv, int chains)
 {
     const int64_t bytes = ncols * (int64_t)sv;
-    SpmmSweep sw = spmm_sweep_shape(m, nnz, ncols, sv);
+    SpmmSweep sw = spmm_sweep_shape(m, nnz, ncols, sv, chains);
     if (sw.slots == 0 || n <= 0) return SpmmSweep{};
     const double mean = (double)nnz / m, mb = 1e-6 * (double)bytes * n;
     if (bytes % 128 == 0 ? mb < 20.0 || n < 40000 : mb < (mean < 14.0 ? 14.0 : 9.0)) return SpmmSweep{};
@@ -564,20 +580,29 @@ inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, si
     return sw;
 }
 // Calls whose columns nobody has looked at: whether asking pays (slots 0: not).  Where the answer is no, the launch is spent: 4.6 us with
-// one round of workgroups (100 columns fp32, 160001 power-law rows of 20: 264 us before), 5.8 with two, 9 with five.  So it is for calls
-// whose rows of B, each fetched by itself, take 240 us and more, for two rounds at most, and where an XCD's waves meet a row of B often
-// (100 columns fp32, 150001 uniform rows of 25, 1.6: 257 us without, 157 with). Rows of B that start on lines, which the merge kernel
+// one round of workgroups (100 columns fp32, 160001 power-law rows of 20: 264 us before), 5.8 with two, 8 with three (250 columns, 100003 rows
+// of 36 within 3000 of the diagonal: 274 us before).  So it is for calls
+// whose rows of B, each fetched by itself, take 240 us and more, for two rounds at most (three where a row is several sums), and
+// where an XCD's waves meet a row of B often (100 columns fp32, 150001 uniform rows of 25, 1.6: 257 us without, 157 with). Rows of B that start on lines, which the merge kernel
 // takes a line or two at a time, gain less (256 columns fp32, 60001 uniform rows of 30, 173 us without and 157 with; 128 fp64, 20 per row
 // within 3000 of the diagonal 165 and 171): from twice as many lines on.  Rows that the merge kernel cuts have to be longer than
 // the sweep takes: it looks at whole rows only.
 constexpr double kSweepAskLines = 240e-6 * 58e9, kSweepAskShared = 0.6;
-constexpr int64_t kSweepAskBlocks = 2048;
+constexpr int64_t kSweepAskBlocks = 3 * 1024;
+constexpr int64_t spmm_sweep_ask_blocks(int chains) { return chains > 1 ? kSweepAskBlocks : 2 * 1024; }
+// The longest row it takes then: rows of up to spmm_dealt elements where the mean is no longer, so that they need one sum each; longer
+// means with two or four sums, but no row that eight groups would share.
+inline int32_t spmm_sweep_ask_longest(int32_t m, int32_t nnz, int groups)
+{
+    const int64_t longest = spmm_sweep_longest(m, nnz), dealt = spmm_dealt(groups);
+    return (int32_t)(nnz <= dealt * m || groups > 4 ? std::min(longest, dealt) : longest);
+}
 inline bool spmm_sweep_askable(const SpmmSweep &sw, int32_t m, int32_t nnz, int64_t ncols, size_t sv, int32_t items)
 {
     const int64_t bytes = ncols * (int64_t)sv;
     return sw.slots > 0 && (double)nnz * ((double)bytes / 128.0 + (bytes % 128 ? 1.0 : 0.0)) >= kSweepAskLines &&
            (bytes % 128 || (double)nnz * (double)bytes / 128.0 >= 2.0 * kSweepAskLines) &&
-           spmm_sweep_longest(m, nnz) <= items && spmm_sweep_blocks(sw, m) <= kSweepAskBlocks;
+           spmm_sweep_longest(m, nnz) <= items && spmm_sweep_blocks(sw, m) <= spmm_sweep_ask_blocks(1);
 }
 inline int32_t spmm_segments(int32_t m, int32_t nnz, int32_t items) { return (int32_t)ceil_div64((int64_t)m + nnz, items); }
 

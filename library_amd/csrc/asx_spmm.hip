@@ -467,7 +467,7 @@ __global__ __launch_bounds__(kChunkThreads, REACH == kRowsFar ? 4 : 6) void k_sp
     // registers of four workgroups a compute unit, eight of three (no plan, 4 columns, 20 per row 49.7 us with eight, 44.1 with six,
     // 43.9 with four; 40 per row 50.1, 47.2, 47.1; 60 52.9, 48.2, 50.9).
     constexpr int U = REACH == kRowsNear && sizeof(T) == 4 && VEC == 4 && LOGG == 0 ? 6 : 8;
-    constexpr int kWide = NG > 4 ? 256 : 64;  // longer rows are taken by all waves (elements)
+    constexpr int kWide = NG > 4 ? 256 : kChunkWideLeast;  // longer rows are taken by all waves (elements)
     constexpr int kDealt = spmm_dealt(NG) < kWide ? spmm_dealt(NG) : kWide;
     constexpr int kWaves = kChunkThreads / kWave, NE = (kChunkElems + kChunkThreads - 1) / kChunkThreads;
     __shared__ int32_t s_col[kChunkElems];

@@ -104,11 +104,13 @@ constexpr int sweep_batch(int slots) { return slots == 20 ? 5 : slots == 12 ? 6 
 // and a load 16 cycles of a compute unit's L1 where all lanes take part, none where none does - slots without an element are
 // masked out, not sent past a buffer's end (119 us against 157 for the first example above) -; and lines past the L2s for what
 // waves are apart.  Batches of G slots, all loads of a batch ahead of its sums.
+// Rows of more than `dealt` elements are `chains` sums of a stretch each, S / chains slots apart, so that most steps have nothing to do for
+// the batches of one stretch or the other.
 //
 // ASK: the call does not know its columns (above).  Rows longer than ask.longest are left to the merge kernel.
 template <typename T, int LOGL, int S, bool ASK>
 __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
-    SweepAsk ask, int32_t m, int32_t nnz, int32_t rows, int32_t cap, uint32_t width, uint32_t last, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
+    SweepAsk ask, int32_t m, int32_t nnz, int32_t rows, int32_t chains, int32_t dealt, int32_t cap, uint32_t width, uint32_t last, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
     const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ B, int64_t ldb, T beta, T *__restrict__ C, int64_t ldc)
 {
     typedef typename Vec16<T>::type V;
@@ -132,9 +134,9 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
     const char *Bc = (const char *)(B + c);
     const uint32_t pitch = (uint32_t)((uint64_t)ldb * sizeof(T));
 
-    // the lane's row: element s up to e
-    const int32_t mine = grp * rows + gl;
-    bool has_row = gl < rows && mine < nrow;
+    // the lane's row, or its part of one: element s up to e
+    const int32_t apart = chains == 1 ? S : chains == 2 ? S / 2 : S / 4, part = (gl >= apart) + (gl >= 2 * apart) + (gl >= 3 * apart), mine = grp * rows + gl - part * apart;
+    bool has_row = part < chains && gl - part * apart < rows && mine < nrow;
     int32_t s = has_row ? row_ptr[x0 + mine] : 0, e = has_row ? row_ptr[x0 + mine + 1] : 0;
     if constexpr (ASK) {
         __shared__ int s_yes, s_long[kBlock / kWave];
@@ -155,7 +157,14 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
         if (!s_yes || x0 >= m) return;
         if (too_long) has_row = false, s = e = 0;
     }
-    const uint64_t kept = __ballot(has_row);
+    const uint64_t kept = __ballot(has_row && part == 0);
+    if (e - s > dealt) {  // of more than one sum: a stretch each
+        const int32_t share = (e - s + chains - 1) / chains;
+        s = s + part * share < e ? s + part * share : e;
+        e = s + share < e ? s + share : e;
+    } else if (part > 0) {
+        s = e;
+    }
     const int32_t begin = __builtin_amdgcn_readfirstlane(row_ptr[x0]), end = __builtin_amdgcn_readfirstlane(row_ptr[x0 + nrow]);
 
     V acc[S];
@@ -239,6 +248,10 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
             }
         }
     }
+    if (chains > 1)
+        static_for<0, S / 2>([&](auto j_) { acc[decltype(j_)::value] += acc[decltype(j_)::value + S / 2]; });
+    if (chains > 2)
+        static_for<0, S / 4>([&](auto j_) { acc[decltype(j_)::value] += acc[decltype(j_)::value + S / 4]; });
     static_for<0, S / G>([&](auto g_) {
         constexpr int j0 = decltype(g_)::value * G;
         V c_old[G];
@@ -266,7 +279,7 @@ static int launch_sweep(const SpmmSweep &sw, const SweepAsk &ask, int32_t m, int
     const uint32_t last = (uint32_t)n > sw.width ? (uint32_t)n - sw.width : 0;
 #define ASX_SWEEP(LOGL, S)                                                                                                              \
     if (sw.log_lanes == LOGL && sw.slots == S) {                                                                                        \
-        hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S, ASK>), grid, dim3(kBlock), lds, s, ask, m, nnz, sw.rows, cap, sw.width, last,      \
+        hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S, ASK>), grid, dim3(kBlock), lds, s, ask, m, nnz, sw.rows, sw.chains, sw.dealt, cap, sw.width, last,      \
                            ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc);                                                      \
         return check_launch();                                                                                                          \
     }
