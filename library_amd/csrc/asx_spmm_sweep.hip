@@ -116,7 +116,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
     typedef typename Vec16<T>::type V;
     constexpr int VEC = Vec16<T>::N, L = 1 << LOGL, NG = kWave / L, G = sweep_batch(S);
     static_assert(S <= L && S % G == 0, "a lane knows where one row of its group is");
-    extern __shared__ char s_all[];
+    extern __shared__ __align__(16) char s_all[];
     const int lane = threadIdx.x & (kWave - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t per_xcd = gridDim.x / kXcds;
@@ -274,7 +274,7 @@ static int launch_sweep(const SpmmSweep &sw, const SweepAsk &ask, int32_t m, int
                         const int32_t *col, const T *val, const T *B, int64_t ldb, T beta, T *C, int64_t ldc, hipStream_t s)
 {
     const dim3 grid((unsigned)spmm_sweep_blocks(sw, m), (unsigned)sw.tiles);
-    const int32_t cap = ASK ? std::min(sw.cap, spmm_sweep_cap(sizeof(T)) - 2) : sw.cap;  // asking takes 20 bytes of LDS
+    const int32_t cap = ASK ? std::min(sw.cap, spmm_sweep_cap(sizeof(T)) - 2) : sw.cap;  // asking takes 20 bytes of LDS, 32 ahead of the aligned rest
     const size_t lds = (size_t)cap * (sizeof(T) + 4) * (kBlock / kWave);
     const uint32_t last = (uint32_t)n > sw.width ? (uint32_t)n - sw.width : 0;
 #define ASX_SWEEP(LOGL, S)                                                                                                              \
