@@ -343,9 +343,12 @@ __device__ __forceinline__ void place_by_column(RowsShared<T, COLS, THREADS> &sh
 constexpr int32_t kLargeBucket = 16 * kSortElems, kLargePiece = 8 * kSortElems;
 
 // A bucket of up to PER elements a thread is sorted in one turn: its elements are loaded once, ranked, and what the waves have counted
-// per column gives the row offsets of A^T as well as the places, which are consecutive then.  Buckets of 4096 to 8192 elements take
-// 1024 threads instead of a count and two turns of 512, one workgroup behind the other on a compute unit being what bounds the kernel;
-// counters and staged elements share LDS and values are loaded late, so that two such workgroups fit (64 registers).
+// per column gives the row offsets of A^T as well as the places, which are consecutive then.  Where buckets of up to 512 columns hold
+// more than 4096 elements on average, all take 1024 threads instead of a count and two turns of 512, one workgroup behind the other on a
+// compute unit being what bounds the kernel; counters and staged elements share LDS and values are loaded late, so that two such
+// workgroups fit (64 registers).  Larger averages take them as well: most of their buckets need several turns either way, and 512
+// threads came out alike (transpose and multiply, 300000 columns, 1024 and 512 threads: 6 M elements fp32 172 and 173 us, fp64 195 and
+// 192; 16 M 415 and 415, 542 and 541; 32 M 921 and 927, 1235 and 1230).
 // 3.6 M elements of 489 buckets, fp32: 25.9 -> 19.6 us.  Transpose and multiply, 4 M uniform elements into 200013 rows: fp32 127 -> 112
 // us, fp64 149 -> 134; 1 M in one turn of 512 threads 62 -> 59.
 template <typename T, int COLS, int THREADS>

@@ -24,6 +24,8 @@ def _shift(n, nnz):
 @pytest.mark.parametrize("n,nnz,shift,mean,turns", [
     (300000, 4000003, 9, 6825, ()),                                    # 1024 threads
     (300000, 4000003, 9, 6825, (8191, 8192, 8193, 20000, 0, 1)),
+    (300000, 6000001, 9, 10238, ()),                                   # 1024 threads, several turns for most
+    (300000, 6000001, 9, 10238, (8191, 8192, 8193, 4095, 4096, 4097)),
     (150000, 1000003, 9, 3412, (4095, 4096, 4097, 9000, 0, 1)),        # 512 threads and up to 512 columns
     (300000, 1000003, 10, 3412, (4095, 4096, 4097, 9000, 0, 1)),       # 1024
     (1000003, 2000003, 11, 4089, (4095, 4096, 4097, 9000, 0, 1)),      # 4096
