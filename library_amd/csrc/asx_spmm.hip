@@ -170,8 +170,8 @@ __global__ __launch_bounds__(kBlock) void k_spmm_splits(int32_t m, int32_t nnz, 
 
 // Boundaries seg and seg + 1 by the wave that owns the segment, for calls without a plan (a launch of k_spmm_splits
 // before it: 13.9 us against 10.0 with 85000 elements and 8 columns, 271 against 266 with 3.8 M and 100): four groups of 16
-// lanes search the points seg - 1 .. seg + 2 side by side, 16 probes at a time.  rest() runs behind the first probes' requests; where it
-// says that nothing is left to do, false comes back.
+// lanes search the points seg - 1 .. seg + 2 side by side, 16 probes at a time.  rest() runs once, behind the first probes' requests; where
+// it says that nothing is left to do, false comes back.
 template <typename F>
 __device__ __forceinline__ bool segment_ends(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nnz, int32_t items,
                                              int32_t nseg, int64_t seg, int32_t &x0, int32_t &y0, int32_t &x1, int32_t &y1,
@@ -195,6 +195,7 @@ __device__ __forceinline__ bool segment_ends(const int32_t *__restrict__ row_ptr
         lo = lo < hi ? at : lo;
         hi = to < hi ? to : hi;
     }
+    if (first && !rest()) return false;  // nothing to search
     int32_t x[4], y[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
