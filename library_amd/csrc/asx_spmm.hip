@@ -14,6 +14,7 @@
 //           separate pass and joins segments with atomicAdd).
 //   chunk : the same with a workgroup per (longer) segment, for narrow rows of B, and for wide ones of small or scattered matrices.
 #include <algorithm>
+#include <type_traits>
 
 #include "asx_internal.hpp"
 
@@ -172,6 +173,9 @@ __global__ __launch_bounds__(kBlock) void k_spmm_splits(int32_t m, int32_t nnz, 
 // before it: 13.9 us against 10.0 with 85000 elements and 8 columns, 271 against 266 with 3.8 M and 100): four groups of 16
 // lanes search the points seg - 1 .. seg + 2 side by side, 16 probes at a time.  rest() runs once, behind the first probes' requests; where
 // it says that nothing is left to do, false comes back.
+struct NothingAsked {
+    __device__ bool operator()() const { return true; }
+};
 template <typename F>
 __device__ __forceinline__ bool segment_ends(const int32_t *__restrict__ row_ptr, int32_t m, int32_t nnz, int32_t items,
                                              int32_t nseg, int64_t seg, int32_t &x0, int32_t &y0, int32_t &x1, int32_t &y1,
@@ -185,11 +189,16 @@ __device__ __forceinline__ bool segment_ends(const int32_t *__restrict__ row_ptr
     bool first = true;
     while (__ballot(lo < hi)) {  // uniform; a group that is done repeats its answer
         const int64_t step = (hi - lo + 15) / 16, p = lo + l * step;
-        const bool in = lo < hi && p < hi;
-        const int32_t end = row_ptr[in ? p + 1 : 0];
-        if (first && !rest()) return false;
-        first = false;
-        const bool before = in && (int64_t)end < d - p;  // the point lies behind p
+        bool before;  // the point lies behind p
+        if constexpr (std::is_same<F, NothingAsked>::value) {
+            before = lo < hi && p < hi && (int64_t)row_ptr[p + 1] < d - p;
+        } else {
+            const bool in = lo < hi && p < hi;
+            const int32_t end = row_ptr[in ? p + 1 : 0];
+            if (first && !rest()) return false;
+            first = false;
+            before = in && (int64_t)end < d - p;
+        }
         const int n = __popc((unsigned)(__ballot(before) >> (q * 16)) & 0xffffu);
         const int64_t at = lo + (n > 0 ? (n - 1) * step + 1 : 0), to = lo + n * step;
         lo = lo < hi ? at : lo;
@@ -282,15 +291,18 @@ __device__ __forceinline__ typename VecOf<T, VEC>::type spmm_staged(int32_t i0, 
 // bits from the same old values of C, in one wave).
 // Consecutive segments run on one XCD, whose L2 then fetches the rows of B that neighbouring rows
 // of A share once.
-// ask: where the sweep kernel has been launched ahead and answered that it takes the call, what is left are rows longer than it takes.
-template <typename T, int VEC, int LOGG, int SEG>
-__global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
-                                                       const int32_t *__restrict__ row_ptr,
-                                                       const int32_t *__restrict__ col, const T *__restrict__ val,
-                                                       const T *__restrict__ B, int64_t ldb, T beta,
-                                                       T *__restrict__ C, int64_t ldc,
-                                                       const int32_t *__restrict__ xs, const int32_t *__restrict__ ys,
-                                                       T *__restrict__ carry, int32_t *__restrict__ carry_row, SweepAsk ask)
+// ASK: the sweep kernel has been launched ahead; where it answered that it takes the call, what is left are rows longer than it takes.
+// That is a kernel of its own, and the usual one has no argument more: with one kernel for both, fp32 calls took 0.3 to 0.5 us
+// longer (5-point stencil of 22680 rows, 64 columns 8.1 us and 8.5, 160 columns 12.1 and 12.5), with an argument that nobody reads, and
+// so the grid's sizes on a third line of arguments, still 0.15.
+template <typename T, int VEC, int LOGG, int SEG, bool ASK>
+__device__ __forceinline__ void spmm_merge_segment(int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
+                                                   const int32_t *__restrict__ row_ptr,
+                                                   const int32_t *__restrict__ col, const T *__restrict__ val,
+                                                   const T *__restrict__ B, int64_t ldb, T beta,
+                                                   T *__restrict__ C, int64_t ldc,
+                                                   const int32_t *__restrict__ xs, const int32_t *__restrict__ ys,
+                                                   T *__restrict__ carry, int32_t *__restrict__ carry_row, const SweepAsk &ask)
 {
     typedef typename VecOf<T, VEC>::type V;
     constexpr int G = 1 << LOGG, NG = kWave / G;
@@ -307,15 +319,8 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     const int64_t seg = blk * (kBlock / kWave) + w;
     if (seg >= nseg) return;  // wave-uniform
     int32_t least = -1;  // only rows of more elements are left to do
-    const int32_t swept = ask.answer ? *ask.answer : 0;
-    const auto rest = [&]() {
-        if (!swept) return true;
-        bool any = false;
-        for (int i = lane * 8; i < ask.blocks; i += kWave * 8) any |= *(const uint64_t *)(ask.too_long + i) != 0;
-        if (__ballot(any) == 0) return false;
-        least = ask.longest;
-        return true;
-    };
+    int32_t swept = 0;
+    if constexpr (ASK) swept = *ask.answer;
     const int grp = lane >> LOGG, gl = lane & (G - 1);
     const int64_t t0 = (int64_t)blockIdx.y * ncols / gridDim.y, t1 = (int64_t)(blockIdx.y + 1) * ncols / gridDim.y;
     int64_t c = t0 + gl * VEC;
@@ -324,15 +329,23 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     const char *Bc = (const char *)(B + c);
     const uint64_t ldb_bytes = (uint64_t)ldb * sizeof(T);
     int32_t x0, y0, x1, y1;
-    if (xs) {  // uniform
+    if (xs)  // uniform
         x0 = xs[seg], y0 = ys[seg], x1 = xs[seg + 1], y1 = ys[seg + 1];
-        if (!rest()) {
+    if constexpr (ASK) {
+        const auto rest = [&]() {
+            if (!swept) return true;
+            bool any = false;
+            for (int i = lane * 8; i < ask.blocks; i += kWave * 8) any |= *(const uint64_t *)(ask.too_long + i) != 0;
+            if (__ballot(any) == 0) return false;
+            least = ask.longest;
+            return true;
+        };
+        if (xs ? !rest() : !segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1, rest)) {
             if (carry_row && lane == 0 && blockIdx.y == 0) carry_row[seg] = -1;
             return;
         }
-    } else if (!segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1, rest)) {
-        if (carry_row && lane == 0 && blockIdx.y == 0) carry_row[seg] = -1;
-        return;
+    } else if (!xs) {
+        segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1, NothingAsked{});
     }
     const int32_t nel = y1 - y0 < kElems ? y1 - y0 : kElems, nrow = x1 - x0 < kEnds ? x1 - x0 : kEnds;
     int32_t *s_col = s_col_all[w];
@@ -392,12 +405,12 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
     };
     const bool stores = active && grp == 0;
     // a row that is cut covers a segment, which holds `least` elements or more
-    const bool first_cut = least >= 0 && row_ptr[x0] != y0;
+    const bool first_cut = ASK && least >= 0 && row_ptr[x0] != y0;
     for (int32_t r0 = 0; r0 < nrow; r0 += NG) {
         const int32_t r = r0 + grp;
         const int32_t k = r < nrow ? s_end[r] : 0, e = r < nrow ? s_end[r + 1] : 0;
-        const bool wanted = r < nrow && (e - k > least || (first_cut && r == 0));
-        const bool dealt = !wanted || e - k <= kDealt;
+        const bool wanted = r < nrow && (!ASK || e - k > least || (first_cut && r == 0));
+        const bool dealt = (ASK && !wanted) || e - k <= kDealt;
         if (wanted && dealt) {
             V *out = (V *)(C + (int64_t)(x0 + r) * ldc + c);
             V c_old = T(0);
@@ -430,6 +443,32 @@ __global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, i
         if (stores) *(V *)(carry + seg * ncols + c) = acc;
     }
     if (carry_row && lane == 0 && blockIdx.y == 0) carry_row[seg] = has_tail ? x1 : -1;
+}
+
+template <typename T, int VEC, int LOGG, int SEG>
+__global__ __launch_bounds__(kBlock) void k_spmm_merge(int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
+                                                       const int32_t *__restrict__ row_ptr,
+                                                       const int32_t *__restrict__ col, const T *__restrict__ val,
+                                                       const T *__restrict__ B, int64_t ldb, T beta,
+                                                       T *__restrict__ C, int64_t ldc,
+                                                       const int32_t *__restrict__ xs, const int32_t *__restrict__ ys,
+                                                       T *__restrict__ carry, int32_t *__restrict__ carry_row)
+{
+    spmm_merge_segment<T, VEC, LOGG, SEG, false>(m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
+                                                 carry_row, SweepAsk{});
+}
+
+template <typename T, int VEC, int LOGG, int SEG>
+__global__ __launch_bounds__(kBlock) void k_spmm_merge_rest(int32_t m, int32_t nnz, int32_t items, int32_t nseg, int32_t ncols, T alpha,
+                                                            const int32_t *__restrict__ row_ptr,
+                                                            const int32_t *__restrict__ col, const T *__restrict__ val,
+                                                            const T *__restrict__ B, int64_t ldb, T beta,
+                                                            T *__restrict__ C, int64_t ldc,
+                                                            const int32_t *__restrict__ xs, const int32_t *__restrict__ ys,
+                                                            T *__restrict__ carry, int32_t *__restrict__ carry_row, SweepAsk ask)
+{
+    spmm_merge_segment<T, VEC, LOGG, SEG, true>(m, nnz, items, nseg, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry,
+                                                carry_row, ask);
 }
 
 // ===========================================================================================
@@ -492,7 +531,7 @@ __global__ __launch_bounds__(kChunkThreads, REACH == kRowsFar ? 4 : 6) void k_sp
         x0 = xs[seg], y0 = ys[seg], x1 = xs[seg + 1], y1 = ys[seg + 1];
     } else {
         if (w == 0) {
-            segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1, [] { return true; });
+            segment_ends(row_ptr, m, nnz, items, nseg, seg, x0, y0, x1, y1, NothingAsked{});
             if (lane == 0) s_cut[0] = x0, s_cut[1] = y0, s_cut[2] = x1, s_cut[3] = y1;
         }
         __syncthreads();
@@ -676,8 +715,14 @@ static void launch_merge_width(const SpmmTiling &tiling, int32_t m, int32_t nnz,
     const dim3 grid((unsigned)(ceil_div64(ceil_div64(nseg, kBlock / kWave), kXcds) * kXcds), (unsigned)tiling.tiles);
 #define ASX_WIDTH(LOGG)                                                                                              \
     if (tiling.log_lanes <= LOGG) {                                                                                      \
+        if constexpr (VEC == 16 / sizeof(T) && LOGG >= 3) /* the sweep's calls: rows of B of more than 64 bytes */       \
+            if (ask.answer) {                                                                                            \
+                hipLaunchKernelGGL((k_spmm_merge_rest<T, VEC, LOGG, SEG>), grid, dim3(kBlock), 0, s, m, nnz, items, nseg, ncols, alpha,  \
+                                   row_ptr, col, val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, ask);          \
+                return;                                                                                                  \
+            }                                                                                                            \
         hipLaunchKernelGGL((k_spmm_merge<T, VEC, LOGG, SEG>), grid, dim3(kBlock), 0, s, m, nnz, items, nseg, ncols, alpha, row_ptr, col, \
-                           val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row, ask);                                \
+                           val, B, ldb, beta, C, ldc, xs, ys, carry, carry_row);                                     \
         return;                                                                                                      \
     }
     ASX_WIDTH(0)

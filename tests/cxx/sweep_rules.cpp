@@ -58,6 +58,7 @@ int main()
             ++asked;
             REQUIRE(longest <= items && spmm_segments(m, nnz, items) >= 2);  // whole rows only, and splits to look for
             REQUIRE(spmm_sweep_ask_blocks(chains) <= kSweepAskBlocks);
+            REQUIRE(t.log_lanes >= 3 && t.vec == (int)(16 / sv));  // the merge kernel has a variant that looks at the answer
         }
     }
     std::printf("taken %ld, several sums %ld, asked %ld\n", taken, several, asked);
