@@ -219,7 +219,7 @@ int asx_spmv_plan_create(asx_plan **plan, int alg, int value_type, int32_t m, in
                          const int32_t *d_row_ptr, const int32_t *d_col, const void *d_val, void *stream);
 /* Brings a plan that holds a copy of A's values (ASX_SPMV_SLICED, ASX_SPMV_WINDOW, ASX_SPMM_BLOCKED) up to date
  * with d_val (same sparsity pattern as when the plan was built); asynchronous on `stream`; one
- * pass over the values (sliced: 156 us for 34 M fp64 values, 38 us for 16.8 M fp32 ones).  For
+ * pass over the values (sliced: 150 us for 34 M fp64 values, 38 us for 16.8 M fp32 ones).  For
  * the other kernels, which read the caller's values in every call, it does nothing.
  * asx_plan_holds_values tells the two kinds apart.  No counterpart in the reference. */
 int asx_plan_update_values(asx_plan *plan, const void *d_val, void *stream);
@@ -370,7 +370,10 @@ size_t asx_spmv_noalloc_max_workspace(void);
  *        spapi.h:1272-1306)
  * ---------------------------------------------------------------------------------- */
 int asx_spmm_resolve_alg(int alg, int32_t m, int32_t nnz, int32_t ncols);
-/* alphasparseSpMM_bufferSize, hip/kernel/level3/alphasparse_spmm.hip:699-850. */
+/* alphasparseSpMM_bufferSize, hip/kernel/level3/alphasparse_spmm.hip:699-850.
+ * A large ASX_SPMM_DEFAULT call without a plan, or with a plan that was made without A's columns, keeps the device's
+ * answer about them in the last bytes: with a buffer that lacks these (an older size) it runs the merge
+ * kernel whatever the columns are, and rows of more than 32 stored elements may be rounded otherwise. */
 size_t asx_spmm_workspace_bytes(int alg, int value_type, int32_t m, int32_t nnz, int32_t ncols);
 
 int asx_spmm_csr_f32(const asx_plan *plan, int alg, int32_t m, int32_t k, int32_t nnz, int32_t ncols,

@@ -511,10 +511,10 @@ inline bool spmm_everywhere(double spread, double span, double falls, double mea
 //   Windows: the more, the less of B a window needs (a wave ahead or behind does less harm), but every window costs its
 //   instructions whether rows have an element in it or not: 1.24 MB(B)^0.35 mean^-0.3 windows an element of a mean row, between 1
 //   and 2.5, fitted to 110 uniform matrices (both types, rows of B of 72 to 2000 bytes, 4 to 64 per row, B of 14 to 317 MB)
-//   timed with 1 to 6: 0.5 % behind the best of these on average; a tenth less where a group has 16 lanes or more, which inputs that
+//   timed with 1 to 6, all with one sum a row: 0.5 % behind the best of these on average; then a tenth less where a group has 16 lanes or more, which inputs that
 //   are not in the Infinity Cache want (74 such matrices, three sets of inputs in turn: 0.986 of the time with the tenth; 100
 //   columns fp32, 150001 rows of 25 150 us and 141).
-//   On those 110 it takes 0.78 of the row-ordered kernels' time on average (100 columns fp32, 160000 rows of 25 270 us against
+//   On those 110 it took 0.78 of the row-ordered kernels' time on average (100 columns fp32, 160000 rows of 25 270 us against
 //   130; 96, 94796 of 49 316 and 136; 64, 573065 of 9 204 and 191; 22, 1 M of 4 138 and 133).  Not taken: a B that the L2s keep
 //   between them (9 MB, 14 where rows of A are short) - where rows of B start on lines the row-ordered kernels work through it
 //   in tiles of one line, which they can keep up to 40000 rows or 20 MB (192 columns fp32, 27903 rows of 8 22.6 us there, 23.4 here;
@@ -581,10 +581,11 @@ inline SpmmSweep spmm_sweep(int32_t m, int32_t n, int32_t nnz, int64_t ncols, si
 }
 // Calls whose columns nobody has looked at: whether asking pays (slots 0: not).  Where the answer is no, the launch is spent: 4.6 us with
 // one round of workgroups (100 columns fp32, 160001 power-law rows of 20: 264 us before), 5.8 with two, 8 with three (250 columns, 100003 rows
-// of 36 within 3000 of the diagonal: 274 us before).  So it is for calls
-// whose rows of B, each fetched by itself, take 240 us and more, for two rounds at most (three where a row is several sums), and
-// where an XCD's waves meet a row of B often (100 columns fp32, 150001 uniform rows of 25, 1.6: 257 us without, 157 with). Rows of B that start on lines, which the merge kernel
-// takes a line or two at a time, gain less (256 columns fp32, 60001 uniform rows of 30, 173 us without and 157 with; 128 fp64, 20 per row
+// of 36 within 3000 of the diagonal: 274 us before).  So it is for calls whose rows of B, each fetched by itself, take 240 us and more,
+// for two rounds at most (three where a row is several sums), and where an XCD's waves meet a row of B often: 100 columns fp32, 150001
+// uniform rows of 25, 3.1 times, 257 us without and 150 with; 250 columns, 80000 rows of 25 and 400000 columns of A, 0.62 times, 359 and 278
+// - below 0.6 a yes still gains (500000, 0.5 times, 359 and 289), but less, for the same price of a no.  Rows of B that start on lines,
+// which the merge kernel takes a line or two at a time, gain less (256 columns fp32, 60001 uniform rows of 30, 173 us without and 157 with; 128 fp64, 20 per row
 // within 3000 of the diagonal 165 and 171): from twice as many lines on.  Rows that the merge kernel cuts have to be longer than
 // the sweep takes: it looks at whole rows only.
 constexpr double kSweepAskLines = 240e-6 * 58e9, kSweepAskShared = 0.6;

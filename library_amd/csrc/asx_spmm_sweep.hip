@@ -7,13 +7,13 @@
 // elements of all rows.  Nothing orders the waves but that they do the same work a window; those ahead wait for memory, those
 // behind find their rows of B in the L2.
 //
-// Calls whose columns nobody has looked at ask the device (sweep_asks): the first wave of every workgroup looks at 64 rows spread over
+// Calls whose columns nobody has looked at ask the device (sweep_suits): the first wave of every workgroup looks at 64 rows spread over
 // A, all workgroups come to the same answer, and where it is no they end; the merge kernel, launched behind them, finds the
 // answer in the call's workspace and does what is left: everything, or the rows that are too long to be walked by one lane group.
 //
-// Uniform columns, 25 per row, 100 columns fp32 of 150001 rows: 258 us with the merge kernel, 15.4 M lines past the L2s; 124 here where B is in
-// the Infinity Cache, 141 where inputs change from call to call.  49 per row, 96 columns of 94796 rows 316 and 136; 24 per row, 103
-// columns fp64 of 97486 337 and 215 (in the cache).
+// Uniform columns, 25 per row, 100 columns fp32 of 150001 rows: 255 us with the merge kernel, 14.7 M lines past the L2s, 4.8 M here; 124 us here
+// where B is in the Infinity Cache, 141 where inputs change from call to call.  49 per row, 96 columns of 94796 rows 316 and 136, 100
+// columns, where such rows are two sums, 289 and 158; 24 per row, 103 columns fp64 of 97486 337 and 215 (in the cache).
 #include "asx_internal.hpp"
 
 namespace asx {
