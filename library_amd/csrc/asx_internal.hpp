@@ -230,8 +230,7 @@ struct SpmmSweep {
     uint32_t width;  // columns a window
     int log_lanes;   // of a group
     int64_t tiles;   // of columns of B
-    int32_t chains;  // sums of stretches that a row of more than `dealt` elements is made of: 1, 2 or 4
-    int32_t dealt;
+    int32_t chains;  // sums of stretches that a row of more than 32 elements is made of: 1, 2 or 4
 };
 template <typename T>
 int launch_spmm_sweep(const SpmmSweep &sw, const SweepAsk *ask, int32_t m, int32_t n, int32_t nnz, int32_t ncols, T alpha,
@@ -548,7 +547,6 @@ inline SpmmSweep spmm_sweep_shape(int32_t m, int32_t nnz, int64_t ncols, size_t 
     rows = ceil_div64(m, round * ceil_div64(m, round * rows));
     sw.rows = (int32_t)rows;
     sw.chains = chains;
-    sw.dealt = chains == 1 ? 0x7fffffff : spmm_dealt(chains);
     const int64_t slots = rows * chains;
     sw.slots = slots <= 4 ? 4 : slots <= 8 ? 8 : slots <= 12 ? 12 : slots <= 16 ? 16 : 20;
     sw.cap = std::min(cap, ((int32_t)(1.1 * mean * (double)(rows * t.groups)) + 2) & ~1);

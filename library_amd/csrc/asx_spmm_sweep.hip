@@ -104,19 +104,22 @@ constexpr int sweep_batch(int slots) { return slots == 20 ? 5 : slots == 12 ? 6 
 // and a load 16 cycles of a compute unit's L1 where all lanes take part, none where none does - slots without an element are
 // masked out, not sent past a buffer's end (119 us against 157 for the first example above) -; and lines past the L2s for what
 // waves are apart.  Batches of G slots, all loads of a batch ahead of its sums.
-// Rows of more than `dealt` elements are `chains` sums of a stretch each, S / chains slots apart, so that most steps have nothing to do for
-// the batches of one stretch or the other.
+// LONG: rows of more than 32 elements are two or four sums of a stretch each (rows >> 8 says how many), S / 2 or S / 4 slots apart, so that
+// most steps have nothing to do for the batches of one stretch or the other.  A variant of its own: the usual one's registers are
+// given out otherwise as soon as it knows of stretches (260 columns fp32, 100001 rows of 10 180 -> 213 us).
 //
 // ASK: the call does not know its columns (above).  Rows longer than ask.longest are left to the merge kernel.
-template <typename T, int LOGL, int S, bool ASK>
+template <typename T, int LOGL, int S, bool ASK, bool LONG>
 __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
-    SweepAsk ask, int32_t m, int32_t nnz, int32_t rows, int32_t chains, int32_t dealt, int32_t cap, uint32_t width, uint32_t last, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
+    SweepAsk ask, int32_t m, int32_t nnz, int32_t rows, int32_t cap, uint32_t width, uint32_t last, int32_t ncols, T alpha, const int32_t *__restrict__ row_ptr,
     const int32_t *__restrict__ col, const T *__restrict__ val, const T *__restrict__ B, int64_t ldb, T beta, T *__restrict__ C, int64_t ldc)
 {
     typedef typename Vec16<T>::type V;
     constexpr int VEC = Vec16<T>::N, L = 1 << LOGL, NG = kWave / L, G = sweep_batch(S);
     static_assert(S <= L && S % G == 0, "a lane knows where one row of its group is");
     extern __shared__ __align__(16) char s_all[];
+    const int32_t chains = LONG ? rows >> 8 : 1;
+    if (LONG) rows &= 255;
     const int lane = threadIdx.x & (kWave - 1);
     const int w = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave);
     const uint32_t per_xcd = gridDim.x / kXcds;
@@ -135,8 +138,10 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
     const uint32_t pitch = (uint32_t)((uint64_t)ldb * sizeof(T));
 
     // the lane's row, or its part of one: element s up to e
-    const int32_t apart = chains == 1 ? S : chains == 2 ? S / 2 : S / 4, part = (gl >= apart) + (gl >= 2 * apart) + (gl >= 3 * apart), mine = grp * rows + gl - part * apart;
-    bool has_row = part < chains && gl - part * apart < rows && mine < nrow;
+    const int32_t apart = chains == 2 ? S / 2 : S / 4, part = LONG ? (gl >= apart) + (gl >= 2 * apart) + (gl >= 3 * apart) : 0;
+    const int32_t mine = grp * rows + gl - (LONG ? part * apart : 0);
+    bool has_row = (LONG ? gl - part * apart : gl) < rows && mine < nrow;
+    if (LONG) has_row = has_row && part < chains;
     int32_t s = has_row ? row_ptr[x0 + mine] : 0, e = has_row ? row_ptr[x0 + mine + 1] : 0;
     if constexpr (ASK) {
         __shared__ int s_yes, s_long[kBlock / kWave];
@@ -157,13 +162,15 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
         if (!s_yes || x0 >= m) return;
         if (too_long) has_row = false, s = e = 0;
     }
-    const uint64_t kept = __ballot(has_row && part == 0);
-    if (e - s > dealt) {  // of more than one sum: a stretch each
-        const int32_t share = (e - s + chains - 1) / chains;
-        s = s + part * share < e ? s + part * share : e;
-        e = s + share < e ? s + share : e;
-    } else if (part > 0) {
-        s = e;
+    const uint64_t kept = __ballot(LONG ? has_row && part == 0 : has_row);
+    if constexpr (LONG) {
+        if (e - s > spmm_dealt(4)) {  // several sums, of a stretch each
+            const int32_t share = (e - s + chains - 1) / chains;
+            s = s + part * share < e ? s + part * share : e;
+            e = s + share < e ? s + share : e;
+        } else if (part > 0) {
+            s = e;
+        }
     }
     const int32_t begin = __builtin_amdgcn_readfirstlane(row_ptr[x0]), end = __builtin_amdgcn_readfirstlane(row_ptr[x0 + nrow]);
 
@@ -248,10 +255,10 @@ __global__ __launch_bounds__(kBlock, 4) void k_spmm_sweep(
             }
         }
     }
-    if (chains > 1)
+    if constexpr (LONG) {
         static_for<0, S / 2>([&](auto j_) { acc[decltype(j_)::value] += acc[decltype(j_)::value + S / 2]; });
-    if (chains > 2)
-        static_for<0, S / 4>([&](auto j_) { acc[decltype(j_)::value] += acc[decltype(j_)::value + S / 4]; });
+        if (chains > 2) static_for<0, S / 4>([&](auto j_) { acc[decltype(j_)::value] += acc[decltype(j_)::value + S / 4]; });
+    }
     static_for<0, S / G>([&](auto g_) {
         constexpr int j0 = decltype(g_)::value * G;
         V c_old[G];
@@ -279,7 +286,13 @@ static int launch_sweep(const SpmmSweep &sw, const SweepAsk &ask, int32_t m, int
     const uint32_t last = (uint32_t)n > sw.width ? (uint32_t)n - sw.width : 0;
 #define ASX_SWEEP(LOGL, S)                                                                                                              \
     if (sw.log_lanes == LOGL && sw.slots == S) {                                                                                        \
-        hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S, ASK>), grid, dim3(kBlock), lds, s, ask, m, nnz, sw.rows, sw.chains, sw.dealt, cap, sw.width, last,      \
+        if constexpr (LOGL >= 4)                                                                                                        \
+            if (sw.chains > 1) {                                                                                                        \
+                hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S, ASK, true>), grid, dim3(kBlock), lds, s, ask, m, nnz, sw.rows | sw.chains << 8, cap, \
+                                   sw.width, last, ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc);                              \
+                return check_launch();                                                                                                  \
+            }                                                                                                                           \
+        hipLaunchKernelGGL((k_spmm_sweep<T, LOGL, S, ASK, false>), grid, dim3(kBlock), lds, s, ask, m, nnz, sw.rows, cap, sw.width, last,      \
                            ncols, alpha, row_ptr, col, val, B, ldb, beta, C, ldc);                                                      \
         return check_launch();                                                                                                          \
     }

@@ -46,7 +46,7 @@ int main()
             several += chains > 1;
             const int groups = kWave >> sw.log_lanes;
             REQUIRE(chains >= 1 && launched(sw) && sw.slots <= 1 << sw.log_lanes && sw.rows >= 1 && sw.rows * chains <= sw.slots && sw.slots % chains == 0);
-            REQUIRE(chains == 1 || sw.dealt == spmm_dealt(chains));
+            REQUIRE(sw.chains == chains && (chains == 1 || (spmm_dealt(chains) == spmm_dealt(4) && sw.log_lanes >= 4)) && sw.rows < 256);
             REQUIRE(sw.cap >= 2 && sw.cap % 2 == 0 && sw.cap <= spmm_sweep_cap(sv));
             REQUIRE(4 * (std::min(sw.cap, spmm_sweep_cap(sv) - 2) * (sv + 4) * (kBlock / kWave) + 32) <= 160 * 1024);
             REQUIRE(sw.tiles >= 1 && sw.tiles <= 65535 && ncols / sw.tiles >= (int64_t)(16 / sv));
